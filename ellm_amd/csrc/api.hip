@@ -266,9 +266,21 @@ static int attn_create(const ellm_attn_desc* d, const ellm_kv_seq_table* table, 
   h->part_rows = ellm::prefill_workspace_rows((uint32_t)d->max_position_interval, (uint32_t)d->batch_size,
                                               (uint32_t)d->attention_head_num, (uint32_t)n_cu);
   h->general = ellm::attn_is_general(*d);
-  if (h->general) {   // the kernel for other head sizes and binary32 keeps nothing between workgroups
-    h->ws = ellm::DecodeWorkspace{0, 0, 0};
-    h->part_rows = 0;
+  if (h->general) {   // other head sizes and binary32: one table of partial rows for both kinds of call
+    const ellm::GeneralWorkspace w = ellm::general_workspace(
+        (uint32_t)d->max_position_interval, (uint32_t)d->batch_size, (uint32_t)d->attention_head_num,
+        (uint32_t)d->kv_head_num, (uint32_t)d->head_size, (uint32_t)n_cu);
+    h->ws = ellm::DecodeWorkspace{0, 0, w.counters};
+    h->part_rows = w.rows;
+    hipError_t e = hipMalloc((void**)&h->part_o, w.rows * w.pitch * sizeof(float));
+    if (e == hipSuccess) e = hipMalloc((void**)&h->part_ml, w.rows * 2 * sizeof(float));
+    if (e == hipSuccess) e = hipMalloc((void**)&h->counters, w.counters * sizeof(uint32_t));
+    if (e == hipSuccess) e = hipMemset(h->counters, 0, w.counters * sizeof(uint32_t));
+    if (e != hipSuccess) {
+      (void)free_workspace(h);
+      delete h;
+      return fail_hip(e, "hipMalloc(workspace)");
+    }
     *out_handle = h;
     return ELLM_OK;
   }
@@ -303,7 +315,6 @@ int ellm_attn_create_ragged(const ellm_attn_desc* d, const ellm_kv_seq_table* ta
 int ellm_attn_reset(ellm_attn* h, void* stream) {
   if (!h) return fail(ELLM_ERR_INVALID_ARGUMENT, "null handle");
   if (int st = ellm::check_current_device(h->device)) return st;
-  if (h->general) return ELLM_OK;   // no counters
   const hipError_t e = ellm::launch_fill_u32(h->counters, h->ws.counters, 0u, (hipStream_t)stream);
   if (e != hipSuccess) return fail_hip(e, "counter reset launch");
   return ELLM_OK;

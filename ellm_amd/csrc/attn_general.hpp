@@ -1,0 +1,290 @@
+// Shared parts of the attention kernels for shapes other than 128-wide 16-bit heads: any head
+// size up to 256 and binary32 storage (attn_general.hip: dispatch and merge;
+// attn_general_chunk.hip: many query rows per K/V plane; attn_general_step.hip: few).
+#pragma once
+
+#include <type_traits>
+
+#include "common.hpp"
+#include "kernels.hpp"
+
+namespace ellm {
+namespace gen {
+
+constexpr int kMaxHead = 256;
+constexpr uint32_t kGeneralTileRows = 128;   // query rows of a workgroup of the chunk kernel
+constexpr uint32_t kGeneralStepRows = 16;    // and of the step kernel
+
+struct F32 {};   // binary32 storage
+
+// What a storage type is to the kernels: its element, how many make a 16-byte piece, and the
+// exponent shift the soft-max weights carry on their way through the second product (binary16
+// weights keep 2^-24 at the small end: moved up, weights down to 2^-31 of the largest count).
+template <typename S>
+struct Store;
+template <>
+struct Store<F16> {
+  typedef uint16_t E;
+  static constexpr int kPiece = 8;
+  static constexpr float kShift = 7.0f;
+  static constexpr uint32_t kExpMask = 0x7c007c00u;
+};
+template <>
+struct Store<BF16> {
+  typedef uint16_t E;
+  static constexpr int kPiece = 8;
+  static constexpr float kShift = 0.0f;
+  static constexpr uint32_t kExpMask = 0x7f807f80u;
+};
+template <>
+struct Store<F32> {
+  typedef float E;
+  static constexpr int kPiece = 4;
+  static constexpr float kShift = 0.0f;
+  static constexpr uint32_t kExpMask = 0x7f800000u;
+};
+
+template <typename S>
+__device__ __forceinline__ float load_elem(const typename Store<S>::E* p) {
+  if constexpr (std::is_same<S, F32>::value) return *p;
+  else return Mfma<S>::to_float(*p);
+}
+template <typename S>
+__device__ __forceinline__ void store_elem(typename Store<S>::E* p, float v) {
+  if constexpr (std::is_same<S, F32>::value) *p = v;
+  else *p = (uint16_t)(Mfma<S>::pack2(v, 0.0f) & 0xffffu);
+}
+
+struct GeneralArgs {
+  const void* q;
+  const void* k;
+  const void* v;
+  void* out;
+  float* lse;
+  const uint32_t* positions;     // single-token calls only
+  const size_t* seq_offsets;
+  const uint32_t* seq_caps;
+  size_t kv_stride_seq, kv_stride_head, kv_stride_pos;
+  uint32_t batch_pitch, n_q_heads, n_kv_heads, group, head_size;
+  uint32_t position_index;       // first query's position, or the bound of the per-sequence positions
+  uint32_t interval;
+  uint32_t rows;                 // query rows of a plane: interval x group; row r = token r / group, head r % group
+  uint32_t negate_q;             // scale < 0: the sign is folded into the query rows so that c > 0
+  float c;                       // |scale| x log2(e), > 0
+  // Key range split over workgroups: n_split pieces of split_len keys.  Partial row of plane row
+  // r and split s: (plane x rows + r) x n_split + s of part_o [..][pitch] (weighted sums) and
+  // part_ml [..][2] (reference exponent in log2 units, denominator).
+  uint32_t n_split, split_len;
+  uint32_t row_tiles;            // workgroups along the rows of a plane
+  float* part_o;
+  float* part_ml;
+  uint32_t* counters;            // arrivals per (plane, row tile); zero between launches
+};
+
+// Position of a plane's query row; for calls with per-sequence positions and capacities too.
+__device__ __forceinline__ uint32_t start_position(const GeneralArgs& p, uint32_t seq) {
+  uint32_t pos = p.position_index;
+  if (p.positions) pos = min(p.positions[seq], p.position_index);
+  if (p.seq_caps) pos = min(pos, p.seq_caps[seq] - 1);   // (shared ranges fit every sequence: checked on the host)
+  return pos;
+}
+
+// Element offset of query row r of a plane in q / out (x head_size) and in lse.
+__device__ __forceinline__ size_t query_row(const GeneralArgs& p, uint32_t seq, uint32_t kvh, uint32_t r) {
+  return ((size_t)(r / p.group) * p.batch_pitch + seq) * p.n_q_heads + kvh * p.group + r % p.group;
+}
+
+__device__ __forceinline__ uint64_t scalar64(uint64_t v) {  // tells the compiler that v is wave-uniform
+  const uint32_t lo = (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)v);
+  const uint32_t hi = (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)(v >> 32));
+  return ((uint64_t)hi << 32) | (uint64_t)lo;
+}
+
+// ---- pieces of K / V rows ------------------------------------------------------------------
+// VEC: rows start on 16-byte boundaries and hold whole 16-byte pieces.  The pieces of a chunk of
+// keys are fetched with buffer loads whose descriptor ends at the last key that counts, so later
+// rows read as zeros; a piece past the head's end is given an offset no descriptor covers.
+// Otherwise a piece is gathered element by element under the same two bounds.
+constexpr uint32_t kNowhere = 0xf0000000u;
+constexpr uint64_t kMaxRecords = 0x80000000u;   // 64 rows of at most 2^25 bytes
+
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t chunk_rsrc(uint64_t plane, uint64_t off, uint64_t valid) {
+  const uint64_t left = valid > off ? valid - off : 0;
+  const uint32_t capped = (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)(left > kMaxRecords ? kMaxRecords : left));
+  return __builtin_amdgcn_make_buffer_rsrc((void*)(plane + off), 0, capped, 0x00020000);
+}
+
+template <typename S>
+__device__ __forceinline__ u32x4 gather_piece(const typename Store<S>::E* plane, size_t stride_pos, uint32_t key,
+                                              uint32_t end, uint32_t e0, uint32_t head_size) {
+  u32x4 w = {0, 0, 0, 0};
+  if (key < end) {
+    const typename Store<S>::E* row = plane + (size_t)key * stride_pos;
+#pragma unroll
+    for (int e = 0; e < Store<S>::kPiece; ++e)
+      if (e0 + e < head_size) {
+        if constexpr (std::is_same<S, F32>::value) w[e] = __builtin_bit_cast(uint32_t, row[e0 + e]);
+        else w[e >> 1] |= (uint32_t)row[e0 + e] << (16 * (e & 1));
+      }
+  }
+  return w;
+}
+
+// Query row piece: elements e0 .. of the row, zeros past the head's end, sign folded in.
+template <typename S, bool VEC>
+__device__ __forceinline__ u32x4 query_piece(const GeneralArgs& p, const typename Store<S>::E* row, uint32_t e0) {
+  u32x4 w = {0, 0, 0, 0};
+  if constexpr (VEC) {
+    if (e0 < p.head_size) w = load16(row + e0);
+  } else {
+    w = gather_piece<S>(row, 0, 0, 1, e0, p.head_size);
+  }
+  if (p.negate_q) w ^= std::is_same<S, F32>::value ? 0x80000000u : 0x80008000u;
+  return w;
+}
+
+// Whether a piece holds an element with all exponent bits set (infinity or NaN).
+template <typename S>
+__device__ __forceinline__ bool piece_not_finite(u32x4 w) {
+  constexpr uint32_t m = Store<S>::kExpMask;
+  bool bad = false;
+#pragma unroll
+  for (int e = 0; e < 4; ++e) {
+    const uint32_t x = w[e] & m;
+    if constexpr (std::is_same<S, F32>::value) bad |= x == m;
+    else bad |= (x & 0xffffu) == (m & 0xffffu) || (x >> 16) == (m >> 16);
+  }
+  return bad;
+}
+
+// Agent-scope accesses for partial rows that another workgroup of the same launch folds.
+__device__ __forceinline__ void store_agent(float* p, float v) {
+  __hip_atomic_store((uint32_t*)p, __builtin_bit_cast(uint32_t, v), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
+__device__ __forceinline__ float wave_sum(float v) {
+#pragma unroll
+  for (int m = 32; m >= 1; m >>= 1) v += __shfl_xor(v, m);
+  return v;
+}
+
+// One query row over keys [k0, end), by one wave and without matrix instructions, result into the
+// output or the partial row.  The matrix kernels multiply every value row of a chunk
+// by every query row, masked pairs with a weight of zero, and 0 x infinity is not 0; a query row
+// must not see what the value rows of later positions hold, so a workgroup that meets a value
+// that is not finite beyond its first row's position takes its rows through here instead.
+template <typename S>
+__device__ __forceinline__ void plain_row(const GeneralArgs& p, const typename Store<S>::E* kp,
+                                                     const typename Store<S>::E* vp, size_t row, size_t prow,
+                                                     uint32_t k0, uint32_t end, uint32_t pitch, bool partial) {
+  typedef typename Store<S>::E E;
+  constexpr int kPerLane = kMaxHead / kWave;
+  const int lane = threadIdx.x & 63;
+  const E* q = (const E*)p.q + row * p.head_size;
+  float qv[kPerLane], o[kPerLane];
+#pragma unroll
+  for (int i = 0; i < kPerLane; ++i) {
+    const uint32_t d = lane + 64 * i;
+    qv[i] = d < p.head_size ? (p.negate_q ? -load_elem<S>(q + d) : load_elem<S>(q + d)) : 0.0f;
+    o[i] = 0.0f;
+  }
+  float m = -INFINITY, l = 0.0f;
+  for (uint32_t j = k0; j < end; ++j) {
+    float part = 0.0f, vv[kPerLane];
+#pragma unroll
+    for (int i = 0; i < kPerLane; ++i) {
+      const uint32_t d = lane + 64 * i;
+      const size_t at = (size_t)j * p.kv_stride_pos + d;
+      part = d < p.head_size ? __builtin_fmaf(qv[i], load_elem<S>(kp + at), part) : part;
+      vv[i] = d < p.head_size ? load_elem<S>(vp + at) : 0.0f;
+    }
+    const float s = wave_sum(part) * p.c;
+    const float m_new = fmaxf(m, s);
+    const float alpha = fast_exp2(m - m_new), w = fast_exp2(s - m_new);
+    l = l * alpha + w;
+#pragma unroll
+    for (int i = 0; i < kPerLane; ++i) o[i] = __builtin_fmaf(w, vv[i], o[i] * alpha);
+    m = m_new;
+  }
+  if (partial) {
+#pragma unroll
+    for (int i = 0; i < kPerLane; ++i)
+      if (lane + 64 * i < (int)pitch) store_agent(p.part_o + prow * pitch + lane + 64 * i, o[i]);
+    if (lane == 0) {
+      store_agent(p.part_ml + 2 * prow, m);
+      store_agent(p.part_ml + 2 * prow + 1, l);
+    }
+  } else {
+    E* out = (E*)p.out + row * p.head_size;
+    const float inv = 1.0f / l;
+#pragma unroll
+    for (int i = 0; i < kPerLane; ++i)
+      if (lane + 64u * i < p.head_size) store_elem<S>(out + lane + 64 * i, o[i] * inv);
+    if (p.lse && lane == 0) p.lse[row] = (m + fast_log2(l)) * kLn2;
+  }
+}
+
+// Four consecutive elements d .. d + 3 of an output row.
+template <typename S, bool VEC>
+__device__ __forceinline__ void store_out4(const GeneralArgs& p, size_t row, uint32_t d, f32x4 v) {
+  typedef typename Store<S>::E E;
+  E* out = (E*)p.out + row * p.head_size + d;
+  if constexpr (VEC) {
+    if (d >= p.head_size) return;
+    if constexpr (std::is_same<S, F32>::value) *(f32x4*)out = v;
+    else *(u32x2*)out = u32x2{Mfma<S>::pack2(v[0], v[1]), Mfma<S>::pack2(v[2], v[3])};
+  } else {
+#pragma unroll
+    for (int e = 0; e < 4; ++e)
+      if (d + e < p.head_size) store_elem<S>(out + e, v[e]);
+  }
+}
+
+// Weights of two keys as operands of the second product.  A 16-bit value keeps 11 (binary16) or 8
+// (bfloat16) significant bits; the weight goes in as two of them, the rounded value and what the
+// rounding left, so that the product carries the weight to 2^-17 or better and the output is
+// rounded once, at the end.
+template <typename S>
+__device__ __forceinline__ void split_pair(float p0, float p1, uint32_t& hi, uint32_t& lo) {
+  hi = Mfma<S>::pack2(p0, p1);
+  lo = Mfma<S>::pack2(p0 - Mfma<S>::to_float((uint16_t)(hi & 0xffffu)), p1 - Mfma<S>::to_float((uint16_t)(hi >> 16)));
+}
+
+// Launchers of the two kernels (grid and workspace fields of the arguments set); nb = blocks of
+// 32 elements of the padded head, vec as above.
+hipError_t launch_general_chunk(const GeneralArgs& p, int dtype, int nb, bool vec, uint32_t planes, hipStream_t stream);
+hipError_t launch_general_step(const GeneralArgs& p, int dtype, int nb, bool vec, uint32_t planes, hipStream_t stream);
+
+// Blocks of 32 elements the kernels pad a head to: 1, 2, 3, 4, 6 or 8 (2, 4 or 8 for rows that are
+// not made of whole aligned 16-byte pieces).
+inline int head_blocks(uint32_t head_size, bool vec) {
+  const int n = (int)((head_size + 31) / 32);
+  if (!vec) return n <= 2 ? 2 : n <= 4 ? 4 : 8;
+  return n <= 4 ? n : n <= 6 ? 6 : 8;
+}
+
+// f(std::integral_constant<int, blocks>, std::bool_constant<vec>) for a value of head_blocks().
+template <typename F>
+inline hipError_t with_head_blocks(int nb, bool vec, F f) {
+  using std::integral_constant;
+  if (vec) {
+    switch (nb) {
+      case 1: return f(integral_constant<int, 1>{}, std::true_type{});
+      case 2: return f(integral_constant<int, 2>{}, std::true_type{});
+      case 3: return f(integral_constant<int, 3>{}, std::true_type{});
+      case 4: return f(integral_constant<int, 4>{}, std::true_type{});
+      case 6: return f(integral_constant<int, 6>{}, std::true_type{});
+      case 8: return f(integral_constant<int, 8>{}, std::true_type{});
+    }
+  } else {
+    switch (nb) {
+      case 2: return f(integral_constant<int, 2>{}, std::false_type{});
+      case 4: return f(integral_constant<int, 4>{}, std::false_type{});
+      case 8: return f(integral_constant<int, 8>{}, std::false_type{});
+    }
+  }
+  return hipErrorInvalidValue;
+}
+
+}  // namespace gen
+}  // namespace ellm

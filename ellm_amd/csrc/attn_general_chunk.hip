@@ -1,0 +1,330 @@
+// Chunks of tokens (or any call with more than 32 query rows per K/V plane) for head sizes other
+// than 128 and for binary32 storage: the formulation of prefill.hip (S^T = K.Q^T, O^T += V^T.P^T, a
+// lane owns one query row, online soft-max in binary32) on 32x32 matrix tiles, templated over the
+// storage type and the padded head size.
+//
+// Four waves of 32 rows share every key step of 32 or 64 keys through LDS (double-buffered, one
+// barrier a step, the next step's rows in registers meanwhile); rows are the (token, head) pairs of a
+// GQA group in order, so a group's heads share the K/V rows whatever the group size.  What bounds it:
+// 16-bit, the vector instructions of the soft-max (twelve a pair of scores, two of them quarter-rate
+// exponentials) beside 6 x 32 matrix cycles per 16 keys and 32 elements; binary32, the matrix pipe
+// (256 flops a cycle and unit).  Two or three workgroups a unit overlap the one with the other.
+// Measured: 2048 tokens, 32 query / 8 key-value heads of 64, bfloat16: 46.5 us (370 TFLOP/s), where one
+// workgroup per query row without matrix instructions took 4360 us; 1019 tokens, 32 / 4 heads of 256,
+// binary16: 80 us (was 2103); 433 tokens x 2 on 369, 32 / 32 heads of 128, binary32: 124 us (was 1127).
+#include "attn_general.hpp"
+
+namespace ellm {
+namespace gen {
+namespace {
+
+constexpr int kWaves = 4;
+constexpr int kThreads = kWaves * kWave;
+constexpr int kTileRows = 32 * kWaves;   // query rows of a workgroup
+static_assert(kTileRows == (int)kGeneralTileRows, "the merge derives a row's live splits from its workgroup's last row");
+constexpr float kRescaleStep = 8.0f;     // log2 units
+
+typedef __attribute__((address_space(3))) uint8_t LdsByte;
+typedef __attribute__((address_space(3))) u32x4 LdsU32x4;
+typedef __attribute__((address_space(3))) float LdsF32;
+typedef short i16x4 __attribute__((ext_vector_type(4)));
+typedef __attribute__((address_space(3))) i16x4 LdsI16x4;
+
+// Shape of a kernel: NB blocks of 32 head elements, MB blocks of 32 keys per step.
+template <typename S, int NB>
+struct Shape {
+  static constexpr bool kF32 = std::is_same<S, F32>::value;
+  static constexpr int kBytes = sizeof(typename Store<S>::E);
+  static constexpr int kHead = 32 * NB;
+  static constexpr int kPiecesRow = kHead * kBytes / 16;
+  static constexpr int MB = (!kF32 && NB <= 4) ? 2 : 1;
+  static constexpr int kKeys = 32 * MB;
+  static constexpr int kPieces = kKeys * kPiecesRow / kThreads;   // 16-byte pieces of K (and of V) a thread moves per step
+  // Row pitches in LDS, bytes.  K rows are read 16 bytes a lane from 32 rows: a pitch of 4 x odd
+  // words spreads 16 of them over all banks.  V rows, 16-bit: a 16-lane block of the transposing read
+  // takes 32 bytes from each of four rows and its neighbour the next 32, so four rows 16 x odd words
+  // apart cover the banks; binary32: lanes 0-31 read 32 words of a row and lanes 32-63 the same
+  // columns four rows on, which 8 x odd words put into the other half of the banks.
+  static constexpr int kKPitch = kHead * kBytes + 16;
+  static constexpr int kVWords = kHead * kBytes / 4;
+  static constexpr int kVPitch = 4 * (kF32 ? kVWords + 8 : (kVWords % 32 == 16 ? kVWords : kVWords + 16));
+  static constexpr int kKBuf = kKeys * kKPitch, kVBuf = kKeys * kVPitch;
+  static constexpr int kLds = 2 * (kKBuf + kVBuf);
+  // Waves per SIMD the registers are planned for: queries, accumulators, scores, weights and the
+  // pieces on their way to LDS are about 40 (32 x 32 x head / 64) registers and a few dozen more.
+  // Binary32 heads of 256 have no registers left to hold the next V rows during a step: those are
+  // requested behind it (a step is 16384 matrix cycles there).
+  static constexpr bool kLateV = kF32 && NB == 8;
+  static constexpr int kOccupancy = kF32 ? (NB <= 2 ? 2 : 1) : NB <= 2 ? 3 : NB <= 4 ? 2 : 1;
+};
+
+template <typename S, int NB, bool VEC>
+__global__ __launch_bounds__(kThreads, (Shape<S, NB>::kOccupancy)) void general_chunk_kernel(GeneralArgs p) {
+  typedef Shape<S, NB> X;
+  typedef typename Store<S>::E E;
+  constexpr int MB = X::MB, kKeys = X::kKeys, kPieces = X::kPieces;
+  constexpr int kQ = X::kPiecesRow / 2;      // query registers: pieces 2 s + g of the row
+  constexpr float kShift = Store<S>::kShift;
+  __shared__ __attribute__((aligned(16))) uint8_t smem[X::kLds];
+  __shared__ uint32_t s_bad;                 // a value beyond the first row's position is not finite
+
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int j = lane & 31, g = lane >> 5;
+  const uint32_t planes = gridDim.x / p.row_tiles;
+  const uint32_t plane = blockIdx.x % planes;
+  const uint32_t tile = p.row_tiles - 1 - blockIdx.x / planes;   // longest rows first
+  const uint32_t seq = plane / p.n_kv_heads, kvh = plane % p.n_kv_heads;
+  const uint32_t P0 = start_position(p, seq);
+  const uint32_t row0 = tile * kTileRows;
+  const uint32_t last_row = min(p.rows, row0 + kTileRows) - 1;
+  const uint32_t k0 = blockIdx.y * p.split_len;
+  // keys [k0, end): up to the last row's position, and to the end of this split
+  const uint32_t end = min(P0 + last_row / p.group + 1, k0 + p.split_len);
+  if (k0 >= end) return;   // (the merge derives the live splits the same way)
+  const uint32_t first_pos = P0 + row0 / p.group;
+  const uint32_t n_steps = (end - k0 + kKeys - 1) / kKeys;
+
+  const uint32_t r = row0 + 32 * wave + j;
+  const bool row_valid = r < p.rows;
+  const uint32_t rc = row_valid ? r : last_row;
+  const uint32_t rowpos = P0 + rc / p.group;
+  const size_t row = query_row(p, seq, kvh, rc);
+  const uint32_t wave_row0 = min(row0 + 32u * wave, last_row), wave_row1 = min(wave_row0 + 31u, last_row);
+  const uint32_t wave_first = P0 + wave_row0 / p.group;    // chunks up to here need no mask,
+  const uint32_t wave_last = P0 + wave_row1 / p.group;     // chunks past here are not this wave's
+  const bool wave_has_rows = __builtin_amdgcn_readfirstlane((int)(row0 + 32u * wave <= last_row));
+
+  u32x4 qreg[kQ];
+  {
+    const E* qrow = (const E*)p.q + row * p.head_size;
+#pragma unroll
+    for (int s = 0; s < kQ; ++s) qreg[s] = query_piece<S, VEC>(p, qrow, (2 * s + g) * Store<S>::kPiece);
+  }
+
+  const size_t plane_at = seq_plane_offset(p.seq_offsets, p.kv_stride_seq, seq) + (size_t)kvh * p.kv_stride_head;
+  const E* kp = (const E*)p.k + plane_at;
+  const E* vp = (const E*)p.v + plane_at;
+  const uint64_t kplane = scalar64((uint64_t)kp), vplane = scalar64((uint64_t)vp);
+  const uint64_t pos_bytes = (uint64_t)p.kv_stride_pos * sizeof(E);
+  const uint64_t valid = scalar64((uint64_t)(end - 1) * pos_bytes + (uint64_t)p.head_size * sizeof(E));
+  uint32_t off[kPieces], lds_k[kPieces], lds_v[kPieces];
+  const uint32_t lds0 = (uint32_t)(uintptr_t)(LdsByte*)smem;
+#pragma unroll
+  for (int i = 0; i < kPieces; ++i) {
+    const uint32_t pi = tid + kThreads * i, krow = pi / X::kPiecesRow, col = pi % X::kPiecesRow;
+    if constexpr (VEC)
+      off[i] = col * Store<S>::kPiece < p.head_size ? (uint32_t)(krow * pos_bytes) + 16 * col : kNowhere;
+    else
+      off[i] = krow | col * Store<S>::kPiece << 16;
+    lds_k[i] = lds0 + krow * X::kKPitch + 16 * col;
+    lds_v[i] = lds0 + 2 * X::kKBuf + krow * X::kVPitch + 16 * col;
+  }
+  u32x4 kst[kPieces], vst[kPieces];
+  auto load_rows = [&](uint32_t step, const E* rows, uint64_t plane_base, u32x4 (&st)[kPieces]) {
+    const uint32_t kb = k0 + step * kKeys;
+    if constexpr (VEC) {
+      const __amdgpu_buffer_rsrc_t rs = chunk_rsrc(plane_base, (uint64_t)kb * pos_bytes, valid);
+#pragma unroll
+      for (int i = 0; i < kPieces; ++i) st[i] = __builtin_amdgcn_raw_buffer_load_b128(rs, off[i], 0, 0);
+    } else {
+#pragma unroll
+      for (int i = 0; i < kPieces; ++i)
+        st[i] = gather_piece<S>(rows, p.kv_stride_pos, kb + (off[i] & 0xffffu), end, off[i] >> 16, p.head_size);
+    }
+  };
+  auto load_step = [&](uint32_t step) {
+    load_rows(step, kp, kplane, kst);
+    if constexpr (!X::kLateV) load_rows(step, vp, vplane, vst);
+  };
+  auto store_step = [&](uint32_t step) {
+    const uint32_t buf = step & 1;
+    if constexpr (X::kLateV) load_rows(step, vp, vplane, vst);
+#pragma unroll
+    for (int i = 0; i < kPieces; ++i) {
+      *(LdsU32x4*)(lds_k[i] + buf * X::kKBuf) = kst[i];
+      *(LdsU32x4*)(lds_v[i] + buf * X::kVBuf) = vst[i];
+    }
+    if (k0 + step * kKeys + kKeys - 1 > first_pos) {   // some row of the workgroup must not see some of these values
+      bool bad = false;
+#pragma unroll
+      for (int i = 0; i < kPieces; ++i) bad |= piece_not_finite<S>(vst[i]);
+      if (bad) s_bad = 1;
+    }
+  };
+
+  float m_run = -INFINITY, l_run = 0.0f;
+  f32x16 oacc[NB];
+#pragma unroll
+  for (int db = 0; db < NB; ++db)
+#pragma unroll
+    for (int e = 0; e < 16; ++e) oacc[db][e] = 0.0f;
+
+  // K as the A operand: key j of a block, the pieces the query registers hold
+  const uint32_t k_read = lds0 + j * X::kKPitch + 16 * g;
+  // V^T as the A operand: 16-bit through the transposing read (see prefill.hip), binary32 element by
+  // element, keys in the order in which the soft-max leaves the weights in registers
+  const uint32_t v_read = X::kF32 ? lds0 + 2 * X::kKBuf + 4 * g * X::kVPitch + 4 * j
+                                  : lds0 + 2 * X::kKBuf + (4 * g + ((lane & 15) >> 2)) * X::kVPitch +
+                                        2 * (16 * ((lane >> 4) & 1) + 4 * (lane & 3));
+
+  auto compute = [&](uint32_t step) __attribute__((always_inline)) {
+    const uint32_t kb = k0 + step * kKeys, buf = step & 1;
+    if (!wave_has_rows || kb > wave_last) return;
+    const uint32_t ks = k_read + buf * X::kKBuf, vs = v_read + buf * X::kVBuf;
+    f32x16 st[MB];
+#pragma unroll
+    for (int mb = 0; mb < MB; ++mb) {
+#pragma unroll
+      for (int e = 0; e < 16; ++e) st[mb][e] = 0.0f;
+    }
+#pragma unroll
+    for (int s = 0; s < kQ; ++s)
+#pragma unroll
+      for (int mb = 0; mb < MB; ++mb) {
+        const u32x4 a = *(const LdsU32x4*)(ks + 32 * mb * X::kKPitch + 32 * s);
+        if constexpr (X::kF32) {
+#pragma unroll
+          for (int e = 0; e < 4; ++e)
+            st[mb] = __builtin_amdgcn_mfma_f32_32x32x2f32(__builtin_bit_cast(float, (uint32_t)a[e]),
+                                                          __builtin_bit_cast(float, (uint32_t)qreg[s][e]), st[mb], 0, 0, 0);
+        } else {
+          st[mb] = Mfma<S>::m32x32x16(a, qreg[s], st[mb]);
+        }
+      }
+    if (kb + kKeys - 1 > wave_first || kb + kKeys > end) {   // some pair of the step is masked
+#pragma unroll
+      for (int mb = 0; mb < MB; ++mb)
+#pragma unroll
+        for (int e = 0; e < 16; ++e) {
+          const uint32_t key = kb + 32 * mb + 8 * (e >> 2) + 4 * g + (e & 3);
+          st[mb][e] = (key <= rowpos && key < end) ? st[mb][e] : -INFINITY;
+        }
+    }
+    float rmax = st[0][0];
+#pragma unroll
+    for (int mb = 0; mb < MB; ++mb)
+#pragma unroll
+      for (int e = 0; e < 16; ++e) rmax = fmaxf(rmax, st[mb][e]);
+    rmax = max_with_partner_half(rmax);
+    const float tmax = rmax * p.c;
+    const bool grow = tmax > m_run + kRescaleStep;
+    if (__any(grow)) {
+      const float m_new = grow ? tmax : m_run;
+      const float alpha = grow ? fast_exp2(m_run - m_new) : 1.0f;
+      m_run = m_new;
+      l_run *= alpha;
+#pragma unroll
+      for (int db = 0; db < NB; ++db) oacc[db] *= alpha;
+    }
+    const float neg_m = (m_run == -INFINITY) ? 0.0f : kShift - m_run;
+    float psum = 0.0f;
+    if constexpr (X::kF32) {
+#pragma unroll
+      for (int e = 0; e < 16; ++e) {
+        st[0][e] = fast_exp2(__builtin_fmaf(st[0][e], p.c, neg_m));
+        psum += st[0][e];
+      }
+#pragma unroll
+      for (int e = 0; e < 16; ++e)
+#pragma unroll
+        for (int db = 0; db < NB; ++db) {
+          const float a = *(const LdsF32*)(vs + (8 * (e >> 2) + (e & 3)) * X::kVPitch + 128 * db);
+          oacc[db] = __builtin_amdgcn_mfma_f32_32x32x2f32(a, st[0][e], oacc[db], 0, 0, 0);
+        }
+    } else {
+      u32x4 hi[2 * MB], lo[2 * MB];
+#pragma unroll
+      for (int cc = 0; cc < 2 * MB; ++cc)
+#pragma unroll
+        for (int w = 0; w < 4; ++w) {
+          const int e = 8 * (cc & 1) + 2 * w;
+          const float p0 = fast_exp2(__builtin_fmaf(st[cc >> 1][e], p.c, neg_m));
+          const float p1 = fast_exp2(__builtin_fmaf(st[cc >> 1][e + 1], p.c, neg_m));
+          uint32_t h, l;
+          split_pair<S>(p0, p1, h, l);
+          hi[cc][w] = h;
+          lo[cc][w] = l;
+          psum += p0 + p1;
+        }
+#pragma unroll
+      for (int cc = 0; cc < 2 * MB; ++cc)
+#pragma unroll
+        for (int db = 0; db < NB; ++db) {
+          const uint32_t at = vs + 16 * cc * X::kVPitch + 64 * db;
+          const i16x4 a0 = __builtin_amdgcn_ds_read_tr16_b64_v4i16((LdsI16x4*)at);
+          const i16x4 a1 = __builtin_amdgcn_ds_read_tr16_b64_v4i16((LdsI16x4*)(at + 8 * X::kVPitch));
+          const u32x2 w0 = __builtin_bit_cast(u32x2, a0), w1 = __builtin_bit_cast(u32x2, a1);
+          const u32x4 a = {w0[0], w0[1], w1[0], w1[1]};
+          oacc[db] = Mfma<S>::m32x32x16(a, hi[cc], oacc[db]);
+          oacc[db] = Mfma<S>::m32x32x16(a, lo[cc], oacc[db]);
+        }
+    }
+    l_run += psum;
+  };
+
+  if (tid == 0) s_bad = 0;
+  load_step(0);
+  __syncthreads();
+  store_step(0);
+  if (n_steps > 1) load_step(1);
+  __syncthreads();
+  for (uint32_t step = 0; step < n_steps; ++step) {
+    compute(step);
+    if (step + 1 < n_steps) {
+      store_step(step + 1);
+      if (step + 2 < n_steps) load_step(step + 2);
+    }
+    __syncthreads();
+  }
+
+  const size_t part_row0 = (size_t)plane * p.rows;
+  if (s_bad) {   // (uniform: the last barrier is behind every write of it)
+    for (uint32_t rr = row0 + wave; rr <= last_row; rr += kWaves)
+      plain_row<S>(p, kp, vp, query_row(p, seq, kvh, rr), (part_row0 + rr) * p.n_split + blockIdx.y, k0,
+                   min(end, P0 + rr / p.group + 1), X::kHead, p.n_split > 1);
+    return;
+  }
+  const float l = sum_with_partner_half(l_run);
+  if (!row_valid) return;
+  if (p.n_split > 1) {
+    const size_t part = (part_row0 + r) * p.n_split + blockIdx.y;
+    float* orow = p.part_o + part * X::kHead;
+#pragma unroll
+    for (int db = 0; db < NB; ++db)
+#pragma unroll
+      for (int q4 = 0; q4 < 4; ++q4)
+        *(f32x4*)(orow + 32 * db + 8 * q4 + 4 * g) =
+            f32x4{oacc[db][4 * q4], oacc[db][4 * q4 + 1], oacc[db][4 * q4 + 2], oacc[db][4 * q4 + 3]};
+    if (g == 0) *(float2*)(p.part_ml + part * 2) = float2{m_run == -INFINITY ? m_run : m_run - kShift, l};
+  } else {
+    const float inv = 1.0f / l;
+#pragma unroll
+    for (int db = 0; db < NB; ++db)
+#pragma unroll
+      for (int q4 = 0; q4 < 4; ++q4)
+        store_out4<S, VEC>(p, row, 32 * db + 8 * q4 + 4 * g,
+                           f32x4{oacc[db][4 * q4] * inv, oacc[db][4 * q4 + 1] * inv, oacc[db][4 * q4 + 2] * inv,
+                                 oacc[db][4 * q4 + 3] * inv});
+    if (p.lse && g == 0) p.lse[row] = (m_run - kShift + fast_log2(l)) * kLn2;
+  }
+}
+
+}  // namespace
+
+hipError_t launch_general_chunk(const GeneralArgs& p, int dtype, int nb, bool vec, uint32_t planes, hipStream_t stream) {
+  const dim3 grid(planes * p.row_tiles, p.n_split), block(kThreads);
+  return with_head_blocks(nb, vec, [&](auto n, auto v) {
+    constexpr int NB = decltype(n)::value;
+    constexpr bool VEC = decltype(v)::value;
+    if (dtype == 0)
+      hipLaunchKernelGGL((general_chunk_kernel<F16, NB, VEC>), grid, block, 0, stream, p);
+    else if (dtype == 1)
+      hipLaunchKernelGGL((general_chunk_kernel<BF16, NB, VEC>), grid, block, 0, stream, p);
+    else
+      hipLaunchKernelGGL((general_chunk_kernel<F32, NB, VEC>), grid, block, 0, stream, p);
+    return hipGetLastError();
+  });
+}
+
+}  // namespace gen
+}  // namespace ellm

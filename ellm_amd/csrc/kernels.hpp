@@ -86,6 +86,14 @@ bool decode_balanced_takes(const DecodeWorkspace& w, uint32_t batch, uint32_t n_
 hipError_t launch_decode_balanced(const AttnArgs& a, uint32_t wgs, hipStream_t stream);
 hipError_t launch_prefill(const AttnArgs& a, hipStream_t stream);
 // Any head size up to 256 and binary32 storage (dtype 2): chunk and single-token calls alike.
+// Workspace of such an operator: partial rows (pitch floats each, then 2 of maximum and sum) and
+// arrival counters, in the chunk path's fields of AttnArgs.
+struct GeneralWorkspace {
+  size_t rows, counters;
+  uint32_t pitch;
+};
+GeneralWorkspace general_workspace(uint32_t max_interval, uint32_t batch_capacity, uint32_t n_q_heads,
+                                   uint32_t n_kv_heads, uint32_t head_size, uint32_t n_cu);
 hipError_t launch_attn_general(const AttnArgs& a, uint32_t head_size, hipStream_t stream);
 
 // Where the rows of a cache layer live: plane of (sequence, head) at

@@ -85,11 +85,12 @@ int ellm_device_count(void);
  *            run() will be given; sizes q/out).
  *
  * head_size 128 with 16-bit storage (every model configuration the reference ships) runs the
- * MFMA kernels.  Any other head_size from 1 to 256, and ELLM_DTYPE_F32 storage (the type of
+ * kernels built for it.  Any other head_size from 1 to 256, and ELLM_DTYPE_F32 storage (the type of
  * the reference's generic leaf and of its operator test, src/kernel/generic/
- * flash_attention.rs:60-89, src/compiler/mul/attention.rs:262-330), run a plain kernel with the
- * same arguments, masks and results (binary32 arithmetic throughout), written to be right and
- * not for a roofline; there kv_strides[0..2] need not be multiples of 8.
+ * flash_attention.rs:60-89, src/compiler/mul/attention.rs:262-330), run MFMA kernels of their own with
+ * the same arguments, masks and results (binary32 accumulation; soft-max weights of at least 16
+ * significant bits, binary32 for binary32 storage); there kv_strides[0..2] need not be multiples of
+ * 8 (rows that are not whole aligned 16-byte pieces, and sequence tables, take element-wise loads).
  * ellm_attn_run_noalloc and ellm_matmul3_attn_run take 128-wide 16-bit heads only.
  */
 typedef struct ellm_attn_desc {

@@ -1,0 +1,90 @@
+"""The matrix kernels for other head sizes and binary32 at the edges of their tiles: rows per
+workgroup (16 and 128), keys per step, padded head blocks, key splits and their folds, rows that are
+not whole 16-byte pieces, values that are not finite beyond a row's position.  Same oracle and
+bounds as tests/test_gpu_general_heads.py: the weights enter the second product with at least 16
+significant bits, so 16-bit results still differ by the one rounding to storage."""
+import numpy as np
+import pytest
+
+import oracle_lib as orc
+from test_gpu_general_heads import _check, _rand, _run
+
+pytestmark = pytest.mark.gpu
+
+# (name, dtype, batch, q heads, kv heads, head size, capacity, position_index, interval)
+CASES = [
+    ("rows_32_step_kernel_two_tiles", orc.F16, 1, 16, 1, 64, 200, 130, 2),
+    ("rows_33_chunk_kernel", orc.BF16, 2, 3, 1, 64, 256, 150, 11),
+    ("rows_128_one_tile", orc.F16, 1, 4, 1, 96, 96, 64, 32),
+    ("rows_129_two_tiles", orc.BF16, 1, 3, 1, 160, 150, 100, 43),
+    ("keys_64_and_65", orc.F16, 1, 2, 1, 32, 65, 0, 65),
+    ("h224_padded_to_256", orc.F16, 1, 2, 1, 224, 120, 5, 70),
+    ("h192_key_split", orc.BF16, 1, 8, 1, 192, 1100, 1040, 5),
+    ("h64_key_split_many_rows", orc.F16, 1, 8, 2, 64, 2100, 2000, 67),
+    ("f32_h64_key_split", orc.F32, 1, 8, 2, 64, 1500, 1400, 40),
+    ("f32_h256", orc.F32, 1, 2, 1, 256, 130, 20, 60),
+    ("f32_h96_three_tiles", orc.F32, 1, 3, 1, 96, 140, 20, 100),
+    ("h33_elements_one_by_one", orc.F16, 2, 4, 2, 33, 180, 30, 50),
+    ("f32_h130_elements_one_by_one", orc.F32, 1, 4, 1, 130, 100, 3, 40),
+    ("step_group_17", orc.F16, 1, 17, 1, 64, 400, 399, 1),
+    ("step_group_40_h256", orc.BF16, 1, 40, 1, 256, 300, 299, 1),
+    ("step_fold_of_33_splits", orc.F16, 1, 4, 1, 128 - 8, 2110, 2109, 1),
+    ("step_f32_h256_splits", orc.F32, 2, 8, 1, 256, 1030, 1027, 1),
+    ("step_f32_h32", orc.F32, 1, 2, 2, 32, 700, 650, 1),
+    ("step_h5_splits", orc.BF16, 1, 3, 1, 5, 600, 599, 1),
+]
+
+
+@pytest.mark.parametrize("case", CASES, ids=[c[0] for c in CASES])
+def test_tile_edges(case):
+    name, dtype, b, hq, hkv, hs, cap, p0, s = case
+    print("case", name, flush=True)
+    q, k, v = _rand((s, b, hq, hs), 31, dtype), _rand((b, hkv, cap, hs), 32, dtype), _rand((b, hkv, cap, hs), 33, dtype)
+    scale = -0.9 / np.sqrt(hs) if hs == 96 else 1.0 / np.sqrt(hs)   # (a negative scale once per type)
+    want, want_lse = orc.attention(q, k, v, scale, dtype, position_index=p0)
+    got, lse = _run(q, k, v, scale, dtype, p0=p0)
+    _check(name, got, lse, want, want_lse, dtype, b)
+
+
+@pytest.mark.parametrize("dtype,hq,hkv,hs,p0,s", [(orc.F16, 8, 2, 64, 100, 70), (orc.BF16, 8, 1, 192, 600, 9),
+                                                   (orc.F32, 4, 1, 128, 40, 3)])
+def test_values_beyond_a_row_are_not_seen(dtype, hq, hkv, hs, p0, s):
+    """The value row of the chunk's last token holds infinities: rows of earlier tokens come out as if
+    it were not there (chunk kernel unsplit and split, step kernel with several tokens)."""
+    cap = p0 + s + 3
+    q, k, v = _rand((s, 1, hq, hs), 41, dtype), _rand((1, hkv, cap, hs), 42, dtype), _rand((1, hkv, cap, hs), 43, dtype)
+    scale = 1.0 / np.sqrt(hs)
+    want, want_lse = orc.attention(q, k, v, scale, dtype, position_index=p0)
+    v2 = v.copy()
+    if dtype == orc.F32:
+        v2[:, :, p0 + s - 1:] = np.inf
+    else:
+        v2.view(np.uint16)[:, :, p0 + s - 1:] = 0x7C00 if dtype == orc.F16 else 0x7F80
+    got, lse = _run(q, k, v2, scale, dtype, p0=p0)
+    _check("infinite_last_value", got[:-1], lse[:-1], want[:-1], want_lse[:-1], dtype, 1)
+    assert np.isposinf(got[-1]).all() and np.abs(lse[-1] - want_lse[-1]).max() <= 1e-4
+
+
+def test_repeated_steps_fold_the_same_bits():
+    """The arrival counters return to zero: the same handle launched many times gives the same bits."""
+    import torch
+
+    import ellm_amd
+
+    b, hq, hkv, hs, cap = 2, 8, 2, 64, 3000
+    q = torch.randn((1, b, hq, hs), device="cuda").to(torch.bfloat16)
+    k = torch.randn((b, hkv, cap, hs), device="cuda").to(torch.bfloat16)
+    v = torch.randn((b, hkv, cap, hs), device="cuda").to(torch.bfloat16)
+    out = torch.zeros_like(q)
+    op = ellm_amd.Attention(q, k, v, out, b, hq, hkv, hs, k.stride(), 0.125)
+    op.run(cap - 1, 1, b)
+    torch.cuda.synchronize()
+    first = out.clone()
+    for i in range(200):
+        op.run(cap - 1 if i % 3 else cap // 2, 1, b)
+    op.reset()
+    out.zero_()
+    op.run(cap - 1, 1, b)
+    torch.cuda.synchronize()
+    assert torch.equal(out, first)
+    op.close()
