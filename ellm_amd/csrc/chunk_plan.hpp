@@ -91,4 +91,68 @@ inline KeySplit plan_key_split(uint32_t tiles, uint32_t items, uint32_t slots, u
   return best;
 }
 
+// ---- short prompts -------------------------------------------------------------------------
+// Estimated time of a chunk call (us, launch included, 256 compute units) through the kernels that
+// can take it.  `planes` K/V planes of interval x group query rows each, the first at position p0.
+// The constants are fits to back-to-back calls (binary16; 32 / 4, 32 / 32 and 64 / 8 heads).
+struct ChunkShape {
+  uint32_t p0, interval, group, planes, n_cu;
+  double rows() const { return (double)interval * group; }
+  double keys() const { return (double)p0 + interval; }
+  double stream_us(double tb_s) const { return planes * keys() * 512 / (tb_s * 1e6); }   // every K/V row once
+};
+inline double whole_up(double x) { return (double)(uint64_t)(x + 0.999999); }
+
+// short_prompt_kernel with wr = 1 (four waves of keys) or 2 (two): workgroup starts and merges plus
+// steps of 32 rows x 32 keys, or the longest walk, or the K/V rows from memory.  Estimated (measured):
+// one row block wide: 512 tokens x 32 heads 11.0 (10.9) us, 1000 x 1 23.3 (23.3), 300 x 4 16 (18),
+// 40 x 8 on 1250 18 (21), 3 x 24 on 300, 32 / 32 heads 29 (23); two wide: 512 tokens, 64 / 8 heads 14.7
+// (14.1), 1000 x 1 20.7 (21.5), 600 x 4 31 (29), 40 x 21 on 1250 33 (33).
+inline double short_prompt_us(const ChunkShape& c, uint32_t wr) {
+  const double wgs = c.planes * whole_up(c.rows() / (32 * wr));
+  const double steps = c.planes * whole_up(c.rows() / 32) * ((c.p0 + 0.5 * c.interval) / 32 + 1);
+  const double work = (wr == 1 ? 0.0052 * wgs + 0.00078 * steps : 0.0065 * wgs + 0.00075 * steps) * 256 / c.n_cu;
+  const double chain = 1.5 + (wr == 1 ? 0.80 : 0.95) * wr * whole_up(c.keys() / 32) / 4;
+  const double t = work > chain ? work : chain, stream = c.stream_us(5.0);
+  return 5.0 + (t > stream ? t : stream);
+}
+
+// The merge launch of a split call and its partial rows, written and read once.
+inline double merge_us(const ChunkShape& c, uint32_t n_split) {
+  return n_split > 1 ? 4.0 + c.planes * c.rows() * n_split * (128 + 2) * 8 / 5e6 : 0.0;
+}
+
+// chunk_stream_kernel: 16 x 24 on 1024 28 (29.5), 40 x 8 on 1250 32 (33.5), 40 x 21 on 1250 44 (42),
+// 46 x 11 on 1713, 32 / 32 heads 58 (58), 24 x 7 on 8724, 64 / 8 heads 80 (86).
+inline double chunk_stream_us(const ChunkShape& c, uint32_t waves, const KeySplit& ks) {
+  const double tile = waves == 4 ? 1.9 : waves == 8 ? 2.0 : 2.5, slots = (waves == 4 ? 2.0 : 1.0) * c.n_cu;
+  double tiles = ks.split_tiles * whole_up(c.planes * (double)ks.n_split / slots);   // equal pieces, whole rounds
+  if (waves != 4) {                                                                  // pieces dealt over the units
+    const double mean = 1.08 * c.planes * whole_up(c.keys() / 64) / slots;
+    tiles = mean > ks.split_tiles ? mean : ks.split_tiles;
+  }
+  const double walk = tiles * tile, stream = c.stream_us(7.0);
+  return 5.0 + (walk > stream ? walk : stream) + merge_us(c, ks.n_split);
+}
+
+// prefill_pingpong_kernel, `wgs` workgroups of one compute unit each: 128 tokens 11.6 (11.7), 512 19.4 (20),
+// 1000 30 (29), 1000 x 4 43 (48); split: 128 on 4096 31 (30).
+inline double pingpong_us(const ChunkShape& c, double wgs, const KeySplit& ks) {
+  if (ks.n_split > 1) return 7.0 + 1.6 * ks.split_tiles + merge_us(c, ks.n_split);
+  const double longest = whole_up(c.keys() / 64), mean = wgs / c.n_cu * ((c.p0 + 0.5 * c.interval) / 64 + 1);
+  return 4.5 + 4.5 * whole_up(wgs / c.n_cu) + 1.3 * (longest > mean ? longest : mean);
+}
+
+// The row blocks per workgroup (1 or 2) short_prompt_kernel should take a call with, or 0: another
+// kernel's estimate `other_us` is not at least 15 % longer (the estimates are).  Up to 1920 keys: there the XCDs' L2s hold
+// the planes that are being walked, which the estimate takes for granted (261 tokens on 4868 keys:
+// 60 us where it says 42).
+constexpr uint32_t kShortPromptKeys = 1920;
+inline uint32_t short_prompt_wr(const ChunkShape& c, double other_us) {
+  if (c.p0 + c.interval > kShortPromptKeys) return 0;
+  const double one = short_prompt_us(c, 1), two = short_prompt_us(c, 2);
+  if ((one < two ? one : two) > 0.87 * other_us) return 0;
+  return one < two ? 1 : 2;
+}
+
 }  // namespace ellm

@@ -689,6 +689,241 @@ __global__ __launch_bounds__(WAVES * kWave, WAVES == 4 ? 2 : 1) void chunk_strea
   }
 }
 
+// ---------------------------------------------------------------------------
+// Short prompts: a call whose whole causal triangle is a few thousand key tiles, where the kernels
+// above leave most of the part idle or pay a merge launch.  A workgroup owns 32 WR query rows (row r of
+// a plane = token r / group, head r % group); its WK groups of WR waves take the keys in turns of 32,
+// each group with tiles of its own in LDS, and meet once at the end: many short workgroups whose
+// longest walk is 1 / WK of the row's keys.  What a wider WR buys is K/V traffic: every 32-key tile is
+// fetched once per workgroup, and a compute unit takes in 55-60 GB/s, which is what bounds the form
+// with one row block (16 KB a step: 15 TB/s over the part).  Two workgroups of four waves a unit.
+// Eight waves of keys (1 x 8) only paid on long walks (128 tokens on 4096 keys 28.7 us, split ping-pong
+// launch 30), four row blocks (4 x 2) nowhere.  Measured against the kernels above, back to back: 512
+// tokens, 32 = 32 heads 20.0 -> 11.3 us; 256 tokens, 32 / 4 heads 14.3 -> 7.3; 1000 tokens 28.9 -> 21.5;
+// 16 x 24 on 1024 30 -> 21; 40 x 21 on 1250 42 -> 33; 128 on 1000 24 -> 13; 50 x 4 on 1620 25 -> 17.
+// ---------------------------------------------------------------------------
+constexpr int kShKsHalves = kSK * kKsPitch, kShVsHalves = kSK * kVsPitch;
+constexpr int kShTileHalves = kShKsHalves + kShVsHalves;
+constexpr int kShRedPitch = kHeadDim + 4;   // floats per row of the merge
+
+template <typename T, int WR, int WK>
+__global__ __launch_bounds__(WR* WK* kWave, 2) void short_prompt_kernel(PrefillKernelArgs p) {
+  constexpr int kThreads = WR * WK * kWave;
+  constexpr int kBufs = WR == 1 ? 1 : 2;        // one wave: its LDS accesses are in order, no second buffer
+  constexpr int kPieces = 8 / WR;               // 16-byte pieces of K (and of V) a thread moves per tile
+  constexpr int kRows = 32 * WR;
+  __shared__ __attribute__((aligned(16))) uint16_t smem[WK * kBufs * kShTileHalves];
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int rw = wave % WR, kg = wave / WR;
+  const int j = lane & 31, g = lane >> 5;
+  // One XCD (workgroup id % 8) takes a plane's row tiles one after the other, longest first, so that
+  // they find its K/V rows in that XCD's L2; with fewer planes than XCDs several share one, with
+  // counts in between the planes are dealt round.
+  const uint32_t planes = p.combos, tiles = p.n_wg_tokens;   // batch * kv_heads
+  uint32_t plane, order;
+  if (p.xcd_mode == 2) {
+    plane = (blockIdx.x & 7) + 8 * ((blockIdx.x >> 3) / tiles);
+    order = (blockIdx.x >> 3) % tiles;
+  } else if (p.xcd_mode == 1) {
+    plane = (blockIdx.x & 7) % planes;
+    order = (blockIdx.x >> 3) * (8 / planes) + (blockIdx.x & 7) / planes;
+  } else {
+    plane = blockIdx.x % planes;
+    order = blockIdx.x / planes;
+  }
+  if (plane >= planes || order >= tiles) return;
+  const uint32_t rows = p.interval * p.group;
+  const uint32_t row0 = kRows * (tiles - 1 - order);
+  const uint32_t seq = plane / p.n_kv_heads, kvh = plane % p.n_kv_heads;
+  const uint32_t P0 = p.position_index;
+  const uint32_t last_row = min(rows, row0 + kRows) - 1;
+  const uint32_t kmax = P0 + last_row / p.group;
+  const uint32_t n_chunks = kmax / kSK + 1;
+  const uint32_t r = row0 + 32 * rw + j;
+  const bool row_valid = r <= last_row;
+  const uint32_t rc = min(r, last_row);
+  const uint32_t tok = rc / p.group, head = kvh * p.group + rc % p.group;
+  const uint32_t rowpos = P0 + tok;
+  const uint32_t wave_row0 = min(row0 + 32u * rw, last_row), wave_row1 = min(wave_row0 + 31u, last_row);
+  const uint32_t wave_first_pos = P0 + wave_row0 / p.group, wave_last_pos = P0 + wave_row1 / p.group;
+
+  const size_t plane_at = seq_plane_offset(p.seq_offsets, p.kv_stride_seq, seq) + kvh * p.kv_stride_head;
+  const uint64_t kplane_u = uniform64(p.k + plane_at), vplane_u = uniform64(p.v + plane_at);
+  const uint32_t stride_pos = (uint32_t)p.kv_stride_pos;
+  const uint32_t chunk_bytes = kSK * stride_pos * 2;
+  const uint64_t valid_bytes = uniform_u64(((uint64_t)kmax * stride_pos + kHeadDim) * 2);
+  const int ld_c = lane & 15, ld_r = 4 * rw + (lane >> 4);   // rows ld_r + 4 WR i of a tile
+  const uint32_t piece_off0 = (ld_r * stride_pos + 8 * ld_c) * 2, piece_step = 4 * WR * stride_pos * 2;
+  u32x4 kst[kPieces], vst[kPieces];
+  auto load_chunk = [&](uint32_t ck) {
+    const uint64_t off = (uint64_t)ck * chunk_bytes;
+    const uint32_t left = bytes_left(valid_bytes, off);
+    const __amdgpu_buffer_rsrc_t kr = __builtin_amdgcn_make_buffer_rsrc((void*)(kplane_u + off), 0, left, kBufferFlags);
+    const __amdgpu_buffer_rsrc_t vr = __builtin_amdgcn_make_buffer_rsrc((void*)(vplane_u + off), 0, left, kBufferFlags);
+#pragma unroll
+    for (int i = 0; i < kPieces; ++i) kst[i] = __builtin_amdgcn_raw_buffer_load_b128(kr, piece_off0 + i * piece_step, 0, 0);
+#pragma unroll
+    for (int i = 0; i < kPieces; ++i) vst[i] = __builtin_amdgcn_raw_buffer_load_b128(vr, piece_off0 + i * piece_step, 0, 0);
+  };
+  if ((uint32_t)kg < n_chunks) load_chunk(kg);
+  u32x4 qreg[8];
+  {
+    const uint16_t* qrow = p.q + (size_t)tok * p.q_token_stride + ((size_t)seq * p.n_q_heads + head) * kHeadDim;
+#pragma unroll
+    for (int s = 0; s < 8; ++s) {
+      qreg[s] = load16(qrow + 16 * s + 8 * g);
+      if (p.negate_q) qreg[s] ^= 0x80008000u;
+    }
+  }
+  const float c = p.c;
+  const uint32_t lds0 = (uint32_t)(uintptr_t)(LdsHalf*)smem + 2 * kg * kBufs * kShTileHalves;
+  const uint32_t ks_store = lds0 + 2 * (ld_r * kKsPitch + 8 * ld_c);
+  const uint32_t vs_store = lds0 + 2 * (kShKsHalves + ld_r * kVsPitch + 8 * ld_c);
+  auto store_chunk = [&](uint32_t buf) {
+#pragma unroll
+    for (int i = 0; i < kPieces; ++i) {
+      *(LdsU32x4*)(ks_store + 2 * (buf * kShTileHalves + 4 * WR * i * kKsPitch)) = kst[i];
+      *(LdsU32x4*)(vs_store + 2 * (buf * kShTileHalves + 4 * WR * i * kVsPitch)) = vst[i];
+    }
+  };
+  // operand addresses as in the kernels above
+  const uint32_t k_read0 = lds0 + 2 * (j * kKsPitch + 8 * g);
+  const uint32_t v_read0 = lds0 + 2 * (kShKsHalves + (4 * g + ((lane & 15) >> 2)) * kVsPitch + 16 * ((lane >> 4) & 1) + 4 * (lane & 3));
+  float m_run = -INFINITY, l_run = 0.0f;
+  f32x16 oacc[4];
+#pragma unroll
+  for (int db = 0; db < 4; ++db)
+#pragma unroll
+    for (int e = 0; e < 16; ++e) oacc[db][e] = 0.0f;
+
+  auto compute = [&](uint32_t ck, uint32_t buf) __attribute__((always_inline)) {
+    const uint32_t kb = ck * kSK;
+    if (kb > wave_last_pos) return;
+    const uint32_t k_read = k_read0 + 2 * buf * kShTileHalves, v_read = v_read0 + 2 * buf * kShTileHalves;
+    f32x16 st;
+#pragma unroll
+    for (int e = 0; e < 16; ++e) st[e] = 0.0f;
+#pragma unroll
+    for (int s = 0; s < 8; ++s) {
+      const u32x4 a = *(const LdsU32x4*)(k_read + 2 * 16 * s);
+      st = Mfma<T>::m32x32x16(a, qreg[s], st);
+    }
+    if (kb + kSK - 1 > wave_first_pos) {   // chunk crosses the diagonal of some row
+#pragma unroll
+      for (int e = 0; e < 16; ++e) {
+        const uint32_t key = kb + 8 * (e >> 2) + 4 * g + (e & 3);
+        st[e] = (key <= rowpos) ? st[e] : -INFINITY;
+      }
+    }
+    float rmax = st[0];
+#pragma unroll
+    for (int e = 1; e < 16; ++e) rmax = fmaxf(rmax, st[e]);
+    rmax = max_with_partner_half(rmax);
+    const float tmax = rmax * c;
+    const bool grow = tmax > m_run + kRescaleStep;
+    if (__any(grow)) {
+      const float m_new = grow ? tmax : m_run;
+      const float alpha = grow ? fast_exp2(m_run - m_new) : 1.0f;
+      m_run = m_new;
+      l_run *= alpha;
+#pragma unroll
+      for (int db = 0; db < 4; ++db) oacc[db] *= alpha;
+    }
+    const float neg_m = (m_run == -INFINITY) ? 0.0f : -m_run;
+    float psum = 0.0f;
+    u32x4 pk[2];
+#pragma unroll
+    for (int cc = 0; cc < 2; ++cc)
+#pragma unroll
+      for (int w = 0; w < 4; ++w) {
+        const float p0 = fast_exp2(__builtin_fmaf(st[8 * cc + 2 * w], c, neg_m));
+        const float p1 = fast_exp2(__builtin_fmaf(st[8 * cc + 2 * w + 1], c, neg_m));
+        pk[cc][w] = Mfma<T>::pack2(p0, p1);
+        psum += p0 + p1;
+      }
+    l_run += psum;
+#pragma unroll
+    for (int cc = 0; cc < 2; ++cc)
+#pragma unroll
+      for (int db = 0; db < 4; ++db) {
+        const uint32_t at = v_read + 2 * (16 * cc * kVsPitch + 32 * db);
+        const i16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((LdsI16x4*)at);
+        const i16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((LdsI16x4*)(at + 2 * 8 * kVsPitch));
+        const u32x2 l2 = __builtin_bit_cast(u32x2, lo), h2 = __builtin_bit_cast(u32x2, hi);
+        oacc[db] = Mfma<T>::m32x32x16(u32x4{l2[0], l2[1], h2[0], h2[1]}, pk[cc], oacc[db]);
+      }
+  };
+  if constexpr (WR == 1) {
+    for (uint32_t ck = kg; ck < n_chunks; ck += WK) {
+      store_chunk(0);
+      if (ck + WK < n_chunks) load_chunk(ck + WK);
+      __builtin_amdgcn_wave_barrier();
+      compute(ck, 0);
+      __builtin_amdgcn_wave_barrier();
+    }
+  } else {   // every group makes the same number of steps, so that all meet at the barriers
+    const uint32_t n_steps = (n_chunks + WK - 1) / WK;
+    if ((uint32_t)kg < n_chunks) store_chunk(0);
+    if ((uint32_t)kg + WK < n_chunks) load_chunk(kg + WK);
+    __syncthreads();
+    for (uint32_t step = 0; step < n_steps; ++step) {
+      const uint32_t ck = kg + WK * step;
+      if (ck < n_chunks) compute(ck, step & 1);
+      if (ck + WK < n_chunks) {
+        store_chunk((step & 1) ^ 1);
+        if (ck + 2 * WK < n_chunks) load_chunk(ck + 2 * WK);
+      }
+      __syncthreads();
+    }
+  }
+  const float l_wave = sum_with_partner_half(l_run);
+  auto store_lse = [&](uint32_t t, uint32_t h, float v) { p.lse[((size_t)t * p.batch_pitch + seq) * p.n_q_heads + h] = v * kLn2; };
+  float* red = (float*)smem;
+  // the groups' rows meet in LDS: red[group][row][128 sums, maximum, denominator]
+  static_assert(WK * kRows * kShRedPitch * 4 <= WK * kBufs * kShTileHalves * 2, "the merge must fit in the staging buffers");
+  __syncthreads();
+  float* mine = red + (kg * kRows + 32 * rw + j) * kShRedPitch;
+#pragma unroll
+  for (int db = 0; db < 4; ++db)
+#pragma unroll
+    for (int q4 = 0; q4 < 4; ++q4)
+      *(f32x4*)(mine + 32 * db + 8 * q4 + 4 * g) =
+          f32x4{oacc[db][4 * q4], oacc[db][4 * q4 + 1], oacc[db][4 * q4 + 2], oacc[db][4 * q4 + 3]};
+  if (g == 0) *(f32x2*)(mine + kHeadDim) = f32x2{m_run, l_wave};
+  __syncthreads();
+  // a thread finishes eight columns of a row, a wave four whole rows at a time
+#pragma unroll
+  for (int n = 0; n < kRows * 16 / kThreads; ++n) {
+    const uint32_t rr = kThreads / 16 * n + (tid >> 4), d8 = tid & 15;
+    if (row0 + rr > last_row) continue;
+    f32x2 ml[WK];
+    float m = -INFINITY;
+#pragma unroll
+    for (int w = 0; w < WK; ++w) {
+      ml[w] = *(const f32x2*)(red + (w * kRows + rr) * kShRedPitch + kHeadDim);
+      m = fmaxf(m, ml[w][0]);
+    }
+    float l = 0.0f;
+    f32x4 o[2] = {{0.0f, 0.0f, 0.0f, 0.0f}, {0.0f, 0.0f, 0.0f, 0.0f}};
+#pragma unroll
+    for (int w = 0; w < WK; ++w) {
+      const float wgt = fast_exp2(ml[w][0] - m);   // (a group without keys left -inf: weight 0; m is finite, key 0 counts)
+      const float* src = red + (w * kRows + rr) * kShRedPitch + 8 * d8;
+      l += wgt * ml[w][1];
+      o[0] += wgt * *(const f32x4*)src;
+      o[1] += wgt * *(const f32x4*)(src + 4);
+    }
+    const float inv = 1.0f / l;
+    const uint32_t t = (row0 + rr) / p.group, h = kvh * p.group + (row0 + rr) % p.group;
+    u32x4 w4;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) w4[e] = Mfma<T>::pack2(o[e >> 1][2 * (e & 1)] * inv, o[e >> 1][2 * (e & 1) + 1] * inv);
+    store16(p.out + (size_t)t * p.q_token_stride + ((size_t)seq * p.n_q_heads + h) * kHeadDim + 8 * d8, w4);
+    if (p.lse && d8 == 0) store_lse(t, h, m + fast_log2(l));
+  }
+}
+
 // Folds the partial results of a split launch: G lanes per (query row, four columns) take
 // the row's splits in turn and combine through lane exchanges (with hundreds of splits and
 // few rows a thread walking them alone would be one long chain of memory round trips).
@@ -801,6 +1036,27 @@ hipError_t launch_pingpong(const AttnArgs& a, hipStream_t stream) {
     return merge(prefill_merge_kernel<T, 1>, 1);
   };
 
+  // Short prompts and short chunks on short caches (short_prompt_wr, chunk_plan.hpp)
+  const ChunkShape shape = {a.position_index, a.position_interval, a.group, a.batch * a.n_kv_heads, a.n_cu};
+  auto short_launch = [&](uint32_t wr) {
+    const uint32_t planes = shape.planes, wg_rows = 32 * wr;
+    p.combos = planes;
+    p.n_wg_tokens = (uint32_t)(((size_t)a.position_interval * a.group + wg_rows - 1) / wg_rows);
+    // Planes that are no multiple of the XCDs, or that together overflow their L2s, go to one XCD each
+    // (40 tokens x 21 sequences on 1250, 84 planes: 55.7 -> 39.9 us); else all planes advance together,
+    // longest rows first over the whole call (512 tokens x 32 heads: 10.8 against 12.8 us).
+    const double xcd_mb = planes / 8.0 * (a.position_index + a.position_interval) * 512e-6;
+    p.xcd_mode = planes <= 8 && 8 % planes == 0 ? 1 : planes >= 32 && (planes % 8 || xcd_mb > 8.0) ? 2 : 0;
+    uint32_t n = planes * p.n_wg_tokens;
+    if (p.xcd_mode == 1) n = 8 * ((p.n_wg_tokens + 8 / planes - 1) / (8 / planes));
+    if (p.xcd_mode == 2) n = (planes + 7) / 8 * 8 * p.n_wg_tokens;
+    if (wr == 2)
+      hipLaunchKernelGGL((short_prompt_kernel<T, 2, 2>), dim3(n), dim3(4 * kWave), 0, stream, p);
+    else
+      hipLaunchKernelGGL((short_prompt_kernel<T, 1, 4>), dim3(n), dim3(4 * kWave), 0, stream, p);
+    return hipGetLastError();
+  };
+
   // Few query rows per plane on a cache long enough to be worth streaming: one workgroup
   // covers all rows of a GQA group, the key range is split until there are two
   // workgroups per compute unit (splits of at least 256 keys), as far as the workspace holds
@@ -837,6 +1093,8 @@ hipError_t launch_pingpong(const AttnArgs& a, hipStream_t stream) {
     }
     // enough workgroups to be worth it (a lone sequence with one split would leave the part idle)
     if ((size_t)planes * p.n_split * 2 >= a.n_cu || planes * p.n_split >= p.combos * p.n_wg_tokens) {
+      if (const uint32_t wr = short_prompt_wr(shape, chunk_stream_us(shape, waves, {p.split_tiles, p.n_split})))
+        return short_launch(wr);
       p.tblocks_per_wg = (a.position_interval + 31) / 32;  // (the merge derives every row's live splits from the chunk's last token)
       const dim3 grid(planes, p.n_split);
       if (waves == 4)
@@ -882,6 +1140,8 @@ hipError_t launch_pingpong(const AttnArgs& a, hipStream_t stream) {
       p.n_split = ks.n_split;
     }
   }
+  if (const uint32_t wr = short_prompt_wr(shape, pingpong_us(shape, base, {p.split_tiles, p.n_split})))
+    return short_launch(wr);
   if (p.n_split <= 1) {
     p.n_split = 1;
     hipLaunchKernelGGL((prefill_pingpong_kernel<T, false>), dim3(n_wg), dim3(kPpThreads), 0, stream, p);

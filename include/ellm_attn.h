@@ -135,7 +135,8 @@ int ellm_attn_reset(ellm_attn* handle, void* stream);
  * intervals the tiled MFMA kernel (with the key range split over workgroups and
  * a merge launch behind it when the call has too few query rows to fill the
  * device; calls with at most 384 query rows per K/V plane on 512 keys or more
- * take a kernel that streams every plane once).  Zero batch_size or
+ * take a kernel that streams every plane once, short prompts and short chunks on short caches one
+ * whose waves share the keys of 32 or 64 rows).  Zero batch_size or
  * position_interval is a no-op returning ELLM_OK.  One run of a handle in flight
  * at a time (see the top of this file).
  * K/V rows at positions up to position_index + position_interval - 1 must hold finite

@@ -1,0 +1,73 @@
+"""Short prompts and short chunks on short caches: the kernel whose waves share a row block's keys
+(short_prompt_kernel) at the edges of its tiles, and the rule that sends calls to it."""
+import os
+import shutil
+import subprocess
+
+import numpy as np
+import pytest
+
+import oracle_lib as orc
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+
+# (batch, q heads, kv heads, position_index, interval, row blocks per workgroup on 256 compute units)
+CASES = [
+    (1, 8, 8, 0, 64, 1),         # one workgroup per 32 tokens, two key chunks for four waves
+    (1, 2, 1, 0, 33, 1),         # 66 rows: two row blocks and two rows of a third
+    (1, 3, 1, 95, 11, 1),        # 33 rows of a group of three, on a cache: one row in the second block
+    (2, 8, 2, 0, 129, 1),        # several tokens per row block, a chunk of one key at the end
+    (9, 8, 4, 7, 31, 1),         # 36 planes: one XCD each, the last four XCDs idle in the last round
+    (3, 6, 1, 500, 65, 1),       # three planes: dealt round
+    (1, 32, 4, 0, 1001, 2),      # two row blocks a workgroup, planes shared by two XCDs, 8 rows in the last
+    (1, 64, 8, 0, 500, 2),       # 500 x 8 rows: the last workgroup holds 32 rows of 64
+    (2, 48, 16, 100, 201, 2),    # 603 rows of a group of three: the last workgroup holds 27
+]
+
+
+def test_the_rule_sends_these_calls_there(tmp_path):
+    gxx = shutil.which("g++")
+    if not gxx:
+        pytest.skip("no g++")
+    src = tmp_path / "probe.cpp"
+    src.write_text(r"""
+#include "chunk_plan.hpp"
+#include <cstdio>
+#include <cstdlib>
+using namespace ellm;
+int main(int, char** v) {
+  const uint32_t b = atoi(v[1]), hq = atoi(v[2]), hkv = atoi(v[3]), p0 = atoi(v[4]), s = atoi(v[5]);
+  const ChunkShape c = {p0, s, hq / hkv, b * hkv, 256};
+  const uint32_t g = hq / hkv, stacked = g % 8 == 0 ? 8 : g % 4 == 0 ? 4 : g % 2 == 0 ? 2 : 1;   // heads a workgroup of the
+  const double wgs = (double)b * hkv * (g / stacked) * ((s * stacked + 255) / 256);             // ping-pong kernel stacks
+  printf("%u\n", short_prompt_wr(c, pingpong_us(c, wgs, {0, 1})));
+}
+""")
+    exe = tmp_path / "probe"
+    subprocess.run([gxx, "-O1", "-std=c++17", "-I", os.path.join(ROOT, "ellm_amd", "csrc"), "-o", str(exe), str(src)], check=True)
+
+    def wr(*a):
+        return int(subprocess.run([str(exe), *map(str, a)], check=True, capture_output=True, text=True).stdout)
+
+    for c in CASES:
+        assert wr(*c[:5]) == c[5], c
+    assert wr(1, 32, 4, 0, 4096) == 0 and wr(1, 32, 4, 8192, 64) == 0      # long walks: the other kernels
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("case", CASES, ids=[f"{c[0]}x{c[4]}on{c[3]}_{c[1]}q{c[2]}kv" for c in CASES])
+def test_short_prompts_match_the_oracle(case):
+    from gpu_util import D, LSE_TOL, compare, gpu_attention, rand_storage
+
+    b, hq, hkv, p0, s, wr = case
+    print("case", case, flush=True)
+    dtype = orc.BF16 if wr == 2 else orc.F16
+    q = rand_storage((s, b + 1, hq, D), 61, dtype)      # one sequence of capacity more than the batch
+    k = rand_storage((b + 1, hkv, p0 + s + 1, D), 62, dtype)
+    v = rand_storage((b + 1, hkv, p0 + s + 1, D), 63, dtype)
+    want, want_lse = orc.attention(q, k, v, D ** -0.5, dtype, position_index=p0, batch=b)
+    got, lse = gpu_attention(q, k, v, D ** -0.5, dtype, position_index=p0, batch=b)
+    res = compare(got[:, :b], orc.from_storage(want, dtype)[:, :b], dtype)
+    assert res["ok"], res
+    assert np.abs(lse[:, :b] - want_lse[:, :b]).max() <= LSE_TOL
+    assert np.isnan(got[:, b:]).all()
