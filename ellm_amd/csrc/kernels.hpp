@@ -161,7 +161,7 @@ struct ProjectArgs {
 bool project_raw_takes(uint32_t rows, uint32_t heads, uint32_t K, bool has_workspace);
 hipError_t launch_project(const ProjectArgs& a, hipStream_t stream);
 // Few-rows kernel: rows it handles at most, floats of partial sums and counters it needs.
-size_t project_workspace_floats(uint32_t heads, uint32_t K);
+size_t project_workspace_floats(uint32_t heads);
 // The kernel a projection of this shape runs (heads = 128-wide output column groups).
 enum { kPathFewRows = 0, kPathTiles128 = 1, kPathTiles256x1 = 2, kPathTiles = 3 };
 int project_path(uint32_t rows, uint32_t heads, uint32_t K, bool has_workspace);

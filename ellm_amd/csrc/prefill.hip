@@ -740,9 +740,7 @@ __global__ __launch_bounds__(WR* WK* kWave, 2) void short_prompt_kernel(PrefillK
   const uint32_t last_row = min(rows, row0 + kRows) - 1;
   const uint32_t kmax = P0 + last_row / p.group;
   const uint32_t n_chunks = kmax / kSK + 1;
-  const uint32_t r = row0 + 32 * rw + j;
-  const bool row_valid = r <= last_row;
-  const uint32_t rc = min(r, last_row);
+  const uint32_t rc = min(row0 + 32 * rw + j, last_row);
   const uint32_t tok = rc / p.group, head = kvh * p.group + rc % p.group;
   const uint32_t rowpos = P0 + tok;
   const uint32_t wave_row0 = min(row0 + 32u * rw, last_row), wave_row1 = min(wave_row0 + 31u, last_row);

@@ -272,10 +272,10 @@ hipError_t launch_project(const ProjectArgs& a, hipStream_t stream) {
   const int path = project_path(a.rows, a.heads0 + 2 * a.heads_kv, a.K, a.ws && a.counters);
   if (a.raw_out) {
     if (path != kPathFewRows || a.residual) return hipErrorInvalidValue;   // (project_raw_takes() said otherwise)
-    return launch_project_small(p, a.ws, a.counters, a.dtype, kModeRaw, stream);
+    return launch_project_small(p, a.ws, a.counters, g_n_cu, a.dtype, kModeRaw, stream);
   }
   if (path == kPathFewRows)
-    return launch_project_small(p, a.ws, a.counters, a.dtype, a.residual ? kModeAdd : kModeQkv, stream);
+    return launch_project_small(p, a.ws, a.counters, g_n_cu, a.dtype, a.residual ? kModeAdd : kModeQkv, stream);
   if (path == kPathTiles128 || path == kPathTiles256x1)
     return launch_project_mid(p, path == kPathTiles128 ? 1 : 2, a.dtype, a.residual != nullptr, stream);
   const uint32_t blocks = p.tiles_m * p.tiles_n;
@@ -301,13 +301,9 @@ hipError_t project_prepare() {
   if (hipGetDevice(&dev) == hipSuccess &&
       hipDeviceGetAttribute(&n_cu, hipDeviceAttributeMultiprocessorCount, dev) == hipSuccess && n_cu > 0)
     g_n_cu = (uint32_t)n_cu;
-  const hipError_t e = mid_prepare();
-  if (e != hipSuccess) return e;
-  return small_prepare();
+  return mid_prepare();
 }
 
-size_t project_workspace_floats(uint32_t heads, uint32_t K) {
-  return small_workspace_floats(heads, K);
-}
+size_t project_workspace_floats(uint32_t heads) { return (size_t)heads * kHeadDim * kSmallRowsMax; }
 
 }  // namespace ellm

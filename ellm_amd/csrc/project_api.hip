@@ -26,14 +26,14 @@ struct ellm_matmul_add {
 namespace {
 // Partial sums and arrival counters of the few-rows kernel; left null (the tile kernel then
 // runs every call) when they would take more than 64 MiB.
-int alloc_small_workspace(uint32_t heads, uint32_t K, int* device, float** ws, uint32_t** counters) {
+int alloc_small_workspace(uint32_t heads, int* device, float** ws, uint32_t** counters) {
   *ws = nullptr;
   *counters = nullptr;
   int n_cu = 0;
   if (int st = ellm::current_gfx950_device(device, &n_cu)) return st;
   const hipError_t prep = ellm::project_prepare();
   if (prep != hipSuccess) return ellm::set_error(ELLM_ERR_HIP, "projection kernels: %s", hipGetErrorString(prep));
-  const size_t floats = ellm::project_workspace_floats(heads, K);
+  const size_t floats = ellm::project_workspace_floats(heads);
   if (floats * sizeof(float) > (size_t)64 << 20) return ELLM_OK;
   hipError_t e = hipMalloc((void**)ws, floats * sizeof(float));
   if (e == hipSuccess) e = hipMalloc((void**)counters, heads * sizeof(uint32_t));
@@ -119,8 +119,8 @@ static int matmul3_create(const ellm_matmul3_desc* d, const ellm_kv_seq_table* t
     h->seq_caps = table->seq_capacity;
     h->caps_host.assign(table->seq_capacity_host, table->seq_capacity_host + d->batch_size);
   }
-  const int rc = alloc_small_workspace((uint32_t)(d->attention_head_num + 2 * d->kv_head_num),
-                                       (uint32_t)d->hidden_size, &h->device, &h->ws, &h->counters);
+  const int rc = alloc_small_workspace((uint32_t)(d->attention_head_num + 2 * d->kv_head_num), &h->device, &h->ws,
+                                       &h->counters);
   if (rc != ELLM_OK) {
     delete h;
     return rc;
@@ -266,7 +266,7 @@ int ellm_matmul_add_create(const ellm_matmul_add_desc* d, ellm_matmul_add** out_
   ellm_matmul_add* h = new (std::nothrow) ellm_matmul_add;
   if (!h) return ellm::set_error(ELLM_ERR_HIP, "out of host memory");
   h->d = *d;
-  const int rc = alloc_small_workspace((uint32_t)(d->n / 128), (uint32_t)d->k, &h->device, &h->ws, &h->counters);
+  const int rc = alloc_small_workspace((uint32_t)(d->n / 128), &h->device, &h->ws, &h->counters);
   if (rc != ELLM_OK) {
     delete h;
     return rc;

@@ -61,16 +61,13 @@ constexpr int kModeAdd = 1;  // plain product plus a residual of the output's la
 constexpr int kModeRaw = 2;  // the binary32 sums of every column to the workspace, [row][column]: a fused
                              // single-token step, whose attention kernel finishes the rows (few-rows kernel only)
 
-// Streaming kernel for a few rows (project_small.hip).  It would take up to 128 rows, but from
-// about 64 on one 128-token tile per head (project_mid.hip) is faster: measured for the
-// 2048 -> 5120 product 19 / 29 us at 64 / 128 rows against a flat 18.5 us.
+// Streaming kernel for a few rows (project_small.hip); from 65 rows on one 128-token tile per head
+// (project_mid.hip) runs.
 constexpr uint32_t kSmallRowsMax = 64;
-hipError_t small_prepare();
 bool small_kernel_takes(uint32_t rows, uint32_t K);
-size_t small_workspace_floats(uint32_t heads, uint32_t K);
-// mode: kModeQkv, kModeAdd or kModeRaw
-hipError_t launch_project_small(const ProjectKernelArgs& p, float* ws, uint32_t* counters, int dtype,
-                                int mode, hipStream_t stream);
+// mode: kModeQkv, kModeAdd or kModeRaw; ws: kSmallRowsMax floats per column, counters: one per head
+hipError_t launch_project_small(const ProjectKernelArgs& p, float* ws, uint32_t* counters, uint32_t n_cu, int dtype,
+                                 int mode, hipStream_t stream);
 
 // Tile kernel with 128-token x one-head tiles (project_mid.hip), for row counts at which
 // the 256 x 256 tiles are fewer than the compute units.

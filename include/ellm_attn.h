@@ -510,8 +510,7 @@ int ellm_matmul3_reset(ellm_matmul3* handle, void* stream);
  * The handles must describe the same step: proj's q_state / k_state / v_state are attn's
  * q / k / v, same dtype, head counts, batch_size, kv_strides, sequence_capacity and (for caches
  * with per-sequence capacities) the same sequence table; else ELLM_ERR_INVALID_ARGUMENT.
- * Shapes the fused form does not take (more than 64 sequences, hidden_size not a multiple of
- * 256 or below 1024) run the two ordinary calls: same results.  ellm_matmul3_attn_path tells
+ * Shapes the fused form does not take (more than 64 sequences, hidden_size below 1024) run the two ordinary calls: same results.  ellm_matmul3_attn_path tells
  * which (1 fused, 0 two ordinary calls, negative: a status).  Neither handle may have
  * another call in flight.
  */
