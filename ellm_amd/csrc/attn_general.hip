@@ -63,7 +63,7 @@ hipError_t launch_merge(const GeneralArgs& p, uint32_t planes, uint32_t pitch, h
   const size_t items = (size_t)planes * p.rows * (pitch / 4);
   auto go = [&](auto kernel, size_t lanes) {
     hipLaunchKernelGGL(kernel, dim3((uint32_t)((items * lanes + 255) / 256)), dim3(256), 0, stream, p, planes, pitch,
-                       (uint32_t)kGeneralTileRows);
+                       p.tile_rows);
     return hipGetLastError();
   };
   if (p.n_split > 8 && items * 8 <= ((size_t)1 << 21)) return go(general_merge_kernel<S, VEC, 8>, 8);
@@ -148,18 +148,35 @@ hipError_t launch_attn_general(const AttnArgs& a, uint32_t head_size, hipStream_
     return gen::launch_general_step(p, a.dtype, nb, vec, planes, stream);
   }
 
-  p.row_tiles = (uint32_t)((rows + gen::kGeneralTileRows - 1) / gen::kGeneralTileRows);
+  const bool f32 = a.dtype == 2;
+  auto tiles_of = [&](size_t n) { return (rows + n - 1) / n; };
+  // Key groups put more waves on a row's keys: 64 rows and four groups while all workgroups find a
+  // unit of their own (131 tokens on 378, 32 / 8 heads of 64: 15.2 -> 9.7 us), else 128 rows.  With
+  // more workgroups than units, heads of 65 to 128 elements keep two small workgroups a unit, whose
+  // starts and ends overlap (408 tokens x 4 on 152, 32 / 32 heads of 96: 26 us, 32 with two groups);
+  // heads up to 64 leave room for two workgroups of two groups, and wider ones have one wave per SIMD
+  // without them.  Up to 128 keys there is nothing to share (21 tokens: 5.8 against 6.2 us).
+  p.tile_rows = 128;
+  p.key_groups = 1;
+  if (max_len > 128) {
+    if (gen::chunk_key_groups(f32, nb, 2) > 1 && planes * tiles_of(64) <= a.n_cu) p.tile_rows = 64;
+    const bool one_each = planes * tiles_of(p.tile_rows) <= a.n_cu;
+    if (one_each || nb <= 2 || nb > 4) p.key_groups = (uint32_t)gen::chunk_key_groups(f32, nb, p.tile_rows / 32);
+  }
+  p.row_tiles = (uint32_t)tiles_of(p.tile_rows);
   if ((size_t)planes * p.row_tiles > 0x7fffffffu) return hipErrorInvalidValue;
   const uint32_t items = planes * p.row_tiles;
   const uint32_t tiles = (max_len + 63) / 64;
   p.n_split = 1;
   p.split_len = tiles * 64;
-  const uint32_t slots = (es == 2 && nb <= 4 ? 2 : 1) * a.n_cu;
-  // too few workgroups to fill the part: split the key range, in pieces of at least 256 keys
+  p.turn_at = items <= 2 * a.n_cu && planes <= a.n_cu ? a.n_cu / planes : p.row_tiles;
+  // too few workgroups to fill the part: split the key range, in pieces of at least 512 keys or, four
+  // waves a workgroup, 256
+  const uint32_t slots = (es == 2 && nb <= 4 && p.key_groups == 1 ? 2 : 1) * a.n_cu;
   if (2 * (size_t)items <= slots && tiles >= 8 && room > 1) {
     const double tile_us = (es == 4 ? 1.7 : 0.5) * nb;
     const double split_us = (double)planes * rows * (32 * nb + 2) * 8 / 4e6;
-    const KeySplit ks = plan_key_split(tiles, items, slots, 4, (uint32_t)(room < 4096 ? room : 4096), split_us / tile_us);
+    const KeySplit ks = plan_key_split(tiles, items, slots, p.key_groups > 1 ? 8 : 4, (uint32_t)(room < 4096 ? room : 4096), split_us / tile_us);
     if (ks.n_split > 1) {
       p.n_split = ks.n_split;
       p.split_len = ks.split_tiles * 64;

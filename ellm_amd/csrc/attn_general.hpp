@@ -12,7 +12,6 @@ namespace ellm {
 namespace gen {
 
 constexpr int kMaxHead = 256;
-constexpr uint32_t kGeneralTileRows = 128;   // query rows of a workgroup of the chunk kernel
 constexpr uint32_t kGeneralStepRows = 16;    // and of the step kernel
 
 struct F32 {};   // binary32 storage
@@ -76,6 +75,9 @@ struct GeneralArgs {
   // part_ml [..][2] (reference exponent in log2 units, denominator).
   uint32_t n_split, split_len;
   uint32_t row_tiles;            // workgroups along the rows of a plane
+  uint32_t tile_rows;            // query rows of a workgroup of the chunk kernel (64 or 128)
+  uint32_t turn_at;              // ... and the row tile of the launch (longest first) from which the order turns
+  uint32_t key_groups;           // groups of waves that share the keys of those rows
   float* part_o;
   float* part_ml;
   uint32_t* counters;            // arrivals per (plane, row tile); zero between launches
@@ -261,6 +263,14 @@ inline int head_blocks(uint32_t head_size, bool vec) {
   const int n = (int)((head_size + 31) / 32);
   if (!vec) return n <= 2 ? 2 : n <= 4 ? 4 : 8;
   return n <= 4 ? n : n <= 6 ? 6 : 8;
+}
+
+// Key groups of a chunk kernel's workgroup of `row_blocks` x 32 query rows: as many as its registers (a
+// wave's queries, accumulators and scores) and LDS (two steps of K and V a group) allow.
+constexpr int chunk_key_groups(bool f32, int nb, int row_blocks) {
+  if (f32) return 1;
+  if (row_blocks == 4) return nb <= 6 ? 2 : 1;
+  return nb <= 4 ? 4 : 1;
 }
 
 // f(std::integral_constant<int, blocks>, std::bool_constant<vec>) for a value of head_blocks().

@@ -3,43 +3,53 @@
 // lane owns one query row, online soft-max in binary32) on 32x32 matrix tiles, templated over the
 // storage type and the padded head size.
 //
-// Four waves of 32 rows share every key step of 32 or 64 keys through LDS (double-buffered, one
-// barrier a step, the next step's rows in registers meanwhile); rows are the (token, head) pairs of a
-// GQA group in order, so a group's heads share the K/V rows whatever the group size.  What bounds it:
-// 16-bit, the vector instructions of the soft-max (twelve a pair of scores, two of them quarter-rate
-// exponentials) beside 6 x 32 matrix cycles per 16 keys and 32 elements; binary32, the matrix pipe
-// (256 flops a cycle and unit).  Two or three workgroups a unit overlap the one with the other.
-// Measured: 2048 tokens, 32 query / 8 key-value heads of 64, bfloat16: 46.5 us (370 TFLOP/s), where one
-// workgroup per query row without matrix instructions took 4360 us; 1019 tokens, 32 / 4 heads of 256,
-// binary16: 80 us (was 2103); 433 tokens x 2 on 369, 32 / 32 heads of 128, binary32: 124 us (was 1127).
+// A key group is two or four waves of 32 rows that share steps of 32 or 64 keys through LDS
+// (double-buffered, one barrier a step, the next step's rows in registers meanwhile); up to four groups
+// take the steps of the same rows in turn and merge their rows in LDS at the end.  Rows are the
+// (token, head) pairs of a GQA group in order, so a group's heads share the K/V rows whatever the
+// group size.  What bounds it: 16-bit, the vector instructions of the soft-max (13 a pair of scores,
+// two of them quarter-rate exponentials; 7 matrix cycles beside them with heads of 64), and one
+// wave issues a vector instruction only every six cycles or so, so that a SIMD wants several waves:
+// two, from two groups or two workgroups, are the least, four the best where registers allow.
+// Groups that take turns at a step's matrix and vector parts, as the 128-wide tile kernel's do, came out
+// slower than groups side by side (a lone wave's vector part is 1.5 x as long as a shared one).
+// Binary32 is bound by the matrix pipe (256 flops a cycle and unit) and keeps one group.
+// Measured, one group before: 2048 tokens, 32 query / 8 key-value heads of 64, bfloat16: 46.0 -> 41.9 us
+// (410 TFLOP/s); 341 tokens, 32 / 32 heads of 96: 16.2 -> 10.2; 603 tokens x 2, 32 / 4 heads of 192: 40.6 -> 29.1.
+// Binary16 heads of 256 (one group: no registers for two): 1019 tokens, 32 / 4 heads 80 us.
 #include "attn_general.hpp"
 
 namespace ellm {
 namespace gen {
 namespace {
 
-constexpr int kWaves = 4;
-constexpr int kThreads = kWaves * kWave;
-constexpr int kTileRows = 32 * kWaves;   // query rows of a workgroup
-static_assert(kTileRows == (int)kGeneralTileRows, "the merge derives a row's live splits from its workgroup's last row");
 constexpr float kRescaleStep = 8.0f;     // log2 units
 
 typedef __attribute__((address_space(3))) uint8_t LdsByte;
 typedef __attribute__((address_space(3))) u32x4 LdsU32x4;
 typedef __attribute__((address_space(3))) float LdsF32;
+typedef __attribute__((address_space(3))) f32x4 LdsF32x4;
+typedef __attribute__((address_space(3))) f32x2 LdsF32x2;
 typedef short i16x4 __attribute__((ext_vector_type(4)));
 typedef __attribute__((address_space(3))) i16x4 LdsI16x4;
 
-// Shape of a kernel: NB blocks of 32 head elements, MB blocks of 32 keys per step.
-template <typename S, int NB>
+// Shape of a kernel: NB blocks of 32 head elements, RB row blocks (waves) of a key group, KG key
+// groups, MB blocks of 32 keys a step of a group.
+template <typename S, int NB, int RB, int KG>
 struct Shape {
   static constexpr bool kF32 = std::is_same<S, F32>::value;
   static constexpr int kBytes = sizeof(typename Store<S>::E);
   static constexpr int kHead = 32 * NB;
   static constexpr int kPiecesRow = kHead * kBytes / 16;
-  static constexpr int MB = (!kF32 && NB <= 4) ? 2 : 1;
+  static constexpr int kWaves = RB * KG, kThreads = kWaves * kWave;
+  static constexpr int kGroupThreads = RB * kWave;
+  static constexpr int kTileRows = 32 * RB;  // query rows of a workgroup
+  static constexpr int MB = (!kF32 && NB <= 4 && KG <= 2 && !(NB == 2 && KG == 2)) ? 2 : 1;
   static constexpr int kKeys = 32 * MB;
-  static constexpr int kPieces = kKeys * kPiecesRow / kThreads;   // 16-byte pieces of K (and of V) a thread moves per step
+  // 16-byte pieces of K (and of V) a thread moves per step, the last one of some threads none
+  static constexpr int kAllPieces = kKeys * kPiecesRow;
+  static constexpr int kPieces = (kAllPieces + kGroupThreads - 1) / kGroupThreads;
+  static constexpr bool kEven = kPieces * kGroupThreads == kAllPieces;
   // Row pitches in LDS, bytes.  K rows are read 16 bytes a lane from 32 rows: a pitch of 4 x odd
   // words spreads 16 of them over all banks.  V rows, 16-bit: a 16-lane block of the transposing read
   // takes 32 bytes from each of four rows and its neighbour the next 32, so four rows 16 x odd words
@@ -49,30 +59,43 @@ struct Shape {
   static constexpr int kVWords = kHead * kBytes / 4;
   static constexpr int kVPitch = 4 * (kF32 ? kVWords + 8 : (kVWords % 32 == 16 ? kVWords : kVWords + 16));
   static constexpr int kKBuf = kKeys * kKPitch, kVBuf = kKeys * kVPitch;
-  static constexpr int kLds = 2 * (kKBuf + kVBuf);
+  static constexpr int kGroupLds = 2 * (kKBuf + kVBuf);
+  // The groups' results meet in the same memory, up to half of them at a time: a wave's
+  // accumulators and, behind all of those, its rows' maxima and sums.
+  static constexpr int kMergeWave = NB * 16 * kWave * 4;
+  static constexpr int kMergeLds = KG / 2 * RB * (kMergeWave + 2 * kWave * 4);
+  static constexpr int kLds = KG * kGroupLds > kMergeLds ? KG * kGroupLds : kMergeLds;
+  static_assert(kLds + 16 <= 160 * 1024, "LDS of a compute unit");
   // Waves per SIMD the registers are planned for: queries, accumulators, scores, weights and the
   // pieces on their way to LDS are about 40 (32 x 32 x head / 64) registers and a few dozen more.
+  // Heads of 64 with two groups take steps of 32 keys to fit twice on a unit.
   // Binary32 heads of 256 have no registers left to hold the next V rows during a step: those are
   // requested behind it (a step is 16384 matrix cycles there).
   static constexpr bool kLateV = kF32 && NB == 8;
-  static constexpr int kOccupancy = kF32 ? (NB <= 2 ? 2 : 1) : NB <= 2 ? 3 : NB <= 4 ? 2 : 1;
+  static constexpr int kOccupancy = KG == 2 && NB <= 2 ? 4 : KG > 1 ? kWaves / 4 : kF32 ? (NB <= 2 ? 2 : 1) : NB <= 2 ? 3 : NB <= 4 ? 2 : 1;
 };
 
-template <typename S, int NB, bool VEC>
-__global__ __launch_bounds__(kThreads, (Shape<S, NB>::kOccupancy)) void general_chunk_kernel(GeneralArgs p) {
-  typedef Shape<S, NB> X;
+template <typename S, int NB, bool VEC, int RB, int KG>
+__global__ __launch_bounds__((Shape<S, NB, RB, KG>::kThreads), (Shape<S, NB, RB, KG>::kOccupancy))
+void general_chunk_kernel(GeneralArgs p) {
+  typedef Shape<S, NB, RB, KG> X;
   typedef typename Store<S>::E E;
-  constexpr int MB = X::MB, kKeys = X::kKeys, kPieces = X::kPieces;
+  constexpr int MB = X::MB, kKeys = X::kKeys, kPieces = X::kPieces, kTileRows = X::kTileRows;
   constexpr int kQ = X::kPiecesRow / 2;      // query registers: pieces 2 s + g of the row
   constexpr float kShift = Store<S>::kShift;
   __shared__ __attribute__((aligned(16))) uint8_t smem[X::kLds];
   __shared__ uint32_t s_bad;                 // a value beyond the first row's position is not finite
 
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int tid = threadIdx.x % X::kGroupThreads, lane = tid & 63, wave = tid >> 6;   // within the key group
+  const uint32_t kg = KG == 1 ? 0u : (uint32_t)__builtin_amdgcn_readfirstlane((int)(threadIdx.x / X::kGroupThreads));
   const int j = lane & 31, g = lane >> 5;
   const uint32_t planes = gridDim.x / p.row_tiles;
   const uint32_t plane = blockIdx.x % planes;
-  const uint32_t tile = p.row_tiles - 1 - blockIdx.x / planes;   // longest rows first
+  // longest rows first; the second workgroup of every unit, where two are resident and there are no
+  // more, in the opposite order, so that the unit with the longest gets the shortest
+  uint32_t order = blockIdx.x / planes;
+  if (order >= p.turn_at) order = p.row_tiles - 1 - (order - p.turn_at);
+  const uint32_t tile = p.row_tiles - 1 - order;
   const uint32_t seq = plane / p.n_kv_heads, kvh = plane % p.n_kv_heads;
   const uint32_t P0 = start_position(p, seq);
   const uint32_t row0 = tile * kTileRows;
@@ -107,13 +130,14 @@ __global__ __launch_bounds__(kThreads, (Shape<S, NB>::kOccupancy)) void general_
   const uint64_t kplane = scalar64((uint64_t)kp), vplane = scalar64((uint64_t)vp);
   const uint64_t pos_bytes = (uint64_t)p.kv_stride_pos * sizeof(E);
   const uint64_t valid = scalar64((uint64_t)(end - 1) * pos_bytes + (uint64_t)p.head_size * sizeof(E));
+  const bool has_last = tid + X::kGroupThreads * (kPieces - 1) < X::kAllPieces;
   uint32_t off[kPieces], lds_k[kPieces], lds_v[kPieces];
-  const uint32_t lds0 = (uint32_t)(uintptr_t)(LdsByte*)smem;
+  const uint32_t lds_all = (uint32_t)(uintptr_t)(LdsByte*)smem, lds0 = lds_all + kg * X::kGroupLds;
 #pragma unroll
   for (int i = 0; i < kPieces; ++i) {
-    const uint32_t pi = tid + kThreads * i, krow = pi / X::kPiecesRow, col = pi % X::kPiecesRow;
+    const uint32_t pi = tid + X::kGroupThreads * i, krow = pi / X::kPiecesRow, col = pi % X::kPiecesRow;
     if constexpr (VEC)
-      off[i] = col * Store<S>::kPiece < p.head_size ? (uint32_t)(krow * pos_bytes) + 16 * col : kNowhere;
+      off[i] = col * Store<S>::kPiece < p.head_size && krow < (uint32_t)kKeys ? (uint32_t)(krow * pos_bytes) + 16 * col : kNowhere;
     else
       off[i] = krow | col * Store<S>::kPiece << 16;
     lds_k[i] = lds0 + krow * X::kKPitch + 16 * col;
@@ -136,20 +160,25 @@ __global__ __launch_bounds__(kThreads, (Shape<S, NB>::kOccupancy)) void general_
     load_rows(step, kp, kplane, kst);
     if constexpr (!X::kLateV) load_rows(step, vp, vplane, vst);
   };
-  auto store_step = [&](uint32_t step) {
-    const uint32_t buf = step & 1;
-    if constexpr (X::kLateV) load_rows(step, vp, vplane, vst);
+  auto store_rows = [&](uint32_t step, const u32x4 (&st)[kPieces], const uint32_t (&at)[kPieces], int bytes)
+      __attribute__((always_inline)) {
 #pragma unroll
-    for (int i = 0; i < kPieces; ++i) {
-      *(LdsU32x4*)(lds_k[i] + buf * X::kKBuf) = kst[i];
-      *(LdsU32x4*)(lds_v[i] + buf * X::kVBuf) = vst[i];
-    }
+    for (int i = 0; i < kPieces; ++i)
+      if (X::kEven || i + 1 < kPieces || has_last) *(LdsU32x4*)(at[i] + (step / KG & 1) * bytes) = st[i];
+  };
+  auto look_at = [&](uint32_t step) {
     if (k0 + step * kKeys + kKeys - 1 > first_pos) {   // some row of the workgroup must not see some of these values
       bool bad = false;
 #pragma unroll
       for (int i = 0; i < kPieces; ++i) bad |= piece_not_finite<S>(vst[i]);
       if (bad) s_bad = 1;
     }
+  };
+  auto store_step = [&](uint32_t step) {
+    if constexpr (X::kLateV) load_rows(step, vp, vplane, vst);
+    store_rows(step, kst, lds_k, X::kKBuf);
+    store_rows(step, vst, lds_v, X::kVBuf);
+    look_at(step);
   };
 
   float m_run = -INFINITY, l_run = 0.0f;
@@ -168,8 +197,8 @@ __global__ __launch_bounds__(kThreads, (Shape<S, NB>::kOccupancy)) void general_
                                         2 * (16 * ((lane >> 4) & 1) + 4 * (lane & 3));
 
   auto compute = [&](uint32_t step) __attribute__((always_inline)) {
-    const uint32_t kb = k0 + step * kKeys, buf = step & 1;
-    if (!wave_has_rows || kb > wave_last) return;
+    const uint32_t kb = k0 + step * kKeys, buf = step / KG & 1;
+    if (step >= n_steps || !wave_has_rows || kb > wave_last) return;
     const uint32_t ks = k_read + buf * X::kKBuf, vs = v_read + buf * X::kVBuf;
     f32x16 st[MB];
 #pragma unroll
@@ -262,28 +291,67 @@ __global__ __launch_bounds__(kThreads, (Shape<S, NB>::kOccupancy)) void general_
     l_run += psum;
   };
 
-  if (tid == 0) s_bad = 0;
-  load_step(0);
+  // step s of the keys belongs to group s mod KG; every group passes every barrier
+  if (threadIdx.x == 0) s_bad = 0;
+  if (kg < n_steps) load_step(kg);
   __syncthreads();
-  store_step(0);
-  if (n_steps > 1) load_step(1);
+  if (kg < n_steps) store_step(kg);
+  if (kg + KG < n_steps) load_step(kg + KG);
   __syncthreads();
-  for (uint32_t step = 0; step < n_steps; ++step) {
+  for (uint32_t first = 0; first < n_steps; first += KG) {
+    const uint32_t step = first + kg;
     compute(step);
-    if (step + 1 < n_steps) {
-      store_step(step + 1);
-      if (step + 2 < n_steps) load_step(step + 2);
+    if (step + KG < n_steps) {
+      store_step(step + KG);
+      if (step + 2 * KG < n_steps) load_step(step + 2 * KG);
     }
     __syncthreads();
   }
 
   const size_t part_row0 = (size_t)plane * p.rows;
   if (s_bad) {   // (uniform: the last barrier is behind every write of it)
-    for (uint32_t rr = row0 + wave; rr <= last_row; rr += kWaves)
+    for (uint32_t rr = row0 + threadIdx.x / kWave; rr <= last_row; rr += X::kWaves)
       plain_row<S>(p, kp, vp, query_row(p, seq, kvh, rr), (part_row0 + rr) * p.n_split + blockIdx.y, k0,
                    min(end, P0 + rr / p.group + 1), X::kHead, p.n_split > 1);
     return;
   }
+  // the groups' rows: the upper half of the groups hands its own over, until one group is left
+#pragma unroll
+  for (int groups = KG; groups > 1; groups = (groups + 1) / 2) {
+    const uint32_t half = (groups + 1) / 2, pairs = groups - half;
+    const bool gives = kg >= half && kg < (uint32_t)groups, takes = kg < pairs;
+    const uint32_t slot = (gives ? kg - half : kg) * RB + wave;
+    const uint32_t at = lds_all + slot * X::kMergeWave + 16 * lane;
+    const uint32_t ml = lds_all + pairs * RB * X::kMergeWave + slot * (2 * kWave * 4) + 8 * lane;
+    if (gives) {
+#pragma unroll
+      for (int db = 0; db < NB; ++db)
+#pragma unroll
+        for (int q4 = 0; q4 < 4; ++q4)
+          *(LdsF32x4*)(at + (4 * db + q4) * (16 * kWave)) =
+              f32x4{oacc[db][4 * q4], oacc[db][4 * q4 + 1], oacc[db][4 * q4 + 2], oacc[db][4 * q4 + 3]};
+      *(LdsF32x2*)ml = f32x2{m_run, l_run};
+    }
+    __syncthreads();
+    if (takes) {
+      const f32x2 other = *(const LdsF32x2*)ml;
+      const float m_new = fmaxf(m_run, other[0]);
+      const float wa = m_run == -INFINITY ? 0.0f : fast_exp2(m_run - m_new);
+      const float wb = other[0] == -INFINITY ? 0.0f : fast_exp2(other[0] - m_new);
+      m_run = m_new;
+      l_run = l_run * wa + other[1] * wb;
+#pragma unroll
+      for (int db = 0; db < NB; ++db)
+#pragma unroll
+        for (int q4 = 0; q4 < 4; ++q4) {
+          const f32x4 o = *(const LdsF32x4*)(at + (4 * db + q4) * (16 * kWave));
+#pragma unroll
+          for (int e = 0; e < 4; ++e) oacc[db][4 * q4 + e] = oacc[db][4 * q4 + e] * wa + o[e] * wb;
+        }
+    }
+    if (groups > 2) __syncthreads();
+  }
+  if (KG > 1 && kg != 0) return;
   const float l = sum_with_partner_half(l_run);
   if (!row_valid) return;
   if (p.n_split > 1) {
@@ -312,17 +380,28 @@ __global__ __launch_bounds__(kThreads, (Shape<S, NB>::kOccupancy)) void general_
 }  // namespace
 
 hipError_t launch_general_chunk(const GeneralArgs& p, int dtype, int nb, bool vec, uint32_t planes, hipStream_t stream) {
-  const dim3 grid(planes * p.row_tiles, p.n_split), block(kThreads);
+  const dim3 grid(planes * p.row_tiles, p.n_split);
   return with_head_blocks(nb, vec, [&](auto n, auto v) {
     constexpr int NB = decltype(n)::value;
     constexpr bool VEC = decltype(v)::value;
-    if (dtype == 0)
-      hipLaunchKernelGGL((general_chunk_kernel<F16, NB, VEC>), grid, block, 0, stream, p);
-    else if (dtype == 1)
-      hipLaunchKernelGGL((general_chunk_kernel<BF16, NB, VEC>), grid, block, 0, stream, p);
-    else
-      hipLaunchKernelGGL((general_chunk_kernel<F32, NB, VEC>), grid, block, 0, stream, p);
-    return hipGetLastError();
+    auto go = [&](auto storage) {
+      typedef decltype(storage) S;
+      constexpr int kLong = chunk_key_groups(std::is_same<S, F32>::value, NB, 4);
+      constexpr int kShort = chunk_key_groups(std::is_same<S, F32>::value, NB, 2);
+      if constexpr (kShort > 1)
+        if (p.tile_rows == 64) {
+          hipLaunchKernelGGL((general_chunk_kernel<S, NB, VEC, 2, kShort>), grid, dim3(128 * kShort), 0, stream, p);
+          return hipGetLastError();
+        }
+      if constexpr (kLong > 1)
+        if (p.key_groups > 1) {
+          hipLaunchKernelGGL((general_chunk_kernel<S, NB, VEC, 4, kLong>), grid, dim3(256 * kLong), 0, stream, p);
+          return hipGetLastError();
+        }
+      hipLaunchKernelGGL((general_chunk_kernel<S, NB, VEC, 4, 1>), grid, dim3(256), 0, stream, p);
+      return hipGetLastError();
+    };
+    return dtype == 0 ? go(F16{}) : dtype == 1 ? go(BF16{}) : go(F32{});
   });
 }
 

@@ -24,6 +24,16 @@ CASES = [
     ("f32_h64_key_split", orc.F32, 1, 8, 2, 64, 1500, 1400, 40),
     ("f32_h256", orc.F32, 1, 2, 1, 256, 130, 20, 60),
     ("f32_h96_three_tiles", orc.F32, 1, 3, 1, 96, 140, 20, 100),
+    ("h64_four_groups_of_64_rows", orc.BF16, 1, 4, 1, 64, 300, 100, 80),
+    ("h96_four_groups_last_steps_uneven", orc.F16, 1, 2, 1, 96, 200, 70, 63),
+    ("h32_four_groups_three_steps", orc.F16, 1, 2, 2, 32, 140, 60, 70),
+    ("h120_four_groups", orc.F16, 1, 3, 1, 120, 290, 150, 90),
+    ("h64_two_groups_two_a_unit", orc.F16, 5, 64, 64, 64, 200, 10, 129),
+    ("h80_two_groups", orc.BF16, 3, 64, 64, 80, 200, 30, 131),
+    ("h96_more_than_one_a_unit", orc.BF16, 5, 64, 64, 96, 180, 0, 135),
+    ("h160_two_groups_one_step_left", orc.F16, 2, 4, 2, 160, 165, 0, 161),
+    ("h64_order_turns", orc.BF16, 4, 32, 32, 64, 390, 0, 385),
+    ("h64_four_groups_key_split", orc.F16, 1, 4, 1, 64, 1700, 1600, 40),
     ("h33_elements_one_by_one", orc.F16, 2, 4, 2, 33, 180, 30, 50),
     ("f32_h130_elements_one_by_one", orc.F32, 1, 4, 1, 130, 100, 3, 40),
     ("step_group_17", orc.F16, 1, 17, 1, 64, 400, 399, 1),
