@@ -23,7 +23,7 @@
 // chunk c + 1, fetched into registers an iteration earlier, is written to the other stage.
 // Calls with at most 64 rows go to the streaming kernel of project_small.hip, calls that would
 // leave these tiles fewer than the compute units to the 128-token tiles of project_mid.hip.
-#include "project_epilogue.hpp"
+#include "project_mid_tile.hpp"
 
 namespace ellm {
 using namespace proj;
@@ -39,8 +39,9 @@ constexpr int kRowPitch = kKc * 2;
 constexpr int kStageBytes = 2 * kTile * kRowPitch;  // X rows then W rows
 constexpr int kStages = 2;
 constexpr int kProjThreads = 256;
-constexpr int kProjLdsBytes = kStages * kStageBytes;
-static_assert(4 * kEpWaveBytes <= kProjLdsBytes, "the epilogue reuses the stages");
+constexpr int kProjLdsBytes = MidShape<2, 4>::kLdsBytes;   // the most of the three forms of a workgroup
+static_assert(kStages * kStageBytes <= kProjLdsBytes && MidShape<1, 4>::kLdsBytes <= kProjLdsBytes, "forms of a workgroup");
+static_assert(4 * kEpWaveBytes <= kStages * kStageBytes, "the epilogue reuses the stages");
 constexpr int kGroupM = 4;                          // token tiles that take turns on one column tile
 
 
@@ -53,12 +54,20 @@ __global__ __launch_bounds__(kProjThreads) void project_kernel(ProjectKernelArgs
   const int wn = wave & 1, wm = wave >> 1;
 
   // workgroup -> tile: ids that share id % 8 (one XCD, one L2) are made consecutive,
-  // then kGroupM token tiles x all column tiles form a band that is walked token-first
-  uint32_t tm, tn;
+  // then kGroupM token tiles x all column tiles form a band that is walked token-first;
+  // the tiles past whole_tiles (a multiple of the compute units, or all) go to tail_parts
+  // workgroups each, likewise consecutive per XCD
+  const bool whole = blockIdx.x < p.whole_tiles;
+  uint32_t tm, tn, part = 0;
   {
-    const uint32_t total = p.tiles_m * p.tiles_n;
-    const uint32_t q = total >> 3, r = total & 7, xcd = blockIdx.x & 7, idx = blockIdx.x >> 3;
-    const uint32_t pid = xcd * q + min(xcd, r) + idx;
+    const uint32_t total = whole ? p.whole_tiles : (p.tiles_m * p.tiles_n - p.whole_tiles) * p.tail_parts;
+    const uint32_t id = whole ? blockIdx.x : blockIdx.x - p.whole_tiles;
+    const uint32_t q = total >> 3, r = total & 7, xcd = id & 7, idx = id >> 3;
+    uint32_t pid = xcd * q + min(xcd, r) + idx;
+    if (!whole) {
+      part = pid % p.tail_parts;
+      pid = p.whole_tiles + pid / p.tail_parts;
+    }
     const uint32_t per_band = kGroupM * p.tiles_n;
     const uint32_t band = pid / per_band, in_band = pid % per_band;
     const uint32_t first_m = band * kGroupM;
@@ -67,6 +76,15 @@ __global__ __launch_bounds__(kProjThreads) void project_kernel(ProjectKernelArgs
     tn = in_band / band_m;
   }
   const uint32_t heads_total = p.heads0 + 2 * p.heads_kv;
+  if (!whole) {   // one head of the tile, all of its tokens or half of them
+    const uint32_t hh = 2 * tn + (part & 1), first = tm * kTile + (part >> 1) * (kTile / 2);
+    if (hh >= heads_total || first >= p.rows) return;
+    if (p.tail_parts == 2)
+      mid_tile<S, MODE, 2, 4>(p, first, hh, proj_smem);
+    else
+      mid_tile<S, MODE, 1, 4>(p, first, hh, proj_smem);
+    return;
+  }
   const uint32_t K = p.K;
   const uint32_t n_chunks = K / kKc;
 
@@ -278,7 +296,21 @@ hipError_t launch_project(const ProjectArgs& a, hipStream_t stream) {
     return launch_project_small(p, a.ws, a.counters, g_n_cu, a.dtype, a.residual ? kModeAdd : kModeQkv, stream);
   if (path == kPathTiles128 || path == kPathTiles256x1)
     return launch_project_mid(p, path == kPathTiles128 ? 1 : 2, a.dtype, a.residual != nullptr, stream);
-  const uint32_t blocks = p.tiles_m * p.tiles_n;
+  // A last round of tiles that would leave half of the compute units without one, or three
+  // quarters, is cut into halves (256 tokens x one head) or quarters (128 x one head), one per unit:
+  // a half takes 0.6 of a tile's time, a quarter 0.4, and what reads more of the L2 lines per flop
+  // runs only where units would idle.  Attention block of a layer, whole tiles -> cut (us): 8000 tokens
+  // 2048 wide, 32 / 4 heads (640 tiles, 128 cut) 741 -> 731; 4300 tokens (340 tiles) 348 -> 335; 1800
+  // tokens 8192 wide, 64 / 8 heads (320 tiles) 619 -> 538; 3300 tokens (520 and 416 tiles) 1155 -> 1089.
+  // More than half a round stays whole: its halves would need two rounds of 0.6.
+  const uint32_t tiles = p.tiles_m * p.tiles_n, last = tiles % g_n_cu;
+  p.whole_tiles = tiles;
+  p.tail_parts = 1;
+  if (tiles > g_n_cu && last && 2 * last <= g_n_cu) {
+    p.whole_tiles = tiles - last;
+    p.tail_parts = 4 * last <= g_n_cu ? 4 : 2;
+  }
+  const uint32_t blocks = p.whole_tiles + (tiles - p.whole_tiles) * p.tail_parts;
   auto go = [&](auto kernel) {
     hipLaunchKernelGGL(kernel, dim3(blocks), dim3(kProjThreads), kProjLdsBytes, stream, p);
     return hipGetLastError();

@@ -555,7 +555,7 @@ int ellm_matmul_add_reset(ellm_matmul_add* handle, void* stream);
  * of 128 (attention_head_num + 2 * kv_head_num, or n / 128) and inner size k runs on the
  * current device: 0 = the weight-streaming kernel for at most 64 rows, 1 = MFMA tiles of
  * 128 tokens x one head, 2 = tiles of 256 tokens x one head, 3 = tiles of 256 tokens x two
- * heads; -1 for sizes no handle accepts.  No
+ * heads (a mostly empty last round as one-head tiles); -1 for sizes no handle accepts.  No
  * counterpart in the reference (its MatMul3::run has one code path); it lets a test or a
  * harness see that its shapes reach every kernel.
  */

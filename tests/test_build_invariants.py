@@ -35,6 +35,15 @@ def test_one_head_tile_kernels_leave_m0_to_the_inline_asm(tmp_path):
     assert not any("movrel" in l or "s_set_gpr_idx" in l for l in code)
 
 
+def test_tile_kernel_leaves_m0_to_the_inline_asm(tmp_path):
+    """The same for project.hip, whose last round runs the one-head tile."""
+    text = _listing("project.hip", tmp_path)
+    code = [l.split(";")[0] for l in text.splitlines()]
+    uses = [l for l in code if re.search(r"\bm0\b", l)]
+    assert uses and all(re.fullmatch(r"\s*s_mov_b32 m0, s\d+\s*", l) for l in uses)
+    assert not any("movrel" in l or "s_set_gpr_idx" in l for l in code)
+
+
 @pytest.mark.parametrize("name", ["project.hip", "project_mid.hip", "project_small.hip", "prefill.hip", "decode.hip",
                                   "decode_balanced.hip", "kv_cache.hip"])
 def test_hot_kernels_do_not_spill(name, tmp_path):
