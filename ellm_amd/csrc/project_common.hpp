@@ -30,6 +30,7 @@ struct ProjectKernelArgs {
   uint32_t heads0, heads_kv;
   uint32_t tiles_m, tiles_n;
   uint32_t whole_tiles, tail_parts;   // project_kernel: tiles of 256 x 256; workgroups per tile of the rest
+  uint32_t band_m;                    // project_mid_kernel: token tiles that take turns on one head
   uint32_t position_index, max_start;
   uint32_t finalize0;        // segment 0 rows are normalised and rotated
   float eps;

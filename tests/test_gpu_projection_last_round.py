@@ -1,5 +1,5 @@
 """The 256 x 256 projection tiles whose last round is cut into halves (256 tokens x one head) or
-quarters (128 tokens x one head).  Same oracle and bound as tests/test_gpu_projection.py."""
+quarters (128 tokens x one head), and one-head tiles walked in bands.  Same oracle and bound as tests/test_gpu_projection.py."""
 import pytest
 
 import oracle_lib as orc
@@ -63,5 +63,25 @@ def test_matmul_add_last_round(rows, k, heads, dtype, parts):
     op.run(0, rows, 1)
     torch.cuda.synchronize()
     res = compare_ulps(to_host(dr, dtype), orc.from_storage(orc.matmul_add(a, w, r, dtype, batch_size=1), dtype), dtype)
+    assert res["ok"], res
+    op.close()
+
+
+@pytest.mark.parametrize("rows,heads,path", [(1601, 16, 1), (3200, 17, 2), (3841, 16, 2)])   # 13 tiles in bands of 4, 4, 4, 1; 16 in bands of 4
+def test_matmul_add_bands(rows, heads, path):
+    import torch
+
+    import ellm_amd
+
+    assert _path(rows, heads, 64) == path
+    a = rand_storage((rows, 1, 64), 51, orc.F16)
+    w = rand_storage((heads * D, 64), 52, orc.F16, scale=0.125)
+    r = rand_storage((rows, 1, heads * D), 53, orc.F16)
+    da, dw, dr = to_dev(a, orc.F16), to_dev(w, orc.F16), to_dev(r, orc.F16)
+    out = torch.zeros_like(dr)
+    op = ellm_amd.MatMulAdd(da, dw, dr, out)
+    op.run(0, rows, 1)
+    torch.cuda.synchronize()
+    res = compare_ulps(to_host(out, orc.F16), orc.from_storage(orc.matmul_add(a, w, r, orc.F16, batch_size=1), orc.F16), orc.F16)
     assert res["ok"], res
     op.close()
