@@ -184,10 +184,6 @@ struct ellm_kv_cache {
 
 static hipError_t free_workspace(ellm_attn* h) {
   hipError_t first = hipSuccess;
-  if (h->general) {   // (parts of part_o)
-    h->part_ml = nullptr;
-    h->counters = nullptr;
-  }
   void* ptrs[] = {h->ws_acc, h->ws_ml, h->ws2_acc, h->ws2_ml, h->counters, h->part_o, h->part_ml};
   for (void* p : ptrs) {
     if (!p) continue;
@@ -276,13 +272,10 @@ static int attn_create(const ellm_attn_desc* d, const ellm_kv_seq_table* table, 
         (uint32_t)d->kv_head_num, (uint32_t)d->head_size, (uint32_t)n_cu);
     h->ws = ellm::DecodeWorkspace{0, 0, w.counters};
     h->part_rows = w.rows;
-    // one allocation: rows, their (max, sum) pairs, counters (26 us of a handle's creation; three took 37)
-    hipError_t e = hipMalloc((void**)&h->part_o, (w.rows * (w.pitch + 2) + w.counters) * sizeof(float));
-    if (e == hipSuccess) {
-      h->part_ml = h->part_o + w.rows * w.pitch;
-      h->counters = (uint32_t*)(h->part_ml + w.rows * 2);
-      e = hipMemset(h->counters, 0, w.counters * sizeof(uint32_t));
-    }
+    hipError_t e = hipMalloc((void**)&h->part_o, w.rows * w.pitch * sizeof(float));
+    if (e == hipSuccess) e = hipMalloc((void**)&h->part_ml, w.rows * 2 * sizeof(float));
+    if (e == hipSuccess) e = hipMalloc((void**)&h->counters, w.counters * sizeof(uint32_t));
+    if (e == hipSuccess) e = hipMemset(h->counters, 0, w.counters * sizeof(uint32_t));
     if (e != hipSuccess) {
       (void)free_workspace(h);
       delete h;
