@@ -206,20 +206,25 @@ void general_chunk_kernel(GeneralArgs p) {
 #pragma unroll
       for (int e = 0; e < 16; ++e) st[mb][e] = 0.0f;
     }
+    f32x16 st2;   // binary32: a second chain of sums, the odd pieces' (half the rounding steps in a row)
+#pragma unroll
+    for (int e = 0; e < 16; ++e) st2[e] = 0.0f;
 #pragma unroll
     for (int s = 0; s < kQ; ++s)
 #pragma unroll
       for (int mb = 0; mb < MB; ++mb) {
         const u32x4 a = *(const LdsU32x4*)(ks + 32 * mb * X::kKPitch + 32 * s);
         if constexpr (X::kF32) {
+          f32x16& sum = s & 1 ? st2 : st[mb];
 #pragma unroll
           for (int e = 0; e < 4; ++e)
-            st[mb] = __builtin_amdgcn_mfma_f32_32x32x2f32(__builtin_bit_cast(float, (uint32_t)a[e]),
-                                                          __builtin_bit_cast(float, (uint32_t)qreg[s][e]), st[mb], 0, 0, 0);
+            sum = __builtin_amdgcn_mfma_f32_32x32x2f32(__builtin_bit_cast(float, (uint32_t)a[e]),
+                                                       __builtin_bit_cast(float, (uint32_t)qreg[s][e]), sum, 0, 0, 0);
         } else {
           st[mb] = Mfma<S>::m32x32x16(a, qreg[s], st[mb]);
         }
       }
+    if constexpr (X::kF32) st[0] += st2;
     if (kb + kKeys - 1 > wave_first || kb + kKeys > end) {   // some pair of the step is masked
 #pragma unroll
       for (int mb = 0; mb < MB; ++mb)
@@ -253,13 +258,19 @@ void general_chunk_kernel(GeneralArgs p) {
         st[0][e] = fast_exp2(__builtin_fmaf(st[0][e], p.c, neg_m));
         psum += st[0][e];
       }
+      // a sum of its own per step: chains of 32 keys and of steps round less than one chain over all keys
 #pragma unroll
-      for (int e = 0; e < 16; ++e)
+      for (int db = 0; db < NB; ++db) {
+        f32x16 part;
 #pragma unroll
-        for (int db = 0; db < NB; ++db) {
+        for (int e = 0; e < 16; ++e) part[e] = 0.0f;
+#pragma unroll
+        for (int e = 0; e < 16; ++e) {
           const float a = *(const LdsF32*)(vs + (8 * (e >> 2) + (e & 3)) * X::kVPitch + 128 * db);
-          oacc[db] = __builtin_amdgcn_mfma_f32_32x32x2f32(a, st[0][e], oacc[db], 0, 0, 0);
+          part = __builtin_amdgcn_mfma_f32_32x32x2f32(a, st[0][e], part, 0, 0, 0);
         }
+        oacc[db] += part;
+      }
     } else {
       u32x4 hi[2 * MB], lo[2 * MB];
 #pragma unroll
