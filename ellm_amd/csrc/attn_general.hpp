@@ -164,6 +164,8 @@ __device__ __forceinline__ void store_agent(float* p, float v) {
   __hip_atomic_store((uint32_t*)p, __builtin_bit_cast(uint32_t, v), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
+__device__ __forceinline__ uint32_t lane_number() { return __builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, 0u)); }
+
 __device__ __forceinline__ float wave_sum(float v) {
 #pragma unroll
   for (int m = 32; m >= 1; m >>= 1) v += __shfl_xor(v, m);
@@ -181,7 +183,7 @@ __device__ __forceinline__ void plain_row(const GeneralArgs& p, const typename S
                                                      uint32_t k0, uint32_t end, uint32_t pitch, bool partial) {
   typedef typename Store<S>::E E;
   constexpr int kPerLane = kMaxHead / kWave;
-  const int lane = threadIdx.x & 63;
+  const int lane = (int)lane_number();
   const E* q = (const E*)p.q + row * p.head_size;
   float qv[kPerLane], o[kPerLane];
 #pragma unroll
@@ -250,6 +252,15 @@ template <typename S>
 __device__ __forceinline__ void split_pair(float p0, float p1, uint32_t& hi, uint32_t& lo) {
   hi = Mfma<S>::pack2(p0, p1);
   lo = Mfma<S>::pack2(p0 - Mfma<S>::to_float((uint16_t)(hi & 0xffffu)), p1 - Mfma<S>::to_float((uint16_t)(hi >> 16)));
+}
+
+// leaf(First) + ... + leaf(First + N - 1), added pairwise.  Binary32 products sum in many short chains of
+// matrix instructions: one chain over a head of 128 rounds 128 times at up to the size of the score, and
+// that error alone is as large as all others of a row together.
+template <int First, int N, typename F>
+__device__ __forceinline__ auto pairwise_sum(F& leaf) {
+  if constexpr (N == 1) return leaf(std::integral_constant<int, First>{});
+  else return pairwise_sum<First, N / 2>(leaf) + pairwise_sum<First + N / 2, N - N / 2>(leaf);
 }
 
 // Launchers of the two kernels (grid and workspace fields of the arguments set); nb = blocks of

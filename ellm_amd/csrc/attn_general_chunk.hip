@@ -13,7 +13,10 @@
 // two, from two groups or two workgroups, are the least, four the best where registers allow.
 // Groups that take turns at a step's matrix and vector parts, as the 128-wide tile kernel's do, came out
 // slower than groups side by side (a lone wave's vector part is 1.5 x as long as a shared one).
-// Binary32 is bound by the matrix pipe (256 flops a cycle and unit) and keeps one group.
+// Binary32 is bound by the matrix pipe (256 flops a cycle and unit) and keeps one group.  Its sums run in
+// chains of eight products; the chains are added up behind the next one's matrix instructions, and that
+// costs: 681 tokens x 3, 32 / 4 heads of 128, 135 us and an error of 2.1e-7 against 64 bits with chains of
+// half a head and of a step's keys, 171 us and 1.3e-7 now (one workgroup per query row: 1673 us, 1.6e-7).
 // Measured, one group before: 2048 tokens, 32 query / 8 key-value heads of 64, bfloat16: 46.0 -> 41.9 us
 // (410 TFLOP/s); 341 tokens, 32 / 32 heads of 96: 16.2 -> 10.2; 603 tokens x 2, 32 / 4 heads of 192: 40.6 -> 29.1.
 // Binary16 heads of 256 (one group: no registers for two): 1019 tokens, 32 / 4 heads 80 us.
@@ -46,10 +49,13 @@ struct Shape {
   static constexpr int kTileRows = 32 * RB;  // query rows of a workgroup
   static constexpr int MB = (!kF32 && NB <= 4 && KG <= 2 && !(NB == 2 && KG == 2)) ? 2 : 1;
   static constexpr int kKeys = 32 * MB;
-  // 16-byte pieces of K (and of V) a thread moves per step, the last one of some threads none
+  // 16-byte pieces of K (and of V) a thread moves per step
   static constexpr int kAllPieces = kKeys * kPiecesRow;
-  static constexpr int kPieces = (kAllPieces + kGroupThreads - 1) / kGroupThreads;
-  static constexpr bool kEven = kPieces * kGroupThreads == kAllPieces;
+  static constexpr int kPieces = kAllPieces / kGroupThreads;
+  static_assert(kPieces * kGroupThreads == kAllPieces, "every thread moves the same number of pieces");
+  // a thread's pieces lie in one column, kRowStep keys apart (or anywhere: 0)
+  static constexpr int kRowStep = kGroupThreads % kPiecesRow == 0 ? kGroupThreads / kPiecesRow : 0;
+  static constexpr int kPlaces = kRowStep ? 1 : kPieces;
   // Row pitches in LDS, bytes.  K rows are read 16 bytes a lane from 32 rows: a pitch of 4 x odd
   // words spreads 16 of them over all banks.  V rows, 16-bit: a 16-lane block of the transposing read
   // takes 32 bytes from each of four rows and its neighbour the next 32, so four rows 16 x odd words
@@ -69,10 +75,10 @@ struct Shape {
   // Waves per SIMD the registers are planned for: queries, accumulators, scores, weights and the
   // pieces on their way to LDS are about 40 (32 x 32 x head / 64) registers and a few dozen more.
   // Heads of 64 with two groups take steps of 32 keys to fit twice on a unit.
-  // Binary32 heads of 256 have no registers left to hold the next V rows during a step: those are
-  // requested behind it (a step is 16384 matrix cycles there).
-  static constexpr bool kLateV = kF32 && NB == 8;
-  static constexpr int kOccupancy = KG == 2 && NB <= 2 ? 4 : KG > 1 ? kWaves / 4 : kF32 ? (NB <= 2 ? 2 : 1) : NB <= 2 ? 3 : NB <= 4 ? 2 : 1;
+  // Wider binary32 heads have no registers left to hold the next V rows beside the partial sums of the
+  // scores: those are requested between the two products (4096 matrix cycles each with heads of 128).
+  static constexpr bool kLateV = kF32 && NB >= 4;
+  static constexpr int kOccupancy = KG == 2 && NB <= 2 ? 4 : KG > 1 ? kWaves / 4 : kF32 ? (NB <= 4 ? 2 : 1) : NB <= 2 ? 3 : NB <= 4 ? 2 : 1;
 };
 
 template <typename S, int NB, bool VEC, int RB, int KG>
@@ -86,7 +92,8 @@ void general_chunk_kernel(GeneralArgs p) {
   __shared__ __attribute__((aligned(16))) uint8_t smem[X::kLds];
   __shared__ uint32_t s_bad;                 // a value beyond the first row's position is not finite
 
-  const int tid = threadIdx.x % X::kGroupThreads, lane = tid & 63, wave = tid >> 6;   // within the key group
+  const int tid = threadIdx.x % X::kGroupThreads, lane = tid & 63;   // within the key group
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const uint32_t kg = KG == 1 ? 0u : (uint32_t)__builtin_amdgcn_readfirstlane((int)(threadIdx.x / X::kGroupThreads));
   const int j = lane & 31, g = lane >> 5;
   const uint32_t planes = gridDim.x / p.row_tiles;
@@ -111,7 +118,6 @@ void general_chunk_kernel(GeneralArgs p) {
   const bool row_valid = r < p.rows;
   const uint32_t rc = row_valid ? r : last_row;
   const uint32_t rowpos = P0 + rc / p.group;
-  const size_t row = query_row(p, seq, kvh, rc);
   const uint32_t wave_row0 = min(row0 + 32u * wave, last_row), wave_row1 = min(wave_row0 + 31u, last_row);
   const uint32_t wave_first = P0 + wave_row0 / p.group;    // chunks up to here need no mask,
   const uint32_t wave_last = P0 + wave_row1 / p.group;     // chunks past here are not this wave's
@@ -119,52 +125,53 @@ void general_chunk_kernel(GeneralArgs p) {
 
   u32x4 qreg[kQ];
   {
-    const E* qrow = (const E*)p.q + row * p.head_size;
+    const E* qrow = (const E*)p.q + query_row(p, seq, kvh, rc) * p.head_size;
 #pragma unroll
     for (int s = 0; s < kQ; ++s) qreg[s] = query_piece<S, VEC>(p, qrow, (2 * s + g) * Store<S>::kPiece);
   }
 
   const size_t plane_at = seq_plane_offset(p.seq_offsets, p.kv_stride_seq, seq) + (size_t)kvh * p.kv_stride_head;
-  const E* kp = (const E*)p.k + plane_at;
-  const E* vp = (const E*)p.v + plane_at;
-  const uint64_t kplane = scalar64((uint64_t)kp), vplane = scalar64((uint64_t)vp);
+  const uint64_t kplane = scalar64((uint64_t)((const E*)p.k + plane_at)), vplane = scalar64((uint64_t)((const E*)p.v + plane_at));
+  const E *kp = (const E*)kplane, *vp = (const E*)vplane;
   const uint64_t pos_bytes = (uint64_t)p.kv_stride_pos * sizeof(E);
   const uint64_t valid = scalar64((uint64_t)(end - 1) * pos_bytes + (uint64_t)p.head_size * sizeof(E));
-  const bool has_last = tid + X::kGroupThreads * (kPieces - 1) < X::kAllPieces;
-  uint32_t off[kPieces], lds_k[kPieces], lds_v[kPieces];
+  uint32_t off0[X::kPlaces], lds_k0[X::kPlaces], lds_v0[X::kPlaces];
   const uint32_t lds_all = (uint32_t)(uintptr_t)(LdsByte*)smem, lds0 = lds_all + kg * X::kGroupLds;
 #pragma unroll
-  for (int i = 0; i < kPieces; ++i) {
+  for (int i = 0; i < X::kPlaces; ++i) {
     const uint32_t pi = tid + X::kGroupThreads * i, krow = pi / X::kPiecesRow, col = pi % X::kPiecesRow;
     if constexpr (VEC)
-      off[i] = col * Store<S>::kPiece < p.head_size && krow < (uint32_t)kKeys ? (uint32_t)(krow * pos_bytes) + 16 * col : kNowhere;
+      off0[i] = col * Store<S>::kPiece < p.head_size ? (uint32_t)(krow * pos_bytes) + 16 * col : kNowhere;
     else
-      off[i] = krow | col * Store<S>::kPiece << 16;
-    lds_k[i] = lds0 + krow * X::kKPitch + 16 * col;
-    lds_v[i] = lds0 + 2 * X::kKBuf + krow * X::kVPitch + 16 * col;
+      off0[i] = krow | col * Store<S>::kPiece << 16;
+    lds_k0[i] = lds0 + krow * X::kKPitch + 16 * col;
+    lds_v0[i] = lds0 + 2 * X::kKBuf + krow * X::kVPitch + 16 * col;
   }
+  // of piece i (a step of 64 keys is at most 2^31 bytes: kNowhere plus its rows stays past every descriptor)
+  const uint32_t row_step = VEC ? (uint32_t)(X::kRowStep * pos_bytes) : (uint32_t)X::kRowStep;
+  auto off = [&](int i) { return X::kRowStep ? off0[0] + i * row_step : off0[i % X::kPlaces]; };
+  auto lds_k = [&](int i) { return X::kRowStep ? lds_k0[0] + i * X::kRowStep * X::kKPitch : lds_k0[i % X::kPlaces]; };
+  auto lds_v = [&](int i) { return X::kRowStep ? lds_v0[0] + i * X::kRowStep * X::kVPitch : lds_v0[i % X::kPlaces]; };
   u32x4 kst[kPieces], vst[kPieces];
   auto load_rows = [&](uint32_t step, const E* rows, uint64_t plane_base, u32x4 (&st)[kPieces]) {
     const uint32_t kb = k0 + step * kKeys;
     if constexpr (VEC) {
       const __amdgpu_buffer_rsrc_t rs = chunk_rsrc(plane_base, (uint64_t)kb * pos_bytes, valid);
 #pragma unroll
-      for (int i = 0; i < kPieces; ++i) st[i] = __builtin_amdgcn_raw_buffer_load_b128(rs, off[i], 0, 0);
+      for (int i = 0; i < kPieces; ++i) st[i] = __builtin_amdgcn_raw_buffer_load_b128(rs, off(i), 0, 0);
     } else {
 #pragma unroll
       for (int i = 0; i < kPieces; ++i)
-        st[i] = gather_piece<S>(rows, p.kv_stride_pos, kb + (off[i] & 0xffffu), end, off[i] >> 16, p.head_size);
+        st[i] = gather_piece<S>(rows, p.kv_stride_pos, kb + (off(i) & 0xffffu), end, off(i) >> 16, p.head_size);
     }
   };
   auto load_step = [&](uint32_t step) {
     load_rows(step, kp, kplane, kst);
     if constexpr (!X::kLateV) load_rows(step, vp, vplane, vst);
   };
-  auto store_rows = [&](uint32_t step, const u32x4 (&st)[kPieces], const uint32_t (&at)[kPieces], int bytes)
-      __attribute__((always_inline)) {
+  auto store_rows = [&](uint32_t step, const u32x4 (&st)[kPieces], auto at, int bytes) __attribute__((always_inline)) {
 #pragma unroll
-    for (int i = 0; i < kPieces; ++i)
-      if (X::kEven || i + 1 < kPieces || has_last) *(LdsU32x4*)(at[i] + (step / KG & 1) * bytes) = st[i];
+    for (int i = 0; i < kPieces; ++i) *(LdsU32x4*)(at(i) + (step / KG & 1) * bytes) = st[i];
   };
   auto look_at = [&](uint32_t step) {
     if (k0 + step * kKeys + kKeys - 1 > first_pos) {   // some row of the workgroup must not see some of these values
@@ -175,7 +182,6 @@ void general_chunk_kernel(GeneralArgs p) {
     }
   };
   auto store_step = [&](uint32_t step) {
-    if constexpr (X::kLateV) load_rows(step, vp, vplane, vst);
     store_rows(step, kst, lds_k, X::kKBuf);
     store_rows(step, vst, lds_v, X::kVBuf);
     look_at(step);
@@ -196,35 +202,63 @@ void general_chunk_kernel(GeneralArgs p) {
                                   : lds0 + 2 * X::kKBuf + (4 * g + ((lane & 15) >> 2)) * X::kVPitch +
                                         2 * (16 * ((lane >> 4) & 1) + 4 * (lane & 3));
 
+  auto load_late = [&](uint32_t step) __attribute__((always_inline)) {
+    if constexpr (X::kLateV)
+      if (step < n_steps) load_rows(step, vp, vplane, vst);
+  };
   auto compute = [&](uint32_t step) __attribute__((always_inline)) {
     const uint32_t kb = k0 + step * kKeys, buf = step / KG & 1;
-    if (step >= n_steps || !wave_has_rows || kb > wave_last) return;
+    if (step >= n_steps || !wave_has_rows || kb > wave_last) {
+      load_late(step + KG);
+      return;
+    }
     const uint32_t ks = k_read + buf * X::kKBuf, vs = v_read + buf * X::kVBuf;
     f32x16 st[MB];
+    f32x16 zero;
 #pragma unroll
-    for (int mb = 0; mb < MB; ++mb) {
-#pragma unroll
-      for (int e = 0; e < 16; ++e) st[mb][e] = 0.0f;
-    }
-    f32x16 st2;   // binary32: a second chain of sums, the odd pieces' (half the rounding steps in a row)
-#pragma unroll
-    for (int e = 0; e < 16; ++e) st2[e] = 0.0f;
-#pragma unroll
-    for (int s = 0; s < kQ; ++s)
-#pragma unroll
-      for (int mb = 0; mb < MB; ++mb) {
-        const u32x4 a = *(const LdsU32x4*)(ks + 32 * mb * X::kKPitch + 32 * s);
-        if constexpr (X::kF32) {
-          f32x16& sum = s & 1 ? st2 : st[mb];
-#pragma unroll
-          for (int e = 0; e < 4; ++e)
+    for (int e = 0; e < 16; ++e) zero[e] = 0.0f;
+    if constexpr (X::kF32) {
+      // Eight products a chain, chains added up in kTotals sums.  A matrix instruction keeps the pipe
+      // busy for 64 cycles: a quarter of the additions of the chain before goes behind each of them.
+      constexpr int kTotals = NB <= 2 ? 4 : 2;   // (what the registers hold)
+      f32x16 total[kTotals], before;
+      u32x4 a = *(const LdsU32x4*)ks;
+      static_for<kQ + 1>([&](auto s_) __attribute__((always_inline)) {
+        constexpr int s = decltype(s_)::value;
+        u32x4 next;
+        if constexpr (s + 1 < kQ) next = *(const LdsU32x4*)(ks + 32 * (s + 1));
+        f32x16 sum = zero;
+        static_for<4>([&](auto e_) __attribute__((always_inline)) {
+          constexpr int e = decltype(e_)::value;
+          if constexpr (s < kQ)
             sum = __builtin_amdgcn_mfma_f32_32x32x2f32(__builtin_bit_cast(float, (uint32_t)a[e]),
                                                        __builtin_bit_cast(float, (uint32_t)qreg[s][e]), sum, 0, 0, 0);
-        } else {
+          __builtin_amdgcn_sched_barrier(0);
+          if constexpr (s > 0) {
+#pragma unroll
+            for (int x = 4 * e; x < 4 * e + 4; ++x) {
+              if constexpr (s <= kTotals) total[(s - 1) % kTotals][x] = before[x];
+              else total[(s - 1) % kTotals][x] += before[x];
+            }
+          }
+          __builtin_amdgcn_sched_barrier(0);
+        });
+        before = sum;
+        if constexpr (s + 1 < kQ) a = next;
+      });
+      auto each = [&](auto n_) { return total[decltype(n_)::value]; };
+      st[0] = pairwise_sum<0, kTotals>(each);
+    } else {
+#pragma unroll
+      for (int mb = 0; mb < MB; ++mb) st[mb] = zero;
+#pragma unroll
+      for (int s = 0; s < kQ; ++s)
+#pragma unroll
+        for (int mb = 0; mb < MB; ++mb) {
+          const u32x4 a = *(const LdsU32x4*)(ks + 32 * mb * X::kKPitch + 32 * s);
           st[mb] = Mfma<S>::m32x32x16(a, qreg[s], st[mb]);
         }
-      }
-    if constexpr (X::kF32) st[0] += st2;
+    }
     if (kb + kKeys - 1 > wave_first || kb + kKeys > end) {   // some pair of the step is masked
 #pragma unroll
       for (int mb = 0; mb < MB; ++mb)
@@ -234,6 +268,7 @@ void general_chunk_kernel(GeneralArgs p) {
           st[mb][e] = (key <= rowpos && key < end) ? st[mb][e] : -INFINITY;
         }
     }
+    load_late(step + KG);
     float rmax = st[0][0];
 #pragma unroll
     for (int mb = 0; mb < MB; ++mb)
@@ -254,23 +289,38 @@ void general_chunk_kernel(GeneralArgs p) {
     float psum = 0.0f;
     if constexpr (X::kF32) {
 #pragma unroll
-      for (int e = 0; e < 16; ++e) {
-        st[0][e] = fast_exp2(__builtin_fmaf(st[0][e], p.c, neg_m));
-        psum += st[0][e];
-      }
-      // a sum of its own per step: chains of 32 keys and of steps round less than one chain over all keys
+      for (int e = 0; e < 16; ++e) st[0][e] = fast_exp2(__builtin_fmaf(st[0][e], p.c, neg_m));
+      auto weight = [&](auto e_) { return st[0][decltype(e_)::value]; };
+      psum = pairwise_sum<0, 16>(weight);
+      // chains of eight keys, added up likewise: a block's four chains, then their sum to the row's
+      f32x16 before, block;
+      float v[4];
+      auto rows_of = [&](int n, float (&to)[4]) __attribute__((always_inline)) {   // chain n: block n / 4, keys 8 (n % 4) ..
 #pragma unroll
-      for (int db = 0; db < NB; ++db) {
-        f32x16 part;
+        for (int e = 0; e < 4; ++e) to[e] = *(const LdsF32*)(vs + (8 * (n & 3) + e) * X::kVPitch + 128 * (n >> 2));
+      };
+      rows_of(0, v);
+      static_for<4 * NB + 2>([&](auto n_) __attribute__((always_inline)) {
+        constexpr int n = decltype(n_)::value, done = n - 1;   // (the chain before)
+        float next[4];
+        if constexpr (n + 1 < 4 * NB) rows_of(n + 1, next);
+        f32x16 sum = zero;
+        static_for<4>([&](auto e_) __attribute__((always_inline)) {
+          constexpr int e = decltype(e_)::value;
+          if constexpr (n < 4 * NB) sum = __builtin_amdgcn_mfma_f32_32x32x2f32(v[e], st[0][4 * (n & 3) + e], sum, 0, 0, 0);
+          __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-        for (int e = 0; e < 16; ++e) part[e] = 0.0f;
+          for (int x = 4 * e; x < 4 * e + 4; ++x) {
+            if constexpr (done > 0 && done % 4 == 0) oacc[done / 4 - 1][x] += block[x];
+            if constexpr (done >= 0 && done < 4 * NB) block[x] = done % 4 == 0 ? before[x] : block[x] + before[x];
+          }
+          __builtin_amdgcn_sched_barrier(0);
+        });
+        before = sum;
+        if constexpr (n + 1 < 4 * NB)
 #pragma unroll
-        for (int e = 0; e < 16; ++e) {
-          const float a = *(const LdsF32*)(vs + (8 * (e >> 2) + (e & 3)) * X::kVPitch + 128 * db);
-          part = __builtin_amdgcn_mfma_f32_32x32x2f32(a, st[0][e], part, 0, 0, 0);
-        }
-        oacc[db] += part;
-      }
+          for (int e = 0; e < 4; ++e) v[e] = next[e];
+      });
     } else {
       u32x4 hi[2 * MB], lo[2 * MB];
 #pragma unroll
@@ -305,6 +355,7 @@ void general_chunk_kernel(GeneralArgs p) {
   // step s of the keys belongs to group s mod KG; every group passes every barrier
   if (threadIdx.x == 0) s_bad = 0;
   if (kg < n_steps) load_step(kg);
+  load_late(kg);
   __syncthreads();
   if (kg < n_steps) store_step(kg);
   if (kg + KG < n_steps) load_step(kg + KG);
@@ -321,7 +372,7 @@ void general_chunk_kernel(GeneralArgs p) {
 
   const size_t part_row0 = (size_t)plane * p.rows;
   if (s_bad) {   // (uniform: the last barrier is behind every write of it)
-    for (uint32_t rr = row0 + threadIdx.x / kWave; rr <= last_row; rr += X::kWaves)
+    for (uint32_t rr = row0 + kg * RB + wave; rr <= last_row; rr += X::kWaves)
       plain_row<S>(p, kp, vp, query_row(p, seq, kvh, rr), (part_row0 + rr) * p.n_split + blockIdx.y, k0,
                    min(end, P0 + rr / p.group + 1), X::kHead, p.n_split > 1);
     return;
@@ -364,27 +415,30 @@ void general_chunk_kernel(GeneralArgs p) {
   }
   if (KG > 1 && kg != 0) return;
   const float l = sum_with_partner_half(l_run);
-  if (!row_valid) return;
+  // (the lane's row again, from the lane's number: kept through the loop it costs registers that are not there)
+  const uint32_t lane_again = lane_number(), g_again = lane_again >> 5, r_again = row0 + 32 * wave + (lane_again & 31);
+  if (r_again >= p.rows) return;
+  const size_t row_again = query_row(p, seq, kvh, r_again);
   if (p.n_split > 1) {
-    const size_t part = (part_row0 + r) * p.n_split + blockIdx.y;
+    const size_t part = (part_row0 + r_again) * p.n_split + blockIdx.y;
     float* orow = p.part_o + part * X::kHead;
 #pragma unroll
     for (int db = 0; db < NB; ++db)
 #pragma unroll
       for (int q4 = 0; q4 < 4; ++q4)
-        *(f32x4*)(orow + 32 * db + 8 * q4 + 4 * g) =
+        *(f32x4*)(orow + 32 * db + 8 * q4 + 4 * g_again) =
             f32x4{oacc[db][4 * q4], oacc[db][4 * q4 + 1], oacc[db][4 * q4 + 2], oacc[db][4 * q4 + 3]};
-    if (g == 0) *(float2*)(p.part_ml + part * 2) = float2{m_run == -INFINITY ? m_run : m_run - kShift, l};
+    if (g_again == 0) *(float2*)(p.part_ml + part * 2) = float2{m_run == -INFINITY ? m_run : m_run - kShift, l};
   } else {
     const float inv = 1.0f / l;
 #pragma unroll
     for (int db = 0; db < NB; ++db)
 #pragma unroll
       for (int q4 = 0; q4 < 4; ++q4)
-        store_out4<S, VEC>(p, row, 32 * db + 8 * q4 + 4 * g,
+        store_out4<S, VEC>(p, row_again, 32 * db + 8 * q4 + 4 * g_again,
                            f32x4{oacc[db][4 * q4] * inv, oacc[db][4 * q4 + 1] * inv, oacc[db][4 * q4 + 2] * inv,
                                  oacc[db][4 * q4 + 3] * inv});
-    if (p.lse && g == 0) p.lse[row] = (m_run - kShift + fast_log2(l)) * kLn2;
+    if (p.lse && g_again == 0) p.lse[row_again] = (m_run - kShift + fast_log2(l)) * kLn2;
   }
 }
 

@@ -9,6 +9,8 @@
 // meet once at the end.  Measured: 8 sequences x 4096 keys, 32 query / 4 key-value heads of 128 in
 // binary32: 27.5 us (4.9 TB/s), where one workgroup per query row took 437 us; 2 x 11046 keys, 32 / 32
 // heads of 256 in bfloat16: 112 us (6.5 TB/s; was 5450); 11 x 131 keys, heads of 96: 6.9 us (was 31).
+// Binary32 products sum in chains of eight, as in the chunk kernel: 11 x 2471 keys, 32 / 32 heads of 128, an error
+// of 2.1e-7 against 64 bits in 162 us, where one chain over the head and one over all keys gave 6.1e-7 in 156.
 #include "attn_general.hpp"
 #include "decode_common.hpp"
 
@@ -23,6 +25,7 @@ constexpr int kRows = (int)kGeneralStepRows;
 typedef __attribute__((address_space(3))) uint8_t LdsByte;
 typedef __attribute__((address_space(3))) u32x4 LdsU32x4;
 typedef __attribute__((address_space(3))) float LdsF32;
+typedef __attribute__((address_space(3))) f32x2 LdsF32x2;
 typedef short i16x4 __attribute__((ext_vector_type(4)));
 typedef __attribute__((address_space(3))) i16x4 LdsI16x4;
 
@@ -147,34 +150,41 @@ __global__ __launch_bounds__(kThreads, (StepShape<S, NB>::kOccupancy)) void gene
     __builtin_amdgcn_wave_barrier();
     // S^T: lane (row c, group g) register r of block mc <-> key kb + 16 mc + 4 g + r
     f32x4 st[MC];
-#pragma unroll
-    for (int mc = 0; mc < MC; ++mc) st[mc] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-#pragma unroll
-    for (int s = 0; s < kQ; ++s)
+    if constexpr (X::kF32) {
 #pragma unroll
       for (int mc = 0; mc < MC; ++mc) {
-        const u32x4 a = *(const LdsU32x4*)(k_read + 16 * mc * X::kKPitch + 64 * s);
-        if constexpr (X::kF32) {
+        auto half_piece = [&](auto n_) __attribute__((always_inline)) {   // eight products a score
+          constexpr int s = decltype(n_)::value / 2, e = decltype(n_)::value % 2 * 2;
+          const f32x2 a = *(const LdsF32x2*)(k_read + 16 * mc * X::kKPitch + 64 * s + 4 * e);
+          const f32x4 sum = __builtin_amdgcn_mfma_f32_16x16x4f32(a[0], __builtin_bit_cast(float, (uint32_t)qreg[s][e]),
+                                                                 f32x4{0.0f, 0.0f, 0.0f, 0.0f}, 0, 0, 0);
+          return __builtin_amdgcn_mfma_f32_16x16x4f32(a[1], __builtin_bit_cast(float, (uint32_t)qreg[s][e + 1]), sum, 0, 0, 0);
+        };
+        st[mc] = pairwise_sum<0, 2 * kQ>(half_piece);
+      }
+    } else {
 #pragma unroll
-          for (int e = 0; e < 4; ++e)
-            st[mc] = __builtin_amdgcn_mfma_f32_16x16x4f32(__builtin_bit_cast(float, (uint32_t)a[e]),
-                                                          __builtin_bit_cast(float, (uint32_t)qreg[s][e]), st[mc], 0, 0, 0);
-        } else {
+      for (int mc = 0; mc < MC; ++mc) st[mc] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+      for (int s = 0; s < kQ; ++s)
+#pragma unroll
+        for (int mc = 0; mc < MC; ++mc) {
+          const u32x4 a = *(const LdsU32x4*)(k_read + 16 * mc * X::kKPitch + 64 * s);
           st[mc] = Mfma<S>::m16x16x32(a, qreg[s], st[mc]);
         }
-      }
+    }
     float tmax = -INFINITY;
 #pragma unroll
     for (int mc = 0; mc < MC; ++mc)
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
         const uint32_t key = kb + 16 * mc + 4 * g + e;
-        st[mc][e] = (key <= rowpos && key < end) ? st[mc][e] * p.c : -INFINITY;
+        st[mc][e] = (key <= rowpos && key < end) ? st[mc][e] : -INFINITY;
         tmax = fmaxf(tmax, st[mc][e]);
       }
     tmax = fmaxf(tmax, xor_shuffle(tmax, 16));
     tmax = fmaxf(tmax, xor_shuffle(tmax, 32));
-    const float m_new = fmaxf(m_run, tmax);   // -inf while the row has seen none of its keys
+    const float m_new = fmaxf(m_run, tmax * p.c);   // -inf while the row has seen none of its keys
     const float ref = m_new == -INFINITY ? 0.0f : m_new;
     const float alpha = fast_exp2(m_run - ref);
     float psum = 0.0f;
@@ -182,25 +192,31 @@ __global__ __launch_bounds__(kThreads, (StepShape<S, NB>::kOccupancy)) void gene
     for (int mc = 0; mc < MC; ++mc)
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
-        st[mc][e] = fast_exp2(st[mc][e] - (ref - kShift));
+        st[mc][e] = fast_exp2(__builtin_fmaf(st[mc][e], p.c, kShift - ref));
         psum += st[mc][e];
       }
     l_run = l_run * alpha + psum;
     m_run = m_new;
+    if constexpr (X::kF32) {   // a sum of its own per request, in chains of eight keys
 #pragma unroll
-    for (int b = 0; b < 2 * NB; ++b) acc[b] *= alpha;
+      for (int b = 0; b < 2 * NB; ++b) {
+        auto key_pair = [&](auto n_) __attribute__((always_inline)) {
+          constexpr int mc = decltype(n_)::value / 2, e = decltype(n_)::value % 2 * 2;
+          const uint32_t vs = v_read + (16 * mc + e) * X::kVPitch + 64 * b;
+          const f32x4 sum = __builtin_amdgcn_mfma_f32_16x16x4f32(*(const LdsF32*)vs, st[mc][e],
+                                                                 f32x4{0.0f, 0.0f, 0.0f, 0.0f}, 0, 0, 0);
+          return __builtin_amdgcn_mfma_f32_16x16x4f32(*(const LdsF32*)(vs + X::kVPitch), st[mc][e + 1], sum, 0, 0, 0);
+        };
+        const f32x4 part = pairwise_sum<0, 2 * MC>(key_pair);
 #pragma unroll
-    for (int mc = 0; mc < MC; ++mc) {
-      const uint32_t vs = v_read + 16 * mc * X::kVPitch;
-      if constexpr (X::kF32) {
+        for (int e = 0; e < 4; ++e) acc[b][e] = __builtin_fmaf(acc[b][e], alpha, part[e]);
+      }
+    } else {
 #pragma unroll
-        for (int e = 0; e < 4; ++e)
+      for (int b = 0; b < 2 * NB; ++b) acc[b] *= alpha;
 #pragma unroll
-          for (int b = 0; b < 2 * NB; ++b) {
-            const float a = *(const LdsF32*)(vs + e * X::kVPitch + 64 * b);
-            acc[b] = __builtin_amdgcn_mfma_f32_16x16x4f32(a, st[mc][e], acc[b], 0, 0, 0);
-          }
-      } else {
+      for (int mc = 0; mc < MC; ++mc) {
+        const uint32_t vs = v_read + 16 * mc * X::kVPitch;
         u32x2 hi, lo;
         uint32_t h, l;
         split_pair<S>(st[mc][0], st[mc][1], h, l);

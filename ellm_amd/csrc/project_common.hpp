@@ -44,14 +44,6 @@ __device__ __forceinline__ size_t kv_row_offset(const ProjectKernelArgs& p, uint
          (size_t)pos * p.kv_stride_pos;
 }
 
-template <int N, typename F>
-__device__ __forceinline__ void static_for(F&& f) {
-  if constexpr (N > 0) {
-    static_for<N - 1>(f);
-    f(std::integral_constant<int, N - 1>{});
-  }
-}
-
 __device__ __forceinline__ uint64_t uniform64(const void* p) {
   const uint32_t lo = (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)(uint64_t)p);
   const uint32_t hi = (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)((uint64_t)p >> 32));
