@@ -176,14 +176,14 @@ __device__ __forceinline__ float wave_sum(float v) {
 // output or the partial row.  The matrix kernels multiply every value row of a chunk
 // by every query row, masked pairs with a weight of zero, and 0 x infinity is not 0; a query row
 // must not see what the value rows of later positions hold, so a workgroup that meets a value
-// that is not finite beyond its first row's position takes its rows through here instead.
+// that is not finite beyond its first row's position takes its rows through here instead.  So do rows
+// whose sums are not finite (not_finite_sum).
 template <typename S>
 __device__ __forceinline__ void plain_row(const GeneralArgs& p, const typename Store<S>::E* kp,
                                                      const typename Store<S>::E* vp, size_t row, size_t prow,
-                                                     uint32_t k0, uint32_t end, uint32_t pitch, bool partial) {
+                                                     uint32_t k0, uint32_t end, uint32_t pitch, bool partial, int lane) {
   typedef typename Store<S>::E E;
   constexpr int kPerLane = kMaxHead / kWave;
-  const int lane = (int)lane_number();
   const E* q = (const E*)p.q + row * p.head_size;
   float qv[kPerLane], o[kPerLane];
 #pragma unroll
@@ -203,8 +203,8 @@ __device__ __forceinline__ void plain_row(const GeneralArgs& p, const typename S
       vv[i] = d < p.head_size ? load_elem<S>(vp + at) : 0.0f;
     }
     const float s = wave_sum(part) * p.c;
-    const float m_new = fmaxf(m, s);
-    const float alpha = fast_exp2(m - m_new), w = fast_exp2(s - m_new);
+    const float m_new = fmaxf(m, s), ref = m_new == -INFINITY ? 0.0f : m_new;
+    const float alpha = fast_exp2(m - ref), w = fast_exp2(s - ref);
     l = l * alpha + w;
 #pragma unroll
     for (int i = 0; i < kPerLane; ++i) o[i] = __builtin_fmaf(w, vv[i], o[i] * alpha);
@@ -261,6 +261,15 @@ template <int First, int N, typename F>
 __device__ __forceinline__ auto pairwise_sum(F& leaf) {
   if constexpr (N == 1) return leaf(std::integral_constant<int, First>{});
   else return pairwise_sum<First, N / 2>(leaf) + pairwise_sum<First + N / 2, N - N / 2>(leaf);
+}
+
+// Whether a row with these sums needs plain_row.  largest: the largest magnitude among its weighted sums (NaN
+// counts as the largest of all); l: the weights' sum (NaN, as from a key that is not a number: every way to add
+// up gives NaN).  A weight in two 16-bit operands on an infinite value gives NaN where it should give the
+// infinity, when its rest is 0 or negative (0 x inf, inf - inf), and then the sum is NaN to the end.
+__device__ __forceinline__ bool not_finite_sum(float largest, float l) { return !(largest < INFINITY) && l == l; }
+__device__ __forceinline__ float largest_of(float m, float a, float b) {   // one instruction
+  return __builtin_elementwise_maximum(__builtin_elementwise_maximum(m, __builtin_fabsf(a)), __builtin_fabsf(b));
 }
 
 // Launchers of the two kernels (grid and workspace fields of the arguments set); nb = blocks of

@@ -374,7 +374,7 @@ void general_chunk_kernel(GeneralArgs p) {
   if (s_bad) {   // (uniform: the last barrier is behind every write of it)
     for (uint32_t rr = row0 + kg * RB + wave; rr <= last_row; rr += X::kWaves)
       plain_row<S>(p, kp, vp, query_row(p, seq, kvh, rr), (part_row0 + rr) * p.n_split + blockIdx.y, k0,
-                   min(end, P0 + rr / p.group + 1), X::kHead, p.n_split > 1);
+                   min(end, P0 + rr / p.group + 1), X::kHead, p.n_split > 1, (int)lane_number());
     return;
   }
   // the groups' rows: the upper half of the groups hands its own over, until one group is left
@@ -415,6 +415,19 @@ void general_chunk_kernel(GeneralArgs p) {
   }
   if (KG > 1 && kg != 0) return;
   const float l = sum_with_partner_half(l_run);
+  // Sums that are not finite: an infinite value under a weight in two operands, or weights above one (up to
+  // 2^kRescaleStep) on values less than that below the largest number.
+  float top[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+  for (int db = 0; db < NB; ++db)
+#pragma unroll
+    for (int e = 0; e < 16; e += 2) top[e >> 2] = largest_of(top[e >> 2], oacc[db][e], oacc[db][e + 1]);
+  if (__any(not_finite_sum(largest_of(top[0], top[1], largest_of(top[2], top[3], 0.0f)), l))) {
+    for (uint32_t rr = row0 + 32 * wave; rr < min(row0 + 32 * wave + 32, last_row + 1); ++rr)
+      plain_row<S>(p, kp, vp, query_row(p, seq, kvh, rr), (part_row0 + rr) * p.n_split + blockIdx.y, k0,
+                   min(end, P0 + rr / p.group + 1), X::kHead, p.n_split > 1, (int)lane_number());
+    return;
+  }
   // (the lane's row again, from the lane's number: kept through the loop it costs registers that are not there)
   const uint32_t lane_again = lane_number(), g_again = lane_again >> 5, r_again = row0 + 32 * wave + (lane_again & 31);
   if (r_again >= p.rows) return;

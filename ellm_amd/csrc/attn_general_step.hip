@@ -236,6 +236,14 @@ __global__ __launch_bounds__(kThreads, (StepShape<S, NB>::kOccupancy)) void gene
   l_run += xor_shuffle(l_run, 16);
   l_run += xor_shuffle(l_run, 32);
 
+  if constexpr (!X::kF32) {
+    float top[2] = {0.0f, 0.0f};
+#pragma unroll
+    for (int b = 0; b < 2 * NB; ++b)
+#pragma unroll
+      for (int e = 0; e < 4; e += 2) top[e >> 1] = largest_of(top[e >> 1], acc[b][e], acc[b][e + 1]);
+    bad |= not_finite_sum(largest_of(top[0], top[1], 0.0f), l_run);
+  }
   // the four waves' rows meet in LDS (the staging buffers are idle behind the barrier)
   if (tid == 0) s_bad = 0;
   __syncthreads();
@@ -259,7 +267,7 @@ __global__ __launch_bounds__(kThreads, (StepShape<S, NB>::kOccupancy)) void gene
   if (s_bad) {
     for (uint32_t rr = wave; rr < rows_here; rr += kWaves)
       plain_row<S>(p, kp, vp, query_row(p, seq, kvh, row0 + rr), prow0 + (size_t)rr * p.n_split + split, k0,
-                   min(end, P0 + (row0 + rr) / p.group + 1), X::kHead, live > 1);
+                   min(end, P0 + (row0 + rr) / p.group + 1), X::kHead, live > 1, lane);
   } else {
     for (uint32_t item = tid; item < n_items; item += kThreads) {
       const uint32_t rr = item / kQuads, dq = item % kQuads;

@@ -103,6 +103,52 @@ def test_values_beyond_a_row_are_not_seen(dtype, hq, hkv, hs, p0, s):
     assert np.isposinf(got[-1]).all() and np.abs(lse[-1] - want_lse[-1]).max() <= 1e-4
 
 
+# (q heads, kv heads, head size, position_index, interval): chunk kernel with one, two and four key groups and with a
+# key split, step kernel with one and several splits, several tokens
+INFINITE = [(8, 8, 64, 20, 40), (8, 2, 64, 400, 40), (4, 4, 192, 300, 140), (8, 1, 96, 1500, 9), (4, 4, 80, 40, 1),
+            (8, 1, 64, 1700, 1), (4, 2, 33, 90, 5)]
+
+
+@pytest.mark.parametrize("dtype", [orc.F16, orc.BF16, orc.F32], ids=["f16", "bf16", "f32"])
+@pytest.mark.parametrize("case", INFINITE, ids=["%dq%dkv_h%d_%d+%d" % c for c in INFINITE])
+def test_an_infinite_value_that_a_row_sees(case, dtype):
+    """Infinities of either sign in the value row of one key that every row sees (the weight is positive, so
+    that is what comes out), and finite values beside them.  As two 16-bit operands the weight has a rest of
+    zero or of either sign, and 0 x inf is not a number."""
+    hq, hkv, hs, p0, s = case
+    print("case", case, dtype, flush=True)
+    cap = p0 + s + 2
+    q, k, v = _rand((s, 1, hq, hs), 61, dtype), _rand((1, hkv, cap, hs), 62, dtype), _rand((1, hkv, cap, hs), 63, dtype)
+    f = v.view(np.float32 if dtype == orc.F32 else np.uint16)
+    plus = np.inf if dtype == orc.F32 else 0x7C00 if dtype == orc.F16 else 0x7F80
+    minus = -np.inf if dtype == orc.F32 else plus | 0x8000
+    f[:, :, 7, 0::3], f[:, :, 7, 1::3] = plus, minus
+    scale = 1.0 / np.sqrt(hs)
+    want, want_lse = orc.attention(q, k, v, scale, dtype, position_index=p0)
+    got, lse = _run(q, k, v, scale, dtype, p0=p0)
+    right = [int(np.isposinf(got[..., 0::3]).sum()), int(np.isneginf(got[..., 1::3]).sum())]
+    assert right == [got[..., 0::3].size, got[..., 1::3].size]
+    w = orc.from_storage(want, dtype)
+    _check("finite_columns", got[..., 2::3], lse, orc.to_storage(np.ascontiguousarray(w[..., 2::3]), dtype), want_lse, dtype, 1)
+
+
+@pytest.mark.parametrize("dtype,hs", [(orc.BF16, 256), (orc.BF16, 64), (orc.F32, 64)], ids=["bf16_h256", "bf16_h64", "f32_h64"])
+def test_large_finite_values_under_rising_scores(dtype, hs):
+    """One value of 1e38 under the highest score, which lies 6.5 binary orders above those of the step of keys
+    before it: less than what makes the chunk kernel move its reference, so the weight is 2^6.5 there."""
+    hq, hkv, s, p0 = 4, 2, 50, 90
+    q, k, v = np.zeros((s, 1, hq, hs), np.float32), np.zeros((1, hkv, p0 + s, hs), np.float32), np.zeros((1, hkv, p0 + s, hs), np.float32)
+    q[..., 0] = 1.0
+    k[:, :, 70, 0] = 6.5
+    v[:, :, 70] = 1e38
+    q, k, v = (orc.to_storage(a, dtype) for a in (q, k, v))
+    got, _ = _run(q, k, v, float(np.log(2.0)), dtype, p0=p0)
+    share = 1.0 / (1.0 + (p0 + np.arange(s)) * 2.0 ** -6.5)          # of the one key among the row's keys
+    want = share[:, None, None, None] * float(orc.from_storage(v, dtype).max())
+    err = float(np.abs(got / want - 1.0).max())
+    assert err <= (2.0 ** -8 if dtype == orc.BF16 else 1e-6)         # half a unit of bfloat16, binary32 sums
+
+
 def test_repeated_steps_fold_the_same_bits():
     """The arrival counters return to zero: the same handle launched many times gives the same bits."""
     import torch
