@@ -9,6 +9,7 @@
 #include <vector>
 
 #include "../../include/ellm_attn.h"
+#include "general_plan.hpp"
 #include "handles.hpp"
 #include "kernels.hpp"
 
@@ -267,7 +268,7 @@ static int attn_create(const ellm_attn_desc* d, const ellm_kv_seq_table* table, 
                                               (uint32_t)d->attention_head_num, (uint32_t)n_cu);
   h->general = ellm::attn_is_general(*d);
   if (h->general) {   // other head sizes and binary32: one table of partial rows for both kinds of call
-    const ellm::GeneralWorkspace w = ellm::general_workspace(
+    const ellm::gen::GeneralWorkspace w = ellm::gen::general_workspace(
         (uint32_t)d->max_position_interval, (uint32_t)d->batch_size, (uint32_t)d->attention_head_num,
         (uint32_t)d->kv_head_num, (uint32_t)d->head_size, (uint32_t)n_cu);
     h->ws = ellm::DecodeWorkspace{0, 0, w.counters};

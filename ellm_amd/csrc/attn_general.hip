@@ -2,10 +2,9 @@
 // binary32 storage.  The reference's generic leaf (src/kernel/generic/flash_attention.rs:60-89)
 // honours whatever `length` and element type its caller hands it, and its operator test runs in
 // f32 (src/compiler/mul/attention.rs:262-330).  Same arguments, masks, position rules and
-// log-sum-exp as the other kernels (ellm_attn_run / ellm_attn_run_ragged).  This file: the choice
-// between the two kernels, their key splits, and the merge of a chunk's splits.
+// log-sum-exp as the other kernels (ellm_attn_run / ellm_attn_run_ragged).  This file: the launches
+// (general_plan.hpp chooses), the kernel for short walks, and the merge of a chunk's splits.
 #include "attn_general.hpp"
-#include "chunk_plan.hpp"
 
 namespace ellm {
 namespace gen {
@@ -58,6 +57,116 @@ __global__ __launch_bounds__(256) void general_merge_kernel(GeneralArgs p, uint3
   if (p.lse && dq == 0) p.lse[row] = (m + fast_log2(l)) * kLn2;
 }
 
+// One workgroup per (token, sequence, query head) row, without matrix instructions: for walks of a few turns,
+// where a launch of the matrix kernels is mostly what their tiles cost whatever is in them, and for few rows of
+// wide heads (general_plan() has the rule and the measured times).  The four waves take the row's keys in turns of four, a
+// lane owns elements lane, lane + 64, ... of the head, scores are sums over the wave, the soft-max runs online
+// and the waves' partial rows meet in LDS.  Bound by the chain of turns: four trips to memory's data, six lane
+// exchanges a score, an exponential.
+constexpr int kRowWaves = 4, kRowKeys = kRowTurn / kRowWaves;
+
+template <typename S>
+__global__ __launch_bounds__(kRowWaves* kWave) void general_rows_kernel(GeneralArgs p) {
+  typedef typename Store<S>::E E;
+  constexpr int kPerLane = kMaxHead / kWave;
+  __shared__ float s_o[kRowWaves][kMaxHead];
+  __shared__ float s_m[kRowWaves], s_l[kRowWaves];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  // longest rows first, the planes side by side
+  const uint32_t hs = p.head_size, planes = gridDim.x / p.rows, plane = blockIdx.x % planes;
+  const uint32_t r = p.rows - 1 - blockIdx.x / planes;
+  const uint32_t seq = plane / p.n_kv_heads, kvh = plane % p.n_kv_heads;
+  const uint32_t pos = start_position(p, seq) + r / p.group;
+  const size_t row = query_row(p, seq, kvh, r);
+  const E* q = (const E*)p.q + row * hs;
+  const size_t plane_at = seq_plane_offset(p.seq_offsets, p.kv_stride_seq, seq) + (size_t)kvh * p.kv_stride_head;
+  const E* kp = (const E*)p.k + plane_at;
+  const E* vp = (const E*)p.v + plane_at;
+
+  float qv[kPerLane], o[kPerLane];
+#pragma unroll
+  for (int i = 0; i < kPerLane; ++i) {
+    const uint32_t d = lane + 64 * i;
+    qv[i] = d < hs ? load_elem<S>(q + d) * p.scale : 0.0f;
+    o[i] = 0.0f;
+  }
+  float m = -INFINITY, l = 0.0f;
+  // wave w takes keys 16 n + 4 w .. + 3 (wave-uniform bounds: no lane leaves the reductions)
+  for (uint32_t j0 = kRowKeys * wave; j0 <= pos; j0 += kRowTurn) {
+    float kk[kRowKeys][kPerLane], vv[kRowKeys][kPerLane];
+#pragma unroll
+    for (int u = 0; u < kRowKeys; ++u) {
+      const size_t at = (size_t)min(j0 + u, pos) * p.kv_stride_pos;   // keys past the row's own position are masked below
+#pragma unroll
+      for (int i = 0; i < kPerLane; ++i) {
+        const uint32_t d = lane + 64 * i;
+        kk[u][i] = d < hs ? load_elem<S>(kp + at + d) : 0.0f;
+        vv[u][i] = d < hs ? load_elem<S>(vp + at + d) : 0.0f;
+      }
+    }
+    float s[kRowKeys];
+#pragma unroll
+    for (int u = 0; u < kRowKeys; ++u) {
+      float part = 0.0f;
+#pragma unroll
+      for (int i = 0; i < kPerLane; ++i) part = __builtin_fmaf(qv[i], kk[u][i], part);
+      s[u] = (j0 + u <= pos) ? wave_sum(part) : -INFINITY;
+    }
+    float m_new = m;
+#pragma unroll
+    for (int u = 0; u < kRowKeys; ++u) m_new = fmaxf(m_new, s[u]);
+    const float alpha = __expf(m - m_new);   // m = -inf on the first turn: exp(-inf) = 0
+    l *= alpha;
+#pragma unroll
+    for (int i = 0; i < kPerLane; ++i) o[i] *= alpha;
+#pragma unroll
+    for (int u = 0; u < kRowKeys; ++u) {
+      const float w = __expf(s[u] - m_new);  // masked keys: exp(-inf) = 0
+      l += w;
+#pragma unroll
+      for (int i = 0; i < kPerLane; ++i) o[i] = __builtin_fmaf(w, vv[u][i], o[i]);
+    }
+    m = m_new;
+  }
+  // the four waves' partial rows meet in LDS (a wave without keys leaves max = -inf, sum = 0)
+#pragma unroll
+  for (int i = 0; i < kPerLane; ++i) s_o[wave][lane + 64 * i] = o[i];
+  if (lane == 0) {
+    s_m[wave] = m;
+    s_l[wave] = l;
+  }
+  __syncthreads();
+  float top = s_m[0];   // finite: wave 0 holds key 0
+#pragma unroll
+  for (int w = 1; w < kRowWaves; ++w) top = fmaxf(top, s_m[w]);
+  float sum = 0.0f, wgt[kRowWaves];
+#pragma unroll
+  for (int w = 0; w < kRowWaves; ++w) {
+    wgt[w] = __expf(s_m[w] - top);
+    sum += wgt[w] * s_l[w];
+  }
+  const float inv = 1.0f / sum;
+  E* out = (E*)p.out + row * hs;
+  for (uint32_t d = threadIdx.x; d < hs; d += blockDim.x) {
+    float acc = 0.0f;
+#pragma unroll
+    for (int w = 0; w < kRowWaves; ++w) acc += wgt[w] * s_o[w][d];
+    store_elem<S>(out + d, acc * inv);
+  }
+  if (p.lse && threadIdx.x == 0) p.lse[row] = top + __logf(sum);
+}
+
+hipError_t launch_rows(const GeneralArgs& p, int dtype, uint32_t planes, hipStream_t stream) {
+  const dim3 grid(planes * p.rows), block(kRowWaves * kWave);
+  if (dtype == 0)
+    hipLaunchKernelGGL(general_rows_kernel<F16>, grid, block, 0, stream, p);
+  else if (dtype == 1)
+    hipLaunchKernelGGL(general_rows_kernel<BF16>, grid, block, 0, stream, p);
+  else
+    hipLaunchKernelGGL(general_rows_kernel<F32>, grid, block, 0, stream, p);
+  return hipGetLastError();
+}
+
 template <typename S, bool VEC>
 hipError_t launch_merge(const GeneralArgs& p, uint32_t planes, uint32_t pitch, hipStream_t stream) {
   const size_t items = (size_t)planes * p.rows * (pitch / 4);
@@ -74,21 +183,6 @@ uint32_t element_bytes(int dtype) { return dtype == 2 ? 4 : 2; }
 
 }  // namespace
 }  // namespace gen
-
-GeneralWorkspace general_workspace(uint32_t max_interval, uint32_t batch_capacity, uint32_t n_q_heads,
-                                   uint32_t n_kv_heads, uint32_t head_size, uint32_t n_cu) {
-  GeneralWorkspace w;
-  const uint32_t group = n_q_heads / n_kv_heads;
-  w.pitch = 32 * (uint32_t)gen::head_blocks(head_size, false);   // (never below the pitch of the vector form)
-  size_t rows = decode_workspace(batch_capacity, n_q_heads, n_kv_heads, n_cu).rows;
-  const size_t chunk = prefill_workspace_rows(max_interval, batch_capacity, n_q_heads, n_cu);
-  if (chunk > rows) rows = chunk;
-  const size_t cap = (size_t)512 * n_cu * 128 / w.pitch;         // 68 MB on 256 units
-  w.rows = rows < cap ? rows : cap;
-  const uint32_t tiles = (group + gen::kGeneralStepRows - 1) / gen::kGeneralStepRows;
-  w.counters = (size_t)batch_capacity * n_kv_heads * (tiles > 2 ? tiles : 2);
-  return w;
-}
 
 hipError_t launch_attn_general(const AttnArgs& a, uint32_t head_size, hipStream_t stream) {
   gen::GeneralArgs p;
@@ -110,6 +204,7 @@ hipError_t launch_attn_general(const AttnArgs& a, uint32_t head_size, hipStream_
   p.head_size = head_size;
   p.position_index = a.position_index;
   p.interval = a.position_interval;
+  p.scale = a.scale;
   const float c = a.scale * kLog2e;
   p.negate_q = c < 0.0f ? 1u : 0u;
   // scale == 0 (uniform attention): a tiny positive c keeps -inf * c == -inf for masked keys
@@ -128,60 +223,27 @@ hipError_t launch_attn_general(const AttnArgs& a, uint32_t head_size, hipStream_
   // offsets lies on the device and may hold anything), 64 rows within a buffer descriptor's reach
   const bool vec = head_size * es % 16 == 0 && p.kv_stride_seq * es % 16 == 0 && p.kv_stride_head * es % 16 == 0 &&
                    p.kv_stride_pos * es % 16 == 0 && p.kv_stride_pos * es <= ((size_t)1 << 25) && !p.seq_offsets;
-  const int nb = gen::head_blocks(head_size, vec);
-  const uint32_t max_len = a.position_index + a.position_interval;
-  const size_t room = p.part_o ? a.prefill_part_rows / ((size_t)planes * rows) : 1;
-
-  // Few query rows per plane: the call is a stream of K and V.  Two workgroups of sixteen rows read a
-  // plane twice (the second time from a cache); from 33 rows on the chunk kernel reads it once.
-  if (p.interval == 1 || rows <= 2 * gen::kGeneralStepRows) {
-    p.row_tiles = (p.rows + gen::kGeneralStepRows - 1) / gen::kGeneralStepRows;
-    DecodePlan plan = decode_plan(max_len, planes * p.row_tiles, 1, a.n_cu);
-    if (plan.n_split > room) {
-      const uint32_t n = room > 1 ? (uint32_t)room : 1;
-      plan.split_len = ((max_len + n - 1) / n + 63) / 64 * 64;
-      plan.n_split = (max_len + plan.split_len - 1) / plan.split_len;
-    }
-    p.split_len = plan.split_len;
-    p.n_split = plan.n_split;
-    if ((size_t)planes * p.row_tiles * p.n_split > 0x7fffffffu) return hipErrorInvalidValue;
-    return gen::launch_general_step(p, a.dtype, nb, vec, planes, stream);
-  }
-
-  const bool f32 = a.dtype == 2;
-  auto tiles_of = [&](size_t n) { return (rows + n - 1) / n; };
-  // Key groups put more waves on a row's keys: 64 rows and four groups while all workgroups find a
-  // unit of their own (131 tokens on 378, 32 / 8 heads of 64: 15.2 -> 9.7 us), else 128 rows.  With
-  // more workgroups than units, heads of 65 to 128 elements keep two small workgroups a unit, whose
-  // starts and ends overlap (408 tokens x 4 on 152, 32 / 32 heads of 96: 26 us, 32 with two groups);
-  // heads up to 64 leave room for two workgroups of two groups, and wider ones have one wave per SIMD
-  // without them.  Up to 128 keys there is nothing to share (21 tokens: 5.8 against 6.2 us).
-  p.tile_rows = 128;
-  p.key_groups = 1;
-  if (max_len > 128) {
-    if (gen::chunk_key_groups(f32, nb, 2) > 1 && planes * tiles_of(64) <= a.n_cu) p.tile_rows = 64;
-    const bool one_each = planes * tiles_of(p.tile_rows) <= a.n_cu;
-    if (one_each || nb <= 2 || nb > 4) p.key_groups = (uint32_t)gen::chunk_key_groups(f32, nb, p.tile_rows / 32);
-  }
-  p.row_tiles = (uint32_t)tiles_of(p.tile_rows);
-  if ((size_t)planes * p.row_tiles > 0x7fffffffu) return hipErrorInvalidValue;
-  const uint32_t items = planes * p.row_tiles;
-  const uint32_t tiles = (max_len + 63) / 64;
-  p.n_split = 1;
-  p.split_len = tiles * 64;
-  p.turn_at = items <= 2 * a.n_cu && planes <= a.n_cu ? a.n_cu / planes : p.row_tiles;
-  // too few workgroups to fill the part: split the key range, in pieces of at least 512 keys or, four
-  // waves a workgroup, 256
-  const uint32_t slots = (es == 2 && nb <= 4 && p.key_groups == 1 ? 2 : 1) * a.n_cu;
-  if (2 * (size_t)items <= slots && tiles >= 8 && room > 1) {
-    const double tile_us = (es == 4 ? 1.7 : 0.5) * nb;
-    const double split_us = (double)planes * rows * (32 * nb + 2) * 8 / 4e6;
-    const KeySplit ks = plan_key_split(tiles, items, slots, p.key_groups > 1 ? 8 : 4, (uint32_t)(room < 4096 ? room : 4096), split_us / tile_us);
-    if (ks.n_split > 1) {
-      p.n_split = ks.n_split;
-      p.split_len = ks.split_tiles * 64;
-    }
-  }
+  gen::GeneralCall call;
+  call.planes = planes;
+  call.group = a.group;
+  call.interval = a.position_interval;
+  call.max_len = a.position_index + a.position_interval;
+  call.n_cu = a.n_cu;
+  call.head_size = head_size;
+  call.f32 = a.dtype == 2;
+  call.vec = vec;
+  call.room = p.part_o ? a.prefill_part_rows / ((size_t)planes * rows) : 1;
+  const gen::GeneralPlan plan = gen::general_plan(call);
+  const int nb = plan.nb;
+  p.row_tiles = plan.row_tiles;
+  p.tile_rows = plan.tile_rows;
+  p.key_groups = plan.key_groups;
+  p.turn_at = plan.turn_at;
+  p.n_split = plan.n_split;
+  p.split_len = plan.split_len;
+  if (plan.kernel == gen::kGeneralRows) return gen::launch_rows(p, a.dtype, planes, stream);
+  if ((size_t)planes * p.row_tiles * (plan.kernel == gen::kGeneralStep ? p.n_split : 1) > 0x7fffffffu) return hipErrorInvalidValue;
+  if (plan.kernel == gen::kGeneralStep) return gen::launch_general_step(p, a.dtype, nb, vec, planes, stream);
   const hipError_t e = gen::launch_general_chunk(p, a.dtype, nb, vec, planes, stream);
   if (e != hipSuccess || p.n_split == 1) return e;
   const uint32_t pitch = 32 * (uint32_t)nb;

@@ -1,18 +1,19 @@
 // Shared parts of the attention kernels for shapes other than 128-wide 16-bit heads: any head
-// size up to 256 and binary32 storage (attn_general.hip: dispatch and merge;
-// attn_general_chunk.hip: many query rows per K/V plane; attn_general_step.hip: few).
+// size up to 256 and binary32 storage (general_plan.hpp: which kernel, what cut; attn_general.hip:
+// launches, merge and the row kernel; attn_general_chunk.hip: many query rows per K/V plane;
+// attn_general_step.hip: few).
 #pragma once
 
 #include <type_traits>
 
 #include "common.hpp"
+#include "general_plan.hpp"
 #include "kernels.hpp"
 
 namespace ellm {
 namespace gen {
 
 constexpr int kMaxHead = 256;
-constexpr uint32_t kGeneralStepRows = 16;    // and of the step kernel
 
 struct F32 {};   // binary32 storage
 
@@ -70,6 +71,7 @@ struct GeneralArgs {
   uint32_t rows;                 // query rows of a plane: interval x group; row r = token r / group, head r % group
   uint32_t negate_q;             // scale < 0: the sign is folded into the query rows so that c > 0
   float c;                       // |scale| x log2(e), > 0
+  float scale;
   // Key range split over workgroups: n_split pieces of split_len keys.  Partial row of plane row
   // r and split s: (plane x rows + r) x n_split + s of part_o [..][pitch] (weighted sums) and
   // part_ml [..][2] (reference exponent in log2 units, denominator).
@@ -106,7 +108,10 @@ __device__ __forceinline__ uint64_t scalar64(uint64_t v) {  // tells the compile
 // VEC: rows start on 16-byte boundaries and hold whole 16-byte pieces.  The pieces of a chunk of
 // keys are fetched with buffer loads whose descriptor ends at the last key that counts, so later
 // rows read as zeros; a piece past the head's end is given an offset no descriptor covers.
-// Otherwise a piece is gathered element by element under the same two bounds.
+// Otherwise a piece is sixteen bytes from anywhere inside its row (global loads need no alignment): the
+// row's last ones where the piece goes past the head, put right (settle_piece) when they have arrived, so
+// that a step's loads are in flight together (element by element under the two bounds, each load was
+// waited for: 64 tokens x 2, 4 / 4 heads of 129, binary16 32 us); heads shorter than a piece by elements.
 constexpr uint32_t kNowhere = 0xf0000000u;
 constexpr uint64_t kMaxRecords = 0x80000000u;   // 64 rows of at most 2^25 bytes
 
@@ -119,17 +124,37 @@ __device__ __forceinline__ __amdgpu_buffer_rsrc_t chunk_rsrc(uint64_t plane, uin
 template <typename S>
 __device__ __forceinline__ u32x4 gather_piece(const typename Store<S>::E* plane, size_t stride_pos, uint32_t key,
                                               uint32_t end, uint32_t e0, uint32_t head_size) {
+  typedef u32x4 AnyPlace __attribute__((aligned(2)));
+  constexpr uint32_t kPiece = Store<S>::kPiece;
+  const typename Store<S>::E* row = plane + (size_t)min(key, end - 1) * stride_pos;
+  if (head_size >= kPiece) return *(const AnyPlace*)(row + min(e0, head_size - kPiece));
   u32x4 w = {0, 0, 0, 0};
-  if (key < end) {
-    const typename Store<S>::E* row = plane + (size_t)key * stride_pos;
 #pragma unroll
-    for (int e = 0; e < Store<S>::kPiece; ++e)
-      if (e0 + e < head_size) {
-        if constexpr (std::is_same<S, F32>::value) w[e] = __builtin_bit_cast(uint32_t, row[e0 + e]);
-        else w[e >> 1] |= (uint32_t)row[e0 + e] << (16 * (e & 1));
-      }
+  for (uint32_t e = 0; e < kPiece; ++e) {
+    const typename Store<S>::E x = row[min(e, head_size - 1)];
+    if constexpr (std::is_same<S, F32>::value) w[e] = e < head_size ? __builtin_bit_cast(uint32_t, x) : 0u;
+    else w[e >> 1] |= (e < head_size ? (uint32_t)x : 0u) << (16 * (e & 1));
   }
   return w;
+}
+
+// The piece that was asked for, of what gather_piece fetched: the row's last elements moved down to its
+// start, zeros past the head and past the keys.
+template <typename S>
+__device__ __forceinline__ u32x4 settle_piece(u32x4 w, uint32_t key, uint32_t end, uint32_t e0, uint32_t head_size) {
+  constexpr uint32_t kPiece = Store<S>::kPiece, kBits = 128 / kPiece;
+  const uint32_t from = head_size >= kPiece ? min(e0, head_size - kPiece) : 0u;
+  const uint32_t bits = (e0 - from) * kBits;
+  uint64_t lo = (uint64_t)w[0] | (uint64_t)w[1] << 32, hi = (uint64_t)w[2] | (uint64_t)w[3] << 32;
+  if (bits >= 64) {
+    lo = hi;
+    hi = 0;
+  }
+  const uint32_t rest = bits & 63;
+  lo = lo >> rest | (hi << 1) << (63 - rest);
+  hi >>= rest;
+  const bool any = key < end && e0 < head_size;
+  return any ? u32x4{(uint32_t)lo, (uint32_t)(lo >> 32), (uint32_t)hi, (uint32_t)(hi >> 32)} : u32x4{0, 0, 0, 0};
 }
 
 // Query row piece: elements e0 .. of the row, zeros past the head's end, sign folded in.
@@ -139,7 +164,7 @@ __device__ __forceinline__ u32x4 query_piece(const GeneralArgs& p, const typenam
   if constexpr (VEC) {
     if (e0 < p.head_size) w = load16(row + e0);
   } else {
-    w = gather_piece<S>(row, 0, 0, 1, e0, p.head_size);
+    w = settle_piece<S>(gather_piece<S>(row, 0, 0, 1, e0, p.head_size), 0, 1, e0, p.head_size);
   }
   if (p.negate_q) w ^= std::is_same<S, F32>::value ? 0x80000000u : 0x80008000u;
   return w;
@@ -276,22 +301,6 @@ __device__ __forceinline__ float largest_of(float m, float a, float b) {   // on
 // 32 elements of the padded head, vec as above.
 hipError_t launch_general_chunk(const GeneralArgs& p, int dtype, int nb, bool vec, uint32_t planes, hipStream_t stream);
 hipError_t launch_general_step(const GeneralArgs& p, int dtype, int nb, bool vec, uint32_t planes, hipStream_t stream);
-
-// Blocks of 32 elements the kernels pad a head to: 1, 2, 3, 4, 6 or 8 (2, 4 or 8 for rows that are
-// not made of whole aligned 16-byte pieces).
-inline int head_blocks(uint32_t head_size, bool vec) {
-  const int n = (int)((head_size + 31) / 32);
-  if (!vec) return n <= 2 ? 2 : n <= 4 ? 4 : 8;
-  return n <= 4 ? n : n <= 6 ? 6 : 8;
-}
-
-// Key groups of a chunk kernel's workgroup of `row_blocks` x 32 query rows: as many as its registers (a
-// wave's queries, accumulators and scores) and LDS (two steps of K and V a group) allow.
-constexpr int chunk_key_groups(bool f32, int nb, int row_blocks) {
-  if (f32) return 1;
-  if (row_blocks == 4) return nb <= 6 ? 2 : 1;
-  return nb <= 4 ? 4 : 1;
-}
 
 // f(std::integral_constant<int, blocks>, std::bool_constant<vec>) for a value of head_blocks().
 template <typename F>

@@ -131,8 +131,9 @@ void general_chunk_kernel(GeneralArgs p) {
   }
 
   const size_t plane_at = seq_plane_offset(p.seq_offsets, p.kv_stride_seq, seq) + (size_t)kvh * p.kv_stride_head;
-  const uint64_t kplane = scalar64((uint64_t)((const E*)p.k + plane_at)), vplane = scalar64((uint64_t)((const E*)p.v + plane_at));
-  const E *kp = (const E*)kplane, *vp = (const E*)vplane;
+  const E* kp = (const E*)p.k + plane_at;
+  const E* vp = (const E*)p.v + plane_at;
+  const uint64_t kplane = scalar64((uint64_t)kp), vplane = scalar64((uint64_t)vp);
   const uint64_t pos_bytes = (uint64_t)p.kv_stride_pos * sizeof(E);
   const uint64_t valid = scalar64((uint64_t)(end - 1) * pos_bytes + (uint64_t)p.head_size * sizeof(E));
   uint32_t off0[X::kPlaces], lds_k0[X::kPlaces], lds_v0[X::kPlaces];
@@ -182,6 +183,14 @@ void general_chunk_kernel(GeneralArgs p) {
     }
   };
   auto store_step = [&](uint32_t step) {
+    if constexpr (!VEC) {
+      const uint32_t kb = k0 + step * kKeys;
+#pragma unroll
+      for (int i = 0; i < kPieces; ++i) {
+        kst[i] = settle_piece<S>(kst[i], kb + (off(i) & 0xffffu), end, off(i) >> 16, p.head_size);
+        vst[i] = settle_piece<S>(vst[i], kb + (off(i) & 0xffffu), end, off(i) >> 16, p.head_size);
+      }
+    }
     store_rows(step, kst, lds_k, X::kKBuf);
     store_rows(step, vst, lds_v, X::kVBuf);
     look_at(step);

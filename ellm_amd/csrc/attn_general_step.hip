@@ -137,6 +137,10 @@ __global__ __launch_bounds__(kThreads, (StepShape<S, NB>::kOccupancy)) void gene
     const uint32_t kb = k0 + chunk * X::kKeys;
 #pragma unroll
     for (int i = 0; i < kPieces; ++i) {
+      if constexpr (!VEC) {
+        kst[i] = settle_piece<S>(kst[i], kb + (off[i] & 0xffffu), end, off[i] >> 16, p.head_size);
+        vst[i] = settle_piece<S>(vst[i], kb + (off[i] & 0xffffu), end, off[i] >> 16, p.head_size);
+      }
       *(LdsU32x4*)lds_k[i] = kst[i];
       // (the V row of a piece: same place in a table of another pitch)
       const uint32_t pi = lane + kWave * i;

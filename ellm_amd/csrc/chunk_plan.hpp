@@ -10,9 +10,19 @@
 // one partial row (128 + 2 floats) per query row, `split_cost` tiles in all.
 #pragma once
 
+#include <stddef.h>
 #include <stdint.h>
 
 namespace ellm {
+
+// Partial rows (128 + 2 floats each) a handle keeps for calls whose key range is split: 256
+// splits of every row it can be asked for, at most 512 per compute unit (68 MB on 256 units).
+inline size_t prefill_workspace_rows(uint32_t max_interval, uint32_t batch_capacity, uint32_t n_q_heads, uint32_t n_cu) {
+  if (max_interval < 2) return 0;  // single-token calls take the other kernel
+  const size_t rows = (size_t)max_interval * batch_capacity * n_q_heads;
+  const size_t cap = (size_t)512 * n_cu;
+  return rows * 256 < cap ? rows * 256 : cap;
+}
 
 struct KeySplit {
   uint32_t split_tiles;  // tiles per piece (the last piece of a walk may be shorter)

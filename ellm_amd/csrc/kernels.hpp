@@ -5,6 +5,7 @@
 #include <stddef.h>
 #include <stdint.h>
 
+#include "chunk_plan.hpp"
 #include "decode_plan.hpp"
 
 struct ellm_attn_desc;
@@ -74,9 +75,6 @@ struct AttnArgs {
   uint32_t n_cu;
   PendingRows pending;   // single-token path only
 };
-// Partial rows the chunk path's workspace holds for an operator of this shape (0: none needed).
-size_t prefill_workspace_rows(uint32_t max_interval, uint32_t batch_capacity, uint32_t n_q_heads,
-                              uint32_t n_cu);
 
 hipError_t launch_decode(const AttnArgs& a, hipStream_t stream);
 // Per-sequence positions, the planes' keys dealt evenly to `wgs` workgroups (decode_balanced.hip):
@@ -86,14 +84,6 @@ bool decode_balanced_takes(const DecodeWorkspace& w, uint32_t batch, uint32_t n_
 hipError_t launch_decode_balanced(const AttnArgs& a, uint32_t wgs, hipStream_t stream);
 hipError_t launch_prefill(const AttnArgs& a, hipStream_t stream);
 // Any head size up to 256 and binary32 storage (dtype 2): chunk and single-token calls alike.
-// Workspace of such an operator: partial rows (pitch floats each, then 2 of maximum and sum) and
-// arrival counters, in the chunk path's fields of AttnArgs.
-struct GeneralWorkspace {
-  size_t rows, counters;
-  uint32_t pitch;
-};
-GeneralWorkspace general_workspace(uint32_t max_interval, uint32_t batch_capacity, uint32_t n_q_heads,
-                                   uint32_t n_kv_heads, uint32_t head_size, uint32_t n_cu);
 hipError_t launch_attn_general(const AttnArgs& a, uint32_t head_size, hipStream_t stream);
 
 // Where the rows of a cache layer live: plane of (sequence, head) at

@@ -1153,16 +1153,6 @@ hipError_t launch_pingpong(const AttnArgs& a, hipStream_t stream) {
 
 }  // namespace
 
-// Partial rows (128 + 2 floats each) a handle keeps for calls whose key range is split: 256
-// splits of every row it can be asked for, at most 512 per compute unit (68 MB on 256 units).
-size_t prefill_workspace_rows(uint32_t max_interval, uint32_t batch_capacity, uint32_t n_q_heads,
-                              uint32_t n_cu) {
-  if (max_interval < 2) return 0;  // single-token calls take the other kernel
-  const size_t rows = (size_t)max_interval * batch_capacity * n_q_heads;
-  const size_t cap = (size_t)512 * n_cu;
-  return rows * 256 < cap ? rows * 256 : cap;
-}
-
 hipError_t launch_prefill(const AttnArgs& a, hipStream_t stream) {
   if (a.dtype == 0) return launch_pingpong<F16>(a, stream);
   return launch_pingpong<BF16>(a, stream);

@@ -1,0 +1,61 @@
+"""The library's own choice of kernel for a call, from the host headers it compiles itself
+(ellm_amd/csrc/*_plan.hpp), for tests that say which kernel their shapes reach.  256 compute units."""
+import atexit
+import functools
+import os
+import shutil
+import subprocess
+import tempfile
+
+import pytest
+
+CSRC = os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))), "ellm_amd", "csrc")
+
+SOURCE = r"""
+#include <cstdio>
+#include <cstdlib>
+#include "general_plan.hpp"
+using namespace ellm;
+// head size, bytes an element, batch capacity, batch, query heads, key-value heads, most positions a call,
+// position_index, interval, whole aligned pieces
+int main(int, char** v) {
+  uint32_t a[11];
+  for (int i = 1; i <= 10; ++i) a[i] = (uint32_t)strtoul(v[i], nullptr, 10);
+  const gen::GeneralWorkspace w = gen::general_workspace(a[7], a[3], a[5], a[6], a[1], 256);
+  gen::GeneralCall c;
+  c.planes = a[4] * a[6];
+  c.group = a[5] / a[6];
+  c.interval = a[9];
+  c.max_len = a[8] + a[9];
+  c.n_cu = 256;
+  c.head_size = a[1];
+  c.f32 = a[2] == 4;
+  c.vec = a[10] != 0;
+  c.room = w.rows / (c.planes * c.rows());
+  const gen::GeneralPlan p = gen::general_plan(c);
+  printf("%d %u %u %u %d\n", (int)p.kernel, p.n_split, p.tile_rows, p.key_groups, p.nb);
+}
+"""
+
+
+@functools.lru_cache(maxsize=None)
+def _program():
+    gxx = shutil.which("g++")
+    if not gxx:
+        pytest.skip("no g++")
+    d = tempfile.mkdtemp(prefix="plan_probe_")
+    atexit.register(shutil.rmtree, d, True)
+    with open(os.path.join(d, "probe.cpp"), "w") as f:
+        f.write(SOURCE)
+    exe = os.path.join(d, "probe")
+    subprocess.run([gxx, "-O1", "-std=c++17", "-I", CSRC, "-o", exe, os.path.join(d, "probe.cpp")], check=True)
+    return exe
+
+
+def general_plan(head_size, element_bytes, batch_capacity, batch, q_heads, kv_heads, position_index, interval, vec=None):
+    """(kernel "rows" / "step" / "chunk", key splits, rows per workgroup, key groups, padded head blocks)"""
+    if vec is None:
+        vec = head_size * element_bytes % 16 == 0
+    args = (head_size, element_bytes, batch_capacity, batch, q_heads, kv_heads, interval, position_index, interval, int(vec))
+    out = subprocess.run([_program(), *map(str, args)], check=True, capture_output=True, text=True).stdout.split()
+    return (("rows", "step", "chunk")[int(out[0])], *map(int, out[1:5]))

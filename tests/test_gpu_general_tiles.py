@@ -7,6 +7,7 @@ import numpy as np
 import pytest
 
 import oracle_lib as orc
+import plan_probe
 from test_gpu_general_heads import _check, _rand, _run
 
 pytestmark = pytest.mark.gpu
@@ -42,13 +43,45 @@ CASES = [
     ("step_f32_h256_splits", orc.F32, 2, 8, 1, 256, 1030, 1027, 1),
     ("step_f32_h32", orc.F32, 1, 2, 2, 32, 700, 650, 1),
     ("step_h5_splits", orc.BF16, 1, 3, 1, 5, 600, 599, 1),
+    # binary32 chunks of more rows than the row kernel is taken for: every padded head, one and several splits
+    ("f32_chunk_h20_one_block", orc.F32, 1, 32, 4, 20, 210, 0, 200),
+    ("f32_chunk_h64", orc.F32, 2, 32, 32, 64, 160, 30, 130),
+    ("f32_chunk_h33_any_place", orc.F32, 1, 64, 8, 33, 150, 0, 150),
+    ("f32_chunk_h96_key_split", orc.F32, 2, 16, 2, 96, 1030, 1000, 30),
+    ("f32_chunk_h128_order_turns", orc.F32, 4, 32, 8, 128, 164, 100, 64),
+    ("f32_chunk_h130_any_place", orc.F32, 4, 32, 8, 130, 164, 100, 64),
+    ("f32_chunk_h192", orc.F32, 1, 64, 8, 192, 150, 0, 150),
+    ("f32_chunk_h256_key_split", orc.F32, 1, 8, 2, 256, 1440, 1400, 40),
+    ("f32_chunk_h256", orc.F32, 4, 32, 8, 256, 164, 100, 64),
+    # the row kernel: one turn of keys, one key more, the widest head, a prompt, heads narrower than a piece
+    ("rows_16_keys", orc.F16, 2, 8, 2, 64, 20, 0, 16),
+    ("rows_17_keys", orc.F32, 1, 16, 4, 250, 20, 16, 1),
+    ("rows_16_keys_h250", orc.BF16, 1, 16, 4, 250, 20, 15, 1),
+    ("rows_h1", orc.F16, 2, 2, 1, 1, 12, 7, 4),
+    ("rows_h256_f32", orc.F32, 1, 4, 4, 256, 140, 33, 100),
+    ("rows_h3_f32", orc.F32, 1, 6, 2, 3, 50, 0, 50),
+    ("chunk_h5_narrower_than_a_piece", orc.F16, 1, 8, 2, 5, 300, 100, 150),
+    ("chunk_h3_f32_narrower_than_a_piece", orc.F32, 1, 64, 8, 3, 150, 0, 150),
 ]
+ON_ROWS = {"f32_h256", "f32_h96_three_tiles", "f32_h130_elements_one_by_one"}
+
+
+def _kernel(name):
+    """The kernel a case is there for: by its name, or the one it takes since short walks have one."""
+    if name in ON_ROWS or name.startswith("rows_") and "kernel" not in name and "_tile" not in name:
+        return "rows"
+    return "step" if name.startswith("step") or "step_kernel" in name else "chunk"
+
+
+def element_bytes(dtype):
+    return 4 if dtype == orc.F32 else 2
 
 
 @pytest.mark.parametrize("case", CASES, ids=[c[0] for c in CASES])
 def test_tile_edges(case):
     name, dtype, b, hq, hkv, hs, cap, p0, s = case
     print("case", name, flush=True)
+    assert plan_probe.general_plan(hs, element_bytes(dtype), b, b, hq, hkv, p0, s)[0] == _kernel(name)
     q, k, v = _rand((s, b, hq, hs), 31, dtype), _rand((b, hkv, cap, hs), 32, dtype), _rand((b, hkv, cap, hs), 33, dtype)
     scale = -0.9 / np.sqrt(hs) if hs == 96 else 1.0 / np.sqrt(hs)   # (a negative scale once per type)
     want, want_lse = orc.attention(q, k, v, scale, dtype, position_index=p0)
@@ -57,17 +90,20 @@ def test_tile_edges(case):
 
 
 # (head size, q heads, kv heads, position_index, interval): chunks and single-token steps, one and several splits
-BINARY32 = [(128, 8, 8, 169, 16), (128, 8, 2, 0, 185), (64, 8, 8, 0, 92), (256, 4, 4, 60, 64), (128, 8, 8, 291, 1),
-            (64, 8, 2, 1900, 1), (256, 4, 1, 700, 1), (100, 4, 4, 60, 1)]
+BINARY32 = [(128, 8, 8, 169, 16), (128, 32, 8, 0, 185), (64, 32, 8, 300, 100), (256, 64, 8, 0, 150), (128, 8, 2, 1400, 40),
+            (128, 8, 8, 291, 1), (64, 8, 2, 1900, 1), (256, 4, 1, 700, 1), (100, 4, 4, 60, 1), (256, 4, 4, 60, 64)]
 
 
 @pytest.mark.parametrize("case", BINARY32, ids=["h%d_%dq%dkv_%d+%d" % c for c in BINARY32])
 def test_binary32_sums_stay_in_short_chains(case):
     """Error against 64-bit arithmetic.  Rounding of a score's sum, of its exponent's argument, of the
     exponential and of the weighted sum each add about 2^-24 to a row (2-norm): together 1.1e-7 to 1.7e-7
-    here, and the bound is 2^-22.  One chain of sums over a head of 128 or 256 gave 2.6e-7 to 5.3e-7."""
+    here, and the bound is 2^-22.  One chain of sums over a head of 128 or 256 gave 2.6e-7 to 5.3e-7.  The last
+    case runs row by row."""
     hs, hq, hkv, p0, s = case
     print("case", case, flush=True)
+    kernel = "step" if s == 1 or s * hq // hkv <= 32 else "rows" if case == BINARY32[-1] else "chunk"
+    assert plan_probe.general_plan(hs, 4, 1, 1, hq, hkv, p0, s)[0] == kernel
     cap = p0 + s
     q, k, v = _rand((s, 1, hq, hs), 51, orc.F32), _rand((1, hkv, cap, hs), 52, orc.F32), _rand((1, hkv, cap, hs), 53, orc.F32)
     scale = np.float32(1.0 / np.sqrt(hs))
@@ -132,11 +168,12 @@ def test_an_infinite_value_that_a_row_sees(case, dtype):
     _check("finite_columns", got[..., 2::3], lse, orc.to_storage(np.ascontiguousarray(w[..., 2::3]), dtype), want_lse, dtype, 1)
 
 
-@pytest.mark.parametrize("dtype,hs", [(orc.BF16, 256), (orc.BF16, 64), (orc.F32, 64)], ids=["bf16_h256", "bf16_h64", "f32_h64"])
-def test_large_finite_values_under_rising_scores(dtype, hs):
+@pytest.mark.parametrize("dtype,hs,hq", [(orc.BF16, 256, 4), (orc.BF16, 64, 4), (orc.F32, 64, 64)], ids=["bf16_h256", "bf16_h64", "f32_h64"])
+def test_large_finite_values_under_rising_scores(dtype, hs, hq):
     """One value of 1e38 under the highest score, which lies 6.5 binary orders above those of the step of keys
     before it: less than what makes the chunk kernel move its reference, so the weight is 2^6.5 there."""
-    hq, hkv, s, p0 = 4, 2, 50, 90
+    hkv, s, p0 = 2, 50, 90
+    assert plan_probe.general_plan(hs, element_bytes(dtype), 1, 1, hq, hkv, p0, s)[0] == "chunk"
     q, k, v = np.zeros((s, 1, hq, hs), np.float32), np.zeros((1, hkv, p0 + s, hs), np.float32), np.zeros((1, hkv, p0 + s, hs), np.float32)
     q[..., 0] = 1.0
     k[:, :, 70, 0] = 6.5
@@ -147,6 +184,17 @@ def test_large_finite_values_under_rising_scores(dtype, hs):
     want = share[:, None, None, None] * float(orc.from_storage(v, dtype).max())
     err = float(np.abs(got / want - 1.0).max())
     assert err <= (2.0 ** -8 if dtype == orc.BF16 else 1e-6)         # half a unit of bfloat16, binary32 sums
+
+
+@pytest.mark.parametrize("dtype,hs", [(orc.F16, 33), (orc.F32, 256), (orc.BF16, 7)])
+def test_row_kernel_with_a_position_per_sequence(dtype, hs):
+    bcap, b, hq, hkv, cap = 4, 3, 8, 2, 30
+    assert plan_probe.general_plan(hs, element_bytes(dtype), bcap, b, hq, hkv, 15, 1)[0] == "rows"
+    q, k, v = _rand((1, bcap, hq, hs), 71, dtype), _rand((bcap, hkv, cap, hs), 72, dtype), _rand((bcap, hkv, cap, hs), 73, dtype)
+    positions = [15, 0, 9]
+    want, want_lse = orc.attention(q, k, v, 0.2, dtype, positions=np.array(positions + [0], dtype=np.uint32), batch=b)
+    got, lse = _run(q, k, v, 0.2, dtype, batch=b, positions=positions)
+    _check("rows_ragged", got, lse, want, want_lse, dtype, b)
 
 
 def test_repeated_steps_fold_the_same_bits():
