@@ -17,10 +17,10 @@ SOURCE = r"""
 #include "general_plan.hpp"
 using namespace ellm;
 // head size, bytes an element, batch capacity, batch, query heads, key-value heads, most positions a call,
-// position_index, interval, whole aligned pieces
+// position_index, interval, whole aligned pieces, and room for partial rows per query row (0: the workspace's)
 int main(int, char** v) {
-  uint32_t a[11];
-  for (int i = 1; i <= 10; ++i) a[i] = (uint32_t)strtoul(v[i], nullptr, 10);
+  uint32_t a[12];
+  for (int i = 1; i <= 11; ++i) a[i] = (uint32_t)strtoul(v[i], nullptr, 10);
   const gen::GeneralWorkspace w = gen::general_workspace(a[7], a[3], a[5], a[6], a[1], 256);
   gen::GeneralCall c;
   c.planes = a[4] * a[6];
@@ -31,9 +31,9 @@ int main(int, char** v) {
   c.head_size = a[1];
   c.f32 = a[2] == 4;
   c.vec = a[10] != 0;
-  c.room = w.rows / (c.planes * c.rows());
+  c.room = a[11] ? a[11] : w.rows / (c.planes * c.rows());
   const gen::GeneralPlan p = gen::general_plan(c);
-  printf("%d %u %u %u %d\n", (int)p.kernel, p.n_split, p.tile_rows, p.key_groups, p.nb);
+  printf("%d %u %u %u %d %zu\n", (int)p.kernel, p.n_split, p.tile_rows, p.key_groups, p.nb, w.rows);
 }
 """
 
@@ -52,10 +52,11 @@ def _program():
     return exe
 
 
-def general_plan(head_size, element_bytes, batch_capacity, batch, q_heads, kv_heads, position_index, interval, vec=None):
-    """(kernel "rows" / "step" / "chunk", key splits, rows per workgroup, key groups, padded head blocks)"""
+def general_plan(head_size, element_bytes, batch_capacity, batch, q_heads, kv_heads, position_index, interval, vec=None, room=0):
+    """(kernel "rows" / "step" / "chunk", key splits, rows per workgroup, key groups, padded head blocks, the
+    workspace's partial rows)"""
     if vec is None:
         vec = head_size * element_bytes % 16 == 0
-    args = (head_size, element_bytes, batch_capacity, batch, q_heads, kv_heads, interval, position_index, interval, int(vec))
+    args = (head_size, element_bytes, batch_capacity, batch, q_heads, kv_heads, interval, position_index, interval, int(vec), room)
     out = subprocess.run([_program(), *map(str, args)], check=True, capture_output=True, text=True).stdout.split()
-    return (("rows", "step", "chunk")[int(out[0])], *map(int, out[1:5]))
+    return (("rows", "step", "chunk")[int(out[0])], *map(int, out[1:]))
