@@ -165,4 +165,145 @@ inline uint32_t short_prompt_wr(const ChunkShape& c, double other_us) {
   return one < two ? 1 : 2;
 }
 
+// ---- the choice ------------------------------------------------------------------------------
+// A chunk call of 128-wide 16-bit heads, the kernel it runs and how the work is cut.
+constexpr uint32_t kChunkTile = 64;         // keys per tile of the ping-pong and streaming kernels
+constexpr uint32_t kPingpongRowBlocks = 8;  // 32-row blocks of a ping-pong workgroup
+
+struct ChunkCall {
+  uint32_t p0, interval;                    // positions p0 .. p0 + interval - 1
+  uint32_t batch, batch_capacity, n_q_heads, n_kv_heads, n_cu;
+  size_t part_rows;                         // partial rows the workspace holds (0: none)
+};
+
+enum ChunkKernel { kChunkStream, kChunkPingpong, kChunkShort };
+
+struct ChunkPlan {
+  ChunkKernel kernel;
+  uint32_t waves;                           // streaming kernel: 4, 8 or 12
+  uint32_t row_blocks;                      // short-prompt kernel: 32-row blocks a workgroup, 1 or 2
+  uint32_t n_split, split_tiles;            // key range of a plane, in tiles (one split: split_tiles may be 0)
+  // ping-pong workgroup: heads_per_wg heads of a group x tblocks_per_wg blocks of 32 tokens
+  uint32_t heads_per_wg, tblocks_per_wg, head_groups;
+  uint32_t combos, n_wg_tokens;             // independent walks x workgroups along their rows
+  uint32_t xcd_mode;                        // how workgroup ids map to those (see the kernels)
+  uint32_t n_wg;                            // workgroups of the launch, per split
+};
+
+inline uint32_t gcd_u32(uint32_t a, uint32_t b) {
+  while (b) {
+    const uint32_t t = a % b;
+    a = b;
+    b = t;
+  }
+  return a;
+}
+
+// Row tiles and workgroup ids of short_prompt_kernel.
+inline void plan_short_prompt(const ChunkShape& shape, uint32_t wr, ChunkPlan* p) {
+  const uint32_t planes = shape.planes, wg_rows = 32 * wr;
+  p->kernel = kChunkShort;
+  p->row_blocks = wr;
+  p->n_split = 1;
+  p->combos = planes;
+  p->n_wg_tokens = (uint32_t)(((size_t)shape.interval * shape.group + wg_rows - 1) / wg_rows);
+  // Planes that are no multiple of the XCDs, or that together overflow their L2s, go to one XCD each
+  // (40 tokens x 21 sequences on 1250, 84 planes: 55.7 -> 39.9 us); else all planes advance together,
+  // longest rows first over the whole call (512 tokens x 32 heads: 10.8 against 12.8 us).
+  const double xcd_mb = planes / 8.0 * shape.keys() * 512e-6;
+  p->xcd_mode = planes <= 8 && 8 % planes == 0 ? 1 : planes >= 32 && (planes % 8 || xcd_mb > 8.0) ? 2 : 0;
+  p->n_wg = planes * p->n_wg_tokens;
+  if (p->xcd_mode == 1) p->n_wg = 8 * ((p->n_wg_tokens + 8 / planes - 1) / (8 / planes));
+  if (p->xcd_mode == 2) p->n_wg = (planes + 7) / 8 * 8 * p->n_wg_tokens;
+}
+
+inline ChunkPlan plan_chunk(const ChunkCall& c) {
+  ChunkPlan p = {};
+  const uint32_t group = c.n_q_heads / c.n_kv_heads, planes = c.batch * c.n_kv_heads;
+  const ChunkShape shape = {c.p0, c.interval, group, planes, c.n_cu};
+  p.heads_per_wg = gcd_u32(group, kPingpongRowBlocks);
+  p.tblocks_per_wg = kPingpongRowBlocks / p.heads_per_wg;
+  p.head_groups = group / p.heads_per_wg;
+  const uint32_t wg_tokens = 32 * p.tblocks_per_wg;
+  p.n_wg_tokens = (c.interval + wg_tokens - 1) / wg_tokens;
+  p.combos = planes * p.head_groups;
+  p.xcd_mode = (p.combos <= 8 && 8 % p.combos == 0) ? 1 : 0;
+
+  // Few query rows per plane on a cache long enough to be worth streaming: one workgroup
+  // covers all rows of a GQA group, the key range is split until there are two
+  // workgroups per compute unit (splits of at least 256 keys), as far as the workspace holds
+  // the partial rows.
+  const uint32_t all_tiles = (c.p0 + c.interval - 1) / kChunkTile + 1;
+  const size_t all_rows = (size_t)c.interval * c.batch_capacity * c.n_q_heads;
+  const size_t plane_rows = (size_t)c.interval * group;
+  const size_t room = c.part_rows ? c.part_rows / all_rows : 1;
+  const uint32_t max_split = (uint32_t)(room < 4096 ? room : 4096);
+  // what one more partial row per query row costs: written and read once, at about 4 TB/s
+  const double split_us = (double)c.interval * c.batch * c.n_q_heads * (128 + 2) * 8 / 4e6;
+  if (plane_rows <= 384 && all_tiles >= 8) {
+    // workgroups of four waves: two per compute unit (with one chunk in flight three were
+    // better); of eight or twelve waves: one.  Pieces of at least four tiles.
+    p.waves = plane_rows <= 128 ? 4 : plane_rows <= 256 ? 8 : 12;
+    const uint32_t slots = (p.waves == 4 ? 2 : 1) * c.n_cu;
+    // a workgroup's time per tile (us, measured on 24 sequences x 8192 keys)
+    const double tile_us = p.waves == 8 ? 2.0 : 2.5;
+    if (p.waves == 4) {
+      // Two workgroups share a compute unit's throughput, so a slot that opens early is not
+      // spare capacity: equal pieces, never more workgroups than slots (24 sequences on 8192
+      // keys, 2 / 8 tokens: 67.6 / 73.1 us; as 5 pieces of 25 tiles and one of 4: 70.1 / 78.9)
+      uint32_t want = slots / planes;
+      if (want > max_split) want = max_split;
+      if (want > all_tiles / 4) want = all_tiles / 4;
+      if (want < 1) want = 1;
+      p.split_tiles = (all_tiles + want - 1) / want;
+      p.n_split = (all_tiles + p.split_tiles - 1) / p.split_tiles;
+    } else {
+      const KeySplit ks = plan_key_split(all_tiles, planes, slots, 4, max_split, split_us / tile_us);
+      p.split_tiles = ks.split_tiles;
+      p.n_split = ks.n_split;
+    }
+    // enough workgroups to be worth it (a lone sequence with one split would leave the part idle)
+    if ((size_t)planes * p.n_split * 2 >= c.n_cu || planes * p.n_split >= p.combos * p.n_wg_tokens) {
+      if (const uint32_t wr = short_prompt_wr(shape, chunk_stream_us(shape, p.waves, {p.split_tiles, p.n_split}))) {
+        plan_short_prompt(shape, wr, &p);
+        return p;
+      }
+      p.kernel = kChunkStream;
+      p.tblocks_per_wg = (c.interval + 31) / 32;  // (the merge derives every row's live splits from the chunk's last token)
+      p.n_wg = planes;
+      return p;
+    }
+  }
+
+  p.kernel = kChunkPingpong;
+  if (p.xcd_mode) {
+    const uint32_t per = 8 / p.combos;
+    p.n_wg = 8 * ((p.n_wg_tokens + per - 1) / per);
+  } else {
+    p.n_wg = p.combos * p.n_wg_tokens;
+  }
+  // Few row blocks on a long cache: split the key range over more workgroups, as far as the
+  // workspace holds the partial rows (plan_key_split weighs the longest chain of pieces a
+  // compute unit runs against the partial rows every piece adds).
+  p.n_split = 1;
+  p.split_tiles = 0;
+  const uint32_t base = p.combos * p.n_wg_tokens;
+  // Only while the unsplit launch leaves at least half of the compute units idle: with more
+  // of them busy the part runs this kernel at its power limit, idle units or not, and a split
+  // only adds the partial rows (64 tokens x 24 sequences on 8192 keys, 192 workgroups: 229 us
+  // unsplit, 235 us as pieces of 97 + 32 tiles on all 256 units).
+  if (c.part_rows && 2 * base <= c.n_cu && all_tiles >= 16) {
+    // pieces of at least eight tiles (each pays the pipeline's first and last step); 1.9 us a
+    // tile and workgroup (measured, 64 tokens x 24 sequences on 8192 keys)
+    const KeySplit ks = plan_key_split(all_tiles, base, c.n_cu, 8, max_split, split_us / 1.9);
+    if (ks.n_split > 1) {
+      p.split_tiles = ks.split_tiles;
+      p.n_split = ks.n_split;
+    }
+  }
+  if (const uint32_t wr = short_prompt_wr(shape, pingpong_us(shape, base, {p.split_tiles, p.n_split})))
+    plan_short_prompt(shape, wr, &p);
+  return p;
+}
+
 }  // namespace ellm

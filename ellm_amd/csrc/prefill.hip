@@ -977,18 +977,20 @@ __global__ __launch_bounds__(256) void prefill_merge_kernel(PrefillKernelArgs p,
   if (p.lse && dq == 0) p.lse[row] = (m + fast_log2(l)) * kLn2;
 }
 
-uint32_t gcd_u32(uint32_t a, uint32_t b) {
-  while (b) {
-    const uint32_t t = a % b;
-    a = b;
-    b = t;
-  }
-  return a;
-}
-
 template <typename T>
-hipError_t launch_pingpong(const AttnArgs& a, hipStream_t stream) {
-  constexpr uint32_t kRowBlocks = kPpWaves;
+hipError_t launch_chunk(const AttnArgs& a, hipStream_t stream) {
+  static_assert(kPingpongRowBlocks == kPpWaves && kChunkTile == kBK, "what the plan is made for");
+  ChunkCall call;
+  call.p0 = a.position_index;
+  call.interval = a.position_interval;
+  call.batch = a.batch;
+  call.batch_capacity = a.batch_pitch;
+  call.n_q_heads = a.n_q_heads;
+  call.n_kv_heads = a.n_kv_heads;
+  call.n_cu = a.n_cu;
+  call.part_rows = a.prefill_part_o ? a.prefill_part_rows : 0;
+  const ChunkPlan plan = plan_chunk(call);
+
   PrefillKernelArgs p;
   p.q = (const uint16_t*)a.q;
   p.k = (const uint16_t*)a.k;
@@ -1004,13 +1006,14 @@ hipError_t launch_pingpong(const AttnArgs& a, hipStream_t stream) {
   p.n_q_heads = a.n_q_heads;
   p.n_kv_heads = a.n_kv_heads;
   p.group = a.group;
-  p.heads_per_wg = gcd_u32(a.group, kRowBlocks);
-  p.tblocks_per_wg = kRowBlocks / p.heads_per_wg;
-  p.head_groups = a.group / p.heads_per_wg;
-  const uint32_t wg_tokens = 32 * p.tblocks_per_wg;
-  p.n_wg_tokens = (a.position_interval + wg_tokens - 1) / wg_tokens;
-  p.combos = a.batch * a.n_kv_heads * p.head_groups;
-  p.xcd_mode = (p.combos <= 8 && 8 % p.combos == 0) ? 1 : 0;
+  p.heads_per_wg = plan.heads_per_wg;
+  p.tblocks_per_wg = plan.tblocks_per_wg;
+  p.head_groups = plan.head_groups;
+  p.n_wg_tokens = plan.n_wg_tokens;
+  p.combos = plan.combos;
+  p.xcd_mode = plan.xcd_mode;
+  p.n_split = plan.n_split;
+  p.split_tiles = plan.split_tiles;
   p.position_index = a.position_index;
   p.interval = a.position_interval;
   float c = a.scale * kLog2e;
@@ -1018,144 +1021,48 @@ hipError_t launch_pingpong(const AttnArgs& a, hipStream_t stream) {
   c = c < 0.0f ? -c : c;
   // scale == 0 (uniform attention): a tiny positive c keeps -inf * c == -inf for masked keys
   p.c = c > 0.0f ? c : 1e-37f;
-
   p.part_o = a.prefill_part_o;
   p.part_ml = a.prefill_part_ml;
-  auto merge_launch = [&]() {
-    const size_t items = (size_t)a.position_interval * a.batch * a.n_q_heads * (kHeadDim / 4);
-    auto merge = [&](auto kernel, size_t lanes) {
-      hipLaunchKernelGGL(kernel, dim3((uint32_t)((items * lanes + 255) / 256)), dim3(256), 0, stream, p, a.batch);
-      return hipGetLastError();
-    };
-    // lanes per item: more when there are many splits to walk, as long as the grid stays small
-    constexpr size_t kLanesMax = (size_t)1 << 21;
-    if (p.n_split > 32 && items * 64 <= kLanesMax) return merge(prefill_merge_kernel<T, 64>, 64);
-    if (p.n_split > 8 && items * 8 <= kLanesMax) return merge(prefill_merge_kernel<T, 8>, 8);
-    return merge(prefill_merge_kernel<T, 1>, 1);
-  };
 
-  // Short prompts and short chunks on short caches (short_prompt_wr, chunk_plan.hpp)
-  const ChunkShape shape = {a.position_index, a.position_interval, a.group, a.batch * a.n_kv_heads, a.n_cu};
-  auto short_launch = [&](uint32_t wr) {
-    const uint32_t planes = shape.planes, wg_rows = 32 * wr;
-    p.combos = planes;
-    p.n_wg_tokens = (uint32_t)(((size_t)a.position_interval * a.group + wg_rows - 1) / wg_rows);
-    // Planes that are no multiple of the XCDs, or that together overflow their L2s, go to one XCD each
-    // (40 tokens x 21 sequences on 1250, 84 planes: 55.7 -> 39.9 us); else all planes advance together,
-    // longest rows first over the whole call (512 tokens x 32 heads: 10.8 against 12.8 us).
-    const double xcd_mb = planes / 8.0 * (a.position_index + a.position_interval) * 512e-6;
-    p.xcd_mode = planes <= 8 && 8 % planes == 0 ? 1 : planes >= 32 && (planes % 8 || xcd_mb > 8.0) ? 2 : 0;
-    uint32_t n = planes * p.n_wg_tokens;
-    if (p.xcd_mode == 1) n = 8 * ((p.n_wg_tokens + 8 / planes - 1) / (8 / planes));
-    if (p.xcd_mode == 2) n = (planes + 7) / 8 * 8 * p.n_wg_tokens;
-    if (wr == 2)
-      hipLaunchKernelGGL((short_prompt_kernel<T, 2, 2>), dim3(n), dim3(4 * kWave), 0, stream, p);
+  const dim3 grid(plan.n_wg, plan.n_split);
+  auto go = [&](auto kernel, uint32_t threads) { hipLaunchKernelGGL(kernel, grid, dim3(threads), 0, stream, p); };
+  if (plan.kernel == kChunkShort) {
+    if (plan.row_blocks == 2)
+      go(short_prompt_kernel<T, 2, 2>, 4 * kWave);
     else
-      hipLaunchKernelGGL((short_prompt_kernel<T, 1, 4>), dim3(n), dim3(4 * kWave), 0, stream, p);
+      go(short_prompt_kernel<T, 1, 4>, 4 * kWave);
+  } else if (plan.kernel == kChunkStream) {
+    if (plan.waves == 4)
+      go(chunk_stream_kernel<T, 4>, 4 * kWave);
+    else if (plan.waves == 8)
+      go(chunk_stream_kernel<T, 8>, 8 * kWave);
+    else
+      go(chunk_stream_kernel<T, 12>, 12 * kWave);
+  } else if (plan.n_split == 1) {
+    go(prefill_pingpong_kernel<T, false>, kPpThreads);
+  } else {
+    go(prefill_pingpong_kernel<T, true>, kPpThreads);
+  }
+  const hipError_t e = hipGetLastError();
+  if (e != hipSuccess || plan.n_split == 1) return e;
+
+  const size_t items = (size_t)a.position_interval * a.batch * a.n_q_heads * (kHeadDim / 4);
+  auto merge = [&](auto kernel, size_t lanes) {
+    hipLaunchKernelGGL(kernel, dim3((uint32_t)((items * lanes + 255) / 256)), dim3(256), 0, stream, p, a.batch);
     return hipGetLastError();
   };
-
-  // Few query rows per plane on a cache long enough to be worth streaming: one workgroup
-  // covers all rows of a GQA group, the key range is split until there are two
-  // workgroups per compute unit (splits of at least 256 keys), as far as the workspace holds
-  // the partial rows.
-  const uint32_t all_tiles = (a.position_index + a.position_interval - 1) / kBK + 1;
-  const size_t all_rows = (size_t)a.position_interval * a.batch_pitch * a.n_q_heads;
-  const size_t plane_rows = (size_t)a.position_interval * a.group;
-  if (plane_rows <= 384 && all_tiles >= 8) {
-    const uint32_t planes = a.batch * a.n_kv_heads;
-    // workgroups of four waves: two per compute unit (with one chunk in flight three were
-    // better: see kStDepth); of eight or twelve waves: one.  Pieces of at least four tiles.
-    const uint32_t waves = plane_rows <= 128 ? 4 : plane_rows <= 256 ? 8 : 12;
-    const uint32_t slots = (waves == 4 ? 2 : 1) * a.n_cu;
-    const size_t room = a.prefill_part_o ? a.prefill_part_rows / all_rows : 1;
-    // a workgroup's time per tile (us, measured on 24 sequences x 8192 keys), and what one more
-    // partial row per query row costs: written and read once, at about 4 TB/s
-    const double tile_us = waves == 8 ? 2.0 : 2.5;
-    const double split_us = (double)a.position_interval * a.batch * a.n_q_heads * (kHeadDim + 2) * 8 / 4e6;
-    const uint32_t max_split = (uint32_t)(room < 4096 ? room : 4096);
-    if (waves == 4) {
-      // Two workgroups share a compute unit's throughput, so a slot that opens early is not
-      // spare capacity: equal pieces, never more workgroups than slots (24 sequences on 8192
-      // keys, 2 / 8 tokens: 67.6 / 73.1 us; as 5 pieces of 25 tiles and one of 4: 70.1 / 78.9)
-      uint32_t want = slots / planes;
-      if (want > max_split) want = max_split;
-      if (want > all_tiles / 4) want = all_tiles / 4;
-      if (want < 1) want = 1;
-      p.split_tiles = (all_tiles + want - 1) / want;
-      p.n_split = (all_tiles + p.split_tiles - 1) / p.split_tiles;
-    } else {
-      const KeySplit ks = plan_key_split(all_tiles, planes, slots, 4, max_split, split_us / tile_us);
-      p.split_tiles = ks.split_tiles;
-      p.n_split = ks.n_split;
-    }
-    // enough workgroups to be worth it (a lone sequence with one split would leave the part idle)
-    if ((size_t)planes * p.n_split * 2 >= a.n_cu || planes * p.n_split >= p.combos * p.n_wg_tokens) {
-      if (const uint32_t wr = short_prompt_wr(shape, chunk_stream_us(shape, waves, {p.split_tiles, p.n_split})))
-        return short_launch(wr);
-      p.tblocks_per_wg = (a.position_interval + 31) / 32;  // (the merge derives every row's live splits from the chunk's last token)
-      const dim3 grid(planes, p.n_split);
-      if (waves == 4)
-        hipLaunchKernelGGL((chunk_stream_kernel<T, 4>), grid, dim3(4 * kWave), 0, stream, p);
-      else if (waves == 8)
-        hipLaunchKernelGGL((chunk_stream_kernel<T, 8>), grid, dim3(8 * kWave), 0, stream, p);
-      else
-        hipLaunchKernelGGL((chunk_stream_kernel<T, 12>), grid, dim3(12 * kWave), 0, stream, p);
-      const hipError_t e = hipGetLastError();
-      if (e != hipSuccess || p.n_split == 1) return e;
-      return merge_launch();
-    }
-  }
-
-  uint32_t n_wg;
-  if (p.xcd_mode) {
-    const uint32_t per = 8 / p.combos;
-    n_wg = 8 * ((p.n_wg_tokens + per - 1) / per);
-  } else {
-    n_wg = p.combos * p.n_wg_tokens;
-  }
-  // Few row blocks on a long cache: split the key range over more workgroups, as far as the
-  // workspace holds the partial rows (plan_key_split weighs the longest chain of pieces a
-  // compute unit runs against the partial rows every piece adds).
-  p.n_split = 1;
-  p.split_tiles = 0;
-  const uint32_t base = p.combos * p.n_wg_tokens;
-  const uint32_t max_tiles = (a.position_index + a.position_interval - 1) / kBK + 1;
-  const size_t rows = (size_t)a.position_interval * a.batch_pitch * a.n_q_heads;
-  // Only while the unsplit launch leaves at least half of the compute units idle: with more
-  // of them busy the part runs this kernel at its power limit, idle units or not, and a split
-  // only adds the partial rows (64 tokens x 24 sequences on 8192 keys, 192 workgroups: 229 us
-  // unsplit, 235 us as pieces of 97 + 32 tiles on all 256 units).
-  if (a.prefill_part_o && 2 * base <= a.n_cu && max_tiles >= 16) {
-    // pieces of at least eight tiles (each pays the pipeline's first and last step); 1.9 us a
-    // tile and workgroup (measured, 64 tokens x 24 sequences on 8192 keys)
-    const size_t room = a.prefill_part_rows / rows;
-    const double split_us = (double)a.position_interval * a.batch * a.n_q_heads * (kHeadDim + 2) * 8 / 4e6;
-    const KeySplit ks = plan_key_split(max_tiles, base, a.n_cu, 8, (uint32_t)(room < 4096 ? room : 4096),
-                                       split_us / 1.9);
-    if (ks.n_split > 1) {
-      p.split_tiles = ks.split_tiles;
-      p.n_split = ks.n_split;
-    }
-  }
-  if (const uint32_t wr = short_prompt_wr(shape, pingpong_us(shape, base, {p.split_tiles, p.n_split})))
-    return short_launch(wr);
-  if (p.n_split <= 1) {
-    p.n_split = 1;
-    hipLaunchKernelGGL((prefill_pingpong_kernel<T, false>), dim3(n_wg), dim3(kPpThreads), 0, stream, p);
-    return hipGetLastError();
-  }
-  hipLaunchKernelGGL((prefill_pingpong_kernel<T, true>), dim3(n_wg, p.n_split), dim3(kPpThreads), 0, stream, p);
-  const hipError_t e = hipGetLastError();
-  if (e != hipSuccess) return e;
-  return merge_launch();
+  // lanes per item: more when there are many splits to walk, as long as the grid stays small
+  constexpr size_t kLanesMax = (size_t)1 << 21;
+  if (p.n_split > 32 && items * 64 <= kLanesMax) return merge(prefill_merge_kernel<T, 64>, 64);
+  if (p.n_split > 8 && items * 8 <= kLanesMax) return merge(prefill_merge_kernel<T, 8>, 8);
+  return merge(prefill_merge_kernel<T, 1>, 1);
 }
 
 }  // namespace
 
 hipError_t launch_prefill(const AttnArgs& a, hipStream_t stream) {
-  if (a.dtype == 0) return launch_pingpong<F16>(a, stream);
-  return launch_pingpong<BF16>(a, stream);
+  if (a.dtype == 0) return launch_chunk<F16>(a, stream);
+  return launch_chunk<BF16>(a, stream);
 }
 
 }  // namespace ellm

@@ -16,9 +16,18 @@ SOURCE = r"""
 #include <cstdlib>
 #include "general_plan.hpp"
 using namespace ellm;
+static int chunk(char** v) {   // batch capacity, batch, query heads, key-value heads, most positions a call, position_index, interval
+  uint32_t a[8];
+  for (int i = 1; i <= 7; ++i) a[i] = (uint32_t)strtoul(v[i + 1], nullptr, 10);
+  const ChunkCall c = {a[6], a[7], a[2], a[1], a[3], a[4], 256, prefill_workspace_rows(a[5], a[1], a[3], 256)};
+  const ChunkPlan p = plan_chunk(c);
+  printf("%d %u %u %u\n", (int)p.kernel, p.kernel == kChunkStream ? p.waves : p.kernel == kChunkShort ? p.row_blocks : 0, p.n_split, p.n_wg);
+  return 0;
+}
 // head size, bytes an element, batch capacity, batch, query heads, key-value heads, most positions a call,
 // position_index, interval, whole aligned pieces, and room for partial rows per query row (0: the workspace's)
 int main(int, char** v) {
+  if (v[1][0] == 'c') return chunk(v);
   uint32_t a[12];
   for (int i = 1; i <= 11; ++i) a[i] = (uint32_t)strtoul(v[i], nullptr, 10);
   const gen::GeneralWorkspace w = gen::general_workspace(a[7], a[3], a[5], a[6], a[1], 256);
@@ -60,3 +69,10 @@ def general_plan(head_size, element_bytes, batch_capacity, batch, q_heads, kv_he
     args = (head_size, element_bytes, batch_capacity, batch, q_heads, kv_heads, interval, position_index, interval, int(vec), room)
     out = subprocess.run([_program(), *map(str, args)], check=True, capture_output=True, text=True).stdout.split()
     return (("rows", "step", "chunk")[int(out[0])], *map(int, out[1:]))
+
+
+def chunk_plan(batch_capacity, batch, q_heads, kv_heads, position_index, interval, most=None):
+    """128-wide 16-bit heads: (kernel "stream" / "pingpong" / "short", its waves or row blocks, key splits, workgroups a split)"""
+    args = ("c", batch_capacity, batch, q_heads, kv_heads, most or interval, position_index, interval)
+    out = subprocess.run([_program(), *map(str, args)], check=True, capture_output=True, text=True).stdout.split()
+    return (("stream", "pingpong", "short")[int(out[0])], *map(int, out[1:]))

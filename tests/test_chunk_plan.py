@@ -7,6 +7,8 @@ import subprocess
 
 import pytest
 
+import plan_probe
+
 ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 CSRC = os.path.join(ROOT, "ellm_amd", "csrc")
 
@@ -95,3 +97,16 @@ def test_known_shapes(rows):
     assert (r[6], r[7], r[8]) == (52, 3, 25) and r[10] == 52
     r = by[(129, 96, 512, 4, 64, 1.0)]
     assert (r[6], r[7]) == (26, 5)
+
+
+def test_the_chunk_cases_reach_the_kernels_they_are_there_for():
+    from test_gpu_parity import PREFILL, kernel_of
+
+    seen = set()
+    for name, bcap, b, hq, hkv, cap, p0, s in PREFILL:
+        kernel, waves, n_split, _ = plan_probe.chunk_plan(bcap, b, hq, hkv, p0, s)
+        want, want_waves = kernel_of(name)
+        assert kernel == want and (want_waves is None or waves == want_waves), (name, kernel, waves)
+        seen.add((kernel, waves, n_split > 1))
+    assert seen >= {("stream", w, True) for w in (4, 8, 12)} | {("stream", 4, False), ("pingpong", 0, True), ("pingpong", 0, False),
+                                                               ("short", 1, False), ("short", 2, False)}

@@ -5,6 +5,7 @@ import numpy as np
 import pytest
 
 import oracle_lib as orc
+import plan_probe
 from gpu_util import (D, LSE_TOL, compare, gpu_attention, rand_storage, to_dev, to_host,
                       torch_dtype)
 
@@ -70,7 +71,40 @@ PREFILL = [
     ("stream_g16_8tok_full_workgroup", 1, 1, 16, 1, 3000, 2900, 8),   # 128 rows exactly
     ("stream_first_split_only_for_early_rows", 2, 2, 8, 2, 700, 500, 5),
     ("stream_unsplit_many_sequences", 160, 160, 32, 4, 600, 560, 16),  # no room for partial rows: one split
+    # the streaming kernel's edges on caches beyond the reach of the short-prompt kernel, which has taken over the
+    # calls on shorter ones above
+    ("long_stream_2tok_on_tile_edge", 6, 6, 32, 4, 2000, 1984, 2),
+    ("long_stream_3tok_off_edge", 6, 6, 32, 4, 2100, 1990, 3),
+    ("long_stream_16tok_across_chunk_edge", 6, 6, 32, 4, 2100, 2039, 16),
+    ("long_stream_16tok_on_chunk_edge", 6, 6, 32, 4, 2100, 2048, 16),
+    ("long_stream_17tok_eight_waves", 6, 6, 32, 4, 2100, 1961, 17),
+    ("long_stream_32tok_eight_waves_full", 6, 6, 32, 4, 2100, 2016, 32),
+    ("long_stream_33tok_twelve_waves", 6, 6, 32, 4, 2100, 1961, 33),
+    ("long_stream_48tok_twelve_waves_full", 6, 6, 32, 4, 2100, 2047, 48),
+    ("long_stream_g16_20tok_twelve_waves_below_capacity", 3, 2, 16, 1, 2300, 2100, 20),
+    ("long_stream_g3_50tok_eight_waves_odd_group", 2, 2, 6, 2, 2300, 2000, 50),
+    ("long_stream_batch_below_capacity_9tok", 5, 3, 8, 2, 2200, 2000, 9),
+    ("long_stream_first_split_only_for_early_rows", 2, 2, 8, 2, 2100, 1950, 5),
+    ("long_pingpong_from_zero_split", 1, 1, 8, 1, 2176, 0, 2100),
+    ("long_pingpong_from_zero_unsplit", 1, 1, 32, 32, 2000, 0, 1990),
 ]
+ON_SHORT = {
+    "one_token_block", "ragged_tail_g8", "mha_two_seq", "chunk_on_cache", "batch_below_capacity_g4", "g2", "g3_odd_group", "g16",
+    "interval_2", "tile_edge_63_64_65", "split_from_zero_later_splits_empty_for_early_rows", "stream_2tok_b24_on_tile_edge",
+    "stream_3tok_b24_off_edge", "stream_16tok_b24_across_chunk_edge", "stream_16tok_b24_on_chunk_edge",
+    "stream_17tok_b24_eight_waves", "stream_32tok_b24_eight_waves_full", "stream_33tok_b24_twelve_waves",
+    "stream_48tok_b6_twelve_waves_full", "stream_g16_20tok_twelve_waves_below_capacity", "stream_g3_50tok_eight_waves_odd_group",
+    "stream_batch_below_capacity_9tok", "stream_first_split_only_for_early_rows",
+}
+
+
+def kernel_of(name):
+    """(kernel, streaming kernel's waves or None) that a case of PREFILL runs."""
+    if name in ON_SHORT:
+        return "short", None
+    if name.startswith(("stream", "long_stream", "split_batch", "split_interval", "split_three")):
+        return "stream", 8 if "eight_waves" in name or "split_batch" in name else 12 if "twelve_waves" in name else 4
+    return "pingpong", None
 
 
 @pytest.mark.parametrize("case", PREFILL, ids=[c[0] for c in PREFILL])
@@ -187,11 +221,13 @@ def test_unusual_scales(scale):
     _check(f"scale {scale} split chunk", q, k2, v2, scale, dtype, p0=1500)
 
 
-def test_garbage_beyond_the_position_does_not_leak():
+@pytest.mark.parametrize("p0,cap,kernel", [(20, 256, "short"), (1930, 2064, "stream")], ids=["short", "stream"])
+def test_garbage_beyond_the_position_does_not_leak(p0, cap, kernel):
     """Cache rows after the last visible position hold NaN / Inf / huge values, and so
     does the output buffer before the call; none of it may reach the result."""
     dtype = orc.F16
-    s, p0, cap = 70, 20, 256
+    s = 70
+    assert plan_probe.chunk_plan(1, 1, 8, 2, p0, s)[0] == kernel
     q = rand_storage((s, 1, 8, D), 19, dtype)
     k = rand_storage((1, 2, cap, D), 20, dtype)
     v = rand_storage((1, 2, cap, D), 21, dtype)
@@ -206,11 +242,14 @@ def test_garbage_beyond_the_position_does_not_leak():
     assert np.array_equal(c1, d1)
 
 
-def test_garbage_beyond_the_position_does_not_leak_into_split_chunks():
+@pytest.mark.parametrize("p0,cap", [(1400, 2048), (1960, 2304)], ids=["1400", "1960"])
+def test_garbage_beyond_the_position_does_not_leak_into_split_chunks(p0, cap):
     """The split chunk path: workgroups of later key ranges see rows whose every key is masked,
     and the cache beyond the last position holds NaN / Inf."""
     dtype = orc.F16
-    s, p0, cap = 40, 1400, 2048
+    s = 40
+    if p0 == 1960:
+        assert plan_probe.chunk_plan(1, 1, 8, 2, p0, s)[0] == "stream" and plan_probe.chunk_plan(1, 1, 8, 2, p0, s)[2] > 1
     q = rand_storage((s, 1, 8, D), 22, dtype)
     k = rand_storage((1, 2, cap, D), 23, dtype)
     v = rand_storage((1, 2, cap, D), 24, dtype)
@@ -225,9 +264,11 @@ def test_garbage_beyond_the_position_does_not_leak_into_split_chunks():
     assert compare(clean, orc.from_storage(want, dtype), dtype)["ok"]
 
 
-def test_causality_rows_ignore_later_keys():
+@pytest.mark.parametrize("s,kernel", [(130, "short"), (1950, "pingpong")], ids=["short", "pingpong"])
+def test_causality_rows_ignore_later_keys(s, kernel):
     dtype = orc.F16
-    s, cap = 130, 192
+    assert plan_probe.chunk_plan(1, 1, 8, 1, 0, s)[0] == kernel
+    cap = s + 62
     q = rand_storage((s, 1, 8, D), 22, dtype)
     k = rand_storage((1, 1, cap, D), 23, dtype)
     v = rand_storage((1, 1, cap, D), 24, dtype)
@@ -240,16 +281,18 @@ def test_causality_rows_ignore_later_keys():
     assert not np.array_equal(base[100:], pert[100:])
 
 
-@pytest.mark.parametrize("shape", [("tile", 130, 60, 256, 8, 1), ("stream", 24, 900, 1024, 8, 2)],
+@pytest.mark.parametrize("shape", [("tile", 130, 60, 256, 8, 1), ("stream", 24, 900, 1024, 8, 2),
+                                   ("long_tile", 130, 1930, 2100, 8, 1), ("long_stream", 24, 1960, 2100, 8, 2)],
                          ids=lambda sh: sh[0])
 def test_value_rows_rule_at_the_boundary_the_header_states(shape):
-    """ellm_attn_run's rule for K/V contents, pinned where it bites, in the tile kernel and in the
-    streaming chunk kernel: (1) rows of the call's own later tokens are read by earlier query rows
+    """ellm_attn_run's rule for K/V contents, pinned where it bites, in the short-prompt kernel and, on
+    longer caches, in the tile kernel and the streaming chunk kernel: (1) rows of the call's own later tokens are read by earlier query rows
     with a probability of exactly 0, so while they are FINITE (whatever their values) the earlier
     rows' bits do not depend on them; (2) rows strictly beyond the call's last position are never
     read: NaN / Inf there change nothing.  (The reference reads neither: flash_attention.rs:57-58.)"""
-    _, s, p0, cap, hq, hkv = shape
+    name, s, p0, cap, hq, hkv = shape
     dtype = orc.F16
+    assert plan_probe.chunk_plan(1, 1, hq, hkv, p0, s)[0] == {"long_tile": "pingpong", "long_stream": "stream"}.get(name, "short")
     q = rand_storage((s, 1, hq, D), 91, dtype)
     k = rand_storage((1, hkv, cap, D), 92, dtype)
     v = rand_storage((1, hkv, cap, D), 93, dtype)

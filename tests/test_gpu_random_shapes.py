@@ -8,6 +8,7 @@ import numpy as np
 import pytest
 
 import oracle_lib as orc
+import plan_probe
 from gpu_util import D, LSE_TOL, compare, gpu_attention, rand_storage
 
 pytestmark = pytest.mark.gpu
@@ -52,6 +53,29 @@ def test_random_chunk_shapes_match_oracle(block):
         lse_err = float(np.abs(got_lse[:, :c["b"]] - want_lse[:, :c["b"]]).max())
         assert res["ok"], (c, res)
         assert lse_err <= LSE_TOL, (c, lse_err)
+
+
+def test_random_chunk_shapes_on_long_caches_match_oracle():
+    """Caches beyond the reach of the short-prompt kernel, which takes most of the draws above: the streaming kernel with
+    four, eight and twelve waves, and the tile kernel."""
+    rng = np.random.default_rng(1100)
+    seen = set()
+    for n in range(24):
+        g, s = [(8, 2), (8, 16), (4, 40), (8, 31), (16, 22), (8, 48), (3, 70), (8, 64), (1, 100), (2, 150), (16, 8), (2, 33)][n % 12]
+        hkv, b = int(rng.choice([1, 2, 4])), int(rng.choice([1, 2, 3]))
+        p0, dtype = int(rng.integers(1921, 4000)), orc.F16 if n % 2 else orc.BF16
+        hq, bcap, cap = hkv * g, b + int(rng.integers(0, 2)), p0 + s + int(rng.integers(0, 5))
+        seen.add(plan_probe.chunk_plan(bcap, b, hq, hkv, p0, s)[:2])
+        print("case", n, g, hkv, b, bcap, p0, s, "f16" if dtype == orc.F16 else "bf16", flush=True)
+        q = rand_storage((s, bcap, hq, D), 7700 + n, dtype)
+        k, v = rand_storage((bcap, hkv, cap, D), 8700 + n, dtype), rand_storage((bcap, hkv, cap, D), 9700 + n, dtype)
+        scale = 1.0 / np.sqrt(D)
+        want, want_lse = orc.attention(q, k, v, scale, dtype, position_index=p0, batch=b)
+        got, got_lse = gpu_attention(q, k, v, scale, dtype, position_index=p0, batch=b)
+        res = compare(got[:, :b], orc.from_storage(want, dtype)[:, :b], dtype)
+        assert res["ok"], (n, res)
+        assert float(np.abs(got_lse[:, :b] - want_lse[:, :b]).max()) <= LSE_TOL, n
+    assert seen >= {("stream", 4), ("stream", 8), ("stream", 12), ("pingpong", 0)}
 
 
 def _draw_ragged(rng):

@@ -1,15 +1,10 @@
 """Short prompts and short chunks on short caches: the kernel whose waves share a row block's keys
 (short_prompt_kernel) at the edges of its tiles, and the rule that sends calls to it."""
-import os
-import shutil
-import subprocess
-
 import numpy as np
 import pytest
 
 import oracle_lib as orc
-
-ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+import plan_probe
 
 # (batch, q heads, kv heads, position_index, interval, row blocks per workgroup on 256 compute units)
 CASES = [
@@ -22,46 +17,29 @@ CASES = [
     (1, 32, 4, 0, 1001, 2),      # two row blocks a workgroup, planes shared by two XCDs, 8 rows in the last
     (1, 64, 8, 0, 500, 2),       # 500 x 8 rows: the last workgroup holds 32 rows of 64
     (2, 48, 16, 100, 201, 2),    # 603 rows of a group of three: the last workgroup holds 27
+    # few rows on a cache, calls that would stream otherwise
+    (4, 32, 4, 700, 13, 1),
+    (21, 32, 4, 1210, 40, 2),    # 84 planes, one XCD each
 ]
 
 
-def test_the_rule_sends_these_calls_there(tmp_path):
-    gxx = shutil.which("g++")
-    if not gxx:
-        pytest.skip("no g++")
-    src = tmp_path / "probe.cpp"
-    src.write_text(r"""
-#include "chunk_plan.hpp"
-#include <cstdio>
-#include <cstdlib>
-using namespace ellm;
-int main(int, char** v) {
-  const uint32_t b = atoi(v[1]), hq = atoi(v[2]), hkv = atoi(v[3]), p0 = atoi(v[4]), s = atoi(v[5]);
-  const ChunkShape c = {p0, s, hq / hkv, b * hkv, 256};
-  const uint32_t g = hq / hkv, stacked = g % 8 == 0 ? 8 : g % 4 == 0 ? 4 : g % 2 == 0 ? 2 : 1;   // heads a workgroup of the
-  const double wgs = (double)b * hkv * (g / stacked) * ((s * stacked + 255) / 256);             // ping-pong kernel stacks
-  printf("%u\n", short_prompt_wr(c, pingpong_us(c, wgs, {0, 1})));
-}
-""")
-    exe = tmp_path / "probe"
-    subprocess.run([gxx, "-O1", "-std=c++17", "-I", os.path.join(ROOT, "ellm_amd", "csrc"), "-o", str(exe), str(src)], check=True)
-
-    def wr(*a):
-        return int(subprocess.run([str(exe), *map(str, a)], check=True, capture_output=True, text=True).stdout)
-
-    for c in CASES:
-        assert wr(*c[:5]) == c[5], c
-    assert wr(1, 32, 4, 0, 4096) == 0 and wr(1, 32, 4, 8192, 64) == 0      # long walks: the other kernels
+def test_the_rule_sends_these_calls_there():
+    for b, hq, hkv, p0, s, wr in CASES:
+        assert plan_probe.chunk_plan(b + 1, b, hq, hkv, p0, s)[:3] == ("short", wr, 1), (b, hq, hkv, p0, s)
+    assert plan_probe.chunk_plan(1, 1, 32, 4, 0, 4096)[0] == "pingpong"       # long walks: the other kernels
+    assert plan_probe.chunk_plan(1, 1, 32, 4, 8192, 64)[0] == "pingpong"
+    assert plan_probe.chunk_plan(24, 24, 32, 4, 8191, 13)[:2] == ("stream", 4)
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("flip", [False, True], ids=["", "other_type"])
 @pytest.mark.parametrize("case", CASES, ids=[f"{c[0]}x{c[4]}on{c[3]}_{c[1]}q{c[2]}kv" for c in CASES])
-def test_short_prompts_match_the_oracle(case):
+def test_short_prompts_match_the_oracle(case, flip):
     from gpu_util import D, LSE_TOL, compare, gpu_attention, rand_storage
 
     b, hq, hkv, p0, s, wr = case
     print("case", case, flush=True)
-    dtype = orc.BF16 if wr == 2 else orc.F16
+    dtype = orc.BF16 if (wr == 2) != flip else orc.F16
     q = rand_storage((s, b + 1, hq, D), 61, dtype)      # one sequence of capacity more than the batch
     k = rand_storage((b + 1, hkv, p0 + s + 1, D), 62, dtype)
     v = rand_storage((b + 1, hkv, p0 + s + 1, D), 63, dtype)
