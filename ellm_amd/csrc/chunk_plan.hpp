@@ -153,15 +153,17 @@ inline double pingpong_us(const ChunkShape& c, double wgs, const KeySplit& ks) {
   return 4.5 + 4.5 * whole_up(wgs / c.n_cu) + 1.3 * (longest > mean ? longest : mean);
 }
 
-// The row blocks per workgroup (1 or 2) short_prompt_kernel should take a call with, or 0: another
-// kernel's estimate `other_us` is not at least 15 % longer (the estimates are).  Up to 1920 keys: there the XCDs' L2s hold
-// the planes that are being walked, which the estimate takes for granted (261 tokens on 4868 keys:
-// 60 us where it says 42).
+// The row blocks per workgroup (1 or 2) short_prompt_kernel should take a call with, or 0: it does not take
+// less than `margin` of another kernel's estimated time (the estimates are no better).  Up to 1920 keys and
+// 115 MB of K and V: there the XCDs' L2s hold the planes that are being walked, which the estimate takes for
+// granted (261 tokens on 4868 keys: 60 us where it says 42; 150 tokens x 6 on 1750, 32 / 32 heads, 187 MB: 71 us
+// where it says 51, and the other kernel takes 67).
 constexpr uint32_t kShortPromptKeys = 1920;
-inline uint32_t short_prompt_wr(const ChunkShape& c, double other_us) {
-  if (c.p0 + c.interval > kShortPromptKeys) return 0;
+constexpr double kShortPromptMb = 115.0;
+inline uint32_t short_prompt_wr(const ChunkShape& c, double other_us, double margin = 0.87) {
+  if (c.p0 + c.interval > kShortPromptKeys || c.planes * c.keys() * 512e-6 > kShortPromptMb) return 0;
   const double one = short_prompt_us(c, 1), two = short_prompt_us(c, 2);
-  if ((one < two ? one : two) > 0.87 * other_us) return 0;
+  if ((one < two ? one : two) > margin * other_us) return 0;
   return one < two ? 1 : 2;
 }
 
@@ -301,7 +303,10 @@ inline ChunkPlan plan_chunk(const ChunkCall& c) {
       p.n_split = ks.n_split;
     }
   }
-  if (const uint32_t wr = short_prompt_wr(shape, pingpong_us(shape, base, {p.split_tiles, p.n_split})))
+  // (beyond 1536 keys pieces of a split walk take less than the estimate: 300 tokens x 2 on 1500, 32 / 4 heads, 34 us
+  // against 38 in the short-prompt kernel)
+  const double margin = all_tiles > 24 ? 0.82 : 0.87;
+  if (const uint32_t wr = short_prompt_wr(shape, pingpong_us(shape, base, {p.split_tiles, p.n_split}), margin))
     plan_short_prompt(shape, wr, &p);
   return p;
 }

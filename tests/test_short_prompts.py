@@ -31,6 +31,17 @@ def test_the_rule_sends_these_calls_there():
     assert plan_probe.chunk_plan(24, 24, 32, 4, 8191, 13)[:2] == ("stream", 4)
 
 
+def test_calls_that_are_shorter_elsewhere_stay_there():
+    """More K and V than the L2s hold, and split walks beyond 1536 keys (measured: 70.6 against 66.5 us, 53.6 against 50.3,
+    38.2 against 34.4); the short-prompt kernel's own neighbours of these calls."""
+    assert plan_probe.chunk_plan(6, 6, 32, 32, 1750, 150)[0] == "stream"
+    assert plan_probe.chunk_plan(22, 22, 64, 8, 1329, 19)[0] == "stream"
+    assert plan_probe.chunk_plan(2, 2, 32, 4, 1500, 300)[0] == "pingpong"
+    assert plan_probe.chunk_plan(4, 4, 32, 32, 1600, 100)[0] == "short"      # 31 against 43 us
+    assert plan_probe.chunk_plan(12, 12, 64, 8, 1506, 37)[0] == "short"      # 41 against 56
+    assert plan_probe.chunk_plan(1, 1, 32, 4, 1600, 300)[0] == "short"       # 26 against 29
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("flip", [False, True], ids=["", "other_type"])
 @pytest.mark.parametrize("case", CASES, ids=[f"{c[0]}x{c[4]}on{c[3]}_{c[1]}q{c[2]}kv" for c in CASES])
