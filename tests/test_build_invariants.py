@@ -45,7 +45,8 @@ def test_tile_kernel_leaves_m0_to_the_inline_asm(tmp_path):
 
 
 @pytest.mark.parametrize("name", ["project.hip", "project_mid.hip", "project_small.hip", "prefill.hip", "decode.hip",
-                                  "decode_balanced.hip", "kv_cache.hip"])
+                                  "decode_balanced.hip", "kv_cache.hip", "attn_general.hip", "attn_general_chunk.hip",
+                                  "attn_general_step.hip"])
 def test_hot_kernels_do_not_spill(name, tmp_path):
     text = _listing(name, tmp_path)
     sizes = [int(x) for x in re.findall(r"\.private_segment_fixed_size:\s*(\d+)", text)]
