@@ -66,7 +66,7 @@ class Attention:
     q, out: [max_position_interval, batch_capacity, attention_head_num, head_size]
     k, v:   any 4-d view [sequence, kv_head, position, head_size] (strides are passed on)
     float16 / bfloat16 tensors with head_size 128 run the MFMA kernels; other head sizes up to
-    256 and float32 tensors run MFMA kernels of their own (same arguments and results).
+    256 and float32 tensors run kernels of their own (same arguments and results).
     """
 
     def __init__(self, q, k, v, out, batch_size, attention_head_num, kv_head_num, head_size,

@@ -271,8 +271,9 @@ __device__ __forceinline__ void store_out4(const GeneralArgs& p, size_t row, uin
 
 // Weights of two keys as operands of the second product.  A 16-bit value keeps 11 (binary16) or 8
 // (bfloat16) significant bits; the weight goes in as two of them, the rounded value and what the
-// rounding left, so that the product carries the weight to 2^-17 or better and the output is
-// rounded once, at the end.
+// rounding left, so that the product carries the weight to 2^-17 of it in bfloat16 and to 2^-22 in
+// binary16, whose rest has steps of 2^-24 (2^-31 after kShift, of the reference weight of 1).  The
+// output is rounded once, at the end.
 template <typename S>
 __device__ __forceinline__ void split_pair(float p0, float p1, uint32_t& hi, uint32_t& lo) {
   hi = Mfma<S>::pack2(p0, p1);

@@ -46,9 +46,9 @@ hipError_t prepare_shape() {
 // Token tiles per band: the eighth of the tiles that an XCD works on side by side is then about
 // band x the heads that make up its number, and the operand rows it takes in from outside its L2,
 // band x tokens + heads x 128 per chunk, are fewer than with all token tiles of a head side by side.
-// Only where that saves a fifth or more: output projection 4096 -> 2048 of 1536 rows (12 x 16 tiles,
-// 24 an XCD: 10 row blocks instead of 14) and 3072 rows (7 instead of 13), attention block of a layer
-// 86.2 -> 84.9 and 152.3 -> 150.4 us; 770 rows (8 instead of 9) 77.0 -> 77.6, not taken.
+// Only where that saves a fifth or more: output projection 4096 -> 2048 of 1280 / 1536 (12 x 16 tiles, 24 an
+// XCD: 10 row blocks instead of 14) / 2048 / 3072 rows (7 instead of 13) 31.7 / 34.0 / 40.3 / 58.6 -> 31.2 / 33.4 /
+// 39.7 / 57.5 us (two runs of each side, 0.1 apart); 770 rows (8 instead of 9) no gain, not taken.
 uint32_t mid_band(uint32_t tiles_m, uint32_t tiles_n, uint32_t tokens) {
   const uint32_t per_xcd = (tiles_m * tiles_n + 7) / 8;
   auto rows_with = [&](uint32_t band) {

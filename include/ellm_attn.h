@@ -21,10 +21,11 @@
  * when it was created: its workspace lives there, and a run or append called
  * while another device is current returns ELLM_ERR_INVALID_ARGUMENT.
  *
- * Only head_size == 128 and 16-bit storage (binary16 / bfloat16) are supported,
- * like the reference's AVX-512 kernel (head_size hard-wired to 128 there,
- * flash_attention.rs:51-56).  Scores, soft-max state and output accumulation are
- * binary32.
+ * Caches, projections and the entry points that fuse them with attention take
+ * head_size == 128 and 16-bit storage (binary16 / bfloat16), like the reference's
+ * AVX-512 kernel (head_size hard-wired to 128 there, flash_attention.rs:51-56);
+ * the attention operator takes any head size up to 256 and binary32 storage too
+ * (ellm_attn_desc).  Scores, soft-max state and output accumulation are binary32.
  */
 #ifndef ELLM_ATTN_H_
 #define ELLM_ATTN_H_
@@ -87,10 +88,14 @@ int ellm_device_count(void);
  * head_size 128 with 16-bit storage (every model configuration the reference ships) runs the
  * kernels built for it.  Any other head_size from 1 to 256, and ELLM_DTYPE_F32 storage (the type of
  * the reference's generic leaf and of its operator test, src/kernel/generic/
- * flash_attention.rs:60-89, src/compiler/mul/attention.rs:262-330), run MFMA kernels of their own with
- * the same arguments, masks and results (binary32 accumulation; soft-max weights of at least 16
- * significant bits, binary32 for binary32 storage); there kv_strides[0..2] need not be multiples of
- * 8 (rows that are not whole aligned 16-byte pieces, and sequence tables, take element-wise loads).
+ * flash_attention.rs:60-89, src/compiler/mul/attention.rs:262-330), run kernels of their own (MFMA, or
+ * row by row where a call is too short for it) with the same arguments, masks and results: binary32
+ * accumulation; soft-max weights in binary32, or, where 16-bit storage meets MFMA, as two 16-bit values
+ * (bfloat16: to 2^-17 of the weight; binary16: to 2^-22 of it, and no finer than 2^-32 of the row's
+ * largest weight).  There kv_strides[0..2] need not be multiples of 8 (rows that are not whole
+ * aligned 16-byte pieces, and sequence tables, take loads of any alignment), and value rows may hold
+ * infinities and NaN: a query row does not see those of later positions, and an infinity that it does
+ * see comes out as one.
  * ellm_attn_run_noalloc and ellm_matmul3_attn_run take 128-wide 16-bit heads only.
  */
 typedef struct ellm_attn_desc {

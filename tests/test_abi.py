@@ -83,7 +83,7 @@ def _desc(**over):
     (dict(k=0x1008), INVALID),                       # not 16-byte aligned
     (dict(dtype=7), INVALID),
     (dict(head_size=0), UNSUPPORTED),
-    (dict(head_size=257), UNSUPPORTED),              # the plain kernel's lanes hold four elements each
+    (dict(head_size=257), UNSUPPORTED),              # eight blocks of 32 elements are the widest head
     (dict(head_size=64, kv_strides=(2 * 64 * 64, 64 * 64, 32, 1)), INVALID),   # rows closer than a head
     (dict(dtype=3), INVALID),
     (dict(attention_head_num=7), INVALID),           # not a multiple of kv_head_num

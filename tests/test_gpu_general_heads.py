@@ -1,9 +1,10 @@
-"""Attention for head sizes other than 128 and for binary32 storage (the library's plain
-kernel, attn_general.hip) against the oracle, through the C ABI.  The reference's generic leaf
-takes any `length` and element type (src/kernel/generic/flash_attention.rs:60-89) and its
-operator test runs in f32 on all-ones tensors (src/compiler/mul/attention.rs:262-330); the
-first test below is that test.  Both sides work in binary32 throughout, so 16-bit results may
-differ by the one rounding to storage and binary32 results by the order of the sums."""
+"""Attention for head sizes other than 128 and for binary32 storage (attn_general*.hip) against
+the oracle, through the C ABI.  The reference's generic leaf takes any `length` and element type
+(src/kernel/generic/flash_attention.rs:60-89) and its operator test runs in f32 on all-ones tensors
+(src/compiler/mul/attention.rs:262-330); the first test below is that test.  Binary32 results may differ
+by the order of the sums, 16-bit results by the one rounding to storage: their soft-max weights go
+through the matrix kernels as two 16-bit values, to 2^-17 of a weight in bfloat16 and, in binary16, to
+2^-22 of it or 2^-32 of the row's largest, whichever is larger, all far below half a unit of the output."""
 import ctypes
 
 import numpy as np
@@ -154,7 +155,7 @@ def test_single_token_steps_match_the_oracle(case):
 
 def test_rows_beyond_the_position_are_never_read():
     """Garbage (NaN) in every K/V row past the call's last position, and for the chunk's earlier
-    tokens in the rows of its later ones, changes nothing: this kernel reads keys 0..=p only."""
+    tokens in the rows of its later ones, changes nothing."""
     dtype, s, b, hq, hkv, hs, cap, p0 = orc.F32, 5, 2, 4, 2, 64, 64, 20
     q, k, v = _rand((s, b, hq, hs), 7, dtype), _rand((b, hkv, cap, hs), 8, dtype), _rand((b, hkv, cap, hs), 9, dtype)
     scale = 0.11

@@ -1,8 +1,7 @@
-"""The matrix kernels for other head sizes and binary32 at the edges of their tiles: rows per
-workgroup (16 and 128), keys per step, padded head blocks, key splits and their folds, rows that are
-not whole 16-byte pieces, values that are not finite beyond a row's position.  Same oracle and
-bounds as tests/test_gpu_general_heads.py: the weights enter the second product with at least 16
-significant bits, so 16-bit results still differ by the one rounding to storage."""
+"""The kernels for other head sizes and binary32 at the edges of their tiles: rows per workgroup (1, 16,
+64 and 128), keys per step and turn, padded head blocks, key splits and their folds, rows that are not
+whole 16-byte pieces, values that are not finite.  Every case says which kernel it is there for
+(general_plan.hpp).  Same oracle and bounds as tests/test_gpu_general_heads.py."""
 import numpy as np
 import pytest
 
