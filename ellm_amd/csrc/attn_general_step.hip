@@ -9,8 +9,9 @@
 // meet once at the end.  Measured: 8 sequences x 4096 keys, 32 query / 4 key-value heads of 128 in
 // binary32: 27.5 us (4.9 TB/s), where one workgroup per query row took 437 us; 2 x 11046 keys, 32 / 32
 // heads of 256 in bfloat16: 112 us (6.5 TB/s; was 5450); 11 x 131 keys, heads of 96: 6.9 us (was 31).
-// Binary32 products sum in chains of eight, as in the chunk kernel: 11 x 2471 keys, 32 / 32 heads of 128, an error
-// of 2.1e-7 against 64 bits in 162 us, where one chain over the head and one over all keys gave 6.1e-7 in 156.
+// Binary32 products sum in short chains (see pairwise_sum): 11 x 2471 keys, 32 / 32 heads of 128, an error of
+// 2.1e-7 against 64 bits in 160 us, where one chain over the head and one over all keys gave 6.1e-7 in 156;
+// chains of eight throughout 2.1e-7 in 161 (11 x 290 keys 16.0 us, sixteen 15.5).
 #include "attn_general.hpp"
 #include "decode_common.hpp"
 
@@ -25,7 +26,6 @@ constexpr int kRows = (int)kGeneralStepRows;
 typedef __attribute__((address_space(3))) uint8_t LdsByte;
 typedef __attribute__((address_space(3))) u32x4 LdsU32x4;
 typedef __attribute__((address_space(3))) float LdsF32;
-typedef __attribute__((address_space(3))) f32x2 LdsF32x2;
 typedef short i16x4 __attribute__((ext_vector_type(4)));
 typedef __attribute__((address_space(3))) i16x4 LdsI16x4;
 
@@ -157,14 +157,20 @@ __global__ __launch_bounds__(kThreads, (StepShape<S, NB>::kOccupancy)) void gene
     if constexpr (X::kF32) {
 #pragma unroll
       for (int mc = 0; mc < MC; ++mc) {
-        auto half_piece = [&](auto n_) __attribute__((always_inline)) {   // eight products a score
-          constexpr int s = decltype(n_)::value / 2, e = decltype(n_)::value % 2 * 2;
-          const f32x2 a = *(const LdsF32x2*)(k_read + 16 * mc * X::kKPitch + 64 * s + 4 * e);
-          const f32x4 sum = __builtin_amdgcn_mfma_f32_16x16x4f32(a[0], __builtin_bit_cast(float, (uint32_t)qreg[s][e]),
-                                                                 f32x4{0.0f, 0.0f, 0.0f, 0.0f}, 0, 0, 0);
-          return __builtin_amdgcn_mfma_f32_16x16x4f32(a[1], __builtin_bit_cast(float, (uint32_t)qreg[s][e + 1]), sum, 0, 0, 0);
+        // chains of sixteen products, of eight up to heads of 64 (131 keys: with sixteen 1.01 of the error of sums
+        // over lanes, with eight 0.91)
+        constexpr int kChain = NB <= 2 ? 2 : 4, kChains = 4 / kChain;
+        auto chain_scores = [&](auto n_) __attribute__((always_inline)) {
+          constexpr int s = decltype(n_)::value / kChains, first = decltype(n_)::value % kChains * kChain;
+          const u32x4 a = *(const LdsU32x4*)(k_read + 16 * mc * X::kKPitch + 64 * s);
+          f32x4 sum = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+          for (int e = first; e < first + kChain; ++e)
+            sum = __builtin_amdgcn_mfma_f32_16x16x4f32(__builtin_bit_cast(float, (uint32_t)a[e]),
+                                                       __builtin_bit_cast(float, (uint32_t)qreg[s][e]), sum, 0, 0, 0);
+          return sum;
         };
-        st[mc] = pairwise_sum<0, 2 * kQ>(half_piece);
+        st[mc] = pairwise_sum<0, kQ * kChains>(chain_scores);
       }
     } else {
 #pragma unroll
