@@ -142,6 +142,27 @@ __device__ __forceinline__ float sum_with_partner_half(float v) {
   return a + b;
 }
 
+// The same between 16-lane rows: v_permlane16_swap exchanges the odd rows of one register with the even
+// rows of the other.
+__device__ __forceinline__ void swap_rows16(float& a, float& b) {
+  asm volatile("s_nop 1\n\tv_permlane16_swap_b32 %0, %1\n\ts_nop 1" : "+v"(a), "+v"(b));
+}
+// Two values whose four lanes l, l ^ 16, l ^ 32, l ^ 48 are to agree on their maximum.  The first
+// exchange leaves the maxima over l, l ^ 32 of x in the lower and of y in the upper half, so that one
+// exchange of 16-lane rows serves both; the last one hands either half the other's value.
+__device__ __forceinline__ void max_over_quarters(float& x, float& y) {
+  swap_halves(x, y);
+  float a = fmaxf(x, y), b = a;
+  swap_rows16(a, b);
+  x = y = fmaxf(a, b);
+  swap_halves(x, y);
+}
+__device__ __forceinline__ float sum_over_quarters(float v) {
+  float a = sum_with_partner_half(v), b = a;
+  swap_rows16(a, b);
+  return a + b;
+}
+
 // Regroup packed 16-bit pairs: given four registers holding (x[k][2c], x[k][2c+1])
 // for k = 0..3, return the two registers holding (x[0][e], x[1][e]) and
 // (x[2][e], x[3][e]) for e = 2c (hi = false) or 2c+1 (hi = true).

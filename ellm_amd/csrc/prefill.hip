@@ -8,13 +8,17 @@
 // walks keys 0..=position once per query row.  Same result per row:
 // softmax(scale * q.K[0..=position]^T) . V[0..=position].
 //
-// Formulation (everything transposed so that one lane owns one query row):
-//   S^T[key][row] = K . Q^T     32x32x16 MFMA, A = K tile from LDS, B = Q in registers
-//   O^T[d][row]  += V^T . P^T   32x32x16 MFMA, A = V^T from LDS (transposing read), B = P^T in registers
+// Formulation (everything transposed so that one lane owns whole query rows):
+//   S^T[key][row] = K . Q^T     A = K tile from LDS, B = Q in registers
+//   O^T[d][row]  += V^T . P^T   A = V^T from LDS (transposing read), B = P^T in registers
 // The C layout of S^T (lane = row, registers = keys) is, up to a fixed
-// permutation of keys inside each 16-key group, the B layout the second MFMA
-// wants; the V^T operand is read with the same permutation, so P never leaves the
-// lane that produced it and row max / row sum need one cross-lane exchange.
+// permutation of keys, the B layout the second MFMA wants; the V^T operand is read with the
+// same permutation, so P never leaves the lane that produced it and row max / row sum need one
+// or two cross-lane exchanges.
+// The tile kernel runs on 16x16x32 instructions, the two kernels for few rows and for short prompts on
+// 32x32x16: on N(0,1) operands a 256 x 256 x 64 loop of the former sustains 1620-1708 TFLOP/s and of the
+// latter 1494-1543 (operands from LDS, nothing else in the loop; on zeros 2111 and 2438: fewer joules a
+// product, more instructions to issue), and what holds the tile kernel back on long calls is the board's power.
 //
 // A workgroup (8 waves) owns 8 blocks of 32 query rows that all read the same
 // K/V plane: up to 8 query heads of one GQA group x consecutive token blocks.
@@ -31,8 +35,8 @@ namespace {
 
 constexpr int kBK = 64;                     // keys per tile
 constexpr int kKsPitch = kHeadDim + 8;      // halves per K row (272 B)
-constexpr int kKsHalves = kBK * kKsPitch;
 constexpr float kRescaleStep = 8.0f;        // log2 units
+constexpr float kMaxSum = 32768.0f;         // of a lane's exponentials of one tile: each fits binary16
 
 struct PrefillKernelArgs {
   const uint16_t* q;
@@ -66,15 +70,27 @@ struct PrefillKernelArgs {
 // ---------------------------------------------------------------------------
 // Ping-pong kernel: 8 waves, two per SIMD.  Waves 0-3 and waves 4-7 run the
 // same per-tile sequence  S^T = K.Q^T -> soft-max -> O^T += V^T.P^T  half a
-// step apart: while one group is in its matrix phase (P.V of the previous tile,
-// then Q.K of the next one, plus moving the following K or V tile into LDS) the
-// other group is in its vector phase (mask, row max, exponentials, packing), and
-// a workgroup barrier flips the roles.  Two waves that share a SIMD are thus
+// step apart: while one group is in its matrix phase (P.V of the previous tile
+// and Q.K of the next one) the other group is in its vector phase (requests of a
+// K or V tile, mask, exponentials, packing), and a workgroup barrier flips the roles.  Two waves that share a SIMD are thus
 // never both in the same phase, which is what lets the MFMA pipe and the vector
 // ALU work at the same time; left to themselves, two identical workgroups on a
 // compute unit run in lockstep and the two pipes take turns instead.
 // Rows: wave w owns row block w (32 rows) of 8; all 256 rows read the same K/V
 // tiles.  Waves 0-3 stage the K tiles, waves 4-7 the V tiles.
+// What bounds it: the board's power on long calls of ordinary operands (1.29-1.32 PFLOP/s at the clock the
+// board allows; 1.65 PFLOP/s on K = V = 0), and a phase of ~1500 clocks for 1024 of matrix work: an
+// instruction of the vector phase takes 8.2 clocks beside 16x16x32 instructions of the other wave (an
+// exponential 15.8; 5.6 and 10.9 beside 32x32x16), the matrix phase has 12 KB of operand reads a wave.
+// Measured, 32x32x16 instructions with a row maximum every tile, K and V through registers -> this form
+// (us): 8192 tokens on 120000, 64 / 8 heads, bf16 26540 -> 25480; 32768 tokens, 32 / 4, f16 7515 -> 7045;
+// 8000 tokens 451 -> 429; 1624 on 10535 295 -> 278; 255 on 11150 (split) 56.7 -> 53.9; 64 tokens x 24 on 4096
+// 119.5 -> 113.9; 412 x 19, 32 / 32 heads 111.1 -> 110.7.  Of that: 16x16x32 alone -1 to +0.5 %, the maximum
+// only where it may have to move 3 to 5 %, tiles straight into LDS 1 to 2 %.  Tried and dropped: Q.K on 32x32x16
+// and P.V on 16x16x32 (eight v_permlane16_swap a tile hand P over: 150 clocks of the vector phase) 26970;
+// all on 32x32x16 with the other two changes 25730 (16x16x32 on the same board 24490); the barrier ahead of a
+// matrix phase's last operands, so that the other group's begins early, 5 % slower than at its end; the
+// tile requests between the matrix instructions instead of ahead of the exponentials 3 % slower.
 // ---------------------------------------------------------------------------
 __device__ __forceinline__ uint64_t uniform64(const void* p) {  // the compiler cannot see that p is wave-uniform
   const uint32_t lo = (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)(uint64_t)p);
@@ -87,8 +103,10 @@ __device__ __forceinline__ uint64_t uniform64(const void* p) {  // the compiler 
 // of the reference's own [position][sequence][kv_head][128] state spans more than 2^32 bytes at
 // 33 sequences x 131072 positions.  Scalar arithmetic (the arguments are wave-uniform).
 __device__ __forceinline__ uint32_t bytes_left(uint64_t valid, uint64_t off) {
-  const uint64_t left = valid > off ? valid - off : 0;
-  const uint32_t capped = left > 0xffffffffull ? 0xffffffffu : (uint32_t)left;
+  // (both below 2^63; told apart by the high word, because the scalar unit has no ordered 64-bit compare)
+  const uint64_t left = valid - off;
+  const int32_t hi = (int32_t)(left >> 32);
+  const uint32_t capped = hi < 0 ? 0u : (hi > 0 ? 0xffffffffu : (uint32_t)left);
   return (uint32_t)__builtin_amdgcn_readfirstlane((int)capped);
 }
 __device__ __forceinline__ uint64_t uniform_u64(uint64_t v) {
@@ -104,22 +122,36 @@ typedef __attribute__((address_space(3))) i16x4 LdsI16x4;
 // V rows in LDS: 288 B apart, so that the four rows a 16-lane block of a
 // transposing read touches (32 B of each) fall into disjoint banks
 constexpr int kVsPitch = kHeadDim + 16;
-constexpr int kVsHalves = kBK * kVsPitch;
 constexpr int kPpWaves = 8;
 constexpr int kPpThreads = kPpWaves * kWave;
-constexpr int kLdsAhead = 8;  // LDS operand reads in flight ahead of their MFMA
+constexpr int kLdsAhead = 8;   // LDS operand reads in flight ahead of their MFMA
+constexpr int kTileHalves = kBK * kHeadDim;
+constexpr int kPpBuffers = 4;                // tiles of K, and of V, in LDS: 128 KB
+constexpr int kPpAhead = kPpBuffers - 1;     // tiles requested ahead of the one being multiplied
+static_assert(kPpAhead == 3, "s_waitcnt vmcnt literals in prefill_pingpong_kernel");
 constexpr int kBufferFlags = 0x00020000;  // raw buffer of 32-bit data, no swizzle (word 3 of the descriptor)
+
+// 16 bytes a lane from memory straight to LDS address lds_at + 16 x lane.  Written as asm: the compiler's
+// own form of this load makes it wait for every outstanding one before each later LDS read (it cannot see
+// that the two touch different buffers).  M0 carries the address; one wait state between its write and the
+// load.  (M0 is a register the compiler reserves and, in the kernel that calls this, never uses itself.)
+__device__ __forceinline__ void load_to_lds(const u32x4& rsrc, uint32_t voff, uint32_t lds_at) {
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, 0 offen lds"
+               :: "s"(lds_at), "v"(voff), "s"(rsrc) : "memory");
+}
 
 template <typename T, bool SPLIT>
 __global__ __launch_bounds__(kPpThreads, 2) void prefill_pingpong_kernel(PrefillKernelArgs p) {
-  // K tiles [2][64][kKsPitch] then V tiles [3][64][kVsPitch]: V is staged one step
-  // earlier than it is read, so that every operand of a matrix step is in LDS a whole
-  // phase before the step starts and can be requested ahead of the barrier.
-  __shared__ __attribute__((aligned(16))) uint16_t smem[2 * kKsHalves + 3 * kVsHalves];
+  // K tiles [4][64][128] then V tiles [4][64][128], rows unpadded: a wave instruction of the staging
+  // below delivers 1 KB, four whole rows.  The sixteen 16-byte pieces of a row are permuted instead, so
+  // that the operand reads meet no bank twice: piece x of K row r sits at x ^ (r & 15) (the sixteen lanes
+  // that a 128-bit read serves at once are rows 0-3 and 12-15 of one piece and 4-11 of its neighbour),
+  // piece x of V row r at x ^ 2 (r & 7) (a transposing read touches two pieces of eight rows).
+  __shared__ __attribute__((aligned(256))) uint16_t smem[2 * kPpBuffers * kTileHalves];
 
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = tid >> 6;
-  const int j = lane & 31, g = lane >> 5;
+  const int c16 = lane & 15, g = lane >> 4;
   const int grp = wave >> 2;  // 0: waves 0-3, 1: waves 4-7
 
   uint32_t combo, order;
@@ -150,19 +182,19 @@ __global__ __launch_bounds__(kPpThreads, 2) void prefill_pingpong_kernel(Prefill
   const uint32_t hg = wave % p.heads_per_wg, tb = wave / p.heads_per_wg;
   const uint32_t head = kvh * p.group + hgrp * p.heads_per_wg + hg;
   const uint32_t tok0 = t_base + 32 * tb;
-  const uint32_t tok = min(tok0 + j, S - 1);
-  const bool row_valid = tok0 + j < S;
-  const uint32_t rowpos = P0 + tok;
+  // this lane's rows: 16 rb + c16 of the wave's 32 (those past the last token repeat its row and are not stored)
+  auto token_of = [&](int rb) { return min(tok0 + 16 * rb + c16, S - 1); };
   const uint32_t first_pos = P0 + min(tok0, S - 1);  // lowest position in this row block
 
-  u32x4 qreg[8];
-  {
-    const uint16_t* qrow =
-        p.q + (size_t)tok * p.q_token_stride + ((size_t)seq * p.n_q_heads + head) * kHeadDim;
+  u32x4 qreg[2][4];   // [row block][32 dims]
 #pragma unroll
-    for (int s = 0; s < 8; ++s) {
-      qreg[s] = load16(qrow + 16 * s + 8 * g);
-      if (p.negate_q) qreg[s] ^= 0x80008000u;
+  for (int rb = 0; rb < 2; ++rb) {
+    const uint16_t* qrow =
+        p.q + (size_t)token_of(rb) * p.q_token_stride + ((size_t)seq * p.n_q_heads + head) * kHeadDim;
+#pragma unroll
+    for (int s = 0; s < 4; ++s) {
+      qreg[rb][s] = load16(qrow + 32 * s + 8 * g);
+      if (p.negate_q) qreg[rb][s] ^= 0x80008000u;
     }
   }
   const float c = p.c;
@@ -171,11 +203,11 @@ __global__ __launch_bounds__(kPpThreads, 2) void prefill_pingpong_kernel(Prefill
   const uint16_t* kplane = p.k + plane_at;
   const uint16_t* vplane = p.v + plane_at;
 
-  // staging: the 256 threads of a group move one 64 x 128 tile, four 16-byte pieces
-  // each (rows ld_r + 16 i, columns 8 ld_c ..), K and V alike: V sits in LDS row by
-  // row as it does in memory and is transposed by the LDS read (ds_read_b64_tr_b16).
-  const int st_tid = tid & 255;
-  const int ld_c = st_tid & 15, ld_r = st_tid >> 4;
+  // staging: the four waves of a group move one 64 x 128 tile straight into LDS, four loads each: rows
+  // ld_r + 16 i, LDS piece tid % 16, K and V alike: V sits in LDS row by row as it does in
+  // memory and is transposed by the LDS read (ds_read_b64_tr_b16).
+  const int ld_r = (tid & 255) >> 4;
+  const int ld_c = (tid & 15) ^ (grp ? 2 * (ld_r & 7) : ld_r);
   const uint16_t* plane = grp ? vplane : kplane;                  // wave-uniform
   const uint32_t stride_pos = (uint32_t)p.kv_stride_pos;
   // Tiles are fetched with buffer loads: the descriptor (base of tile kt, bytes
@@ -193,191 +225,190 @@ __global__ __launch_bounds__(kPpThreads, 2) void prefill_pingpong_kernel(Prefill
   uint32_t piece_off[4];
 #pragma unroll
   for (int i = 0; i < 4; ++i) piece_off[i] = ((ld_r + 16 * i) * stride_pos + 8 * ld_c) * 2;
-  // LDS addresses are kept as byte offsets: the buffers span more than the 64 KB an
-  // instruction's immediate offset reaches, so each step forms one base register
-  // per tile (step_base) and everything else is an immediate on top of it.
   const uint32_t lds0 = (uint32_t)(uintptr_t)(LdsHalf*)smem;
   auto step_base = [](uint32_t addr) {
     asm volatile("" : "+v"(addr));  // opaque: keeps the compiler from folding the sum another way
     return addr;
   };
-  const uint32_t ks_store = lds0 + 2 * (ld_r * kKsPitch + 8 * ld_c);
-  const uint32_t vs_store = lds0 + 2 * (2 * kKsHalves + ld_r * kVsPitch + 8 * ld_c);
-  u32x4 stg[4];
-  auto load_piece = [&](uint32_t kt, int i) {  // kt (relative to kt0) must be wave-uniform to the compiler
-    const uint64_t off = (uint64_t)(kt0 + kt) * tile_bytes;
-    const uint32_t left = bytes_left(valid_bytes, off);
-    const __amdgpu_buffer_rsrc_t rsrc =
-        __builtin_amdgcn_make_buffer_rsrc((void*)(plane_u + off), 0, left, kBufferFlags);
-    stg[i] = __builtin_amdgcn_raw_buffer_load_b128(rsrc, piece_off[i], 0, 0);
-  };
   // (the group comes as a compile-time constant where the caller runs behind the scalar
   // branch on the group, as the run-time value in the prologue)
-  // base: step_base of this lane's place in the destination buffer
-  auto store_piece = [&](auto group, uint32_t base, int i) {
-    *(LdsU32x4*)(base + 2 * 16 * i * (group ? kVsPitch : kKsPitch)) = stg[i];
-  };
-  auto load_tile = [&](uint32_t kt) {
+  const uint32_t wave_lds = lds0 + 4 * 2 * kHeadDim * ((uint32_t)__builtin_amdgcn_readfirstlane(wave) & 3);
+  auto load_tile = [&](auto group, uint32_t kt) __attribute__((always_inline)) {  // kt (relative to kt0): wave-uniform
+    const uint64_t off = (uint64_t)(kt0 + kt) * tile_bytes;
+    const uint64_t at = plane_u + off;
+    const u32x4 rsrc = {(uint32_t)at, (uint32_t)(at >> 32) & 0xffffu, bytes_left(valid_bytes, off), (uint32_t)kBufferFlags};
+    const uint32_t to = wave_lds + (uint32_t)__builtin_amdgcn_readfirstlane((int)(((group ? kPpBuffers : 0) + (kt & (kPpBuffers - 1))) * 2 * kTileHalves));
 #pragma unroll
-    for (int i = 0; i < 4; ++i) load_piece(kt, i);
-  };
-  auto store_base = [&](auto group, int buf) {
-    return step_base(group ? vs_store + 2 * buf * kVsHalves : ks_store + 2 * buf * kKsHalves);
-  };
-  auto store_tile = [&](int buf) {
-    const uint32_t base = store_base(grp, buf);
-#pragma unroll
-    for (int i = 0; i < 4; ++i) store_piece(grp, base, i);
+    for (int i = 0; i < 4; ++i) load_to_lds(rsrc, piece_off[i], to + 16 * i * 2 * kHeadDim);
   };
 
-  float m_run = -INFINITY, l_run = 0.0f;
-  f32x16 oacc[4];
+  // per row: minus its reference maximum (log2 units; +inf: no key seen yet), this lane's share of
+  // the denominator
+  float neg_m[2] = {INFINITY, INFINITY}, l_run[2] = {0.0f, 0.0f};
+  f32x4 oacc[8][2];   // [16 dims][row block]
 #pragma unroll
-  for (int db = 0; db < 4; ++db)
+  for (int db = 0; db < 8; ++db)
 #pragma unroll
-    for (int r = 0; r < 16; ++r) oacc[db][r] = 0.0f;
-  f32x16 st[2];
-  u32x4 pk[4];
+    for (int rb = 0; rb < 2; ++rb) oacc[db][rb] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+  f32x4 st[4][2];     // [16 keys][row block]
+  u32x4 pk[2][2];     // [32 keys][row block]
 #pragma unroll
-  for (int cc = 0; cc < 4; ++cc) pk[cc] = u32x4{0u, 0u, 0u, 0u};  // P(-1) = 0
+  for (int kc = 0; kc < 2; ++kc)
+#pragma unroll
+    for (int rb = 0; rb < 2; ++rb) pk[kc][rb] = u32x4{0u, 0u, 0u, 0u};  // P(-1) = 0
 
   // Every matrix step runs the same straight-line code, the first and the last
   // included: step 0 multiplies P(-1) = 0 by a zeroed "V(-1)" buffer, step n_tiles
   // multiplies Q by whatever finite K tile its buffer still holds and nobody reads
   // the result; tiles past the last one are fetched as zeros (the buffer
   // descriptor has no bytes left) and stored where nothing reads them.
-  // prologue: K(0) and V(0) into LDS, K(1) and V(1) on their way into the staging
-  // registers, zeros into the V^T buffer that step 0 reads.
+  // prologue: zeros into the V buffer that step 0 reads, the first kPpAhead tiles on their way.
   if (grp) {
 #pragma unroll
-    for (int i = 0; i < 4; ++i) stg[i] = u32x4{0u, 0u, 0u, 0u};
-    store_tile(2);
+    for (int i = 0; i < 4; ++i)
+      *(LdsU32x4*)(lds0 + 2 * ((2 * kPpBuffers - 1) * kTileHalves) + (tid & 255) * 16 + i * 4096) = u32x4{0u, 0u, 0u, 0u};
   }
-  load_tile(0);
-  store_tile(0);
-  load_tile(1);
+#pragma unroll
+  for (int kt = 0; kt < kPpAhead; ++kt) load_tile(grp, kt);
+  asm volatile("s_waitcnt vmcnt(8)" ::: "memory");   // 4 (kPpAhead - 1): tile 0 is there
   __syncthreads();
 
-  // Matrix step kt = P.V of tile kt-1 and Q.K of tile kt, their MFMAs interleaved
-  // (six accumulator chains instead of four or two, so no MFMA waits on the
-  // one before it); then the group stores its tile kt+1 (group 0: K, group 1: V)
-  // and fetches tile kt+2.  K(kt) sits in buffer kt % 2, V(kt) in buffer kt % 3: V is
-  // staged one step before the first step that reads it, so that all operands of
-  // a matrix step are in LDS a whole phase before it starts.  Operands come from
+  // Matrix step kt = P.V of tile kt-1 and Q.K of tile kt, their MFMAs interleaved (no MFMA waits on the
+  // one before it).  Tile kt of K and of V sits in buffer kt % 4 of its own.  A vector step
+  // kt requests tile kt + 3 (group 0: K, group 1: V) into the buffer of tile kt - 1, whose last reader,
+  // matrix step kt (V) or kt - 1 (K) of either group, has ended; the matrix step that
+  // follows waits for tile kt + 2 and the barrier at its end shows it to all, one matrix step ahead
+  // of its first reader: three phases for a tile to arrive, and all operands of a
+  // matrix step are in LDS a whole phase before it starts.  Operands come from
   // LDS kLdsAhead reads ahead of the MFMA that consumes them: issued just in
-  // time, every pair of MFMAs (64 cycles) would wait out a full LDS round trip
+  // time, every operand's MFMAs (32 cycles) would wait out a full LDS round trip
   // (100+ cycles).  The first kLdsAhead are requested before the barrier that
   // opens the step (prefetch_ring), so the round trip overlaps the barrier wait.
-  // A operand of P.V (rows = 32 dims, 16 keys): lane (dim j, key half g) holds keys
-  // {4g..4g+3, 8+4g..8+4g+3} of the 16, the order in which the soft-max leaves P in
+  // A operand of P.V (rows = 16 dims, 32 keys): lane (dim c16, key quarter g) holds keys
+  // {4g..4g+3, 16+4g..16+4g+3} of the 32, the order in which the soft-max leaves P in
   // registers.  ds_read_b64_tr_b16 hands lane t of a 16-lane block element
   // (t & 3) of what lanes 4e + (t >> 2), e = 0..3, of that block address: with lane
-  // s pointing at key s >> 2, dims 4 (s & 3).. of the block's 16 dims, lane t ends
-  // up with dim t of 4 consecutive keys.  Two such reads (keys +0 and +8) make one operand.
-  const uint32_t k_read = lds0 + 2 * (j * kKsPitch + 8 * g);
-  const uint32_t v_read = lds0 + 2 * (2 * kKsHalves + (4 * g + ((lane & 15) >> 2)) * kVsPitch +
-                                      16 * ((lane >> 4) & 1) + 4 * (lane & 3));
-  auto mod3 = [](uint32_t x) { return x % 3u; };
+  // s pointing at key s >> 2, dims 4 (s & 3).. of the 16 dims, lane t ends
+  // up with dim t of 4 consecutive keys.  Two such reads (keys +0 and +16) make one operand.
+  const uint32_t k_read = lds0 + 2 * kHeadDim * c16 + 16 * (g ^ c16);
+  const uint32_t v_read = lds0 + 2 * kPpBuffers * kTileHalves + 2 * kHeadDim * (4 * g + (c16 >> 2)) +
+                          32 * (4 * (g & 1) + (c16 >> 2)) + 8 * (c16 & 3);
+  auto k_base = [&](uint32_t kt) { return step_base(k_read + 2 * (kt & (kPpBuffers - 1)) * kTileHalves); };
+  auto v_base = [&](uint32_t kt) { return step_base(v_read + 2 * ((kt - 1) & (kPpBuffers - 1)) * kTileHalves); };
   // operand n of the stream of matrix step kt: P.V 0, Q.K 0, P.V 1, Q.K 1, ...
   // (lane part of the address once per step, operand part as a compile-time offset)
   auto stream_operand = [&](uint32_t ks, uint32_t vs, int n) {
     const int i = n >> 1;
-    if (n & 1) {  // K rows: i = 2 s + mb
-      const int s = i >> 1, mb = i & 1;
-      return (u32x4) * (const LdsU32x4*)(ks + 2 * (32 * mb * kKsPitch + 16 * s));
+    if (n & 1) {  // K: i = 4 s + kb, keys 16 kb.., dims 32 s..
+      const int s = i >> 2, kb = i & 3;
+      return (u32x4) * (const LdsU32x4*)((ks ^ (64 * s)) + 2 * 16 * kb * kHeadDim);
     }
-    // V: i = 4 cc + db, keys 16 cc.., dims 32 db..
-    const int cc = i >> 2, db = i & 3;
-    const uint32_t at = vs + 2 * (16 * cc * kVsPitch + 32 * db);
+    // V: i = 8 kc + db, keys 32 kc.., dims 16 db..
+    const int kc = i >> 3, db = i & 7;
+    const uint32_t at = (vs ^ (32 * db)) + 2 * 32 * kc * kHeadDim;
     const i16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((LdsI16x4*)at);
-    const i16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((LdsI16x4*)(at + 2 * 8 * kVsPitch));
+    const i16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((LdsI16x4*)(at + 2 * 16 * kHeadDim));
     const u32x2 l2 = __builtin_bit_cast(u32x2, lo), h2 = __builtin_bit_cast(u32x2, hi);
     return u32x4{l2[0], l2[1], h2[0], h2[1]};
   };
   u32x4 ring[kLdsAhead];
   auto prefetch_ring = [&](uint32_t kt) __attribute__((always_inline)) {
-    const uint32_t ks = step_base(k_read + 2 * (kt & 1) * kKsHalves);
-    const uint32_t vs = step_base(v_read + 2 * mod3(kt + 2) * kVsHalves);  // V(kt-1)
+    const uint32_t ks = k_base(kt), vs = v_base(kt);
 #pragma unroll
     for (int n = 0; n < kLdsAhead; ++n) ring[n] = stream_operand(ks, vs, n);
   };
-  auto matrix_step = [&](auto group, uint32_t kt) __attribute__((always_inline)) {
-    const uint32_t ks = step_base(k_read + 2 * (kt & 1) * kKsHalves);
-    const uint32_t vs = step_base(v_read + 2 * mod3(kt + 2) * kVsHalves);
-    const uint32_t store_at = store_base(group, group ? (int)mod3(kt + 1) : (int)((kt + 1) & 1));
-    // staging work is dealt out between the MFMAs, and a full scheduling barrier
-    // after every MFMA keeps the compiler from regrouping any of it
+  auto matrix_step = [&](uint32_t kt) __attribute__((always_inline)) {
+    __builtin_amdgcn_s_setprio(0);
+    const uint32_t ks = k_base(kt), vs = v_base(kt);
+    // a full scheduling barrier after every operand's MFMAs keeps the compiler from regrouping them
     __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
     for (int n = 0; n < 32; ++n) {
       const int i = n >> 1;
-      if (n & 1) {
-        const int s = i >> 1, mb = i & 1;
-        if (s == 0) {
-          f32x16 z;
+      const u32x4 a = ring[n % kLdsAhead];
 #pragma unroll
-          for (int r = 0; r < 16; ++r) z[r] = 0.0f;
-          st[mb] = Mfma<T>::m32x32x16(ring[n % kLdsAhead], qreg[s], z);
-        } else {
-          st[mb] = Mfma<T>::m32x32x16(ring[n % kLdsAhead], qreg[s], st[mb]);
-        }
-      } else {
-        oacc[i & 3] = Mfma<T>::m32x32x16(ring[n % kLdsAhead], pk[i >> 2], oacc[i & 3]);
+      for (int rb = 0; rb < 2; ++rb) {
+        if (n & 1)
+          st[i & 3][rb] = Mfma<T>::m16x16x32(a, qreg[rb][i >> 2], i < 4 ? f32x4{0.0f, 0.0f, 0.0f, 0.0f} : st[i & 3][rb]);
+        else
+          oacc[i & 7][rb] = Mfma<T>::m16x16x32(a, pk[i >> 3][rb], oacc[i & 7][rb]);
       }
       if (n + kLdsAhead < 32) ring[n % kLdsAhead] = stream_operand(ks, vs, n + kLdsAhead);
-      // staging last: the loads issued at the end of the previous matrix step have had
-      // almost a whole iteration (~2 us) to arrive before their registers are stored
-      if (n >= 24 && n < 28) store_piece(group, store_at, n - 24);
-      if (n >= 28 && n < 32) load_piece(kt + 2, n - 28);
       __builtin_amdgcn_sched_barrier(0);
     }
-    // the barrier that follows carries no wait of its own: wait here for the LDS stores
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
+    // tile kt + 1 has landed (kPpAhead - 2 younger ones are on their way), operand reads have returned
+    asm volatile("s_waitcnt vmcnt(4) lgkmcnt(0)" ::: "memory");
   };
 
-  // Vector step kt = soft-max of tile kt: mask on the diagonal, row max, lazy
-  // rescale of O^T, exponentials, packing, row sum.
-  auto vector_step = [&](uint32_t kt) __attribute__((always_inline)) {
-    const uint32_t kb = (kt0 + kt) * kBK;
-    if (kb + kBK - 1 > first_pos) {  // tile crosses this row block's diagonal
+  const int last_key = (int)(P0 + tok0 + c16) - 4 * g;   // relative to the lane's first key of a tile
+  // P = exp2(c s + neg) of the tile's scores, packed, and this lane's sums of it
+  auto exponentials = [&](const float (&neg)[2], float (&psum)[2]) __attribute__((always_inline)) {
 #pragma unroll
-      for (int mb = 0; mb < 2; ++mb)
+    for (int rb = 0; rb < 2; ++rb) {
+      psum[rb] = 0.0f;
 #pragma unroll
-        for (int r = 0; r < 16; ++r) {
-          const uint32_t key = kb + 32 * mb + 8 * (r >> 2) + 4 * g + (r & 3);
-          st[mb][r] = (key <= rowpos) ? st[mb][r] : -INFINITY;
+      for (int kc = 0; kc < 2; ++kc)
+#pragma unroll
+        for (int w = 0; w < 4; ++w) {
+          const f32x4& s4 = st[2 * kc + (w >> 1)][rb];
+          const float p0 = fast_exp2(__builtin_fmaf(s4[2 * (w & 1)], c, neg[rb]));
+          const float p1 = fast_exp2(__builtin_fmaf(s4[2 * (w & 1) + 1], c, neg[rb]));
+          pk[kc][rb][w] = Mfma<T>::pack2(p0, p1);
+          psum[rb] += p0 + p1;
         }
     }
-    float rmax = st[0][0];
+  };
+
+  // Vector step kt = request of tile kt + 3, then soft-max of tile kt: mask on the diagonal, exponentials,
+  // packing, row sum; row maximum and rescaling of O^T where they are due.  (Its wave goes first where both
+  // waves of a SIMD have something to issue: 0.5 to 1 % on long calls.)
+  auto vector_step = [&](auto group, uint32_t kt) __attribute__((always_inline)) {
+    load_tile(group, kt + kPpAhead);
+    __builtin_amdgcn_s_setprio(2);
+    const uint32_t kb = (kt0 + kt) * kBK;
+    if (kb + kBK - 1 > first_pos) {  // tile crosses this row block's diagonal
+      const int past = last_key - (int)kb;   // row block 0 sees keys 0 .. past of this lane's, row block 1 sixteen more
 #pragma unroll
-    for (int mb = 0; mb < 2; ++mb)
+      for (int b = 0; b < 4; ++b)
 #pragma unroll
-      for (int r = 0; r < 16; ++r) rmax = fmaxf(rmax, st[mb][r]);
-    rmax = max_with_partner_half(rmax);
-    const float tmax = rmax * c;
-    const bool grow = tmax > m_run + kRescaleStep;
-    if (__any(grow)) {
-      const float m_new = grow ? tmax : m_run;
-      const float alpha = grow ? fast_exp2(m_run - m_new) : 1.0f;
-      m_run = m_new;
-      l_run *= alpha;
+        for (int r = 0; r < 4; ++r)
 #pragma unroll
-      for (int db = 0; db < 4; ++db) oacc[db] *= alpha;
+          for (int rb = 0; rb < 2; ++rb) st[b][rb][r] = 16 * (b - rb) + r <= past ? st[b][rb][r] : -INFINITY;
     }
-    const float neg_m = (m_run == -INFINITY) ? 0.0f : -m_run;
-    float psum = 0.0f;
+    // Exponentials against the reference maximum each row already has: while no lane's sum of them
+    // passes kMaxSum, the true maximum is not looked for.  A row without a reference (neg_m = +inf)
+    // makes its sums infinite or NaN and so asks for one; so does a score that is not finite.
+    float psum[2];
+    exponentials(neg_m, psum);
+    const uint64_t over[2] = {__ballot(!(psum[0] <= kMaxSum)), __ballot(!(psum[1] <= kMaxSum))};
+    if (over[0] | over[1]) {
+      float rmax[2], safe[2];
 #pragma unroll
-    for (int cc = 0; cc < 4; ++cc) {
-      const int mb = cc >> 1, r0 = 8 * (cc & 1);
+      for (int rb = 0; rb < 2; ++rb) {
+        rmax[rb] = st[0][rb][0];
 #pragma unroll
-      for (int w = 0; w < 4; ++w) {
-        const float p0 = fast_exp2(__builtin_fmaf(st[mb][r0 + 2 * w], c, neg_m));
-        const float p1 = fast_exp2(__builtin_fmaf(st[mb][r0 + 2 * w + 1], c, neg_m));
-        pk[cc][w] = Mfma<T>::pack2(p0, p1);
-        psum += p0 + p1;
+        for (int b = 0; b < 4; ++b)
+#pragma unroll
+          for (int r = 0; r < 4; ++r) rmax[rb] = fmaxf(rmax[rb], st[b][rb][r]);
       }
+      max_over_quarters(rmax[0], rmax[1]);
+#pragma unroll
+      for (int rb = 0; rb < 2; ++rb) {
+        // (a row moves by what its own four lanes saw: its bits do not depend on its neighbours)
+        const uint64_t any = over[rb] >> c16;
+        const bool moves = ((any | any >> 16 | any >> 32 | any >> 48) & 1) != 0;
+        const float neg_new = moves ? fminf(neg_m[rb], -(rmax[rb] * c)) : neg_m[rb];   // (+inf while no key of the row is visible)
+        safe[rb] = neg_new == INFINITY ? 0.0f : neg_new;
+        const float alpha = fast_exp2(safe[rb] - neg_m[rb]);       // (a row's first reference: exp2(-inf) = 0)
+        neg_m[rb] = neg_new;
+        l_run[rb] *= alpha;
+#pragma unroll
+        for (int db = 0; db < 8; ++db) oacc[db][rb] *= alpha;
+      }
+      exponentials(safe, psum);
     }
-    l_run += psum;
+    l_run[0] += psum[0];
+    l_run[1] += psum[1];
   };
 
   // Phases, one workgroup barrier apart: group 0 runs matrix(0) | vector(0) |
@@ -391,60 +422,55 @@ __global__ __launch_bounds__(kPpThreads, 2) void prefill_pingpong_kernel(Prefill
   constexpr std::integral_constant<int, 1> kGroup1;
   if (__builtin_amdgcn_readfirstlane(grp) == 0) {
     prefetch_ring(0);
-    matrix_step(kGroup0, 0);
+    matrix_step(0);
     __builtin_amdgcn_s_barrier();
     for (uint32_t kt = 0; kt < n_tiles; ++kt) {
-      vector_step(kt);
+      vector_step(kGroup0, kt);
       prefetch_ring(kt + 1);
       __builtin_amdgcn_s_barrier();
-      matrix_step(kGroup0, kt + 1);
+      matrix_step(kt + 1);
       __builtin_amdgcn_s_barrier();
     }
   } else {
     prefetch_ring(0);
     __builtin_amdgcn_s_barrier();
     for (uint32_t kt = 0; kt < n_tiles; ++kt) {
-      matrix_step(kGroup1, kt);
+      matrix_step(kt);
       __builtin_amdgcn_s_barrier();
-      vector_step(kt);
+      vector_step(kGroup1, kt);
       prefetch_ring(kt + 1);
       __builtin_amdgcn_s_barrier();
     }
-    matrix_step(kGroup1, n_tiles);
+    matrix_step(n_tiles);
   }
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // the last requests still write LDS
 
-
-  if constexpr (SPLIT) {
-    const float l = sum_with_partner_half(l_run);
-    if (row_valid) {
+#pragma unroll
+  for (int rb = 0; rb < 2; ++rb) {
+    const float l = sum_over_quarters(l_run[rb]);
+    const float m = -neg_m[rb];
+    const uint32_t tok = tok0 + 16 * rb + c16;
+    if (tok >= S) continue;
+    if constexpr (SPLIT) {
       const size_t part = (((size_t)tok * p.batch_pitch + seq) * p.n_q_heads + head) * p.n_split + blockIdx.y;
       float* orow = p.part_o + part * kHeadDim;
 #pragma unroll
-      for (int db = 0; db < 4; ++db)
-#pragma unroll
-        for (int q4 = 0; q4 < 4; ++q4)
-          *(f32x4*)(orow + 32 * db + 8 * q4 + 4 * g) =
-              f32x4{oacc[db][4 * q4], oacc[db][4 * q4 + 1], oacc[db][4 * q4 + 2], oacc[db][4 * q4 + 3]};
-      if (g == 0) *(float2*)(p.part_ml + part * 2) = float2{m_run, l};
-    }
-  } else {
-    const float l = sum_with_partner_half(l_run);
-    if (row_valid) {
+      for (int db = 0; db < 8; ++db) *(f32x4*)(orow + 16 * db + 4 * g) = oacc[db][rb];
+      if (g == 0) *(float2*)(p.part_ml + part * 2) = float2{m, l};
+    } else {
       const float inv = 1.0f / l;
       uint16_t* orow =
           p.out + (size_t)tok * p.q_token_stride + ((size_t)seq * p.n_q_heads + head) * kHeadDim;
 #pragma unroll
-      for (int db = 0; db < 4; ++db)
-#pragma unroll
-        for (int q4 = 0; q4 < 4; ++q4) {
-          u32x2 w;
-          w[0] = Mfma<T>::pack2(oacc[db][4 * q4] * inv, oacc[db][4 * q4 + 1] * inv);
-          w[1] = Mfma<T>::pack2(oacc[db][4 * q4 + 2] * inv, oacc[db][4 * q4 + 3] * inv);
-          *(u32x2*)(orow + 32 * db + 8 * q4 + 4 * g) = w;
-        }
+      for (int db = 0; db < 8; ++db) {
+        u32x2 w;
+        w[0] = Mfma<T>::pack2(oacc[db][rb][0] * inv, oacc[db][rb][1] * inv);
+        w[1] = Mfma<T>::pack2(oacc[db][rb][2] * inv, oacc[db][rb][3] * inv);
+        *(u32x2*)(orow + 16 * db + 4 * g) = w;
+      }
       if (p.lse && g == 0)
         p.lse[((size_t)tok * p.batch_pitch + seq) * p.n_q_heads + head] =
-            (m_run + fast_log2(l)) * kLn2;
+            (m + fast_log2(l)) * kLn2;
     }
   }
 }

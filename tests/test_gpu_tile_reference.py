@@ -1,0 +1,48 @@
+"""The tile kernel's reference maximum: exponentials are taken against the one a row has until a lane's
+sum of them passes 2^15, then the row's true maximum is looked for and its sums are rescaled.  Score
+levels that stay below that step, pass it once, again and again, fall back and pass it in some rows of a
+block only; whole rows and a key range in splits, whose later splits some rows see nothing of."""
+import math
+
+import numpy as np
+import pytest
+
+import oracle_lib as orc
+import plan_probe
+from gpu_util import D, LSE_TOL, gpu_attention, rand_storage, storage_ulp
+
+pytestmark = pytest.mark.gpu
+
+# levels of successive 64-key tiles, in units of the score's log2: below the step of 15, once past it,
+# rising all along, falling, up and down
+LEVELS = {"below": [0, 13, 14, 12], "once": [0, 0, 17, 17], "rising": [0, 16, 40, 300], "falling": [300, 30, 10, 0],
+          "waves": [0, 40, -40, 60]}
+
+
+@pytest.mark.parametrize("b,hq,hkv,s,p0,split", [(16, 32, 4, 49, 200, False), (1, 8, 1, 70, 2400, True)], ids=["whole", "split"])
+@pytest.mark.parametrize("name", LEVELS)
+@pytest.mark.parametrize("dtype", [orc.F16, orc.BF16], ids=["f16", "bf16"])
+def test_scores_that_outgrow_the_reference(b, hq, hkv, s, p0, split, name, dtype):
+    cap = p0 + s
+    kernel, _, n_split = plan_probe.chunk_plan(b, b, hq, hkv, p0, s)[:3]
+    assert kernel == "pingpong" and (n_split > 1) == split
+    scale = 1.0 / math.sqrt(D)
+    q = orc.from_storage(rand_storage((s, b, hq, D), 5, dtype), dtype)
+    k = orc.from_storage(rand_storage((b, hkv, cap, D), 6, dtype), dtype)
+    v = rand_storage((b, hkv, cap, D), 7, dtype)
+    q[..., 0] = 8.0 * (np.arange(s)[:, None, None] % 3 - 1)    # of three rows one rises, one falls, one stays
+    level = np.array([LEVELS[name][(i // 64) % 4] for i in range(cap)], dtype=np.float32)
+    k[..., 0] = level * np.float32(math.log(2.0) / (8.0 * scale))
+    q, k = orc.to_storage(q, dtype), orc.to_storage(k, dtype)
+    got, lse = gpu_attention(q, k, v, scale, dtype, position_index=p0)
+    want, want_lse = orc.attention(q, k, v, scale, dtype, position_index=p0)
+    want = orc.from_storage(want, dtype)
+    # Every weight is rounded to the storage type once, by half of its last place: at most 2^-11 (2^-8) of
+    # what the row's weights make of the values' magnitudes; both sides round the output once.  (A row
+    # with few keys that count may cancel to far less than that, so no bound relative to the output.)
+    mags = orc.to_storage(np.abs(orc.from_storage(v, dtype)), dtype)
+    size = orc.from_storage(orc.attention(q, k, mags, scale, dtype, position_index=p0)[0], dtype)
+    err, bound = np.abs(got - want), (2.0 ** -11 if dtype == orc.F16 else 2.0 ** -8) * size + storage_ulp(want, dtype)
+    assert (err <= bound).all(), float((err / bound).max())
+    # (a log-sum-exp of up to 208 is spaced 2^-16; the bound leaves it a dozen roundings)
+    assert np.abs(lse - want_lse).max() <= LSE_TOL + 12 * 2.0 ** -16
