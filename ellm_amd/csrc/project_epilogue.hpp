@@ -1,5 +1,5 @@
 // Epilogue shared by the MFMA tile kernels of the projections: a wave that holds one head
-// (128 output columns) of 32 * MB tokens as transposed 32x32 accumulator blocks finishes
+// (128 output columns) of 32 * MB tokens as transposed 16x16 accumulator blocks finishes
 // the head rows (RMS norm + rotary rotation, or residual add), rounds them and writes
 // them to their destinations.
 #pragma once
@@ -18,13 +18,13 @@ constexpr int kEpWaveBytes = 2 * 32 * kEpPitch;       // per wave: 32 output row
 
 typedef __attribute__((address_space(1))) u32x4 GlobalVec4;
 
-// acc[nb][mb]: column block nb (32 columns) x token block mb (32 tokens) of head `hh`;
-// `first_row` is the row of the activations that token block 0, lane row 0 stands for;
-// `ep_rows` is the LDS byte address of kEpWaveBytes that belong to this wave alone.
-// In the accumulator layout lane (j, g) holds, for token 32 mb + j, the
-// columns 32 nb + 8 b + 4 g + (0..3) of the head: four consecutive columns = two rotation
+// acc[nb][t]: column block nb (16 columns) x token block t (16 tokens) of head `hh`, 32 tokens (two
+// blocks, mb below) at a time; `first_row` is the row of the activations that token block 0, lane row 0
+// stands for; `ep_rows` is the LDS byte address of kEpWaveBytes that belong to this wave alone.
+// In the accumulator layout lane (c16, g) holds, for token 16 t + c16, the
+// columns 16 nb + 4 g + (0..3) of the head: four consecutive columns = two rotation
 // pairs = one 8-byte piece of the rotary row, of the residual row and of the output
-// row; lanes l and l ^ 32 together own the token's 128 columns.
+// row; lanes l, l ^ 16, l ^ 32, l ^ 48 together own the token's 128 columns.
 // Memory is touched in whole rows only, in both directions: a wave instruction moves four
 // 256-byte rows (16 lanes a row), and LDS turns rows into the accumulator layout and back.
 // (Fetching the extra operand in the accumulator layout directly, 8 bytes a lane from 32
@@ -41,7 +41,7 @@ typedef __attribute__((address_space(1))) u32x4 GlobalVec4;
 // residual rows are waited for after it.
 template <int MB>
 struct HeadRows {
-  uint16_t* out_row[MB];        // this lane's token: destination row (g == 0 and g == 1 alike)
+  uint16_t* out_row[MB];        // token lane % 32 of a block of 32: destination row
   const uint16_t* ext_row[MB];  // ... and row of the extra operand; null: none (scale 1, no rotation)
   bool present;    // false: the head lies beyond the last one (odd head count), nothing to do
   bool finalize;   // normalise + rotate
@@ -116,17 +116,18 @@ __device__ __forceinline__ HeadRows<MB> prepare_head(const ProjectKernelArgs& p,
 }
 
 template <typename S, int MODE, int MB>
-__device__ __forceinline__ void finish_head(const ProjectKernelArgs& p, f32x16 (&acc)[4][MB],
+__device__ __forceinline__ void finish_head(const ProjectKernelArgs& p, f32x4 (&acc)[8][2 * MB],
                                             const HeadRows<MB>& h, uint32_t ep_rows, int lane) {
   using M = Mfma<S>;
-  const int j = lane & 31, g = lane >> 5;
+  const int c16 = lane & 15, g = lane >> 4;
   if (!h.present) return;
   const bool finalize = h.finalize;
   const uint32_t ep_ext = ep_rows + 32 * kEpPitch;
   // this lane's place as a mover of whole rows (row lane / 16 + 4 i, piece lane % 16) and as the
-  // owner of token j (8-byte pieces at columns 32 nb + 8 b + 4 g)
+  // owner of tokens c16 and 16 + c16 (8-byte pieces at columns 16 nb + 4 g)
   const uint32_t row_piece = (lane >> 4) * kEpPitch + 16 * (lane & 15);
-  const uint32_t own_piece = j * kEpPitch + 8 * g;
+  const uint32_t own_piece = c16 * kEpPitch + 8 * g;
+  auto piece_at = [](int i) { return 16 * (i & 1) * kEpPitch + 32 * (i >> 1); };   // i: token block i & 1, column block i / 2
   u32x4 raw[8];
 #pragma unroll
   for (int i = 0; i < 8; ++i) raw[i] = h.ext0[i];
@@ -142,30 +143,32 @@ __device__ __forceinline__ void finish_head(const ProjectKernelArgs& p, f32x16 (
   static_for<MB>([&](auto mb_) {
     constexpr int mb = decltype(mb_)::value;
     __builtin_amdgcn_sched_barrier(0);  // one token block's accumulators at a time leave the AGPRs
-    float inv = 1.0f;
+    float inv[2] = {1.0f, 1.0f};
     if (MODE == kModeQkv) {
-      float ss = 0.0f;
 #pragma unroll
-      for (int nb = 0; nb < 4; ++nb)
+      for (int t = 0; t < 2; ++t) {
+        float ss = 0.0f;
 #pragma unroll
-        for (int r = 0; r < 16; ++r) ss = fmaf(acc[nb][mb][r], acc[nb][mb][r], ss);
-      ss = sum_with_partner_half(ss);
-      inv = finalize ? 1.0f / (sqrtf(ss / (float)kHeadDim) + p.eps) : 1.0f;
+        for (int nb = 0; nb < 8; ++nb)
+#pragma unroll
+          for (int r = 0; r < 4; ++r) ss = fmaf(acc[nb][2 * mb + t][r], acc[nb][2 * mb + t][r], ss);
+        ss = sum_over_quarters(ss);
+        inv[t] = finalize ? 1.0f / (sqrtf(ss / (float)kHeadDim) + p.eps) : 1.0f;
+      }
     }
     u32x2 ext[16];
 #pragma unroll
-    for (int i = 0; i < 16; ++i) ext[i] = *(const LdsVec2*)(ep_ext + own_piece + 2 * (32 * (i >> 2) + 8 * (i & 3)));
+    for (int i = 0; i < 16; ++i) ext[i] = *(const LdsVec2*)(ep_ext + own_piece + piece_at(i));
     u32x2 packed[16];
 #pragma unroll
     for (int i = 0; i < 16; ++i) {
-      const int nb = i >> 2, b4 = i & 3;
-      float o0 = acc[nb][mb][4 * b4], o1 = acc[nb][mb][4 * b4 + 1];
-      float o2 = acc[nb][mb][4 * b4 + 2], o3 = acc[nb][mb][4 * b4 + 3];
+      const f32x4& v4 = acc[i >> 1][2 * mb + (i & 1)];
+      float o0 = v4[0], o1 = v4[1], o2 = v4[2], o3 = v4[3];
       const u32x2 rr = ext[i];
       const float e0 = M::to_float((uint16_t)(rr[0] & 0xffffu)), e1 = M::to_float((uint16_t)(rr[0] >> 16));
       const float e2 = M::to_float((uint16_t)(rr[1] & 0xffffu)), e3 = M::to_float((uint16_t)(rr[1] >> 16));
       if (MODE == kModeQkv) {
-        const float y0 = o0 * inv, y1 = o1 * inv, y2 = o2 * inv, y3 = o3 * inv;
+        const float y0 = o0 * inv[i & 1], y1 = o1 * inv[i & 1], y2 = o2 * inv[i & 1], y3 = o3 * inv[i & 1];
         o0 = y0 * e0 - y1 * e1;
         o1 = y0 * e1 + y1 * e0;
         o2 = y2 * e2 - y3 * e3;
@@ -182,7 +185,7 @@ __device__ __forceinline__ void finish_head(const ProjectKernelArgs& p, f32x16 (
     // up all eight of theirs before the first store
 #pragma unroll
     for (int i = 0; i < 16; ++i)
-      *(LdsVec2*)(ep_rows + own_piece + 2 * (32 * (i >> 2) + 8 * (i & 3))) = packed[i];
+      *(LdsVec2*)(ep_rows + own_piece + piece_at(i)) = packed[i];
     if constexpr (mb + 1 < MB) stage_ext(mb + 2);
     uint64_t to[8];
     u32x4 v[8];

@@ -2,13 +2,9 @@
 // tiles of project.hip leave most compute units without a workgroup (1536 rows, the
 // reference's own serving shape of 64 positions x 24 sequences, src/serving/start copy.rs:30,
 // make 6 x 20 of them for the fused Q/K/V projection and 6 x 8 for the output projection).
-// Same formulation (C^T = W . X^T on v_mfma_f32_32x32x16, a lane owns a token), same LDS
-// layout and the same epilogue; the tile is 128 or 256 tokens x one head (a wave owns one or
-// two 32-token blocks x the head's four column blocks).  Tiles this small move up to twice
+// The same tile code (project_mid_tile.hpp) at 128 or 256 tokens x one head.  Tiles this small move up to twice
 // the LDS bytes per MFMA, and 128-bit LDS stores are slow (13 cycles an instruction against
-// 4.7 for a read): here the operand tiles go from memory straight into LDS (buffer loads
-// with the LDS bit) through four (three) stages, and the LDS instruction pipe carries the
-// operand reads only.
+// 4.7 for a read), one more reason why operands go from memory straight into LDS.
 #include "project_mid_tile.hpp"
 
 namespace ellm {
@@ -26,7 +22,7 @@ __global__ __launch_bounds__(64 * WAVES) void project_mid_kernel(ProjectKernelAr
   const uint32_t per_band = p.band_m * p.tiles_n;
   const uint32_t first_m = pid / per_band * p.band_m, in_band = pid % per_band;
   const uint32_t here = min(p.tiles_m - first_m, p.band_m);
-  mid_tile<S, MODE, MB, WAVES>(p, (first_m + in_band % here) * MidShape<MB, WAVES>::kTokens, in_band / here, mid_smem);
+  mid_tile<S, MODE, MB, WAVES, 1>(p, (first_m + in_band % here) * MidShape<MB, WAVES, 1>::kTokens, in_band / here, mid_smem);
 }
 
 template <int MB, int WAVES>
@@ -37,7 +33,7 @@ hipError_t prepare_shape() {
                            (const void*)project_mid_kernel<BF16, kModeAdd, MB, WAVES>};
   for (const void* k : kernels) {
     const hipError_t e =
-        hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, MidShape<MB, WAVES>::kLdsBytes);
+        hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, MidShape<MB, WAVES, 1>::kLdsBytes);
     if (e != hipSuccess) return e;
   }
   return hipSuccess;
@@ -68,7 +64,7 @@ uint32_t mid_band(uint32_t tiles_m, uint32_t tiles_n, uint32_t tokens) {
 
 template <int MB, int WAVES>
 hipError_t launch_shape(ProjectKernelArgs p, int dtype, bool add, hipStream_t stream) {
-  using Shape = MidShape<MB, WAVES>;
+  using Shape = MidShape<MB, WAVES, 1>;
   p.tiles_m = (p.rows + Shape::kTokens - 1) / Shape::kTokens;
   p.tiles_n = p.heads0 + 2 * p.heads_kv;
   p.band_m = mid_band(p.tiles_m, p.tiles_n, Shape::kTokens);
@@ -89,10 +85,11 @@ hipError_t mid_prepare() {
   return e != hipSuccess ? e : prepare_shape<1, 8>();
 }
 
-// The 256-token tile runs as eight waves of one token block each: measured against four waves of two
-// blocks at 1536 rows x 2048 -> 5120, 36.9 against 39.5 us (either way a compute unit takes in
-// (256 + 128) x 128 bytes of operands per chunk at the 55-60 GB/s one unit streams from L2, which is
-// what sets the chunk time of 0.8 us; the second wave per SIMD only hides the stalls around it).
+// 32x32x16 instructions -> this tile code (us, Q/K/V | output projection): 2048 wide 100 rows 18.0 | 29.1 ->
+// 17.1 | 27.1, 1536 rows 37.2 | 34.6 -> 31.9 | 31.6; 4096 wide 256 rows 39.7 | 30.5 -> 35.3 | 28.4; 8192 wide 768 rows
+// 132 | 118 -> 116 | 104.  One wave a SIMD (128 tokens) issues 16x16x32 instructions as fast only while it has
+// little else to issue: with a register sum per operand read and a descriptor select per load it took 19.0 | 30.4 at
+// 100 rows, with neither 17.1 | 27.1.
 hipError_t launch_project_mid(ProjectKernelArgs p, uint32_t token_blocks, int dtype, bool add,
                               hipStream_t stream) {
   if (token_blocks != 2) return launch_shape<1, 4>(p, dtype, add, stream);
