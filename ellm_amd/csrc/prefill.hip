@@ -487,7 +487,11 @@ __global__ __launch_bounds__(kPpThreads, 2) void prefill_pingpong_kernel(Prefill
 // workgroups (36 KB of LDS each), which leave partial rows for prefill_merge_kernel as the
 // split form of the kernel above does.  Chunks of 32 keys go memory -> registers -> LDS
 // (double-buffered, one barrier a chunk, the next chunks' loads in flight during the MFMAs of
-// this one); operands and soft-max as above.
+// this one); operands and soft-max as above.  What bounds it: the stream up to 8 tokens, from 16 on the
+// board's power; 32x32x16 instructions with a row maximum every chunk -> 16x16x32 and none (24 sequences on 8191
+// keys, 32 / 4 heads, us): 2 tokens 67.3 -> 67.2, 8 72.9 -> 72.3, 13 88.6 -> 84.1, 24 129.4 -> 114.8, 33 161 ->
+// 146, 48 195 -> 175; 17 x 5 on 6487 34.3 -> 32.3.  Rows and tokens are worked out again behind the loop: kept
+// across it they cost 14 registers, and the form with twelve waves (168) spilled.
 // ---------------------------------------------------------------------------
 constexpr int kSK = 32;                        // keys per compute step
 constexpr int kStStagersMax = 8 * kWave;       // one 16-byte piece of K and of V each moves a whole chunk
@@ -508,15 +512,14 @@ __global__ __launch_bounds__(WAVES * kWave, WAVES == 4 ? 2 : 1) void chunk_strea
   constexpr int kThreads = WAVES * kWave;
   constexpr int kStagers = kThreads < kStStagersMax ? kThreads : kStStagersMax;  // threads that move K/V
   constexpr int kCK = kSK;                       // keys per staged chunk
-  constexpr int kStKsHalves = kCK * kKsPitch;
-  constexpr int kStVsHalves = kCK * kVsPitch;
+  constexpr int kStHalves = kCK * kVsPitch;      // K and V rows alike 288 B apart: operand reads meet no bank twice
   constexpr int kPieces = kCK * 16 / kStagers;   // 16-byte pieces of K (and of V) a staging thread moves per chunk
   constexpr int kPieceRows = kStagers / 16;      // rows between a thread's pieces
   static_assert(kPieces * kStagers == kCK * 16, "the staging threads must tile a chunk");
-  __shared__ __attribute__((aligned(16))) uint16_t smem[2 * kStKsHalves + 2 * kStVsHalves];
+  __shared__ __attribute__((aligned(16))) uint16_t smem[4 * kStHalves];
 
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int j = lane & 31, g = lane >> 5;
+  const int c16 = lane & 15, g = lane >> 4;
   const uint32_t seq = blockIdx.x / p.n_kv_heads, kvh = blockIdx.x % p.n_kv_heads;
   const uint32_t S = p.interval, P0 = p.position_index;
   const uint32_t kmax = P0 + S - 1;
@@ -528,25 +531,29 @@ __global__ __launch_bounds__(WAVES * kWave, WAVES == 4 ? 2 : 1) void chunk_strea
   const uint32_t n_chunks = (min(kmax + 1, k0 + n_tiles * kBK) - k0 + kCK - 1) / kCK;
 
   const uint32_t rows = S * p.group;                                // query rows of the plane, <= 32 WAVES
-  const uint32_t r = 32 * wave + j;
-  const bool row_valid = r < rows;
-  const uint32_t rc = row_valid ? r : rows - 1;
-  const uint32_t tok = rc / p.group, head = kvh * p.group + rc % p.group;
-  const uint32_t rowpos = P0 + tok;
+  // this lane's rows: 16 rb + c16 of the wave's 32 (those past the last one repeat it and are not stored)
+  uint32_t first_row = 32 * wave + c16;
+  auto row_of = [&](int rb) { return first_row + 16 * rb; };
+  auto token_of = [&](int rb) { return min(row_of(rb), rows - 1) / p.group; };
+  auto head_of = [&](int rb) { return kvh * p.group + min(row_of(rb), rows - 1) % p.group; };
+  uint32_t rowpos[2];
   // positions of the wave's first and last row: chunks past the last are skipped, chunks up to
   // the first need no mask
   const uint32_t wave_first_pos = P0 + min(32u * wave, rows - 1) / p.group;
   const uint32_t wave_last_pos = P0 + min(32u * wave + 31u, rows - 1) / p.group;
   const bool wave_has_rows = 32u * wave < rows;
 
-  u32x4 qreg[8];
-  {
-    const uint16_t* qrow =
-        p.q + (size_t)tok * p.q_token_stride + ((size_t)seq * p.n_q_heads + head) * kHeadDim;
+  u32x4 qreg[2][4];   // [row block][32 dims]
 #pragma unroll
-    for (int s = 0; s < 8; ++s) {
-      qreg[s] = load16(qrow + 16 * s + 8 * g);
-      if (p.negate_q) qreg[s] ^= 0x80008000u;
+  for (int rb = 0; rb < 2; ++rb) {
+    const uint32_t tok = token_of(rb);
+    rowpos[rb] = P0 + tok;
+    const uint16_t* qrow =
+        p.q + (size_t)tok * p.q_token_stride + ((size_t)seq * p.n_q_heads + head_of(rb)) * kHeadDim;
+#pragma unroll
+    for (int s = 0; s < 4; ++s) {
+      qreg[rb][s] = load16(qrow + 32 * s + 8 * g);
+      if (p.negate_q) qreg[rb][s] ^= 0x80008000u;
     }
   }
   const float c = p.c;
@@ -579,87 +586,110 @@ __global__ __launch_bounds__(WAVES * kWave, WAVES == 4 ? 2 : 1) void chunk_strea
     }
   };
   const uint32_t lds0 = (uint32_t)(uintptr_t)(LdsHalf*)smem;
-  const uint32_t ks_store = lds0 + 2 * (ld_r * kKsPitch + 8 * ld_c);
-  const uint32_t vs_store = lds0 + 2 * (2 * kStKsHalves + ld_r * kVsPitch + 8 * ld_c);
+  const uint32_t ks_store = lds0 + 2 * (ld_r * kVsPitch + 8 * ld_c), vs_store = ks_store + 2 * 2 * kStHalves;
   auto store_chunk = [&](uint32_t buf, const u32x4 (&st)[2 * kPieces]) {
     if (!stager) return;
 #pragma unroll
     for (int i = 0; i < kPieces; ++i) {
-      *(LdsU32x4*)(ks_store + 2 * (buf * kStKsHalves + kPieceRows * i * kKsPitch)) = st[i];
-      *(LdsU32x4*)(vs_store + 2 * (buf * kStVsHalves + kPieceRows * i * kVsPitch)) = st[kPieces + i];
+      *(LdsU32x4*)(ks_store + 2 * (buf * kStHalves + kPieceRows * i * kVsPitch)) = st[i];
+      *(LdsU32x4*)(vs_store + 2 * (buf * kStHalves + kPieceRows * i * kVsPitch)) = st[kPieces + i];
     }
   };
   // operand addresses: as in the kernel above (K rows as the A operand of S^T = K.Q^T, V through
   // the transposing read as the A operand of O^T += V^T.P^T, keys in the order P is left in)
-  const uint32_t k_read = lds0 + 2 * (j * kKsPitch + 8 * g);
-  const uint32_t v_read = lds0 + 2 * (2 * kStKsHalves + (4 * g + ((lane & 15) >> 2)) * kVsPitch +
-                                      16 * ((lane >> 4) & 1) + 4 * (lane & 3));
+  const uint32_t k_read = lds0 + 2 * (c16 * kVsPitch + 8 * g);
+  const uint32_t v_read = lds0 + 2 * (2 * kStHalves + (4 * g + (c16 >> 2)) * kVsPitch + 4 * (c16 & 3));
 
-  float m_run = -INFINITY, l_run = 0.0f;
-  f32x16 oacc[4];
+  // per row: minus its reference maximum (+inf: no key seen yet), this lane's share of the denominator
+  float neg_m[2] = {INFINITY, INFINITY}, l_run[2] = {0.0f, 0.0f};
+  f32x4 oacc[8][2];   // [16 dims][row block]
 #pragma unroll
-  for (int db = 0; db < 4; ++db)
+  for (int db = 0; db < 8; ++db)
 #pragma unroll
-    for (int e = 0; e < 16; ++e) oacc[db][e] = 0.0f;
+    for (int rb = 0; rb < 2; ++rb) oacc[db][rb] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
 
   auto compute = [&](uint32_t ck) __attribute__((always_inline)) {
     const uint32_t kb = k0 + ck * kCK;
     const uint32_t buf = ck & 1;
     if (wave_has_rows && kb <= wave_last_pos) {
-      const uint32_t ks = k_read + 2 * buf * kStKsHalves;
-      const uint32_t vs = v_read + 2 * buf * kStVsHalves;
-      f32x16 st;
+      const uint32_t ks = k_read + 2 * buf * kStHalves;
+      const uint32_t vs = v_read + 2 * buf * kStHalves;
+      f32x4 st[2][2];   // [16 keys][row block]
 #pragma unroll
-      for (int e = 0; e < 16; ++e) st[e] = 0.0f;
+      for (int s = 0; s < 4; ++s) {
 #pragma unroll
-      for (int s = 0; s < 8; ++s) {
-        const u32x4 a = *(const LdsU32x4*)(ks + 2 * 16 * s);
-        st = Mfma<T>::m32x32x16(a, qreg[s], st);
+        for (int b = 0; b < 2; ++b) {
+          const u32x4 a = *(const LdsU32x4*)(ks + 2 * (16 * b * kVsPitch + 32 * s));
+#pragma unroll
+          for (int rb = 0; rb < 2; ++rb)
+            st[b][rb] = Mfma<T>::m16x16x32(a, qreg[rb][s], s ? st[b][rb] : f32x4{0.0f, 0.0f, 0.0f, 0.0f});
+        }
       }
       if (kb + kSK - 1 > wave_first_pos) {  // chunk crosses the diagonal of some row of this wave
 #pragma unroll
-        for (int e = 0; e < 16; ++e) {
-          const uint32_t key = kb + 8 * (e >> 2) + 4 * g + (e & 3);
-          st[e] = (key <= rowpos) ? st[e] : -INFINITY;
-        }
+        for (int b = 0; b < 2; ++b)
+#pragma unroll
+          for (int r = 0; r < 4; ++r)
+#pragma unroll
+            for (int rb = 0; rb < 2; ++rb)
+              st[b][rb][r] = (kb + 16 * b + 4 * g + r <= rowpos[rb]) ? st[b][rb][r] : -INFINITY;
       }
-      float rmax = st[0];
+      u32x4 pk[2];   // [row block]
+      float psum[2];
+      auto exponentials = [&](const float (&neg)[2]) __attribute__((always_inline)) {
 #pragma unroll
-      for (int e = 1; e < 16; ++e) rmax = fmaxf(rmax, st[e]);
-      rmax = max_with_partner_half(rmax);
-      const float tmax = rmax * c;
-      const bool grow = tmax > m_run + kRescaleStep;
-      if (__any(grow)) {
-        const float m_new = grow ? tmax : m_run;
-        const float alpha = grow ? fast_exp2(m_run - m_new) : 1.0f;
-        m_run = m_new;
-        l_run *= alpha;
+        for (int rb = 0; rb < 2; ++rb) {
+          psum[rb] = 0.0f;
 #pragma unroll
-        for (int db = 0; db < 4; ++db) oacc[db] *= alpha;
+          for (int w = 0; w < 4; ++w) {
+            const f32x4& s4 = st[w >> 1][rb];
+            const float p0 = fast_exp2(__builtin_fmaf(s4[2 * (w & 1)], c, neg[rb]));
+            const float p1 = fast_exp2(__builtin_fmaf(s4[2 * (w & 1) + 1], c, neg[rb]));
+            pk[rb][w] = Mfma<T>::pack2(p0, p1);
+            psum[rb] += p0 + p1;
+          }
+        }
+      };
+      // (the reference maximum moves where a lane's sum passes kMaxSum: as in the kernel above)
+      exponentials(neg_m);
+      const uint64_t over[2] = {__ballot(!(psum[0] <= kMaxSum)), __ballot(!(psum[1] <= kMaxSum))};
+      if (over[0] | over[1]) {
+        float rmax[2], safe[2];
+#pragma unroll
+        for (int rb = 0; rb < 2; ++rb) {
+          rmax[rb] = st[0][rb][0];
+#pragma unroll
+          for (int b = 0; b < 2; ++b)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) rmax[rb] = fmaxf(rmax[rb], st[b][rb][r]);
+        }
+        max_over_quarters(rmax[0], rmax[1]);
+#pragma unroll
+        for (int rb = 0; rb < 2; ++rb) {
+          const uint64_t any = over[rb] >> c16;
+          const bool moves = ((any | any >> 16 | any >> 32 | any >> 48) & 1) != 0;
+          const float neg_new = moves ? fminf(neg_m[rb], -(rmax[rb] * c)) : neg_m[rb];
+          safe[rb] = neg_new == INFINITY ? 0.0f : neg_new;
+          const float alpha = fast_exp2(safe[rb] - neg_m[rb]);
+          neg_m[rb] = neg_new;
+          l_run[rb] *= alpha;
+#pragma unroll
+          for (int db = 0; db < 8; ++db) oacc[db][rb] *= alpha;
+        }
+        exponentials(safe);
       }
-      const float neg_m = (m_run == -INFINITY) ? 0.0f : -m_run;
-      float psum = 0.0f;
-      u32x4 pk[2];
+      l_run[0] += psum[0];
+      l_run[1] += psum[1];
 #pragma unroll
-      for (int cc = 0; cc < 2; ++cc)
+      for (int db = 0; db < 8; ++db) {
+        const uint32_t at = vs + 2 * 16 * db;
+        const i16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((LdsI16x4*)at);
+        const i16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((LdsI16x4*)(at + 2 * 16 * kVsPitch));
+        const u32x2 l2 = __builtin_bit_cast(u32x2, lo), h2 = __builtin_bit_cast(u32x2, hi);
 #pragma unroll
-        for (int w = 0; w < 4; ++w) {
-          const float p0 = fast_exp2(__builtin_fmaf(st[8 * cc + 2 * w], c, neg_m));
-          const float p1 = fast_exp2(__builtin_fmaf(st[8 * cc + 2 * w + 1], c, neg_m));
-          pk[cc][w] = Mfma<T>::pack2(p0, p1);
-          psum += p0 + p1;
-        }
-      l_run += psum;
-#pragma unroll
-      for (int cc = 0; cc < 2; ++cc)
-#pragma unroll
-        for (int db = 0; db < 4; ++db) {
-          const uint32_t at = vs + 2 * (16 * cc * kVsPitch + 32 * db);
-          const i16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((LdsI16x4*)at);
-          const i16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((LdsI16x4*)(at + 2 * 8 * kVsPitch));
-          const u32x2 l2 = __builtin_bit_cast(u32x2, lo), h2 = __builtin_bit_cast(u32x2, hi);
-          oacc[db] = Mfma<T>::m32x32x16(u32x4{l2[0], l2[1], h2[0], h2[1]}, pk[cc], oacc[db]);
-        }
+        for (int rb = 0; rb < 2; ++rb)
+          oacc[db][rb] = Mfma<T>::m16x16x32(u32x4{l2[0], l2[1], h2[0], h2[1]}, pk[rb], oacc[db][rb]);
+      }
     }
   };
   // chunk n travels through register set n % DEPTH; LDS is double-buffered by chunk parity
@@ -685,33 +715,31 @@ __global__ __launch_bounds__(WAVES * kWave, WAVES == 4 ? 2 : 1) void chunk_strea
     }
   }
 
-  const float l = sum_with_partner_half(l_run);
-  if (!row_valid) return;
-  if (p.n_split > 1) {
-    const size_t part = (((size_t)tok * p.batch_pitch + seq) * p.n_q_heads + head) * p.n_split + blockIdx.y;
-    float* orow = p.part_o + part * kHeadDim;
+  asm volatile("" : "+v"(first_row));   // (tokens and heads are worked out again instead of being kept)
 #pragma unroll
-    for (int db = 0; db < 4; ++db)
+  for (int rb = 0; rb < 2; ++rb) {
+    const float l = sum_over_quarters(l_run[rb]), m = -neg_m[rb];
+    if (row_of(rb) >= rows) continue;
+    const uint32_t tok = token_of(rb), head = head_of(rb);
+    if (p.n_split > 1) {
+      const size_t part = (((size_t)tok * p.batch_pitch + seq) * p.n_q_heads + head) * p.n_split + blockIdx.y;
+      float* orow = p.part_o + part * kHeadDim;
 #pragma unroll
-      for (int q4 = 0; q4 < 4; ++q4)
-        *(f32x4*)(orow + 32 * db + 8 * q4 + 4 * g) =
-            f32x4{oacc[db][4 * q4], oacc[db][4 * q4 + 1], oacc[db][4 * q4 + 2], oacc[db][4 * q4 + 3]};
-    if (g == 0) *(float2*)(p.part_ml + part * 2) = float2{m_run, l};
-  } else {
-    const float inv = 1.0f / l;
-    uint16_t* orow =
-        p.out + (size_t)tok * p.q_token_stride + ((size_t)seq * p.n_q_heads + head) * kHeadDim;
+      for (int db = 0; db < 8; ++db) *(f32x4*)(orow + 16 * db + 4 * g) = oacc[db][rb];
+      if (g == 0) *(float2*)(p.part_ml + part * 2) = float2{m, l};
+    } else {
+      const float inv = 1.0f / l;
+      uint16_t* orow =
+          p.out + (size_t)tok * p.q_token_stride + ((size_t)seq * p.n_q_heads + head) * kHeadDim;
 #pragma unroll
-    for (int db = 0; db < 4; ++db)
-#pragma unroll
-      for (int q4 = 0; q4 < 4; ++q4) {
+      for (int db = 0; db < 8; ++db) {
         u32x2 w;
-        w[0] = Mfma<T>::pack2(oacc[db][4 * q4] * inv, oacc[db][4 * q4 + 1] * inv);
-        w[1] = Mfma<T>::pack2(oacc[db][4 * q4 + 2] * inv, oacc[db][4 * q4 + 3] * inv);
-        *(u32x2*)(orow + 32 * db + 8 * q4 + 4 * g) = w;
+        w[0] = Mfma<T>::pack2(oacc[db][rb][0] * inv, oacc[db][rb][1] * inv);
+        w[1] = Mfma<T>::pack2(oacc[db][rb][2] * inv, oacc[db][rb][3] * inv);
+        *(u32x2*)(orow + 16 * db + 4 * g) = w;
       }
-    if (p.lse && g == 0)
-      p.lse[((size_t)tok * p.batch_pitch + seq) * p.n_q_heads + head] = (m_run + fast_log2(l)) * kLn2;
+      if (p.lse && g == 0) p.lse[((size_t)tok * p.batch_pitch + seq) * p.n_q_heads + head] = (m + fast_log2(l)) * kLn2;
+    }
   }
 }
 

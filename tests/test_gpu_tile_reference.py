@@ -1,4 +1,4 @@
-"""The tile kernel's reference maximum: exponentials are taken against the one a row has until a lane's
+"""The reference maximum of the tile kernel and the streaming chunk kernel: exponentials are taken against the one a row has until a lane's
 sum of them passes 2^15, then the row's true maximum is looked for and its sums are rescaled.  Score
 levels that stay below that step, pass it once, again and again, fall back and pass it in some rows of a
 block only; whole rows and a key range in splits, whose later splits some rows see nothing of."""
@@ -19,13 +19,15 @@ LEVELS = {"below": [0, 13, 14, 12], "once": [0, 0, 17, 17], "rising": [0, 16, 40
           "waves": [0, 40, -40, 60]}
 
 
-@pytest.mark.parametrize("b,hq,hkv,s,p0,split", [(16, 32, 4, 49, 200, False), (1, 8, 1, 70, 2400, True)], ids=["whole", "split"])
+@pytest.mark.parametrize("b,hq,hkv,s,p0,want_kernel,split", [
+    (16, 32, 4, 49, 200, "pingpong", False), (1, 8, 1, 70, 2400, "pingpong", True), (2, 8, 1, 13, 2400, "stream", True),
+    (2, 8, 1, 45, 2400, "stream", True)], ids=["whole", "split", "stream_13", "stream_45"])
 @pytest.mark.parametrize("name", LEVELS)
 @pytest.mark.parametrize("dtype", [orc.F16, orc.BF16], ids=["f16", "bf16"])
-def test_scores_that_outgrow_the_reference(b, hq, hkv, s, p0, split, name, dtype):
+def test_scores_that_outgrow_the_reference(b, hq, hkv, s, p0, want_kernel, split, name, dtype):
     cap = p0 + s
     kernel, _, n_split = plan_probe.chunk_plan(b, b, hq, hkv, p0, s)[:3]
-    assert kernel == "pingpong" and (n_split > 1) == split
+    assert kernel == want_kernel and (n_split > 1) == split
     scale = 1.0 / math.sqrt(D)
     q = orc.from_storage(rand_storage((s, b, hq, D), 5, dtype), dtype)
     k = orc.from_storage(rand_storage((b, hkv, cap, D), 6, dtype), dtype)
