@@ -83,13 +83,15 @@ static uint32_t g_n_cu = 256;
 // Which kernel a call runs: the few-rows streaming kernel when the handle has its workspace
 // and the shape fits it; else the smallest tile whose workgroups all fit the part at once, one
 // per compute unit (128 tokens x one head, then 256 tokens x one head); else 256 x 256 tiles,
-// whose traffic per flop is the lowest.  Measured on 256 compute units for 2048 -> 5120: 128-token
-// tiles 20 us up to 768 rows, 256-token tiles 38-42 us up to 1536 rows (128-token tiles in two
-// rounds: 40-44 us), 256 x 256 tiles 58 us at 2048 rows (61 and 70 us for the other two).
+// whose traffic per flop is the lowest.  Measured on 256 compute units for 2048 -> 5120 (us, 128-token / 256-token /
+// 256 x 256 tiles): 640 rows 20 / 25 / 46, 1024 rows 36 / 28 / 46, 1536 rows 42 / 32 / 47, 2048 rows 58 / 53 / 49.
+// Where the 256 x 256 tiles would leave two fifths of the units without one and two rounds of 128-token
+// tiles suffice, those are faster still: 4096 -> 12288, 640 rows (480 of them, 144 of 256 x 256) 69 / 91 / 85.
 int project_path(uint32_t rows, uint32_t heads, uint32_t K, bool has_workspace) {
   if (has_workspace && small_kernel_takes(rows, K)) return kPathFewRows;
   if (((rows + 127) / 128) * heads <= g_n_cu) return kPathTiles128;
   if (((rows + 255) / 256) * heads <= g_n_cu) return kPathTiles256x1;
+  if (((rows + 127) / 128) * heads <= 2 * g_n_cu && 5 * ((rows + 255) / 256) * ((heads + 1) / 2) <= 3 * g_n_cu) return kPathTiles128;
   return kPathTiles;
 }
 
