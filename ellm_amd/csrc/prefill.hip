@@ -71,26 +71,28 @@ struct PrefillKernelArgs {
 // Ping-pong kernel: 8 waves, two per SIMD.  Waves 0-3 and waves 4-7 run the
 // same per-tile sequence  S^T = K.Q^T -> soft-max -> O^T += V^T.P^T  half a
 // step apart: while one group is in its matrix phase (P.V of the previous tile
-// and Q.K of the next one) the other group is in its vector phase (requests of a
-// K or V tile, mask, exponentials, packing), and a workgroup barrier flips the roles.  Two waves that share a SIMD are thus
+// and Q.K of the next one, plus moving the following K or V tile into LDS) the
+// other group is in its vector phase (mask, exponentials, packing), and
+// a workgroup barrier flips the roles.  Two waves that share a SIMD are thus
 // never both in the same phase, which is what lets the MFMA pipe and the vector
 // ALU work at the same time; left to themselves, two identical workgroups on a
 // compute unit run in lockstep and the two pipes take turns instead.
 // Rows: wave w owns row block w (32 rows) of 8; all 256 rows read the same K/V
 // tiles.  Waves 0-3 stage the K tiles, waves 4-7 the V tiles.
-// What bounds it: the board's power on long calls of ordinary operands (1.29-1.32 PFLOP/s at the clock the
-// board allows; 1.65 PFLOP/s on K = V = 0), and a phase of ~1500 clocks for 1024 of matrix work: an
+// What bounds it: the board's power on long calls of ordinary operands (1.25-1.30 PFLOP/s at the clock the
+// board allows; 1.68 PFLOP/s on K = V = 0), and a phase of ~1500 clocks for 1024 of matrix work: an
 // instruction of the vector phase takes 8.2 clocks beside 16x16x32 instructions of the other wave (an
-// exponential 15.8; 5.6 and 10.9 beside 32x32x16), the matrix phase has 12 KB of operand reads a wave.
-// Measured, 32x32x16 instructions with a row maximum every tile, K and V through registers -> this form
-// (us): 8192 tokens on 120000, 64 / 8 heads, bf16 26540 -> 25480; 32768 tokens, 32 / 4, f16 7515 -> 7045;
-// 8000 tokens 451 -> 429; 1624 on 10535 295 -> 278; 255 on 11150 (split) 56.7 -> 53.9; 64 tokens x 24 on 4096
-// 119.5 -> 113.9; 412 x 19, 32 / 32 heads 111.1 -> 110.7.  Of that: 16x16x32 alone -1 to +0.5 %, the maximum
-// only where it may have to move 3 to 5 %, tiles straight into LDS 1 to 2 %.  Tried and dropped: Q.K on 32x32x16
-// and P.V on 16x16x32 (eight v_permlane16_swap a tile hand P over: 150 clocks of the vector phase) 26970;
-// all on 32x32x16 with the other two changes 25730 (16x16x32 on the same board 24490); the barrier ahead of a
-// matrix phase's last operands, so that the other group's begins early, 5 % slower than at its end; the
-// tile requests between the matrix instructions instead of ahead of the exponentials 3 % slower.
+// exponential 15.8; 5.6 and 10.9 beside 32x32x16), staging and operand reads cost the matrix phase 190 clocks each.
+// Measured, 32x32x16 instructions with a row maximum every tile -> this form
+// (us, in turn on one board): 8192 tokens on 120000, 64 / 8 heads, bf16 27390 -> 26230; 32768 tokens, 32 / 4, f16 7820
+// -> 7370; 8000 tokens 469 -> 444; 1624 on 10535 306 -> 291; 255 on 11150 (split) 57.6 -> 55.3; 64 tokens x 24 on 4096
+// 120.8 -> 118.1; 412 x 19, 32 / 32 heads 108.4 -> 103.1.  Of that: 16x16x32 alone -1 to +0.5 %, the maximum only where
+// it may have to move 3 to 5 %, going first in the vector phase 1 %, the mask from one register 4 % of short
+// calls.  Tried and dropped: tiles straight into LDS, three ahead (1.5 % faster on long calls, but 120 x 8 on 1400,
+// 32 / 32 heads, 57 -> 59 to 65 us and 412 x 19 no faster than at first); Q.K on 32x32x16 and P.V on 16x16x32 (eight
+// v_permlane16_swap a tile hand P over: 150 clocks of the vector phase), 6 % slower than this; all on 32x32x16
+// with the other changes 5 % slower; the barrier ahead of a matrix phase's last operands, so that the other
+// group's begins early, 5 %; the tile's stores earlier in the phase 2 %; six or seven operands ahead instead of eight 1 to 3 %.
 // ---------------------------------------------------------------------------
 __device__ __forceinline__ uint64_t uniform64(const void* p) {  // the compiler cannot see that p is wave-uniform
   const uint32_t lo = (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)(uint64_t)p);
@@ -122,32 +124,19 @@ typedef __attribute__((address_space(3))) i16x4 LdsI16x4;
 // V rows in LDS: 288 B apart, so that the four rows a 16-lane block of a
 // transposing read touches (32 B of each) fall into disjoint banks
 constexpr int kVsPitch = kHeadDim + 16;
+constexpr int kVsHalves = kBK * kVsPitch;
 constexpr int kPpWaves = 8;
 constexpr int kPpThreads = kPpWaves * kWave;
 constexpr int kLdsAhead = 8;   // LDS operand reads in flight ahead of their MFMA
-constexpr int kTileHalves = kBK * kHeadDim;
-constexpr int kPpBuffers = 4;                // tiles of K, and of V, in LDS: 128 KB
-constexpr int kPpAhead = kPpBuffers - 1;     // tiles requested ahead of the one being multiplied
-static_assert(kPpAhead == 3, "s_waitcnt vmcnt literals in prefill_pingpong_kernel");
 constexpr int kBufferFlags = 0x00020000;  // raw buffer of 32-bit data, no swizzle (word 3 of the descriptor)
-
-// 16 bytes a lane from memory straight to LDS address lds_at + 16 x lane.  Written as asm: the compiler's
-// own form of this load makes it wait for every outstanding one before each later LDS read (it cannot see
-// that the two touch different buffers).  M0 carries the address; one wait state between its write and the
-// load.  (M0 is a register the compiler reserves and, in the kernel that calls this, never uses itself.)
-__device__ __forceinline__ void load_to_lds(const u32x4& rsrc, uint32_t voff, uint32_t lds_at) {
-  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, 0 offen lds"
-               :: "s"(lds_at), "v"(voff), "s"(rsrc) : "memory");
-}
 
 template <typename T, bool SPLIT>
 __global__ __launch_bounds__(kPpThreads, 2) void prefill_pingpong_kernel(PrefillKernelArgs p) {
-  // K tiles [4][64][128] then V tiles [4][64][128], rows unpadded: a wave instruction of the staging
-  // below delivers 1 KB, four whole rows.  The sixteen 16-byte pieces of a row are permuted instead, so
-  // that the operand reads meet no bank twice: piece x of K row r sits at x ^ (r & 15) (the sixteen lanes
-  // that a 128-bit read serves at once are rows 0-3 and 12-15 of one piece and 4-11 of its neighbour),
-  // piece x of V row r at x ^ 2 (r & 7) (a transposing read touches two pieces of eight rows).
-  __shared__ __attribute__((aligned(256))) uint16_t smem[2 * kPpBuffers * kTileHalves];
+  // K tiles [2][64][kVsPitch] then V tiles [3][64][kVsPitch]: V is staged one step
+  // earlier than it is read, so that every operand of a matrix step is in LDS a whole
+  // phase before the step starts and can be requested ahead of the barrier.  (288-byte rows: the sixteen lanes that
+  // a 128-bit read serves at once, rows 0-3 and 12-15 of one piece and 4-11 of its neighbour, meet no bank twice.)
+  __shared__ __attribute__((aligned(16))) uint16_t smem[5 * kVsHalves];
 
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = tid >> 6;
@@ -203,11 +192,11 @@ __global__ __launch_bounds__(kPpThreads, 2) void prefill_pingpong_kernel(Prefill
   const uint16_t* kplane = p.k + plane_at;
   const uint16_t* vplane = p.v + plane_at;
 
-  // staging: the four waves of a group move one 64 x 128 tile straight into LDS, four loads each: rows
-  // ld_r + 16 i, LDS piece tid % 16, K and V alike: V sits in LDS row by row as it does in
-  // memory and is transposed by the LDS read (ds_read_b64_tr_b16).
-  const int ld_r = (tid & 255) >> 4;
-  const int ld_c = (tid & 15) ^ (grp ? 2 * (ld_r & 7) : ld_r);
+  // staging: the 256 threads of a group move one 64 x 128 tile, four 16-byte pieces
+  // each (rows ld_r + 16 i, columns 8 ld_c ..), K and V alike: V sits in LDS row by
+  // row as it does in memory and is transposed by the LDS read (ds_read_b64_tr_b16).
+  const int st_tid = tid & 255;
+  const int ld_c = st_tid & 15, ld_r = st_tid >> 4;
   const uint16_t* plane = grp ? vplane : kplane;                  // wave-uniform
   const uint32_t stride_pos = (uint32_t)p.kv_stride_pos;
   // Tiles are fetched with buffer loads: the descriptor (base of tile kt, bytes
@@ -225,21 +214,41 @@ __global__ __launch_bounds__(kPpThreads, 2) void prefill_pingpong_kernel(Prefill
   uint32_t piece_off[4];
 #pragma unroll
   for (int i = 0; i < 4; ++i) piece_off[i] = ((ld_r + 16 * i) * stride_pos + 8 * ld_c) * 2;
+  // LDS addresses are kept as byte offsets: the buffers span more than the 64 KB an
+  // instruction's immediate offset reaches, so each step forms one base register
+  // per tile (step_base) and everything else is an immediate on top of it.
   const uint32_t lds0 = (uint32_t)(uintptr_t)(LdsHalf*)smem;
   auto step_base = [](uint32_t addr) {
     asm volatile("" : "+v"(addr));  // opaque: keeps the compiler from folding the sum another way
     return addr;
   };
+  const uint32_t ks_store = lds0 + 2 * (ld_r * kVsPitch + 8 * ld_c);
+  const uint32_t vs_store = ks_store + 2 * 2 * kVsHalves;
+  u32x4 stg[4];
+  auto load_piece = [&](uint32_t kt, int i) {  // kt (relative to kt0) must be wave-uniform to the compiler
+    const uint64_t off = (uint64_t)(kt0 + kt) * tile_bytes;
+    const uint32_t left = bytes_left(valid_bytes, off);
+    const __amdgpu_buffer_rsrc_t rsrc =
+        __builtin_amdgcn_make_buffer_rsrc((void*)(plane_u + off), 0, left, kBufferFlags);
+    stg[i] = __builtin_amdgcn_raw_buffer_load_b128(rsrc, piece_off[i], 0, 0);
+  };
   // (the group comes as a compile-time constant where the caller runs behind the scalar
   // branch on the group, as the run-time value in the prologue)
-  const uint32_t wave_lds = lds0 + 4 * 2 * kHeadDim * ((uint32_t)__builtin_amdgcn_readfirstlane(wave) & 3);
-  auto load_tile = [&](auto group, uint32_t kt) __attribute__((always_inline)) {  // kt (relative to kt0): wave-uniform
-    const uint64_t off = (uint64_t)(kt0 + kt) * tile_bytes;
-    const uint64_t at = plane_u + off;
-    const u32x4 rsrc = {(uint32_t)at, (uint32_t)(at >> 32) & 0xffffu, bytes_left(valid_bytes, off), (uint32_t)kBufferFlags};
-    const uint32_t to = wave_lds + (uint32_t)__builtin_amdgcn_readfirstlane((int)(((group ? kPpBuffers : 0) + (kt & (kPpBuffers - 1))) * 2 * kTileHalves));
+  // base: step_base of this lane's place in the destination buffer
+  auto store_piece = [&](uint32_t base, int i) {
+    *(LdsU32x4*)(base + 2 * 16 * i * kVsPitch) = stg[i];
+  };
+  auto load_tile = [&](uint32_t kt) {
 #pragma unroll
-    for (int i = 0; i < 4; ++i) load_to_lds(rsrc, piece_off[i], to + 16 * i * 2 * kHeadDim);
+    for (int i = 0; i < 4; ++i) load_piece(kt, i);
+  };
+  auto store_base = [&](auto group, int buf) {
+    return step_base((group ? vs_store : ks_store) + 2 * buf * kVsHalves);
+  };
+  auto store_tile = [&](int buf) {
+    const uint32_t base = store_base(grp, buf);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) store_piece(base, i);
   };
 
   // per row: minus its reference maximum (log2 units; +inf: no key seen yet), this lane's share of
@@ -262,24 +271,23 @@ __global__ __launch_bounds__(kPpThreads, 2) void prefill_pingpong_kernel(Prefill
   // multiplies Q by whatever finite K tile its buffer still holds and nobody reads
   // the result; tiles past the last one are fetched as zeros (the buffer
   // descriptor has no bytes left) and stored where nothing reads them.
-  // prologue: zeros into the V buffer that step 0 reads, the first kPpAhead tiles on their way.
+  // prologue: K(0) and V(0) into LDS, K(1) and V(1) on their way into the staging
+  // registers, zeros into the V^T buffer that step 0 reads.
   if (grp) {
 #pragma unroll
-    for (int i = 0; i < 4; ++i)
-      *(LdsU32x4*)(lds0 + 2 * ((2 * kPpBuffers - 1) * kTileHalves) + (tid & 255) * 16 + i * 4096) = u32x4{0u, 0u, 0u, 0u};
+    for (int i = 0; i < 4; ++i) stg[i] = u32x4{0u, 0u, 0u, 0u};
+    store_tile(2);
   }
-#pragma unroll
-  for (int kt = 0; kt < kPpAhead; ++kt) load_tile(grp, kt);
-  asm volatile("s_waitcnt vmcnt(8)" ::: "memory");   // 4 (kPpAhead - 1): tile 0 is there
+  load_tile(0);
+  store_tile(0);
+  load_tile(1);
   __syncthreads();
 
-  // Matrix step kt = P.V of tile kt-1 and Q.K of tile kt, their MFMAs interleaved (no MFMA waits on the
-  // one before it).  Tile kt of K and of V sits in buffer kt % 4 of its own.  A vector step
-  // kt requests tile kt + 3 (group 0: K, group 1: V) into the buffer of tile kt - 1, whose last reader,
-  // matrix step kt (V) or kt - 1 (K) of either group, has ended; the matrix step that
-  // follows waits for tile kt + 2 and the barrier at its end shows it to all, one matrix step ahead
-  // of its first reader: three phases for a tile to arrive, and all operands of a
-  // matrix step are in LDS a whole phase before it starts.  Operands come from
+  // Matrix step kt = P.V of tile kt-1 and Q.K of tile kt, their MFMAs interleaved
+  // (no MFMA waits on the one before it); then the group stores its tile kt+1 (group 0: K, group 1: V)
+  // and fetches tile kt+2.  K(kt) sits in buffer kt % 2, V(kt) in buffer kt % 3: V is
+  // staged one step before the first step that reads it, so that all operands of
+  // a matrix step are in LDS a whole phase before it starts.  Operands come from
   // LDS kLdsAhead reads ahead of the MFMA that consumes them: issued just in
   // time, every operand's MFMAs (32 cycles) would wait out a full LDS round trip
   // (100+ cycles).  The first kLdsAhead are requested before the barrier that
@@ -290,37 +298,39 @@ __global__ __launch_bounds__(kPpThreads, 2) void prefill_pingpong_kernel(Prefill
   // (t & 3) of what lanes 4e + (t >> 2), e = 0..3, of that block address: with lane
   // s pointing at key s >> 2, dims 4 (s & 3).. of the 16 dims, lane t ends
   // up with dim t of 4 consecutive keys.  Two such reads (keys +0 and +16) make one operand.
-  const uint32_t k_read = lds0 + 2 * kHeadDim * c16 + 16 * (g ^ c16);
-  const uint32_t v_read = lds0 + 2 * kPpBuffers * kTileHalves + 2 * kHeadDim * (4 * g + (c16 >> 2)) +
-                          32 * (4 * (g & 1) + (c16 >> 2)) + 8 * (c16 & 3);
-  auto k_base = [&](uint32_t kt) { return step_base(k_read + 2 * (kt & (kPpBuffers - 1)) * kTileHalves); };
-  auto v_base = [&](uint32_t kt) { return step_base(v_read + 2 * ((kt - 1) & (kPpBuffers - 1)) * kTileHalves); };
+  const uint32_t k_read = lds0 + 2 * (c16 * kVsPitch + 8 * g);
+  const uint32_t v_read = lds0 + 2 * (2 * kVsHalves + (4 * g + (c16 >> 2)) * kVsPitch + 4 * (c16 & 3));
+  auto mod3 = [](uint32_t x) { return x % 3u; };
   // operand n of the stream of matrix step kt: P.V 0, Q.K 0, P.V 1, Q.K 1, ...
   // (lane part of the address once per step, operand part as a compile-time offset)
   auto stream_operand = [&](uint32_t ks, uint32_t vs, int n) {
     const int i = n >> 1;
     if (n & 1) {  // K: i = 4 s + kb, keys 16 kb.., dims 32 s..
       const int s = i >> 2, kb = i & 3;
-      return (u32x4) * (const LdsU32x4*)((ks ^ (64 * s)) + 2 * 16 * kb * kHeadDim);
+      return (u32x4) * (const LdsU32x4*)(ks + 2 * (16 * kb * kVsPitch + 32 * s));
     }
     // V: i = 8 kc + db, keys 32 kc.., dims 16 db..
     const int kc = i >> 3, db = i & 7;
-    const uint32_t at = (vs ^ (32 * db)) + 2 * 32 * kc * kHeadDim;
+    const uint32_t at = vs + 2 * (32 * kc * kVsPitch + 16 * db);
     const i16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((LdsI16x4*)at);
-    const i16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((LdsI16x4*)(at + 2 * 16 * kHeadDim));
+    const i16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((LdsI16x4*)(at + 2 * 16 * kVsPitch));
     const u32x2 l2 = __builtin_bit_cast(u32x2, lo), h2 = __builtin_bit_cast(u32x2, hi);
     return u32x4{l2[0], l2[1], h2[0], h2[1]};
   };
   u32x4 ring[kLdsAhead];
   auto prefetch_ring = [&](uint32_t kt) __attribute__((always_inline)) {
-    const uint32_t ks = k_base(kt), vs = v_base(kt);
+    const uint32_t ks = step_base(k_read + 2 * (kt & 1) * kVsHalves);
+    const uint32_t vs = step_base(v_read + 2 * mod3(kt + 2) * kVsHalves);  // V(kt-1)
 #pragma unroll
     for (int n = 0; n < kLdsAhead; ++n) ring[n] = stream_operand(ks, vs, n);
   };
-  auto matrix_step = [&](uint32_t kt) __attribute__((always_inline)) {
+  auto matrix_step = [&](auto group, uint32_t kt) __attribute__((always_inline)) {
     __builtin_amdgcn_s_setprio(0);
-    const uint32_t ks = k_base(kt), vs = v_base(kt);
-    // a full scheduling barrier after every operand's MFMAs keeps the compiler from regrouping them
+    const uint32_t ks = step_base(k_read + 2 * (kt & 1) * kVsHalves);
+    const uint32_t vs = step_base(v_read + 2 * mod3(kt + 2) * kVsHalves);
+    const uint32_t store_at = store_base(group, group ? (int)mod3(kt + 1) : (int)((kt + 1) & 1));
+    // staging work is dealt out between the MFMAs, and a full scheduling barrier
+    // after every MFMA keeps the compiler from regrouping any of it
     __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
     for (int n = 0; n < 32; ++n) {
@@ -334,10 +344,14 @@ __global__ __launch_bounds__(kPpThreads, 2) void prefill_pingpong_kernel(Prefill
           oacc[i & 7][rb] = Mfma<T>::m16x16x32(a, pk[i >> 3][rb], oacc[i & 7][rb]);
       }
       if (n + kLdsAhead < 32) ring[n % kLdsAhead] = stream_operand(ks, vs, n + kLdsAhead);
+      // staging last: the loads issued at the end of the previous matrix step have had
+      // almost a whole iteration (~2 us) to arrive before their registers are stored
+      if (n >= 24 && n < 28) store_piece(store_at, n - 24);
+      if (n >= 28 && n < 32) load_piece(kt + 2, n - 28);
       __builtin_amdgcn_sched_barrier(0);
     }
-    // tile kt + 1 has landed (kPpAhead - 2 younger ones are on their way), operand reads have returned
-    asm volatile("s_waitcnt vmcnt(4) lgkmcnt(0)" ::: "memory");
+    // the barrier that follows carries no wait of its own: wait here for the LDS stores
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
   };
 
   const int last_key = (int)(P0 + tok0 + c16) - 4 * g;   // relative to the lane's first key of a tile
@@ -359,11 +373,10 @@ __global__ __launch_bounds__(kPpThreads, 2) void prefill_pingpong_kernel(Prefill
     }
   };
 
-  // Vector step kt = request of tile kt + 3, then soft-max of tile kt: mask on the diagonal, exponentials,
-  // packing, row sum; row maximum and rescaling of O^T where they are due.  (Its wave goes first where both
-  // waves of a SIMD have something to issue: 0.5 to 1 % on long calls.)
-  auto vector_step = [&](auto group, uint32_t kt) __attribute__((always_inline)) {
-    load_tile(group, kt + kPpAhead);
+  // Vector step kt = soft-max of tile kt: mask on the diagonal, exponentials, packing, row sum; row maximum
+  // and rescaling of O^T where they are due.  (Its wave goes first where both waves of a SIMD have something
+  // to issue: 0.5 to 1 % on long calls.)
+  auto vector_step = [&](uint32_t kt) __attribute__((always_inline)) {
     __builtin_amdgcn_s_setprio(2);
     const uint32_t kb = (kt0 + kt) * kBK;
     if (kb + kBK - 1 > first_pos) {  // tile crosses this row block's diagonal
@@ -422,28 +435,27 @@ __global__ __launch_bounds__(kPpThreads, 2) void prefill_pingpong_kernel(Prefill
   constexpr std::integral_constant<int, 1> kGroup1;
   if (__builtin_amdgcn_readfirstlane(grp) == 0) {
     prefetch_ring(0);
-    matrix_step(0);
+    matrix_step(kGroup0, 0);
     __builtin_amdgcn_s_barrier();
     for (uint32_t kt = 0; kt < n_tiles; ++kt) {
-      vector_step(kGroup0, kt);
+      vector_step(kt);
       prefetch_ring(kt + 1);
       __builtin_amdgcn_s_barrier();
-      matrix_step(kt + 1);
+      matrix_step(kGroup0, kt + 1);
       __builtin_amdgcn_s_barrier();
     }
   } else {
     prefetch_ring(0);
     __builtin_amdgcn_s_barrier();
     for (uint32_t kt = 0; kt < n_tiles; ++kt) {
-      matrix_step(kt);
+      matrix_step(kGroup1, kt);
       __builtin_amdgcn_s_barrier();
-      vector_step(kGroup1, kt);
+      vector_step(kt);
       prefetch_ring(kt + 1);
       __builtin_amdgcn_s_barrier();
     }
-    matrix_step(n_tiles);
+    matrix_step(kGroup1, n_tiles);
   }
-  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // the last requests still write LDS
 
 #pragma unroll
   for (int rb = 0; rb < 2; ++rb) {
