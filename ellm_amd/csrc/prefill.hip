@@ -88,8 +88,7 @@ struct PrefillKernelArgs {
 // -> 7370; 8000 tokens 469 -> 444; 1624 on 10535 306 -> 291; 255 on 11150 (split) 57.6 -> 55.3; 64 tokens x 24 on 4096
 // 120.8 -> 118.1; 412 x 19, 32 / 32 heads 108.4 -> 103.1.  Of that: 16x16x32 alone -1 to +0.5 %, the maximum only where
 // it may have to move 3 to 5 %, going first in the vector phase 1 %, the mask from one register 4 % of short
-// calls.  Tried and dropped: tiles straight into LDS, three ahead (1.5 % faster on long calls, but 120 x 8 on 1400,
-// 32 / 32 heads, 57 -> 59 to 65 us and 412 x 19 no faster than at first); Q.K on 32x32x16 and P.V on 16x16x32 (eight
+// calls.  Tried and dropped: Q.K on 32x32x16 and P.V on 16x16x32 (eight
 // v_permlane16_swap a tile hand P over: 150 clocks of the vector phase), 6 % slower than this; all on 32x32x16
 // with the other changes 5 % slower; the barrier ahead of a matrix phase's last operands, so that the other
 // group's begins early, 5 %; the tile's stores earlier in the phase 2 %; six or seven operands ahead instead of eight 1 to 3 %.
@@ -128,15 +127,31 @@ constexpr int kVsHalves = kBK * kVsPitch;
 constexpr int kPpWaves = 8;
 constexpr int kPpThreads = kPpWaves * kWave;
 constexpr int kLdsAhead = 8;   // LDS operand reads in flight ahead of their MFMA
+constexpr int kTileHalves = kBK * kHeadDim;
+constexpr int kPpBuffers = 4;                // DIRECT: tiles of K, and of V, in LDS: 128 KB
+constexpr int kPpAhead = kPpBuffers - 1;     // DIRECT: tiles requested ahead of the one being multiplied
+static_assert(kPpAhead == 3, "s_waitcnt vmcnt literals in prefill_pingpong_kernel");
 constexpr int kBufferFlags = 0x00020000;  // raw buffer of 32-bit data, no swizzle (word 3 of the descriptor)
 
-template <typename T, bool SPLIT>
+// 16 bytes a lane from memory straight to LDS address lds_at + 16 x lane.  Written as asm: the compiler's
+// own form of this load makes it wait for every outstanding one before each later LDS read (it cannot see
+// that the two touch different buffers).  M0 carries the address; one wait state between its write and the
+// load.  (M0 is a register the compiler reserves and, in the kernel that calls this, never uses itself.)
+__device__ __forceinline__ void load_to_lds(const u32x4& rsrc, uint32_t voff, uint32_t lds_at) {
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, 0 offen lds"
+               :: "s"(lds_at), "v"(voff), "s"(rsrc) : "memory");
+}
+
+template <typename T, bool SPLIT, bool DIRECT>
 __global__ __launch_bounds__(kPpThreads, 2) void prefill_pingpong_kernel(PrefillKernelArgs p) {
-  // K tiles [2][64][kVsPitch] then V tiles [3][64][kVsPitch]: V is staged one step
+  // Through registers: K tiles [2][64][kVsPitch] then V tiles [3][64][kVsPitch]; V is staged one step
   // earlier than it is read, so that every operand of a matrix step is in LDS a whole
   // phase before the step starts and can be requested ahead of the barrier.  (288-byte rows: the sixteen lanes that
   // a 128-bit read serves at once, rows 0-3 and 12-15 of one piece and 4-11 of its neighbour, meet no bank twice.)
-  __shared__ __attribute__((aligned(16))) uint16_t smem[5 * kVsHalves];
+  // DIRECT: K tiles [4][64][128] then V tiles [4][64][128], rows unpadded (a wave instruction delivers four
+  // whole rows), their sixteen 16-byte pieces permuted to the same end: piece x of K row r sits at x ^ (r & 15),
+  // of V row r at x ^ 2 (r & 7).
+  __shared__ __attribute__((aligned(256))) uint16_t smem[DIRECT ? 2 * kPpBuffers * kTileHalves : 5 * kVsHalves];
 
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = tid >> 6;
@@ -196,7 +211,8 @@ __global__ __launch_bounds__(kPpThreads, 2) void prefill_pingpong_kernel(Prefill
   // each (rows ld_r + 16 i, columns 8 ld_c ..), K and V alike: V sits in LDS row by
   // row as it does in memory and is transposed by the LDS read (ds_read_b64_tr_b16).
   const int st_tid = tid & 255;
-  const int ld_c = st_tid & 15, ld_r = st_tid >> 4;
+  const int ld_r = st_tid >> 4;
+  const int ld_c = DIRECT ? (st_tid & 15) ^ (grp ? 2 * (ld_r & 7) : ld_r) : st_tid & 15;
   const uint16_t* plane = grp ? vplane : kplane;                  // wave-uniform
   const uint32_t stride_pos = (uint32_t)p.kv_stride_pos;
   // Tiles are fetched with buffer loads: the descriptor (base of tile kt, bytes
@@ -251,6 +267,16 @@ __global__ __launch_bounds__(kPpThreads, 2) void prefill_pingpong_kernel(Prefill
     for (int i = 0; i < 4; ++i) store_piece(base, i);
   };
 
+  const uint32_t wave_lds = lds0 + 4 * 2 * kHeadDim * ((uint32_t)__builtin_amdgcn_readfirstlane(wave) & 3);
+  auto load_direct = [&](auto group, uint32_t kt) __attribute__((always_inline)) {   // tile kt into its buffer
+    const uint64_t off = (uint64_t)(kt0 + kt) * tile_bytes, at = plane_u + off;
+    const u32x4 rsrc = {(uint32_t)at, (uint32_t)(at >> 32) & 0xffffu, bytes_left(valid_bytes, off), (uint32_t)kBufferFlags};
+    const uint32_t to = wave_lds + (uint32_t)__builtin_amdgcn_readfirstlane(
+                                       (int)(((group ? kPpBuffers : 0) + (kt & (kPpBuffers - 1))) * 2 * kTileHalves));
+#pragma unroll
+    for (int i = 0; i < 4; ++i) load_to_lds(rsrc, piece_off[i], to + 16 * i * 2 * kHeadDim);
+  };
+
   // per row: minus its reference maximum (log2 units; +inf: no key seen yet), this lane's share of
   // the denominator
   float neg_m[2] = {INFINITY, INFINITY}, l_run[2] = {0.0f, 0.0f};
@@ -273,14 +299,26 @@ __global__ __launch_bounds__(kPpThreads, 2) void prefill_pingpong_kernel(Prefill
   // descriptor has no bytes left) and stored where nothing reads them.
   // prologue: K(0) and V(0) into LDS, K(1) and V(1) on their way into the staging
   // registers, zeros into the V^T buffer that step 0 reads.
-  if (grp) {
+  // (DIRECT: V(-1) is buffer 3, and the first kPpAhead tiles are on their way)
+  if constexpr (DIRECT) {
+    if (grp) {
 #pragma unroll
-    for (int i = 0; i < 4; ++i) stg[i] = u32x4{0u, 0u, 0u, 0u};
-    store_tile(2);
+      for (int i = 0; i < 4; ++i)
+        *(LdsU32x4*)(lds0 + 2 * (2 * kPpBuffers - 1) * kTileHalves + st_tid * 16 + i * 4096) = u32x4{0u, 0u, 0u, 0u};
+    }
+#pragma unroll
+    for (int kt = 0; kt < kPpAhead; ++kt) load_direct(grp, kt);
+    asm volatile("s_waitcnt vmcnt(8)" ::: "memory");   // 4 (kPpAhead - 1): tile 0 is there
+  } else {
+    if (grp) {
+#pragma unroll
+      for (int i = 0; i < 4; ++i) stg[i] = u32x4{0u, 0u, 0u, 0u};
+      store_tile(2);
+    }
+    load_tile(0);
+    store_tile(0);
+    load_tile(1);
   }
-  load_tile(0);
-  store_tile(0);
-  load_tile(1);
   __syncthreads();
 
   // Matrix step kt = P.V of tile kt-1 and Q.K of tile kt, their MFMAs interleaved
@@ -292,43 +330,54 @@ __global__ __launch_bounds__(kPpThreads, 2) void prefill_pingpong_kernel(Prefill
   // time, every operand's MFMAs (32 cycles) would wait out a full LDS round trip
   // (100+ cycles).  The first kLdsAhead are requested before the barrier that
   // opens the step (prefetch_ring), so the round trip overlaps the barrier wait.
+  // DIRECT: tile kt of K and of V sits in buffer kt % 4 of its own.  A vector step kt requests tile kt + 3
+  // into the buffer of tile kt - 1, whose last reader, matrix step kt (V) or kt - 1 (K) of either group, has
+  // ended; matrix step kt + 1 waits for tile kt + 2 at its end, where the barrier shows it to all.
   // A operand of P.V (rows = 16 dims, 32 keys): lane (dim c16, key quarter g) holds keys
   // {4g..4g+3, 16+4g..16+4g+3} of the 32, the order in which the soft-max leaves P in
   // registers.  ds_read_b64_tr_b16 hands lane t of a 16-lane block element
   // (t & 3) of what lanes 4e + (t >> 2), e = 0..3, of that block address: with lane
   // s pointing at key s >> 2, dims 4 (s & 3).. of the 16 dims, lane t ends
   // up with dim t of 4 consecutive keys.  Two such reads (keys +0 and +16) make one operand.
-  const uint32_t k_read = lds0 + 2 * (c16 * kVsPitch + 8 * g);
-  const uint32_t v_read = lds0 + 2 * (2 * kVsHalves + (4 * g + (c16 >> 2)) * kVsPitch + 4 * (c16 & 3));
+  const uint32_t k_read = lds0 + (DIRECT ? 2 * kHeadDim * c16 + 16 * (g ^ c16) : 2 * (c16 * kVsPitch + 8 * g));
+  const int v_row = 4 * g + (c16 >> 2);
+  const uint32_t v_read = lds0 + (DIRECT ? 2 * (kPpBuffers * kTileHalves + v_row * kHeadDim) + 32 * (v_row & 7) + 8 * (c16 & 3)
+                                         : 2 * (2 * kVsHalves + v_row * kVsPitch + 4 * (c16 & 3)));
   auto mod3 = [](uint32_t x) { return x % 3u; };
+  constexpr int kPitch = DIRECT ? kHeadDim : kVsPitch;
+  auto k_base = [&](uint32_t kt) __attribute__((always_inline)) {
+    return step_base(k_read + (DIRECT ? 2 * (kt & (kPpBuffers - 1)) * kTileHalves : 2 * (kt & 1) * kVsHalves));
+  };
+  auto v_base = [&](uint32_t kt) __attribute__((always_inline)) {   // V(kt - 1)
+    return step_base(v_read + (DIRECT ? 2 * ((kt - 1) & (kPpBuffers - 1)) * kTileHalves : 2 * mod3(kt + 2) * kVsHalves));
+  };
   // operand n of the stream of matrix step kt: P.V 0, Q.K 0, P.V 1, Q.K 1, ...
   // (lane part of the address once per step, operand part as a compile-time offset)
   auto stream_operand = [&](uint32_t ks, uint32_t vs, int n) {
     const int i = n >> 1;
     if (n & 1) {  // K: i = 4 s + kb, keys 16 kb.., dims 32 s..
       const int s = i >> 2, kb = i & 3;
-      return (u32x4) * (const LdsU32x4*)(ks + 2 * (16 * kb * kVsPitch + 32 * s));
+      return (u32x4) * (const LdsU32x4*)((DIRECT ? ks ^ (64 * s) : ks + 64 * s) + 2 * 16 * kb * kPitch);
     }
     // V: i = 8 kc + db, keys 32 kc.., dims 16 db..
     const int kc = i >> 3, db = i & 7;
-    const uint32_t at = vs + 2 * (32 * kc * kVsPitch + 16 * db);
+    const uint32_t at = (DIRECT ? vs ^ (32 * db) : vs + 32 * db) + 2 * 32 * kc * kPitch;
     const i16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((LdsI16x4*)at);
-    const i16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((LdsI16x4*)(at + 2 * 16 * kVsPitch));
+    const i16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((LdsI16x4*)(at + 2 * 16 * kPitch));
     const u32x2 l2 = __builtin_bit_cast(u32x2, lo), h2 = __builtin_bit_cast(u32x2, hi);
     return u32x4{l2[0], l2[1], h2[0], h2[1]};
   };
   u32x4 ring[kLdsAhead];
   auto prefetch_ring = [&](uint32_t kt) __attribute__((always_inline)) {
-    const uint32_t ks = step_base(k_read + 2 * (kt & 1) * kVsHalves);
-    const uint32_t vs = step_base(v_read + 2 * mod3(kt + 2) * kVsHalves);  // V(kt-1)
+    const uint32_t ks = k_base(kt), vs = v_base(kt);
 #pragma unroll
     for (int n = 0; n < kLdsAhead; ++n) ring[n] = stream_operand(ks, vs, n);
   };
   auto matrix_step = [&](auto group, uint32_t kt) __attribute__((always_inline)) {
     __builtin_amdgcn_s_setprio(0);
-    const uint32_t ks = step_base(k_read + 2 * (kt & 1) * kVsHalves);
-    const uint32_t vs = step_base(v_read + 2 * mod3(kt + 2) * kVsHalves);
-    const uint32_t store_at = store_base(group, group ? (int)mod3(kt + 1) : (int)((kt + 1) & 1));
+    const uint32_t ks = k_base(kt), vs = v_base(kt);
+    uint32_t store_at = 0;
+    if constexpr (!DIRECT) store_at = store_base(group, group ? (int)mod3(kt + 1) : (int)((kt + 1) & 1));
     // staging work is dealt out between the MFMAs, and a full scheduling barrier
     // after every MFMA keeps the compiler from regrouping any of it
     __builtin_amdgcn_sched_barrier(0);
@@ -346,12 +395,16 @@ __global__ __launch_bounds__(kPpThreads, 2) void prefill_pingpong_kernel(Prefill
       if (n + kLdsAhead < 32) ring[n % kLdsAhead] = stream_operand(ks, vs, n + kLdsAhead);
       // staging last: the loads issued at the end of the previous matrix step have had
       // almost a whole iteration (~2 us) to arrive before their registers are stored
-      if (n >= 24 && n < 28) store_piece(store_at, n - 24);
-      if (n >= 28 && n < 32) load_piece(kt + 2, n - 28);
+      if (!DIRECT && n >= 24 && n < 28) store_piece(store_at, n - 24);
+      if (!DIRECT && n >= 28 && n < 32) load_piece(kt + 2, n - 28);
       __builtin_amdgcn_sched_barrier(0);
     }
     // the barrier that follows carries no wait of its own: wait here for the LDS stores
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
+    // (DIRECT: for tile kt + 1, behind which one younger one is on its way, and for the operand reads)
+    if constexpr (DIRECT)
+      asm volatile("s_waitcnt vmcnt(4) lgkmcnt(0)" ::: "memory");
+    else
+      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
   };
 
   const int last_key = (int)(P0 + tok0 + c16) - 4 * g;   // relative to the lane's first key of a tile
@@ -376,7 +429,8 @@ __global__ __launch_bounds__(kPpThreads, 2) void prefill_pingpong_kernel(Prefill
   // Vector step kt = soft-max of tile kt: mask on the diagonal, exponentials, packing, row sum; row maximum
   // and rescaling of O^T where they are due.  (Its wave goes first where both waves of a SIMD have something
   // to issue: 0.5 to 1 % on long calls.)
-  auto vector_step = [&](uint32_t kt) __attribute__((always_inline)) {
+  auto vector_step = [&](auto group, uint32_t kt) __attribute__((always_inline)) {
+    if constexpr (DIRECT) load_direct(group, kt + kPpAhead);
     __builtin_amdgcn_s_setprio(2);
     const uint32_t kb = (kt0 + kt) * kBK;
     if (kb + kBK - 1 > first_pos) {  // tile crosses this row block's diagonal
@@ -438,7 +492,7 @@ __global__ __launch_bounds__(kPpThreads, 2) void prefill_pingpong_kernel(Prefill
     matrix_step(kGroup0, 0);
     __builtin_amdgcn_s_barrier();
     for (uint32_t kt = 0; kt < n_tiles; ++kt) {
-      vector_step(kt);
+      vector_step(kGroup0, kt);
       prefetch_ring(kt + 1);
       __builtin_amdgcn_s_barrier();
       matrix_step(kGroup0, kt + 1);
@@ -450,12 +504,13 @@ __global__ __launch_bounds__(kPpThreads, 2) void prefill_pingpong_kernel(Prefill
     for (uint32_t kt = 0; kt < n_tiles; ++kt) {
       matrix_step(kGroup1, kt);
       __builtin_amdgcn_s_barrier();
-      vector_step(kt);
+      vector_step(kGroup1, kt);
       prefetch_ring(kt + 1);
       __builtin_amdgcn_s_barrier();
     }
     matrix_step(kGroup1, n_tiles);
   }
+  if constexpr (DIRECT) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // the last requests still write LDS
 
 #pragma unroll
   for (int rb = 0; rb < 2; ++rb) {
@@ -1105,9 +1160,16 @@ hipError_t launch_chunk(const AttnArgs& a, hipStream_t stream) {
     else
       go(chunk_stream_kernel<T, 12>, 12 * kWave);
   } else if (plan.n_split == 1) {
-    go(prefill_pingpong_kernel<T, false>, kPpThreads);
+    // Tiles straight into LDS, three ahead, from walks of 64 tiles on (through registers / straight, us): 8192
+    // tokens on 120000 26230 / 25810, 8000 tokens 444 / 437, 1624 on 10535 291 / 287, layer of 64 x 24 on 4096 189 /
+    // 181-187, 3140 x 3, 32 / 32 heads 284 / 282; but 412 x 19, 32 / 32 heads, 103 / 108, 519 x 3 36 / 38, 120 x 8 on
+    // 1400 57 / 59-65; 255 on 11150 in splits 55.3 / 55.3.
+    if (a.position_index + a.position_interval >= 64u * kBK)
+      go(prefill_pingpong_kernel<T, false, true>, kPpThreads);
+    else
+      go(prefill_pingpong_kernel<T, false, false>, kPpThreads);
   } else {
-    go(prefill_pingpong_kernel<T, true>, kPpThreads);
+    go(prefill_pingpong_kernel<T, true, false>, kPpThreads);
   }
   const hipError_t e = hipGetLastError();
   if (e != hipSuccess || plan.n_split == 1) return e;

@@ -44,6 +44,15 @@ def test_tile_kernel_leaves_m0_to_the_inline_asm(tmp_path):
     assert not any("movrel" in l or "s_set_gpr_idx" in l for l in code)
 
 
+def test_chunk_kernels_leave_m0_to_the_inline_asm(tmp_path):
+    """The same for prefill.hip, whose tile kernel fetches the tiles of long walks straight into LDS."""
+    text = _listing("prefill.hip", tmp_path)
+    code = [l.split(";")[0] for l in text.splitlines()]
+    uses = [l for l in code if re.search(r"\bm0\b", l)]
+    assert uses and all(re.fullmatch(r"\s*s_mov_b32 m0, s\d+\s*", l) for l in uses)
+    assert not any("movrel" in l or "s_set_gpr_idx" in l for l in code)
+
+
 @pytest.mark.parametrize("name", ["project.hip", "project_mid.hip", "project_small.hip", "prefill.hip", "decode.hip",
                                   "decode_balanced.hip", "kv_cache.hip", "attn_general.hip", "attn_general_chunk.hip",
                                   "attn_general_step.hip"])
