@@ -42,6 +42,9 @@ struct Mfma;
 template <>
 struct Mfma<F16> {
   typedef F16 storage;
+  // What a lane's weights of one step may add up to before the row's reference maximum moves: each fits the type
+  // (values are below 2^16, so the binary32 sums have room).
+  static constexpr float kMaxSum = 32768.0f;
   static __device__ __forceinline__ f32x16 m32x32x16(u32x4 a, u32x4 b, f32x16 c) {
     return __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(f16x8, a),
                                                   __builtin_bit_cast(f16x8, b), c, 0, 0, 0);
@@ -72,6 +75,9 @@ struct Mfma<F16> {
 template <>
 struct Mfma<BF16> {
   typedef BF16 storage;
+  // (the same; values have binary32's range here, and a weight above one narrows what the sums can take: 2^8, as
+  // where the reference moves for a score 8 binary orders above it)
+  static constexpr float kMaxSum = 256.0f;
   static __device__ __forceinline__ f32x16 m32x32x16(u32x4 a, u32x4 b, f32x16 c) {
     return __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, a),
                                                    __builtin_bit_cast(bf16x8, b), c, 0, 0, 0);

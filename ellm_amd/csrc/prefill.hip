@@ -38,7 +38,6 @@ namespace {
 constexpr int kBK = 64;                     // keys per tile
 constexpr int kKsPitch = kHeadDim + 8;      // halves per K row (272 B)
 constexpr float kRescaleStep = 8.0f;        // log2 units
-constexpr float kMaxSum = 32768.0f;         // of a lane's exponentials of one tile: each fits binary16
 
 struct PrefillKernelArgs {
   const uint16_t* q;
@@ -449,7 +448,7 @@ __global__ __launch_bounds__(kPpThreads, 2) void prefill_pingpong_kernel(Prefill
     // makes its sums infinite or NaN and so asks for one; so does a score that is not finite.
     float psum[2];
     exponentials(neg_m, psum);
-    const uint64_t over[2] = {__ballot(!(psum[0] <= kMaxSum)), __ballot(!(psum[1] <= kMaxSum))};
+    const uint64_t over[2] = {__ballot(!(psum[0] <= Mfma<T>::kMaxSum)), __ballot(!(psum[1] <= Mfma<T>::kMaxSum))};
     if (over[0] | over[1]) {
       float rmax[2], safe[2];
 #pragma unroll
@@ -721,7 +720,7 @@ __global__ __launch_bounds__(WAVES * kWave, WAVES == 4 ? 2 : 1) void chunk_strea
       };
       // (the reference maximum moves where a lane's sum passes kMaxSum: as in the kernel above)
       exponentials(neg_m);
-      const uint64_t over[2] = {__ballot(!(psum[0] <= kMaxSum)), __ballot(!(psum[1] <= kMaxSum))};
+      const uint64_t over[2] = {__ballot(!(psum[0] <= Mfma<T>::kMaxSum)), __ballot(!(psum[1] <= Mfma<T>::kMaxSum))};
       if (over[0] | over[1]) {
         float rmax[2], safe[2];
 #pragma unroll

@@ -1,5 +1,5 @@
 """The reference maximum of the tile kernel and the streaming chunk kernel: exponentials are taken against the one a row has until a lane's
-sum of them passes 2^15, then the row's true maximum is looked for and its sums are rescaled.  Score
+sum of them passes 2^15 (2^8 in bfloat16), then the row's true maximum is looked for and its sums are rescaled.  Score
 levels that stay below that step, pass it once, again and again, fall back and pass it in some rows of a
 block only; whole rows and a key range in splits, whose later splits some rows see nothing of."""
 import math
@@ -13,7 +13,7 @@ from gpu_util import D, LSE_TOL, gpu_attention, rand_storage, storage_ulp
 
 pytestmark = pytest.mark.gpu
 
-# levels of successive 64-key tiles, in units of the score's log2: below the step of 15, once past it,
+# levels of successive 64-key tiles, in units of the score's log2: below binary16's step of 15, once past it,
 # rising all along, falling, up and down
 LEVELS = {"below": [0, 13, 14, 12], "once": [0, 0, 17, 17], "rising": [0, 16, 40, 300], "falling": [300, 30, 10, 0],
           "waves": [0, 40, -40, 60]}
@@ -48,3 +48,28 @@ def test_scores_that_outgrow_the_reference(b, hq, hkv, s, p0, want_kernel, split
     assert (err <= bound).all(), float((err / bound).max())
     # (a log-sum-exp of up to 208 is spaced 2^-16; the bound leaves it a dozen roundings)
     assert np.abs(lse - want_lse).max() <= LSE_TOL + 12 * 2.0 ** -16
+
+
+@pytest.mark.parametrize("b,hq,hkv,s,p0,want_kernel,split", [
+    (16, 32, 4, 49, 200, "pingpong", False), (2, 32, 4, 600, 4060, "pingpong", False), (1, 8, 1, 70, 2400, "pingpong", True),
+    (300, 8, 1, 13, 520, "stream", False), (2, 8, 1, 13, 2400, "stream", True), (2, 8, 1, 45, 2400, "stream", True)],
+    ids=["whole", "whole_4660_keys", "split", "stream_whole", "stream_13", "stream_45"])
+@pytest.mark.parametrize("rise", [7.5, 14.0])
+def test_large_bfloat16_values_under_rising_scores(b, hq, hkv, s, p0, want_kernel, split, rise):
+    """A value of 2^115 under the one score that lies 7.5 or 14 binary orders above those before it, in another
+    place of the key range for every head: a weight of 2^14 would carry it past binary32's range."""
+    kernel, _, n_split = plan_probe.chunk_plan(b, b, hq, hkv, p0, s)[:3]
+    assert kernel == want_kernel and (n_split > 1) == split
+    q, k, v = (np.zeros(n, np.float32) for n in ((s, b, hq, D), (b, hkv, p0 + s, D), (b, hkv, p0 + s, D)))
+    q[..., 0] = 1.0
+    planes = b * hkv
+    hot = (np.arange(planes) * 37 % (p0 - 110)).reshape(b, hkv) + 100
+    for i in range(b):
+        for h in range(hkv):
+            k[i, h, hot[i, h], 0] = rise
+            v[i, h, hot[i, h]] = 2.0 ** 115
+    q, k, v = (orc.to_storage(a, orc.BF16) for a in (q, k, v))
+    got, _ = gpu_attention(q, k, v, float(np.log(2.0)), orc.BF16, position_index=p0)
+    share = 1.0 / (1.0 + (p0 + np.arange(s)) * 2.0 ** -rise)          # of the one key among the row's keys
+    err = np.abs(got / (share[:, None, None, None] * 2.0 ** 115) - 1.0)
+    assert err.max() <= 2.0 ** -8 + 2.0 ** -9                         # the weights rounded once, the output once
