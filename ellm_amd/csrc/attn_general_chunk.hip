@@ -27,7 +27,6 @@ namespace gen {
 namespace {
 
 constexpr float kRescaleStep = 8.0f;     // log2 units
-constexpr float kMaxSum = 32768.0f;      // of a lane's weights of one step: each fits binary16
 
 typedef __attribute__((address_space(3))) uint8_t LdsByte;
 typedef __attribute__((address_space(3))) u32x4 LdsU32x4;
@@ -280,7 +279,7 @@ void general_chunk_kernel(GeneralArgs p) {
     }
     load_late(step + KG);
     // 16-bit storage and heads up to 128: exponentials against the reference maximum the row already has, and
-    // its true maximum looked for only where a lane's sum of them passes kMaxSum (below).  Else (wider heads
+    // its true maximum looked for only where a lane's sum of them passes Mfma<S>::kMaxSum (below).  Else (wider heads
     // keep their pipe busy with products, and binary32 its own way to add up) the maximum first, every step.
     // Maximum first -> here (us): 2048 tokens, 32 / 8 heads of 64, bf16 42.0 -> 40.4; 1500 on 300, 32 / 4 of 80 56.3 ->
     // 51.8; 400 x 3 on 1000, 32 / 8 of 96 49.2 -> 46.4; heads of 192 and 256 1.3 % slower.
@@ -361,7 +360,7 @@ void general_chunk_kernel(GeneralArgs p) {
       weights();
       if constexpr (kLazy) {
         // (a row without a reference makes its sum infinite or NaN; a row moves by what its own two lanes saw)
-        const uint64_t over = __ballot(!(psum <= kMaxSum));
+        const uint64_t over = __ballot(!(psum <= Mfma<S>::kMaxSum));
         if (over) {
           float rmax = st[0][0];
 #pragma unroll
@@ -460,7 +459,7 @@ void general_chunk_kernel(GeneralArgs p) {
   if (KG > 1 && kg != 0) return;
   const float l = sum_with_partner_half(l_run);
   // Sums that are not finite: an infinite value under a weight in two operands, or weights above one (up to
-  // kMaxSum) on values less than that below the largest number.
+  // 2^8 in bfloat16) on values less than that below the largest number.
   float top[4] = {0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
   for (int db = 0; db < NB; ++db)

@@ -168,18 +168,20 @@ def test_an_infinite_value_that_a_row_sees(case, dtype):
 
 
 @pytest.mark.parametrize("dtype,hs,hq", [(orc.BF16, 256, 4), (orc.BF16, 64, 4), (orc.F32, 64, 64)], ids=["bf16_h256", "bf16_h64", "f32_h64"])
-def test_large_finite_values_under_rising_scores(dtype, hs, hq):
-    """One value of 1e38 under the highest score, which lies 6.5 binary orders above those of the step of keys
-    before it: less than what makes the chunk kernel move its reference, so the weight is 2^6.5 there."""
+@pytest.mark.parametrize("rise", [6.5, 14.0])
+def test_large_finite_values_under_rising_scores(dtype, hs, hq, rise):
+    """One value of 1e38 under the highest score, which lies 6.5 or 14 binary orders above those of the step of keys
+    before it: less and more than what makes the chunk kernel move its reference (by 8), so the weight is 2^6.5
+    or 1 there."""
     hkv, s, p0 = 2, 50, 90
     assert plan_probe.general_plan(hs, element_bytes(dtype), 1, 1, hq, hkv, p0, s)[0] == "chunk"
     q, k, v = np.zeros((s, 1, hq, hs), np.float32), np.zeros((1, hkv, p0 + s, hs), np.float32), np.zeros((1, hkv, p0 + s, hs), np.float32)
     q[..., 0] = 1.0
-    k[:, :, 70, 0] = 6.5
+    k[:, :, 70, 0] = rise
     v[:, :, 70] = 1e38
     q, k, v = (orc.to_storage(a, dtype) for a in (q, k, v))
     got, _ = _run(q, k, v, float(np.log(2.0)), dtype, p0=p0)
-    share = 1.0 / (1.0 + (p0 + np.arange(s)) * 2.0 ** -6.5)          # of the one key among the row's keys
+    share = 1.0 / (1.0 + (p0 + np.arange(s)) * 2.0 ** -rise)          # of the one key among the row's keys
     want = share[:, None, None, None] * float(orc.from_storage(v, dtype).max())
     err = float(np.abs(got / want - 1.0).max())
     assert err <= (2.0 ** -8 if dtype == orc.BF16 else 1e-6)         # half a unit of bfloat16, binary32 sums
