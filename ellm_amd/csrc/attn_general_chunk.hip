@@ -88,6 +88,7 @@ void general_chunk_kernel(GeneralArgs p) {
   typedef typename Store<S>::E E;
   constexpr int MB = X::MB, kKeys = X::kKeys, kPieces = X::kPieces, kTileRows = X::kTileRows;
   constexpr int kQ = X::kPiecesRow / 2;      // query registers: pieces 2 s + g of the row
+  constexpr bool kLazy = !X::kF32 && NB <= 4;   // see compute()
   constexpr float kShift = Store<S>::kShift;
   __shared__ __attribute__((aligned(16))) uint8_t smem[X::kLds];
   __shared__ uint32_t s_bad;                 // a value beyond the first row's position is not finite
@@ -215,7 +216,8 @@ void general_chunk_kernel(GeneralArgs p) {
     if constexpr (X::kLateV)
       if (step < n_steps) load_rows(step, vp, vplane, vst);
   };
-  auto compute = [&](uint32_t step) __attribute__((always_inline)) {
+  auto compute = [&](uint32_t step, auto first_) __attribute__((always_inline)) {
+    constexpr bool kFirst = decltype(first_)::value;   // the group's first step: no row has a reference maximum yet
     const uint32_t kb = k0 + step * kKeys, buf = step / KG & 1;
     if (step >= n_steps || !wave_has_rows || kb > wave_last) {
       load_late(step + KG);
@@ -281,9 +283,11 @@ void general_chunk_kernel(GeneralArgs p) {
     // 16-bit storage and heads up to 128: exponentials against the reference maximum the row already has, and
     // its true maximum looked for only where a lane's sum of them passes Mfma<S>::kMaxSum (below).  Else (wider heads
     // keep their pipe busy with products, and binary32 its own way to add up) the maximum first, every step.
-    // Maximum first -> here (us): 2048 tokens, 32 / 8 heads of 64, bf16 42.0 -> 40.4; 1500 on 300, 32 / 4 of 80 56.3 ->
-    // 51.8; 400 x 3 on 1000, 32 / 8 of 96 49.2 -> 46.4; heads of 192 and 256 1.3 % slower.
-    constexpr bool kLazy = !X::kF32 && NB <= 4;
+    // Maximum first -> here (us): 2048 tokens, 32 / 8 heads of 64, bf16 42.0 -> 40.0; 1500 on 300, 32 / 4 of 80 57.0 ->
+    // 52.2; 400 x 3 on 1000, 32 / 8 of 96 49.1 -> 45.5; heads of 192 and 256 1.3 % slower.  Short walks gain or lose
+    // nothing (300 x 2, 32 / 8 of 80 11.0 -> 11.0, of 32 7.7 -> 7.6; 119 x 3 on 125, 32 / 32 of 64 7.4 -> 7.4), but only
+    // because a group's first step, when no row has a reference, goes to the maximum at once: with a pass over
+    // the weights before it they took 2 to 5 % longer (11.5, 8.0, 7.5).
     float neg_m = kShift - m_run;
     if constexpr (!kLazy) {
       float rmax = st[0][0];
@@ -357,10 +361,10 @@ void general_chunk_kernel(GeneralArgs p) {
             psum += p0 + p1;
           }
       };
-      weights();
+      if constexpr (!kLazy || !kFirst) weights();
       if constexpr (kLazy) {
         // (a row without a reference makes its sum infinite or NaN; a row moves by what its own two lanes saw)
-        const uint64_t over = __ballot(!(psum <= Mfma<S>::kMaxSum));
+        const uint64_t over = kFirst ? ~(uint64_t)0 : __ballot(!(psum <= Mfma<S>::kMaxSum));
         if (over) {
           float rmax = st[0][0];
 #pragma unroll
@@ -403,15 +407,17 @@ void general_chunk_kernel(GeneralArgs p) {
   if (kg < n_steps) store_step(kg);
   if (kg + KG < n_steps) load_step(kg + KG);
   __syncthreads();
-  for (uint32_t first = 0; first < n_steps; first += KG) {
-    const uint32_t step = first + kg;
-    compute(step);
+  auto turn = [&](uint32_t step, auto first) __attribute__((always_inline)) {
+    compute(step, first);
     if (step + KG < n_steps) {
       store_step(step + KG);
       if (step + 2 * KG < n_steps) load_step(step + 2 * KG);
     }
     __syncthreads();
-  }
+  };
+  // (the first turn apart where it skips a pass over the weights: a branch in the loop costs 2048 tokens 1.5 %)
+  if constexpr (kLazy) turn(kg, std::true_type{});
+  for (uint32_t first = kLazy ? KG : 0; first < n_steps; first += KG) turn(first + kg, std::false_type{});
 
   const size_t part_row0 = (size_t)plane * p.rows;
   if (s_bad) {   // (uniform: the last barrier is behind every write of it)
