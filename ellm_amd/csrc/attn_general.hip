@@ -239,6 +239,7 @@ hipError_t launch_attn_general(const AttnArgs& a, uint32_t head_size, hipStream_
   p.tile_rows = plan.tile_rows;
   p.key_groups = plan.key_groups;
   p.turn_at = plan.turn_at;
+  p.max_first = plan.max_first;
   p.n_split = plan.n_split;
   p.split_len = plan.split_len;
   if (plan.kernel == gen::kGeneralRows) return gen::launch_rows(p, a.dtype, planes, stream);

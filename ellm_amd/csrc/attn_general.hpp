@@ -80,6 +80,7 @@ struct GeneralArgs {
   uint32_t tile_rows;            // query rows of a workgroup of the chunk kernel (64 or 128)
   uint32_t turn_at;              // ... and the row tile of the launch (longest first) from which the order turns
   uint32_t key_groups;           // groups of waves that share the keys of those rows
+  uint32_t max_first;            // (host) which form of the chunk kernel: GeneralPlan
   float* part_o;
   float* part_ml;
   uint32_t* counters;            // arrivals per (plane, row tile); zero between launches

@@ -81,14 +81,23 @@ struct Shape {
   static constexpr int kOccupancy = KG == 2 && NB <= 2 ? 4 : KG > 1 ? kWaves / 4 : kF32 ? (NB <= 4 ? 2 : 1) : NB <= 2 ? 3 : NB <= 4 ? 2 : 1;
 };
 
-template <typename S, int NB, bool VEC, int RB, int KG>
-__global__ __launch_bounds__((Shape<S, NB, RB, KG>::kThreads), (Shape<S, NB, RB, KG>::kOccupancy))
+// The weights of two keys as operands of the second product, and their sum.
+template <typename S>
+__device__ __forceinline__ float weigh_pair(float s0, float s1, float c, float shift, uint32_t& hi, uint32_t& lo) {
+  const float p0 = fast_exp2(__builtin_fmaf(s0, c, shift)), p1 = fast_exp2(__builtin_fmaf(s1, c, shift));
+  split_pair<S>(p0, p1, hi, lo);
+  return p0 + p1;
+}
+
+// (heads of 65 to 96 with the maximum every step: 160 registers, three workgroups a unit, which is what that form is for)
+template <typename S, int NB, bool VEC, int RB, int KG, bool LAZY>
+__global__ __launch_bounds__((Shape<S, NB, RB, KG>::kThreads),
+                             (NB == 3 && KG == 1 && !LAZY && !Shape<S, NB, RB, KG>::kF32 ? 3 : Shape<S, NB, RB, KG>::kOccupancy))
 void general_chunk_kernel(GeneralArgs p) {
   typedef Shape<S, NB, RB, KG> X;
   typedef typename Store<S>::E E;
   constexpr int MB = X::MB, kKeys = X::kKeys, kPieces = X::kPieces, kTileRows = X::kTileRows;
   constexpr int kQ = X::kPiecesRow / 2;      // query registers: pieces 2 s + g of the row
-  constexpr bool kLazy = !X::kF32 && NB <= 4;   // see compute()
   constexpr float kShift = Store<S>::kShift;
   __shared__ __attribute__((aligned(16))) uint8_t smem[X::kLds];
   __shared__ uint32_t s_bad;                 // a value beyond the first row's position is not finite
@@ -280,16 +289,17 @@ void general_chunk_kernel(GeneralArgs p) {
         }
     }
     load_late(step + KG);
-    // 16-bit storage and heads up to 128: exponentials against the reference maximum the row already has, and
+    // LAZY (16-bit storage, heads up to 128): exponentials against the reference maximum the row already has, and
     // its true maximum looked for only where a lane's sum of them passes Mfma<S>::kMaxSum (below).  Else (wider heads
-    // keep their pipe busy with products, and binary32 its own way to add up) the maximum first, every step.
+    // keep their pipe busy with products, binary32 its own way to add up, and chunk_max_first() says where heads of 65
+    // to 96 are better off) the maximum first, every step.
     // Maximum first -> here (us): 2048 tokens, 32 / 8 heads of 64, bf16 42.0 -> 40.0; 1500 on 300, 32 / 4 of 80 57.0 ->
     // 52.2; 400 x 3 on 1000, 32 / 8 of 96 49.1 -> 45.5; heads of 192 and 256 1.3 % slower.  Short walks gain or lose
     // nothing (300 x 2, 32 / 8 of 80 11.0 -> 11.0, of 32 7.7 -> 7.6; 119 x 3 on 125, 32 / 32 of 64 7.4 -> 7.4), but only
     // because a group's first step, when no row has a reference, goes to the maximum at once: with a pass over
     // the weights before it they took 2 to 5 % longer (11.5, 8.0, 7.5).
     float neg_m = kShift - m_run;
-    if constexpr (!kLazy) {
+    if constexpr (!LAZY) {
       float rmax = st[0][0];
 #pragma unroll
       for (int mb = 0; mb < MB; ++mb)
@@ -345,24 +355,20 @@ void general_chunk_kernel(GeneralArgs p) {
       });
     } else {
       u32x4 hi[2 * MB], lo[2 * MB];
-      auto weights = [&]() __attribute__((always_inline)) {
-        psum = 0.0f;
+      // (the loop stands here and below: as a lambda it takes 9 registers more where LAZY is off)
+      if constexpr (!LAZY || !kFirst) {
 #pragma unroll
         for (int cc = 0; cc < 2 * MB; ++cc)
 #pragma unroll
           for (int w = 0; w < 4; ++w) {
             const int e = 8 * (cc & 1) + 2 * w;
-            const float p0 = fast_exp2(__builtin_fmaf(st[cc >> 1][e], p.c, neg_m));
-            const float p1 = fast_exp2(__builtin_fmaf(st[cc >> 1][e + 1], p.c, neg_m));
             uint32_t h, l;
-            split_pair<S>(p0, p1, h, l);
+            psum += weigh_pair<S>(st[cc >> 1][e], st[cc >> 1][e + 1], p.c, neg_m, h, l);
             hi[cc][w] = h;
             lo[cc][w] = l;
-            psum += p0 + p1;
           }
-      };
-      if constexpr (!kLazy || !kFirst) weights();
-      if constexpr (kLazy) {
+      }
+      if constexpr (LAZY) {
         // (a row without a reference makes its sum infinite or NaN; a row moves by what its own two lanes saw)
         const uint64_t over = kFirst ? ~(uint64_t)0 : __ballot(!(psum <= Mfma<S>::kMaxSum));
         if (over) {
@@ -380,7 +386,17 @@ void general_chunk_kernel(GeneralArgs p) {
 #pragma unroll
           for (int db = 0; db < NB; ++db) oacc[db] *= alpha;
           neg_m = (m_run == -INFINITY) ? 0.0f : kShift - m_run;
-          weights();
+          psum = 0.0f;
+#pragma unroll
+          for (int cc = 0; cc < 2 * MB; ++cc)
+#pragma unroll
+            for (int w = 0; w < 4; ++w) {
+              const int e = 8 * (cc & 1) + 2 * w;
+              uint32_t h, l;
+              psum += weigh_pair<S>(st[cc >> 1][e], st[cc >> 1][e + 1], p.c, neg_m, h, l);
+              hi[cc][w] = h;
+              lo[cc][w] = l;
+            }
         }
       }
 #pragma unroll
@@ -416,8 +432,8 @@ void general_chunk_kernel(GeneralArgs p) {
     __syncthreads();
   };
   // (the first turn apart where it skips a pass over the weights: a branch in the loop costs 2048 tokens 1.5 %)
-  if constexpr (kLazy) turn(kg, std::true_type{});
-  for (uint32_t first = kLazy ? KG : 0; first < n_steps; first += KG) turn(first + kg, std::false_type{});
+  if constexpr (LAZY) turn(kg, std::true_type{});
+  for (uint32_t first = LAZY ? KG : 0; first < n_steps; first += KG) turn(first + kg, std::false_type{});
 
   const size_t part_row0 = (size_t)plane * p.rows;
   if (s_bad) {   // (uniform: the last barrier is behind every write of it)
@@ -514,18 +530,25 @@ hipError_t launch_general_chunk(const GeneralArgs& p, int dtype, int nb, bool ve
     auto go = [&](auto storage) {
       typedef decltype(storage) S;
       constexpr int kLong = chunk_key_groups(std::is_same<S, F32>::value, NB, 4);
+      // (one key group: not with heads up to 64, whose walks are two steps then, and with NB 3 as the plan says)
+      constexpr bool kLazy = !std::is_same<S, F32>::value && NB <= 4;
       constexpr int kShort = chunk_key_groups(std::is_same<S, F32>::value, NB, 2);
       if constexpr (kShort > 1)
         if (p.tile_rows == 64) {
-          hipLaunchKernelGGL((general_chunk_kernel<S, NB, VEC, 2, kShort>), grid, dim3(128 * kShort), 0, stream, p);
+          hipLaunchKernelGGL((general_chunk_kernel<S, NB, VEC, 2, kShort, kLazy>), grid, dim3(128 * kShort), 0, stream, p);
           return hipGetLastError();
         }
       if constexpr (kLong > 1)
         if (p.key_groups > 1) {
-          hipLaunchKernelGGL((general_chunk_kernel<S, NB, VEC, 4, kLong>), grid, dim3(256 * kLong), 0, stream, p);
+          hipLaunchKernelGGL((general_chunk_kernel<S, NB, VEC, 4, kLong, kLazy>), grid, dim3(256 * kLong), 0, stream, p);
           return hipGetLastError();
         }
-      hipLaunchKernelGGL((general_chunk_kernel<S, NB, VEC, 4, 1>), grid, dim3(256), 0, stream, p);
+      if constexpr (NB == 3 && kLazy)
+        if (p.max_first) {
+          hipLaunchKernelGGL((general_chunk_kernel<S, NB, VEC, 4, 1, false>), grid, dim3(256), 0, stream, p);
+          return hipGetLastError();
+        }
+      hipLaunchKernelGGL((general_chunk_kernel<S, NB, VEC, 4, 1, (kLazy && NB > 2)>), grid, dim3(256), 0, stream, p);
       return hipGetLastError();
     };
     return dtype == 0 ? go(F16{}) : dtype == 1 ? go(BF16{}) : go(F32{});

@@ -69,6 +69,7 @@ struct GeneralPlan {
   int nb;                                                  // matrix kernels: padded head blocks
   uint32_t row_tiles, n_split, split_len;
   uint32_t tile_rows, key_groups, turn_at;                 // chunk kernel
+  bool max_first;                                          // ... its form that looks for the row maximum every step
 };
 
 // Estimated times (us, 256 units) of a call, fitted to graph replays of calls of 4 to 32 heads; measured ones in
@@ -107,6 +108,25 @@ inline double general_chunk_us(const GeneralCall& c, const GeneralPlan& p) {
   const double mean = (c.max_len - 0.5 * (c.interval - 1)) / c.max_len;
   const double work = rounds > 1 ? (1 + (rounds - 1) * mean) * walk : walk;
   return (c.f32 ? 3.8 : 4.5 + 0.2 * p.nb + (c.vec ? 0.0 : 0.4 * p.nb)) + step * work + (p.n_split > 1 ? 6.0 : 0.0);
+}
+
+// Whether the chunk kernel looks for a row's maximum every step (16-bit heads; see its compute()): with heads above 128
+// always; with one key group and heads up to 64, whose walks are two steps, too (128 tokens x 40, 32 / 32 heads of 32: 16.5
+// us, else 17.7, for the registers it takes); with heads of 65 to 96 and one key group, whose other form has registers for two workgroups a unit
+// instead of three, where the third is worth more than the maxima.  That is from three workgroups a unit on
+// (us, every step / only where it may have to move, heads of 80 and 96: 700 tokens x 4, 32 / 32 heads 32.0 / 36.4, 300 x 12
+// 31.8 / 37.8, 2048 x 4 174 / 180), and from two on unless what the first two leave are short walks: those of
+// the shortest rows, at most a third of the longest walk or, with few row tiles a plane, a fifth (1400 x 2, 32 / 8 heads
+// 50.3 / 45.5, 1500 x 2, 32 / 4 56.9 / 51.2, 700 x 3, 32 / 32 28.9 / 27.8; but 300 x 7, 32 / 32 20.0 / 24.3, 500 x 5 on 300
+// 42.0 / 51.3).  Up to two a unit: 1600 tokens, 32 / 8 51.2 / 47.5.
+inline bool chunk_max_first(const GeneralCall& c, const GeneralPlan& p) {
+  if (c.f32 || p.nb > 4 || (p.nb <= 2 && p.key_groups == 1)) return true;
+  const size_t workgroups = (size_t)c.planes * p.row_tiles * p.n_split, pair = 2 * (size_t)c.n_cu;
+  if (p.nb != 3 || p.key_groups != 1 || workgroups <= pair) return false;
+  if (workgroups >= 3 * (size_t)c.n_cu) return true;
+  const size_t left = p.row_tiles - pair / c.planes;          // row tiles of a plane behind the first two a unit
+  const double longest = c.max_len, tail = c.max_len - c.interval + (double)left * p.tile_rows / c.group;
+  return tail * (p.row_tiles >= 16 ? 3 : 5) > longest;
 }
 
 // The matrix kernel of a call and its cut.
@@ -164,6 +184,7 @@ inline GeneralPlan general_matrix_plan(const GeneralCall& c) {
       p.split_len = ks.split_tiles * 64;
     }
   }
+  p.max_first = chunk_max_first(c, p);
   return p;
 }
 

@@ -42,7 +42,7 @@ int main(int, char** v) {
   c.vec = a[10] != 0;
   c.room = a[11] ? a[11] : w.rows / (c.planes * c.rows());
   const gen::GeneralPlan p = gen::general_plan(c);
-  printf("%d %u %u %u %d %zu\n", (int)p.kernel, p.n_split, p.tile_rows, p.key_groups, p.nb, w.rows);
+  printf("%d %u %u %u %d %zu %d\n", (int)p.kernel, p.n_split, p.tile_rows, p.key_groups, p.nb, w.rows, (int)p.max_first);
 }
 """
 
@@ -63,7 +63,7 @@ def _program():
 
 def general_plan(head_size, element_bytes, batch_capacity, batch, q_heads, kv_heads, position_index, interval, vec=None, room=0):
     """(kernel "rows" / "step" / "chunk", key splits, rows per workgroup, key groups, padded head blocks, the
-    workspace's partial rows)"""
+    workspace's partial rows, whether a chunk kernel looks for the row maximum every step)"""
     if vec is None:
         vec = head_size * element_bytes % 16 == 0
     args = (head_size, element_bytes, batch_capacity, batch, q_heads, kv_heads, interval, position_index, interval, int(vec), room)

@@ -18,6 +18,20 @@ def test_known_calls():
     assert plan(64, 4, 1, 1, 8, 2, 1900, 1)[0] == "step"
 
 
+def test_the_form_of_the_chunk_kernel():
+    """Heads of 65 to 96 with one key group: the maximum every step from three workgroups a unit (256) on, and from
+    two on where what those leave is not short."""
+    def every_step(*call):
+        return plan_probe.general_plan(96, 2, call[0], *call)[6]
+
+    assert not every_step(4, 32, 32, 0, 512) and not every_step(1, 32, 8, 0, 1600)      # 512, 400 workgroups
+    assert every_step(4, 32, 32, 0, 700) and every_step(4, 32, 32, 0, 2048)             # 768, 2048
+    assert not every_step(2, 32, 8, 0, 1400) and every_step(2, 32, 8, 500, 1300)        # 704, the last short; 656, all long
+    assert not every_step(3, 32, 32, 0, 700) and every_step(7, 32, 32, 0, 300)          # 576 and 672 with few row tiles a plane
+    for hs, want in ((64, 0), (128 - 8, 0), (192, 1)):
+        assert plan_probe.general_plan(hs, 2, 4, 4, 32, 32, 0, 700)[6] == want
+
+
 def test_a_plan_depends_on_the_rows_not_on_how_the_capacity_is_named():
     for hs, es, s in itertools.product((33, 64, 256), (2, 4), (1, 40)):
         a = plan_probe.general_plan(hs, es, 4, 2, 8, 2, 500, s)
