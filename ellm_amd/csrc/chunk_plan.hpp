@@ -171,6 +171,11 @@ inline uint32_t short_prompt_wr(const ChunkShape& c, double other_us, double mar
 // A chunk call of 128-wide 16-bit heads, the kernel it runs and how the work is cut.
 constexpr uint32_t kChunkTile = 64;         // keys per tile of the ping-pong and streaming kernels
 constexpr uint32_t kPingpongRowBlocks = 8;  // 32-row blocks of a ping-pong workgroup
+// Unsplit ping-pong walks of this many keys and more fetch their tiles straight into LDS, three ahead (through
+// registers / straight, us): 8192 tokens on 120000 26230 / 25810, 8000 tokens 444 / 437, 1624 on 10535 291 / 287,
+// layer of 64 x 24 on 4096 189 / 181-187, 3140 x 3, 32 / 32 heads 284 / 282; but 412 x 19, 32 / 32 heads, 103 / 108,
+// 519 x 3 36 / 38, 120 x 8 on 1400 57 / 59-65; 255 on 11150 in splits 55.3 / 55.3.
+constexpr uint32_t kDirectKeys = 64 * kChunkTile;
 
 struct ChunkCall {
   uint32_t p0, interval;                    // positions p0 .. p0 + interval - 1
@@ -184,6 +189,7 @@ struct ChunkPlan {
   ChunkKernel kernel;
   uint32_t waves;                           // streaming kernel: 4, 8 or 12
   uint32_t row_blocks;                      // short-prompt kernel: 32-row blocks a workgroup, 1 or 2
+  bool direct;                              // ping-pong kernel: tiles straight into LDS
   uint32_t n_split, split_tiles;            // key range of a plane, in tiles (one split: split_tiles may be 0)
   // ping-pong workgroup: heads_per_wg heads of a group x tblocks_per_wg blocks of 32 tokens
   uint32_t heads_per_wg, tblocks_per_wg, head_groups;
@@ -308,6 +314,7 @@ inline ChunkPlan plan_chunk(const ChunkCall& c) {
   const double margin = all_tiles > 24 ? 0.82 : 0.87;
   if (const uint32_t wr = short_prompt_wr(shape, pingpong_us(shape, base, {p.split_tiles, p.n_split}), margin))
     plan_short_prompt(shape, wr, &p);
+  p.direct = p.kernel == kChunkPingpong && p.n_split == 1 && c.p0 + c.interval >= kDirectKeys;
   return p;
 }
 

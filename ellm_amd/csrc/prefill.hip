@@ -1161,11 +1161,7 @@ hipError_t launch_chunk(const AttnArgs& a, hipStream_t stream) {
     else
       go(chunk_stream_kernel<T, 12>, 12 * kWave);
   } else if (plan.n_split == 1) {
-    // Tiles straight into LDS, three ahead, from walks of 64 tiles on (through registers / straight, us): 8192
-    // tokens on 120000 26230 / 25810, 8000 tokens 444 / 437, 1624 on 10535 291 / 287, layer of 64 x 24 on 4096 189 /
-    // 181-187, 3140 x 3, 32 / 32 heads 284 / 282; but 412 x 19, 32 / 32 heads, 103 / 108, 519 x 3 36 / 38, 120 x 8 on
-    // 1400 57 / 59-65; 255 on 11150 in splits 55.3 / 55.3.
-    if (a.position_index + a.position_interval >= 64u * kBK)
+    if (plan.direct)
       go(prefill_pingpong_kernel<T, false, true>, kPpThreads);
     else
       go(prefill_pingpong_kernel<T, false, false>, kPpThreads);

@@ -21,7 +21,8 @@ static int chunk(char** v) {   // batch capacity, batch, query heads, key-value 
   for (int i = 1; i <= 7; ++i) a[i] = (uint32_t)strtoul(v[i + 1], nullptr, 10);
   const ChunkCall c = {a[6], a[7], a[2], a[1], a[3], a[4], 256, prefill_workspace_rows(a[5], a[1], a[3], 256)};
   const ChunkPlan p = plan_chunk(c);
-  printf("%d %u %u %u\n", (int)p.kernel, p.kernel == kChunkStream ? p.waves : p.kernel == kChunkShort ? p.row_blocks : 0, p.n_split, p.n_wg);
+  printf("%d %u %u %u %d\n", (int)p.kernel, p.kernel == kChunkStream ? p.waves : p.kernel == kChunkShort ? p.row_blocks : 0, p.n_split, p.n_wg,
+         (int)p.direct);
   return 0;
 }
 // head size, bytes an element, batch capacity, batch, query heads, key-value heads, most positions a call,
@@ -71,8 +72,18 @@ def general_plan(head_size, element_bytes, batch_capacity, batch, q_heads, kv_he
     return (("rows", "step", "chunk")[int(out[0])], *map(int, out[1:]))
 
 
-def chunk_plan(batch_capacity, batch, q_heads, kv_heads, position_index, interval, most=None):
-    """128-wide 16-bit heads: (kernel "stream" / "pingpong" / "short", its waves or row blocks, key splits, workgroups a split)"""
+def _chunk(batch_capacity, batch, q_heads, kv_heads, position_index, interval, most=None):
     args = ("c", batch_capacity, batch, q_heads, kv_heads, most or interval, position_index, interval)
-    out = subprocess.run([_program(), *map(str, args)], check=True, capture_output=True, text=True).stdout.split()
-    return (("stream", "pingpong", "short")[int(out[0])], *map(int, out[1:]))
+    return subprocess.run([_program(), *map(str, args)], check=True, capture_output=True, text=True).stdout.split()
+
+
+def chunk_plan(*call, **most):
+    """128-wide 16-bit heads: (kernel "stream" / "pingpong" / "short", its waves or row blocks, key splits, workgroups a split).
+    Arguments: batch capacity, batch, query heads, key-value heads, position_index, interval[, most positions a call]"""
+    out = _chunk(*call, **most)
+    return (("stream", "pingpong", "short")[int(out[0])], *map(int, out[1:4]))
+
+
+def chunk_is_direct(*call, **most):
+    """Whether the same call runs the tile kernel's form that fetches K and V straight into LDS."""
+    return _chunk(*call, **most)[4] == "1"

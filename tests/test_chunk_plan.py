@@ -110,3 +110,13 @@ def test_the_chunk_cases_reach_the_kernels_they_are_there_for():
         seen.add((kernel, waves, n_split > 1))
     assert seen >= {("stream", w, True) for w in (4, 8, 12)} | {("stream", 4, False), ("pingpong", 0, True), ("pingpong", 0, False),
                                                                ("short", 1, False), ("short", 2, False)}
+
+
+def test_tiles_go_straight_to_lds_in_unsplit_tile_walks_of_4096_keys_and_more():
+    direct, plan = plan_probe.chunk_is_direct, plan_probe.chunk_plan
+    for b, hq, hkv, s in ((17, 64, 1, 9), (17, 32, 4, 49), (2, 32, 4, 600), (24, 32, 4, 64)):
+        for keys, want in ((4095, False), (4096, True), (4097, True), (131072, True)):
+            assert plan(b, b, hq, hkv, keys - s, s)[:3] == ("pingpong", 0, 1)
+            assert direct(b, b, hq, hkv, keys - s, s) == want, (b, hq, hkv, s, keys)
+    assert plan(1, 1, 32, 4, 8192, 64)[0] == "pingpong" and plan(1, 1, 32, 4, 8192, 64)[2] > 1 and not direct(1, 1, 32, 4, 8192, 64)
+    assert plan(24, 24, 32, 4, 8191, 13)[0] == "stream" and not direct(24, 24, 32, 4, 8191, 13)
