@@ -309,6 +309,26 @@ inline ChunkPlan plan_chunk(const ChunkCall& c) {
       p.n_split = ks.n_split;
     }
   }
+  // More than half of the units, but not most of them: two pieces a walk, sized for how the hardware deals them.  A
+  // launch fills its shader engines (groups of eight units) in turn, so with m long first pieces on each the
+  // second ones run on the other 8 - m units, in r = m / (8 - m) rounds, and should take 1 / r of a first one.
+  // (168 workgroups, m = 6, cut for r = 2 as the count of all free units has it: 281 us against 278 unsplit.)
+  // A tile takes 1.35 us, 1.56 with all units at work; K and V, which unsplit workgroups read in step, cost a split
+  // call their bytes at 12 TB/s.  Unsplit / split (us): 32 / 4 heads, bf16, 1030 tokens on 4100 113.6 / 99.9, on 12000 270
+  // / 226, 1167 on 12000 273 / 243, 1344 on 4100 119.7 / 113.3, 1536 on 4100 128.9 / 124.6, on 12000 312 / 300; 600 on
+  // 12000, 64 / 8 heads 262 / 237; 1089 on 4100, 32 / 32 heads 114.3 / 104.7; 64 x 18 on 8192, f16 190 / 184; 5000 tokens,
+  // 8 / 1 heads 108 / 88.  Left whole: 64 x 18 on 4096 95.6 / 99.0, 660 on 4100, 64 / 8 heads 109 / 111.
+  if (c.part_rows && 2 * base > c.n_cu && 4 * base <= 3 * c.n_cu && max_split >= 2) {
+    const uint32_t m = (8 * base + c.n_cu - 1) / c.n_cu, r = (m + (8 - m) - 1) / (8 - m);   // m: 5 or 6
+    const uint32_t len = (all_tiles * r + r) / (r + 1);
+    const double mean = (c.p0 + 0.5 * c.interval) / kChunkTile + 1;
+    const double chain = 1.35 * len, work = 1.56 * base * mean / c.n_cu;
+    const double split = (chain > work ? chain : work) + merge_us(shape, 2) + shape.stream_us(12.0);
+    if (split < 0.98 * 1.35 * all_tiles) {
+      p.split_tiles = len;
+      p.n_split = 2;
+    }
+  }
   // (beyond 1536 keys pieces of a split walk take less than the estimate: 300 tokens x 2 on 1500, 32 / 4 heads, 34 us
   // against 38 in the short-prompt kernel)
   const double margin = all_tiles > 24 ? 0.82 : 0.87;

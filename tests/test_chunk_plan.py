@@ -114,9 +114,23 @@ def test_the_chunk_cases_reach_the_kernels_they_are_there_for():
 
 def test_tiles_go_straight_to_lds_in_unsplit_tile_walks_of_4096_keys_and_more():
     direct, plan = plan_probe.chunk_is_direct, plan_probe.chunk_plan
-    for b, hq, hkv, s in ((17, 64, 1, 9), (17, 32, 4, 49), (2, 32, 4, 600), (24, 32, 4, 64)):
+    for b, hq, hkv, s in ((25, 64, 1, 9), (25, 32, 4, 49), (3, 32, 4, 600), (26, 32, 4, 64)):
         for keys, want in ((4095, False), (4096, True), (4097, True), (131072, True)):
             assert plan(b, b, hq, hkv, keys - s, s)[:3] == ("pingpong", 0, 1)
             assert direct(b, b, hq, hkv, keys - s, s) == want, (b, hq, hkv, s, keys)
     assert plan(1, 1, 32, 4, 8192, 64)[0] == "pingpong" and plan(1, 1, 32, 4, 8192, 64)[2] > 1 and not direct(1, 1, 32, 4, 8192, 64)
     assert plan(24, 24, 32, 4, 8191, 13)[0] == "stream" and not direct(24, 24, 32, 4, 8191, 13)
+
+
+def test_walks_of_129_to_192_workgroups_are_cut_in_two_where_that_is_faster():
+    """Five of eight units of a shader engine busy: the second pieces run in two rounds on the other three; six:
+    in three rounds on two.  Not where the partial rows cost more than that gives, nor with most units busy."""
+    plan = plan_probe.chunk_plan
+    for s, p0, pieces in ((1030, 4100, 2), (1030, 30000, 2), (1167, 12000, 2), (1344, 4100, 2), (1344, 12000, 2), (1536, 12000, 2),
+                          (1536, 4100, 2),
+                          (1030, 1000, 1), (1480, 2000, 1), (1537, 30000, 1)):
+        assert plan(1, 1, 32, 4, p0, s)[:3] == ("pingpong", 0, pieces), (s, p0)
+    assert plan(18, 18, 32, 4, 4096, 64)[2] == 1 and plan(18, 18, 32, 4, 8192, 64)[2] == 2    # 99 us against 96, 184 against 190
+    assert plan(1, 1, 64, 8, 4100, 660)[2] == 1 and plan(1, 1, 64, 8, 12000, 660)[2] == 2     # 111 against 109, 262 against 272
+    assert plan(1, 1, 8, 1, 0, 5000)[2] == 2
+    assert plan(40, 1, 32, 4, 12000, 1536, most=1536)[2] == 1                                 # no room for the partial rows

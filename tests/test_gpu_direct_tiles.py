@@ -14,8 +14,8 @@ from test_gpu_tile_reference import LEVELS
 pytestmark = pytest.mark.gpu
 
 # (sequences, query heads, key-value heads, tokens, position of the first)
-SHAPES = {"last_tile_of_1": (17, 64, 1, 7, 4090), "whole_tiles": (17, 64, 1, 9, 4087), "two_row_blocks": (17, 32, 4, 49, 4060),
-          "chunk_of_600": (2, 32, 4, 600, 4060)}
+SHAPES = {"last_tile_of_1": (25, 64, 1, 7, 4090), "whole_tiles": (25, 64, 1, 9, 4087), "two_row_blocks": (25, 32, 4, 49, 4060),
+          "chunk_of_600": (3, 32, 4, 600, 4060)}
 
 
 def _shape(name):

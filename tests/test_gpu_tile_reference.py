@@ -51,7 +51,7 @@ def test_scores_that_outgrow_the_reference(b, hq, hkv, s, p0, want_kernel, split
 
 
 @pytest.mark.parametrize("b,hq,hkv,s,p0,want_kernel,split", [
-    (16, 32, 4, 49, 200, "pingpong", False), (2, 32, 4, 600, 4060, "pingpong", False), (1, 8, 1, 70, 2400, "pingpong", True),
+    (16, 32, 4, 49, 200, "pingpong", False), (3, 32, 4, 600, 4060, "pingpong", False), (1, 8, 1, 70, 2400, "pingpong", True),
     (300, 8, 1, 13, 520, "stream", False), (2, 8, 1, 13, 2400, "stream", True), (2, 8, 1, 45, 2400, "stream", True)],
     ids=["whole", "whole_4660_keys", "split", "stream_whole", "stream_13", "stream_45"])
 @pytest.mark.parametrize("rise", [7.5, 14.0])
