@@ -176,20 +176,37 @@ constexpr uint32_t kPingpongRowBlocks = 8;  // 32-row blocks of a ping-pong work
 // layer of 64 x 24 on 4096 189 / 181-187, 3140 x 3, 32 / 32 heads 284 / 282; but 412 x 19, 32 / 32 heads, 103 / 108,
 // 519 x 3 36 / 38, 120 x 8 on 1400 57 / 59-65; 255 on 11150 in splits 55.3 / 55.3.
 constexpr uint32_t kDirectKeys = 64 * kChunkTile;
+// Other walks of the ping-pong kernel run on 32x32x16 instructions while the units are busy for at most this share of
+// the longest walk or piece (then the board's power does not set the time) and the XCDs' L2s serve K and V.  16x16x32
+// / 32x32x16, us:
+//   bf16  busy 0.53 (1030 tokens on 1400, 32 / 4 heads) 59.9 / 54.8   0.57 (1536 on 1400) 72.5 / 71.3   0.58 (2048 on 300)
+//         61.3 / 60.3   0.64 (2048 on 700) 73.2 / 73.2   0.67 (2048 on 1400) 92.2 / 93.2
+//   f16   0.48 (900 tokens, 64 / 8 heads) 29.2 / 27.8   0.53 (600 on 2000) 63.6 / 62.3   0.55 (700 on 1000) 46.2 / 46.1   0.60
+//         (768 on 1400) 57.5 / 58.5   0.67 (900 on 2000) 82.4 / 85.4
+//   split: 2000 / 3000 / 4000 tokens, 8 / 1 heads, f16 32.5 / 31.3, 45.0 / 42.3, 61.0 / 57.1; 0.59 (300 on 2000,
+//         32 / 4) 31.0 / 30.0   0.86 (300 on 3000) 32.6 / 33.1
+//   K and V of 70 MB (250 x 5 on 600, 32 / 32 heads, f16) 34.2 / 37.0; of 49 MB (64 x 19 on 1200, bf16) 37.6 / 36.0; of 41 MB
+//         (64 x 19 on 1000, f16) 33.9 / 34.5
+constexpr double kWideBusy = 0.6, kWideBusyF16 = 0.55;   // (bfloat16 and splits; unsplit binary16)
+constexpr double kWideMbBf16 = 56.0, kWideMbF16 = 32.0;
 
 struct ChunkCall {
   uint32_t p0, interval;                    // positions p0 .. p0 + interval - 1
   uint32_t batch, batch_capacity, n_q_heads, n_kv_heads, n_cu;
   size_t part_rows;                         // partial rows the workspace holds (0: none)
+  bool bf16;                                // storage: bfloat16, else binary16
 };
 
 enum ChunkKernel { kChunkStream, kChunkPingpong, kChunkShort };
+// Forms of the ping-pong kernel: 16x16x32 instructions with tiles through registers or straight into LDS;
+// 32x32x16 instructions
+enum PingpongForm { kPingpongRegisters, kPingpongDirect, kPingpongWide };
 
 struct ChunkPlan {
   ChunkKernel kernel;
   uint32_t waves;                           // streaming kernel: 4, 8 or 12
   uint32_t row_blocks;                      // short-prompt kernel: 32-row blocks a workgroup, 1 or 2
-  bool direct;                              // ping-pong kernel: tiles straight into LDS
+  PingpongForm form;                        // ping-pong kernel
   uint32_t n_split, split_tiles;            // key range of a plane, in tiles (one split: split_tiles may be 0)
   // ping-pong workgroup: heads_per_wg heads of a group x tblocks_per_wg blocks of 32 tokens
   uint32_t heads_per_wg, tblocks_per_wg, head_groups;
@@ -334,7 +351,15 @@ inline ChunkPlan plan_chunk(const ChunkCall& c) {
   const double margin = all_tiles > 24 ? 0.82 : 0.87;
   if (const uint32_t wr = short_prompt_wr(shape, pingpong_us(shape, base, {p.split_tiles, p.n_split}), margin))
     plan_short_prompt(shape, wr, &p);
-  p.direct = p.kernel == kChunkPingpong && p.n_split == 1 && c.p0 + c.interval >= kDirectKeys;
+  if (p.kernel == kChunkPingpong) {
+    const uint32_t longest = p.n_split > 1 ? p.split_tiles : all_tiles;
+    const double busy = base * ((c.p0 + 0.5 * c.interval) / kChunkTile + 0.5) / ((double)c.n_cu * longest);
+    if (p.n_split == 1 && c.p0 + c.interval >= kDirectKeys)
+      p.form = kPingpongDirect;
+    else if (base <= c.n_cu && busy <= (c.bf16 || p.n_split > 1 ? kWideBusy : kWideBusyF16) &&
+             planes * shape.keys() * 512e-6 <= (c.bf16 ? kWideMbBf16 : kWideMbF16))
+      p.form = kPingpongWide;
+  }
   return p;
 }
 

@@ -125,6 +125,7 @@ typedef __attribute__((address_space(3))) i16x4 LdsI16x4;
 // transposing read touches (32 B of each) fall into disjoint banks
 constexpr int kVsPitch = kHeadDim + 16;
 constexpr int kVsHalves = kBK * kVsPitch;
+constexpr int kKsHalves = kBK * kKsPitch;
 constexpr int kPpWaves = 8;
 constexpr int kPpThreads = kPpWaves * kWave;
 constexpr int kLdsAhead = 8;   // LDS operand reads in flight ahead of their MFMA
@@ -540,6 +541,290 @@ __global__ __launch_bounds__(kPpThreads, 2) void prefill_pingpong_kernel(Prefill
         p.lse[((size_t)tok * p.batch_pitch + seq) * p.n_q_heads + head] =
             (m + fast_log2(l)) * kLn2;
     }
+  }
+}
+
+// ---------------------------------------------------------------------------
+// The same kernel on 32x32x16 instructions, tiles through registers and a row maximum every tile: a wave owns its 32
+// rows as one block, lane (j, g) row j and half g of the keys.  For unsplit walks that leave a quarter of the units
+// idle: there the board's power holds nothing back, and a phase is shorter where the matrix instructions leave the
+// vector phase of the other wave more of the issue (5.6 clocks an instruction against 8.2).  Phases, buffers, prefetch
+// ring and scheduling barriers are those of the kernel above.
+// 16x16x32 form / this one (us, in turn on one board): 1030 tokens on 1000, 32 / 4 heads, bf16 52.0 / 48.0, 1200 on 1400
+// 64.0 / 58.8, 1480 tokens 41.0 / 37.9; 520 on 2000, 64 / 8, f16 62.2 / 56.8; 120 x 9 on 1200, 32 / 4, bf16 38.4 / 36.0.
+// ---------------------------------------------------------------------------
+template <typename T, bool SPLIT>
+__global__ __launch_bounds__(kPpThreads, 2) void prefill_pingpong32_kernel(PrefillKernelArgs p) {
+  // K tiles [2][64][kKsPitch] then V tiles [3][64][kVsPitch]
+  __shared__ __attribute__((aligned(16))) uint16_t smem[2 * kKsHalves + 3 * kVsHalves];
+
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = tid >> 6;
+  const int j = lane & 31, g = lane >> 5;
+  const int grp = wave >> 2;  // 0: waves 0-3, 1: waves 4-7
+
+  uint32_t combo, order;
+  if (p.xcd_mode) {
+    const uint32_t xcd = blockIdx.x & 7, slot = blockIdx.x >> 3;
+    const uint32_t per = 8 / p.combos;
+    combo = xcd % p.combos;
+    order = slot * per + xcd / p.combos;
+  } else {
+    combo = blockIdx.x % p.combos;
+    order = blockIdx.x / p.combos;
+  }
+  if (order >= p.n_wg_tokens) return;
+  const uint32_t wg_tok = p.n_wg_tokens - 1 - order;
+  const uint32_t seq = combo / (p.n_kv_heads * p.head_groups);
+  const uint32_t kvh = (combo / p.head_groups) % p.n_kv_heads;
+  const uint32_t hgrp = combo % p.head_groups;
+  const uint32_t t_base = wg_tok * 32 * p.tblocks_per_wg;
+  const uint32_t S = p.interval, P0 = p.position_index;
+  const uint32_t wg_last_tok = min(S, t_base + 32 * p.tblocks_per_wg) - 1;
+  const uint32_t kmax = P0 + wg_last_tok;
+  const uint32_t all_tiles = kmax / kBK + 1;
+  const uint32_t kt0 = SPLIT ? blockIdx.y * p.split_tiles : 0u;
+  if (SPLIT && kt0 >= all_tiles) return;  // (prefill_merge_kernel derives the live splits the same way)
+  const uint32_t n_tiles = SPLIT ? min(all_tiles - kt0, p.split_tiles) : all_tiles;
+
+  const uint32_t hg = wave % p.heads_per_wg, tb = wave / p.heads_per_wg;
+  const uint32_t head = kvh * p.group + hgrp * p.heads_per_wg + hg;
+  const uint32_t tok0 = t_base + 32 * tb;
+  const uint32_t tok = min(tok0 + j, S - 1);
+  const bool row_valid = tok0 + j < S;
+  const uint32_t rowpos = P0 + tok;
+  const uint32_t first_pos = P0 + min(tok0, S - 1);  // lowest position in this row block
+
+  u32x4 qreg[8];
+  {
+    const uint16_t* qrow =
+        p.q + (size_t)tok * p.q_token_stride + ((size_t)seq * p.n_q_heads + head) * kHeadDim;
+#pragma unroll
+    for (int s = 0; s < 8; ++s) {
+      qreg[s] = load16(qrow + 16 * s + 8 * g);
+      if (p.negate_q) qreg[s] ^= 0x80008000u;
+    }
+  }
+  const float c = p.c;
+
+  const size_t plane_at = seq_plane_offset(p.seq_offsets, p.kv_stride_seq, seq) + kvh * p.kv_stride_head;
+  const uint16_t* kplane = p.k + plane_at;
+  const uint16_t* vplane = p.v + plane_at;
+
+  const int st_tid = tid & 255;
+  const int ld_c = st_tid & 15, ld_r = st_tid >> 4;
+  const uint16_t* plane = grp ? vplane : kplane;                  // wave-uniform
+  const uint32_t stride_pos = (uint32_t)p.kv_stride_pos;
+  const uint64_t plane_u = uniform64(plane);
+  const uint32_t tile_bytes = kBK * stride_pos * 2;   // (API bound: 64 rows span < 2^32 bytes)
+  const uint64_t valid_bytes = uniform_u64(((uint64_t)kmax * stride_pos + kHeadDim) * 2);
+  uint32_t piece_off[4];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) piece_off[i] = ((ld_r + 16 * i) * stride_pos + 8 * ld_c) * 2;
+  const uint32_t lds0 = (uint32_t)(uintptr_t)(LdsHalf*)smem;
+  auto step_base = [](uint32_t addr) {
+    asm volatile("" : "+v"(addr));  // opaque: keeps the compiler from folding the sum another way
+    return addr;
+  };
+  const uint32_t ks_store = lds0 + 2 * (ld_r * kKsPitch + 8 * ld_c);
+  const uint32_t vs_store = lds0 + 2 * (2 * kKsHalves + ld_r * kVsPitch + 8 * ld_c);
+  u32x4 stg[4];
+  auto load_piece = [&](uint32_t kt, int i) {  // kt (relative to kt0) must be wave-uniform to the compiler
+    const uint64_t off = (uint64_t)(kt0 + kt) * tile_bytes;
+    const uint32_t left = bytes_left(valid_bytes, off);
+    const __amdgpu_buffer_rsrc_t rsrc =
+        __builtin_amdgcn_make_buffer_rsrc((void*)(plane_u + off), 0, left, kBufferFlags);
+    stg[i] = __builtin_amdgcn_raw_buffer_load_b128(rsrc, piece_off[i], 0, 0);
+  };
+  auto store_piece = [&](auto group, uint32_t base, int i) {
+    *(LdsU32x4*)(base + 2 * 16 * i * (group ? kVsPitch : kKsPitch)) = stg[i];
+  };
+  auto load_tile = [&](uint32_t kt) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) load_piece(kt, i);
+  };
+  auto store_base = [&](auto group, int buf) {
+    return step_base(group ? vs_store + 2 * buf * kVsHalves : ks_store + 2 * buf * kKsHalves);
+  };
+  auto store_tile = [&](int buf) {
+    const uint32_t base = store_base(grp, buf);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) store_piece(grp, base, i);
+  };
+
+  float m_run = -INFINITY, l_run = 0.0f;
+  f32x16 oacc[4];
+#pragma unroll
+  for (int db = 0; db < 4; ++db)
+#pragma unroll
+    for (int r = 0; r < 16; ++r) oacc[db][r] = 0.0f;
+  f32x16 st[2];
+  u32x4 pk[4];
+#pragma unroll
+  for (int cc = 0; cc < 4; ++cc) pk[cc] = u32x4{0u, 0u, 0u, 0u};  // P(-1) = 0
+
+  if (grp) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) stg[i] = u32x4{0u, 0u, 0u, 0u};
+    store_tile(2);
+  }
+  load_tile(0);
+  store_tile(0);
+  load_tile(1);
+  __syncthreads();
+
+  // A operand of P.V (rows = 32 dims, 16 keys): lane (dim j, key half g) holds keys {4g..4g+3, 8+4g..8+4g+3} of the
+  // 16, in two transposing reads (keys +0 and +8).
+  const uint32_t k_read = lds0 + 2 * (j * kKsPitch + 8 * g);
+  const uint32_t v_read = lds0 + 2 * (2 * kKsHalves + (4 * g + ((lane & 15) >> 2)) * kVsPitch +
+                                      16 * ((lane >> 4) & 1) + 4 * (lane & 3));
+  auto mod3 = [](uint32_t x) { return x % 3u; };
+  auto stream_operand = [&](uint32_t ks, uint32_t vs, int n) {
+    const int i = n >> 1;
+    if (n & 1) {  // K rows: i = 2 s + mb
+      const int s = i >> 1, mb = i & 1;
+      return (u32x4) * (const LdsU32x4*)(ks + 2 * (32 * mb * kKsPitch + 16 * s));
+    }
+    // V: i = 4 cc + db, keys 16 cc.., dims 32 db..
+    const int cc = i >> 2, db = i & 3;
+    const uint32_t at = vs + 2 * (16 * cc * kVsPitch + 32 * db);
+    const i16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((LdsI16x4*)at);
+    const i16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((LdsI16x4*)(at + 2 * 8 * kVsPitch));
+    const u32x2 l2 = __builtin_bit_cast(u32x2, lo), h2 = __builtin_bit_cast(u32x2, hi);
+    return u32x4{l2[0], l2[1], h2[0], h2[1]};
+  };
+  u32x4 ring[kLdsAhead];
+  auto prefetch_ring = [&](uint32_t kt) __attribute__((always_inline)) {
+    const uint32_t ks = step_base(k_read + 2 * (kt & 1) * kKsHalves);
+    const uint32_t vs = step_base(v_read + 2 * mod3(kt + 2) * kVsHalves);  // V(kt-1)
+#pragma unroll
+    for (int n = 0; n < kLdsAhead; ++n) ring[n] = stream_operand(ks, vs, n);
+  };
+  auto matrix_step = [&](auto group, uint32_t kt) __attribute__((always_inline)) {
+    const uint32_t ks = step_base(k_read + 2 * (kt & 1) * kKsHalves);
+    const uint32_t vs = step_base(v_read + 2 * mod3(kt + 2) * kVsHalves);
+    const uint32_t store_at = store_base(group, group ? (int)mod3(kt + 1) : (int)((kt + 1) & 1));
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int n = 0; n < 32; ++n) {
+      const int i = n >> 1;
+      if (n & 1) {
+        const int s = i >> 1, mb = i & 1;
+        if (s == 0) {
+          f32x16 z;
+#pragma unroll
+          for (int r = 0; r < 16; ++r) z[r] = 0.0f;
+          st[mb] = Mfma<T>::m32x32x16(ring[n % kLdsAhead], qreg[s], z);
+        } else {
+          st[mb] = Mfma<T>::m32x32x16(ring[n % kLdsAhead], qreg[s], st[mb]);
+        }
+      } else {
+        oacc[i & 3] = Mfma<T>::m32x32x16(ring[n % kLdsAhead], pk[i >> 2], oacc[i & 3]);
+      }
+      if (n + kLdsAhead < 32) ring[n % kLdsAhead] = stream_operand(ks, vs, n + kLdsAhead);
+      if (n >= 24 && n < 28) store_piece(group, store_at, n - 24);
+      if (n >= 28 && n < 32) load_piece(kt + 2, n - 28);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
+  };
+
+  // mask on the diagonal, row maximum, rescaling of O^T where it passed the step, exponentials, packing, row sum
+  auto vector_step = [&](uint32_t kt) __attribute__((always_inline)) {
+    const uint32_t kb = (kt0 + kt) * kBK;
+    if (kb + kBK - 1 > first_pos) {  // tile crosses this row block's diagonal
+#pragma unroll
+      for (int mb = 0; mb < 2; ++mb)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+          const uint32_t key = kb + 32 * mb + 8 * (r >> 2) + 4 * g + (r & 3);
+          st[mb][r] = (key <= rowpos) ? st[mb][r] : -INFINITY;
+        }
+    }
+    float rmax = st[0][0];
+#pragma unroll
+    for (int mb = 0; mb < 2; ++mb)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) rmax = fmaxf(rmax, st[mb][r]);
+    rmax = max_with_partner_half(rmax);
+    const float tmax = rmax * c;
+    const bool grow = tmax > m_run + kRescaleStep;
+    if (__any(grow)) {
+      const float m_new = grow ? tmax : m_run;
+      const float alpha = grow ? fast_exp2(m_run - m_new) : 1.0f;
+      m_run = m_new;
+      l_run *= alpha;
+#pragma unroll
+      for (int db = 0; db < 4; ++db) oacc[db] *= alpha;
+    }
+    const float neg_m = (m_run == -INFINITY) ? 0.0f : -m_run;
+    float psum = 0.0f;
+#pragma unroll
+    for (int cc = 0; cc < 4; ++cc) {
+      const int mb = cc >> 1, r0 = 8 * (cc & 1);
+#pragma unroll
+      for (int w = 0; w < 4; ++w) {
+        const float p0 = fast_exp2(__builtin_fmaf(st[mb][r0 + 2 * w], c, neg_m));
+        const float p1 = fast_exp2(__builtin_fmaf(st[mb][r0 + 2 * w + 1], c, neg_m));
+        pk[cc][w] = Mfma<T>::pack2(p0, p1);
+        psum += p0 + p1;
+      }
+    }
+    l_run += psum;
+  };
+
+  constexpr std::integral_constant<int, 0> kGroup0;
+  constexpr std::integral_constant<int, 1> kGroup1;
+  if (__builtin_amdgcn_readfirstlane(grp) == 0) {
+    prefetch_ring(0);
+    matrix_step(kGroup0, 0);
+    __builtin_amdgcn_s_barrier();
+    for (uint32_t kt = 0; kt < n_tiles; ++kt) {
+      vector_step(kt);
+      prefetch_ring(kt + 1);
+      __builtin_amdgcn_s_barrier();
+      matrix_step(kGroup0, kt + 1);
+      __builtin_amdgcn_s_barrier();
+    }
+  } else {
+    prefetch_ring(0);
+    __builtin_amdgcn_s_barrier();
+    for (uint32_t kt = 0; kt < n_tiles; ++kt) {
+      matrix_step(kGroup1, kt);
+      __builtin_amdgcn_s_barrier();
+      vector_step(kt);
+      prefetch_ring(kt + 1);
+      __builtin_amdgcn_s_barrier();
+    }
+    matrix_step(kGroup1, n_tiles);
+  }
+
+  const float l = sum_with_partner_half(l_run);
+  if (!row_valid) return;
+  if constexpr (SPLIT) {
+    const size_t part = (((size_t)tok * p.batch_pitch + seq) * p.n_q_heads + head) * p.n_split + blockIdx.y;
+    float* orow = p.part_o + part * kHeadDim;
+#pragma unroll
+    for (int db = 0; db < 4; ++db)
+#pragma unroll
+      for (int q4 = 0; q4 < 4; ++q4)
+        *(f32x4*)(orow + 32 * db + 8 * q4 + 4 * g) =
+            f32x4{oacc[db][4 * q4], oacc[db][4 * q4 + 1], oacc[db][4 * q4 + 2], oacc[db][4 * q4 + 3]};
+    if (g == 0) *(float2*)(p.part_ml + part * 2) = float2{m_run, l};
+  } else {
+    const float inv = 1.0f / l;
+    uint16_t* orow = p.out + (size_t)tok * p.q_token_stride + ((size_t)seq * p.n_q_heads + head) * kHeadDim;
+#pragma unroll
+    for (int db = 0; db < 4; ++db)
+#pragma unroll
+      for (int q4 = 0; q4 < 4; ++q4) {
+        u32x2 w;
+        w[0] = Mfma<T>::pack2(oacc[db][4 * q4] * inv, oacc[db][4 * q4 + 1] * inv);
+        w[1] = Mfma<T>::pack2(oacc[db][4 * q4 + 2] * inv, oacc[db][4 * q4 + 3] * inv);
+        *(u32x2*)(orow + 32 * db + 8 * q4 + 4 * g) = w;
+      }
+    if (p.lse && g == 0)
+      p.lse[((size_t)tok * p.batch_pitch + seq) * p.n_q_heads + head] = (m_run + fast_log2(l)) * kLn2;
   }
 }
 
@@ -1110,6 +1395,7 @@ hipError_t launch_chunk(const AttnArgs& a, hipStream_t stream) {
   call.n_q_heads = a.n_q_heads;
   call.n_kv_heads = a.n_kv_heads;
   call.n_cu = a.n_cu;
+  call.bf16 = a.dtype != 0;
   call.part_rows = a.prefill_part_o ? a.prefill_part_rows : 0;
   const ChunkPlan plan = plan_chunk(call);
 
@@ -1161,10 +1447,14 @@ hipError_t launch_chunk(const AttnArgs& a, hipStream_t stream) {
     else
       go(chunk_stream_kernel<T, 12>, 12 * kWave);
   } else if (plan.n_split == 1) {
-    if (plan.direct)
+    if (plan.form == kPingpongDirect)
       go(prefill_pingpong_kernel<T, false, true>, kPpThreads);
+    else if (plan.form == kPingpongWide)
+      go(prefill_pingpong32_kernel<T, false>, kPpThreads);
     else
       go(prefill_pingpong_kernel<T, false, false>, kPpThreads);
+  } else if (plan.form == kPingpongWide) {
+    go(prefill_pingpong32_kernel<T, true>, kPpThreads);
   } else {
     go(prefill_pingpong_kernel<T, true, false>, kPpThreads);
   }

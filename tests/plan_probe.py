@@ -16,13 +16,13 @@ SOURCE = r"""
 #include <cstdlib>
 #include "general_plan.hpp"
 using namespace ellm;
-static int chunk(char** v) {   // batch capacity, batch, query heads, key-value heads, most positions a call, position_index, interval
-  uint32_t a[8];
-  for (int i = 1; i <= 7; ++i) a[i] = (uint32_t)strtoul(v[i + 1], nullptr, 10);
-  const ChunkCall c = {a[6], a[7], a[2], a[1], a[3], a[4], 256, prefill_workspace_rows(a[5], a[1], a[3], 256)};
+static int chunk(char** v) {   // batch capacity, batch, query heads, key-value heads, most positions a call, position_index, interval, bfloat16
+  uint32_t a[9];
+  for (int i = 1; i <= 8; ++i) a[i] = (uint32_t)strtoul(v[i + 1], nullptr, 10);
+  const ChunkCall c = {a[6], a[7], a[2], a[1], a[3], a[4], 256, prefill_workspace_rows(a[5], a[1], a[3], 256), a[8] != 0};
   const ChunkPlan p = plan_chunk(c);
   printf("%d %u %u %u %d\n", (int)p.kernel, p.kernel == kChunkStream ? p.waves : p.kernel == kChunkShort ? p.row_blocks : 0, p.n_split, p.n_wg,
-         (int)p.direct);
+         (int)p.form);
   return 0;
 }
 // head size, bytes an element, batch capacity, batch, query heads, key-value heads, most positions a call,
@@ -72,8 +72,8 @@ def general_plan(head_size, element_bytes, batch_capacity, batch, q_heads, kv_he
     return (("rows", "step", "chunk")[int(out[0])], *map(int, out[1:]))
 
 
-def _chunk(batch_capacity, batch, q_heads, kv_heads, position_index, interval, most=None):
-    args = ("c", batch_capacity, batch, q_heads, kv_heads, most or interval, position_index, interval)
+def _chunk(batch_capacity, batch, q_heads, kv_heads, position_index, interval, most=None, bf16=False):
+    args = ("c", batch_capacity, batch, q_heads, kv_heads, most or interval, position_index, interval, int(bf16))
     return subprocess.run([_program(), *map(str, args)], check=True, capture_output=True, text=True).stdout.split()
 
 
@@ -84,6 +84,11 @@ def chunk_plan(*call, **most):
     return (("stream", "pingpong", "short")[int(out[0])], *map(int, out[1:4]))
 
 
-def chunk_is_direct(*call, **most):
-    """Whether the same call runs the tile kernel's form that fetches K and V straight into LDS."""
-    return _chunk(*call, **most)[4] == "1"
+def chunk_form(*call, **more):
+    """The form of the tile kernel that an unsplit call of it runs: "registers", "direct" or "wide"; for the last one
+    the storage type counts (bf16=True)."""
+    return ("registers", "direct", "wide")[int(_chunk(*call, **more)[4])]
+
+
+def chunk_is_direct(*call, **more):
+    return chunk_form(*call, **more) == "direct"

@@ -134,3 +134,18 @@ def test_walks_of_129_to_192_workgroups_are_cut_in_two_where_that_is_faster():
     assert plan(1, 1, 64, 8, 4100, 660)[2] == 1 and plan(1, 1, 64, 8, 12000, 660)[2] == 2     # 111 against 109, 262 against 272
     assert plan(1, 1, 8, 1, 0, 5000)[2] == 2
     assert plan(40, 1, 32, 4, 12000, 1536, most=1536)[2] == 1                                 # no room for the partial rows
+
+
+def test_short_walks_that_leave_units_idle_run_on_32x32x16():
+    form, plan = plan_probe.chunk_form, plan_probe.chunk_plan
+    for bf16, want in ((True, "wide"), (False, "registers")):
+        assert form(1, 1, 32, 4, 1400, 1536, bf16=bf16) == want                               # units busy for 0.57 of the time
+        assert form(19, 19, 32, 4, 1200, 64, bf16=bf16) == want                               # 49 MB of K and V
+    for bf16 in (True, False):
+        assert form(1, 1, 32, 4, 1000, 1200, bf16=bf16) == "wide"                             # 0.47
+        assert form(1, 1, 32, 4, 700, 2048, bf16=bf16) == "registers"                         # 0.64
+        assert form(22, 22, 32, 4, 2000, 64, bf16=bf16) == "registers"                        # 93 MB
+        assert form(1, 1, 32, 4, 4100, 1600, bf16=bf16) == "direct"
+        assert plan(1, 1, 8, 1, 0, 4000)[2] == 2 and form(1, 1, 8, 1, 0, 4000, bf16=bf16) == "wide"           # cut in two, 0.37
+        assert plan(1, 1, 32, 4, 2000, 300)[2] > 2 and form(1, 1, 32, 4, 2000, 300, bf16=bf16) == "wide"     # pieces of 9 tiles, 0.59
+        assert plan(1, 1, 32, 4, 6000, 300)[2] > 2 and form(1, 1, 32, 4, 6000, 300, bf16=bf16) == "registers"

@@ -1,7 +1,8 @@
 """The reference maximum of the tile kernel and the streaming chunk kernel: exponentials are taken against the one a row has until a lane's
 sum of them passes 2^15 (2^8 in bfloat16), then the row's true maximum is looked for and its sums are rescaled.  Score
 levels that stay below that step, pass it once, again and again, fall back and pass it in some rows of a
-block only; whole rows and a key range in splits, whose later splits some rows see nothing of."""
+block only; whole rows and a key range in splits, whose later splits some rows see nothing of, both on 32x32x16 instructions
+("whole", "split") and on 16x16x32."""
 import math
 
 import numpy as np
@@ -20,14 +21,17 @@ LEVELS = {"below": [0, 13, 14, 12], "once": [0, 0, 17, 17], "rising": [0, 16, 40
 
 
 @pytest.mark.parametrize("b,hq,hkv,s,p0,want_kernel,split", [
-    (16, 32, 4, 49, 200, "pingpong", False), (1, 8, 1, 70, 2400, "pingpong", True), (2, 8, 1, 13, 2400, "stream", True),
-    (2, 8, 1, 45, 2400, "stream", True)], ids=["whole", "split", "stream_13", "stream_45"])
+    (16, 32, 4, 49, 200, "pingpong", False), (26, 32, 4, 49, 200, "pingpong", False), (1, 8, 1, 70, 2400, "pingpong", True),
+    (16, 32, 1, 13, 2600, "pingpong", True), (2, 8, 1, 13, 2400, "stream", True), (2, 8, 1, 45, 2400, "stream", True)],
+    ids=["whole", "whole_26", "split", "split_16", "stream_13", "stream_45"])
 @pytest.mark.parametrize("name", LEVELS)
 @pytest.mark.parametrize("dtype", [orc.F16, orc.BF16], ids=["f16", "bf16"])
 def test_scores_that_outgrow_the_reference(b, hq, hkv, s, p0, want_kernel, split, name, dtype):
     cap = p0 + s
     kernel, _, n_split = plan_probe.chunk_plan(b, b, hq, hkv, p0, s)[:3]
     assert kernel == want_kernel and (n_split > 1) == split
+    if kernel == "pingpong":
+        assert plan_probe.chunk_form(b, b, hq, hkv, p0, s) == ("wide" if p0 + s == 249 and b == 16 or b == 1 else "registers")
     scale = 1.0 / math.sqrt(D)
     q = orc.from_storage(rand_storage((s, b, hq, D), 5, dtype), dtype)
     k = orc.from_storage(rand_storage((b, hkv, cap, D), 6, dtype), dtype)
@@ -51,9 +55,9 @@ def test_scores_that_outgrow_the_reference(b, hq, hkv, s, p0, want_kernel, split
 
 
 @pytest.mark.parametrize("b,hq,hkv,s,p0,want_kernel,split", [
-    (16, 32, 4, 49, 200, "pingpong", False), (3, 32, 4, 600, 4060, "pingpong", False), (1, 8, 1, 70, 2400, "pingpong", True),
-    (300, 8, 1, 13, 520, "stream", False), (2, 8, 1, 13, 2400, "stream", True), (2, 8, 1, 45, 2400, "stream", True)],
-    ids=["whole", "whole_4660_keys", "split", "stream_whole", "stream_13", "stream_45"])
+    (16, 32, 4, 49, 200, "pingpong", False), (26, 32, 4, 49, 200, "pingpong", False), (3, 32, 4, 600, 4060, "pingpong", False), (1, 8, 1, 70, 2400, "pingpong", True),
+    (16, 32, 1, 13, 2600, "pingpong", True), (300, 8, 1, 13, 520, "stream", False), (2, 8, 1, 13, 2400, "stream", True), (2, 8, 1, 45, 2400, "stream", True)],
+    ids=["whole", "whole_26", "whole_4660_keys", "split", "split_16", "stream_whole", "stream_13", "stream_45"])
 @pytest.mark.parametrize("rise", [7.5, 14.0])
 def test_large_bfloat16_values_under_rising_scores(b, hq, hkv, s, p0, want_kernel, split, rise):
     """A value of 2^115 under the one score that lies 7.5 or 14 binary orders above those before it, in another
