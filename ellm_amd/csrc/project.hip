@@ -86,7 +86,9 @@ static uint32_t g_n_cu = 256;
 // whose traffic per flop is the lowest.  Measured on 256 compute units for 2048 -> 5120 (us, 128-token / 256-token /
 // 256 x 256 tiles): 640 rows 20 / 25 / 46, 1024 rows 36 / 28 / 46, 1536 rows 42 / 32 / 47, 2048 rows 58 / 53 / 49.
 // Where the 256 x 256 tiles would leave two fifths of the units without one and two rounds of 128-token
-// tiles suffice, those are faster still: 4096 -> 12288, 640 rows (480 of them, 144 of 256 x 256) 69 / 91 / 85.
+// tiles suffice, those are faster still (256 x 256 / 128-token tiles, bf16, us): 640 rows 4096 -> 12288 80 / 65, 520 rows
+// 79 / 62, 600 rows 2048 -> 12288 45 / 37, 896 rows 7168 -> 9216 132 / 109, 1152 rows 4096 -> 7168 80 / 66, 300 rows 8192
+// -> 18432 149 / 122, 384 rows 152 / 141 (thirteen such shapes, 1.08 to 1.28).
 int project_path(uint32_t rows, uint32_t heads, uint32_t K, bool has_workspace) {
   if (has_workspace && small_kernel_takes(rows, K)) return kPathFewRows;
   if (((rows + 127) / 128) * heads <= g_n_cu) return kPathTiles128;

@@ -55,27 +55,16 @@ __device__ __forceinline__ uint64_t from_lane(uint64_t v, int from) {
   return ((uint64_t)hi << 32) | lo;
 }
 
-// The residual rows of the 128-token-a-wave tiles (thousands of rows a call, each piece read by
-// one workgroup) are marked non-temporal: 1.5 % on 32768 rows; with the smaller tiles' few
-// hundred rows, which their producer may have left in a cache, the mark cost 1 %.
-template <int MODE, int MB>
-constexpr bool kStreamedResidual = MODE == kModeAdd && MB >= 4;
-
 // Rows lane / 16 + 4 i, i = 0..7, of the extra operand of one token block; rows without one
-// read as (1, 0) pairs.  ONCE: rows nobody reads again, marked non-temporal.
-template <typename S, bool ONCE>
+// read as (1, 0) pairs.
+template <typename S>
 __device__ __forceinline__ void fetch_ext_rows(const uint16_t* my_row, int lane, u32x4 (&v)[8]) {
   const uint32_t one_zero = Mfma<S>::pack2(1.0f, 0.0f);
 #pragma unroll
   for (int i = 0; i < 8; ++i) {
     const uint64_t row = from_lane((uint64_t)my_row, 4 * i + (lane >> 4));
     v[i] = u32x4{one_zero, one_zero, one_zero, one_zero};
-    if (row) {
-      if constexpr (ONCE)
-        v[i] = __builtin_nontemporal_load((const GlobalVec4*)(row + 16 * (lane & 15)));
-      else
-        v[i] = *(const GlobalVec4*)(row + 16 * (lane & 15));
-    }
+    if (row) v[i] = *(const GlobalVec4*)(row + 16 * (lane & 15));
   }
 }
 
@@ -111,7 +100,7 @@ __device__ __forceinline__ HeadRows<MB> prepare_head(const ProjectKernelArgs& p,
         h.ext_row[mb] = p.rope + (size_t)pos * p.rope_pos_stride + (size_t)hs * p.rope_head_stride;
     }
   }
-  fetch_ext_rows<S, kStreamedResidual<MODE, MB>>(h.ext_row[0], lane, h.ext0);
+  fetch_ext_rows<S>(h.ext_row[0], lane, h.ext0);
   return h;
 }
 
@@ -137,7 +126,7 @@ __device__ __forceinline__ void finish_head(const ProjectKernelArgs& p, f32x4 (&
   auto stage_ext = [&](int next) __attribute__((always_inline)) {
 #pragma unroll
     for (int i = 0; i < 8; ++i) *(LdsVec4*)(ep_ext + row_piece + 4 * i * kEpPitch) = raw[i];
-    if (next < MB) fetch_ext_rows<S, kStreamedResidual<MODE, MB>>(h.ext_row[next < MB ? next : 0], lane, raw);
+    if (next < MB) fetch_ext_rows<S>(h.ext_row[next < MB ? next : 0], lane, raw);
   };
   stage_ext(1);
   static_for<MB>([&](auto mb_) {
