@@ -928,9 +928,9 @@ def cpu_baseline_ragged_decode(lengths, hq=32, hkv=4, sample_seqs=4, seed=19):
 
 
 def bench_mfma_stream(mode, dtype_name, n_cu, seconds=0.6, zeros=False, per_cu=1):
-    """What a pure stream of v_mfma_f32_32x32x16 sustains on N(0,1) operands on this box now
-    (libellm_diag.so: one wave per SIMD, four accumulators, no global memory access in the loop;
-    mode 0 register operands, mode 1 the A operand re-read from LDS for every MFMA, mode 2 the
+    """What a pure stream of v_mfma_f32_16x16x32 sustains on N(0,1) operands on this box now
+    (libellm_diag.so: one wave per SIMD, eight accumulators, no global memory access in the loop;
+    mode 0 register operands, mode 1 the A operand re-read from LDS for every two MFMAs, mode 2 the
     same plus the vector instructions of a soft-max of that tile shape in the same wave)."""
     import ctypes
 
@@ -949,7 +949,7 @@ def bench_mfma_stream(mode, dtype_name, n_cu, seconds=0.6, zeros=False, per_cu=1
     n_wg = n_cu * per_cu     # per_cu = 2: two waves per SIMD, so one wave's vector work overlaps the other's MFMAs
     sink = torch.zeros((n_wg * 256,), dtype=torch.float32, device="cuda")
     flops = ctypes.c_double()
-    iters = 4000      # 128000 MFMAs a wave: ~2.5 ms a launch
+    iters = 4000      # 256000 MFMAs a wave: ~2.5 ms a launch
     stream = ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
 
     def launch(_i):
@@ -1045,7 +1045,7 @@ def main():
                 "zero_kv": None if pf_zero is None else dict(pf_zero["power"] or {}, ms_per_step=round(pf_zero["ms_per_step"], 4),
                                                              tflops=round(pf_zero["tflops"], 1)),
             },
-            # pure v_mfma_f32_32x32x16_f16 streams on N(0,1) operands on every compute unit, timed in
+            # pure v_mfma_f32_16x16x32_f16 streams on N(0,1) operands on every compute unit, timed in
             # this run (libellm_diag.so): operands in registers / A operand from LDS / LDS-fed plus
             # the vector instructions of a soft-max of the same tile shape
             "mfma_stream_on_n01_fp16": {
