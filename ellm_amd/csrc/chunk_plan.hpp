@@ -313,10 +313,9 @@ inline ChunkPlan plan_chunk(const ChunkCall& c) {
   p.n_split = 1;
   p.split_tiles = 0;
   const uint32_t base = p.combos * p.n_wg_tokens;
-  // Only while the unsplit launch leaves at least half of the compute units idle: with more
-  // of them busy the part runs this kernel at its power limit, idle units or not, and a split
-  // only adds the partial rows (64 tokens x 24 sequences on 8192 keys, 192 workgroups: 229 us
-  // unsplit, 235 us as pieces of 97 + 32 tiles on all 256 units).
+  // This search only while the unsplit launch leaves at least half of the compute units idle: the more of them are
+  // busy, the less the board's power leaves for the others, and the partial rows are added (64 tokens x 24 sequences
+  // on 8192 keys, 192 workgroups: 229 us unsplit, 235 us as pieces of 97 + 32 tiles on all 256 units).
   if (c.part_rows && 2 * base <= c.n_cu && all_tiles >= 16) {
     // pieces of at least eight tiles (each pays the pipeline's first and last step); 1.9 us a
     // tile and workgroup (measured, 64 tokens x 24 sequences on 8192 keys)

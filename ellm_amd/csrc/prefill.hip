@@ -15,8 +15,8 @@
 // permutation of keys, the B layout the second MFMA wants; the V^T operand is read with the
 // same permutation, so P never leaves the lane that produced it and row max / row sum need one
 // or two cross-lane exchanges.
-// The tile kernel and the one for few rows run on 16x16x32 instructions, the one for short prompts on
-// 32x32x16: on N(0,1) operands a 256 x 256 x 64 loop of the former sustains 1620-1708 TFLOP/s and of the
+// The tile kernel and the one for few rows run on 16x16x32 instructions, the one for short prompts and the tile
+// kernel's form for calls that leave units idle on 32x32x16: on N(0,1) operands a 256 x 256 x 64 loop of the former sustains 1620-1708 TFLOP/s and of the
 // latter 1494-1543 (operands from LDS, nothing else in the loop; on zeros 2111 and 2438: fewer joules a
 // product, more instructions to issue).  What holds long calls back is the board's power; a short prompt is a
 // chain of latencies, 1 to 6 % longer on 16x16x32 (512 tokens, 32 / 32 heads 10.9 -> 11.0 us, 700 tokens, 64 / 8
