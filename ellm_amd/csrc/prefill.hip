@@ -546,8 +546,8 @@ __global__ __launch_bounds__(kPpThreads, 2) void prefill_pingpong_kernel(Prefill
 
 // ---------------------------------------------------------------------------
 // The same kernel on 32x32x16 instructions, tiles through registers and a row maximum every tile: a wave owns its 32
-// rows as one block, lane (j, g) row j and half g of the keys.  For unsplit walks that leave a quarter of the units
-// idle: there the board's power holds nothing back, and a phase is shorter where the matrix instructions leave the
+// rows as one block, lane (j, g) row j and half g of the keys.  For walks, whole or in splits, that leave units idle
+// (kWideBusy): there the board's power holds nothing back, and a phase is shorter where the matrix instructions leave the
 // vector phase of the other wave more of the issue (5.6 clocks an instruction against 8.2).  Phases, buffers, prefetch
 // ring and scheduling barriers are those of the kernel above.
 // 16x16x32 form / this one (us, in turn on one board): 1030 tokens on 1000, 32 / 4 heads, bf16 52.0 / 48.0, 1200 on 1400
