@@ -114,12 +114,15 @@ __device__ __forceinline__ uint64_t scalar64(uint64_t v) {  // tells the compile
 // that a step's loads are in flight together (element by element under the two bounds, each load was
 // waited for: 64 tokens x 2, 4 / 4 heads of 129, binary16 32 us); heads shorter than a piece by elements.
 constexpr uint32_t kNowhere = 0xf0000000u;
-constexpr uint64_t kMaxRecords = 0x80000000u;   // 64 rows of at most 2^25 bytes
+constexpr uint32_t kMaxRecords = 0x80000000u;   // 64 rows of at most 2^25 bytes
 
 __device__ __forceinline__ __amdgpu_buffer_rsrc_t chunk_rsrc(uint64_t plane, uint64_t off, uint64_t valid) {
-  const uint64_t left = valid > off ? valid - off : 0;
-  const uint32_t capped = (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)(left > kMaxRecords ? kMaxRecords : left));
-  return __builtin_amdgcn_make_buffer_rsrc((void*)(plane + off), 0, capped, 0x00020000);
+  // (both offsets below 2^63, told apart by the high word: the scalar unit has no ordered 64-bit compare)
+  const uint64_t left = valid - off;
+  const int32_t hi = (int32_t)(left >> 32);
+  const uint32_t lo = (uint32_t)left;
+  const uint32_t capped = hi < 0 ? 0u : hi > 0 || lo > kMaxRecords ? kMaxRecords : lo;
+  return __builtin_amdgcn_make_buffer_rsrc((void*)(plane + off), 0, (uint32_t)__builtin_amdgcn_readfirstlane((int)capped), 0x00020000);
 }
 
 template <typename S>
@@ -171,18 +174,17 @@ __device__ __forceinline__ u32x4 query_piece(const GeneralArgs& p, const typenam
   return w;
 }
 
-// Whether a piece holds an element with all exponent bits set (infinity or NaN).
+// Whether a piece holds an element with all exponent bits set (infinity or NaN): one more in the exponent's last
+// place carries into the sign's, and no further.
+template <typename S>
+__device__ __forceinline__ uint32_t exponent_carry(uint32_t x) {
+  constexpr uint32_t m = Store<S>::kExpMask;
+  return (x & m) + (m & ~(m << 1));
+}
 template <typename S>
 __device__ __forceinline__ bool piece_not_finite(u32x4 w) {
-  constexpr uint32_t m = Store<S>::kExpMask;
-  bool bad = false;
-#pragma unroll
-  for (int e = 0; e < 4; ++e) {
-    const uint32_t x = w[e] & m;
-    if constexpr (std::is_same<S, F32>::value) bad |= x == m;
-    else bad |= (x & 0xffffu) == (m & 0xffffu) || (x >> 16) == (m >> 16);
-  }
-  return bad;
+  constexpr uint32_t sign = std::is_same<S, F32>::value ? 0x80000000u : 0x80008000u;
+  return ((exponent_carry<S>(w[0]) | exponent_carry<S>(w[1]) | exponent_carry<S>(w[2]) | exponent_carry<S>(w[3])) & sign) != 0;
 }
 
 // Agent-scope accesses for partial rows that another workgroup of the same launch folds.

@@ -20,6 +20,10 @@
 // Measured, one group before: 2048 tokens, 32 query / 8 key-value heads of 64, bfloat16: 46.0 -> 41.9 us
 // (410 TFLOP/s); 341 tokens, 32 / 32 heads of 96: 16.2 -> 10.2; 603 tokens x 2, 32 / 4 heads of 192: 40.6 -> 29.1.
 // Binary16 heads of 256 (one group: no registers for two): 1019 tokens, 32 / 4 heads 80 us.
+// Operands of both products read ahead of their use, values looked at for infinities only in the steps whose keys some
+// row must not see, a step's place worked out without vector compares; before -> with it: 2048 tokens, 32 / 8 heads of 64,
+// bf16 40.3 -> 36.5 us; 512 x 4 on 7680 220 -> 208; 2048, 32 / 32 heads of 96, f16 64.2 -> 55.7; 512 x 4 on 7680, 32 / 8
+// heads of 256, bf16 986 -> 895 (a step of 32 keys x 32 rows of 64: 126 vector instructions, 150 before).
 #include "attn_general.hpp"
 
 namespace ellm {
@@ -81,14 +85,6 @@ struct Shape {
   static constexpr int kOccupancy = KG == 2 && NB <= 2 ? 4 : KG > 1 ? kWaves / 4 : kF32 ? (NB <= 4 ? 2 : 1) : NB <= 2 ? 3 : NB <= 4 ? 2 : 1;
 };
 
-// The weights of two keys as operands of the second product, and their sum.
-template <typename S>
-__device__ __forceinline__ float weigh_pair(float s0, float s1, float c, float shift, uint32_t& hi, uint32_t& lo) {
-  const float p0 = fast_exp2(__builtin_fmaf(s0, c, shift)), p1 = fast_exp2(__builtin_fmaf(s1, c, shift));
-  split_pair<S>(p0, p1, hi, lo);
-  return p0 + p1;
-}
-
 // (heads of 65 to 96 with the maximum every step: 160 registers, three workgroups a unit, which is what that form is for)
 template <typename S, int NB, bool VEC, int RB, int KG, bool LAZY>
 __global__ __launch_bounds__((Shape<S, NB, RB, KG>::kThreads),
@@ -132,6 +128,12 @@ void general_chunk_kernel(GeneralArgs p) {
   const uint32_t wave_first = P0 + wave_row0 / p.group;    // chunks up to here need no mask,
   const uint32_t wave_last = P0 + wave_row1 / p.group;     // chunks past here are not this wave's
   const bool wave_has_rows = __builtin_amdgcn_readfirstlane((int)(row0 + 32u * wave <= last_row));
+  // steps of this split that end beyond key x: from this one on
+  auto steps_beyond = [&](uint32_t x) { return x + 1 > k0 ? (x + 1 - k0) / kKeys : 0u; };
+  auto uniform = [](uint32_t x) { return (uint32_t)__builtin_amdgcn_readfirstlane((int)x); };
+  const uint32_t wave_steps = uniform(wave_has_rows && wave_last >= k0 ? min(n_steps, (wave_last - k0) / kKeys + 1) : 0u);
+  const uint32_t mask_from = uniform(min(steps_beyond(wave_first), (end - k0) / kKeys));   // some pair is masked: by position, or past the end
+  const uint32_t look_from = uniform(steps_beyond(first_pos));
 
   u32x4 qreg[kQ];
   {
@@ -176,16 +178,29 @@ void general_chunk_kernel(GeneralArgs p) {
         st[i] = gather_piece<S>(rows, p.kv_stride_pos, kb + (off(i) & 0xffffu), end, off(i) >> 16, p.head_size);
     }
   };
+  // (steps are asked for in order: kg, kg + KG, ...)
+  uint64_t next_off = scalar64((uint64_t)(k0 + kg * kKeys) * pos_bytes);
+  const uint64_t off_step = scalar64((uint64_t)(KG * kKeys) * pos_bytes);
   auto load_step = [&](uint32_t step) {
-    load_rows(step, kp, kplane, kst);
-    if constexpr (!X::kLateV) load_rows(step, vp, vplane, vst);
+    if constexpr (VEC && !X::kLateV) {
+      const __amdgpu_buffer_rsrc_t kr = chunk_rsrc(kplane, next_off, valid), vr = chunk_rsrc(vplane, next_off, valid);
+      next_off += off_step;
+#pragma unroll
+      for (int i = 0; i < kPieces; ++i) kst[i] = __builtin_amdgcn_raw_buffer_load_b128(kr, off(i), 0, 0);
+#pragma unroll
+      for (int i = 0; i < kPieces; ++i) vst[i] = __builtin_amdgcn_raw_buffer_load_b128(vr, off(i), 0, 0);
+    } else {
+      load_rows(step, kp, kplane, kst);
+      if constexpr (!X::kLateV) load_rows(step, vp, vplane, vst);
+    }
   };
   auto store_rows = [&](uint32_t step, const u32x4 (&st)[kPieces], auto at, int bytes) __attribute__((always_inline)) {
 #pragma unroll
     for (int i = 0; i < kPieces; ++i) *(LdsU32x4*)(at(i) + (step / KG & 1) * bytes) = st[i];
   };
   auto look_at = [&](uint32_t step) {
-    if (k0 + step * kKeys + kKeys - 1 > first_pos) {   // some row of the workgroup must not see some of these values
+    if (step >= look_from) {   // some row of the workgroup must not see some of these values
+      asm volatile("");   // (a branch, not a condition: few steps of a walk come here)
       bool bad = false;
 #pragma unroll
       for (int i = 0; i < kPieces; ++i) bad |= piece_not_finite<S>(vst[i]);
@@ -221,6 +236,17 @@ void general_chunk_kernel(GeneralArgs p) {
                                   : lds0 + 2 * X::kKBuf + (4 * g + ((lane & 15) >> 2)) * X::kVPitch +
                                         2 * (16 * ((lane >> 4) & 1) + 4 * (lane & 3));
 
+  // 16-bit: operand n of the second product, keys 16 (n / NB) .., columns 32 (n % NB) ..
+  auto v_operand = [&](uint32_t vs, int n) __attribute__((always_inline)) {
+    const uint32_t at = vs + 16 * (n / NB) * X::kVPitch + 64 * (n % NB);
+    const i16x4 a0 = __builtin_amdgcn_ds_read_tr16_b64_v4i16((LdsI16x4*)at);
+    const i16x4 a1 = __builtin_amdgcn_ds_read_tr16_b64_v4i16((LdsI16x4*)(at + 8 * X::kVPitch));
+    const u32x2 w0 = __builtin_bit_cast(u32x2, a0), w1 = __builtin_bit_cast(u32x2, a1);
+    return u32x4{w0[0], w0[1], w1[0], w1[1]};
+  };
+  // operand reads ahead of the products (three are what 168 registers hold)
+  constexpr int kAheadMax = NB == 3 && KG == 1 && !LAZY ? 3 : 4, kAheadK = kQ * MB < kAheadMax ? kQ * MB : kAheadMax;
+  constexpr int kAhead = 2 * MB * NB < kAheadMax ? 2 * MB * NB : kAheadMax;
   auto load_late = [&](uint32_t step) __attribute__((always_inline)) {
     if constexpr (X::kLateV)
       if (step < n_steps) load_rows(step, vp, vplane, vst);
@@ -228,12 +254,13 @@ void general_chunk_kernel(GeneralArgs p) {
   auto compute = [&](uint32_t step, auto first_) __attribute__((always_inline)) {
     constexpr bool kFirst = decltype(first_)::value;   // the group's first step: no row has a reference maximum yet
     const uint32_t kb = k0 + step * kKeys, buf = step / KG & 1;
-    if (step >= n_steps || !wave_has_rows || kb > wave_last) {
+    if (step >= wave_steps) {
       load_late(step + KG);
       return;
     }
     const uint32_t ks = k_read + buf * X::kKBuf, vs = v_read + buf * X::kVBuf;
     f32x16 st[MB];
+    u32x4 va[2 * MB * NB];
     f32x16 zero;
 #pragma unroll
     for (int e = 0; e < 16; ++e) zero[e] = 0.0f;
@@ -269,17 +296,23 @@ void general_chunk_kernel(GeneralArgs p) {
       auto each = [&](auto n_) { return total[decltype(n_)::value]; };
       st[0] = pairwise_sum<0, kTotals>(each);
     } else {
+      // (operands a few reads ahead of their products; those of the second product, as far as they fit the registers the
+      // first one's leave, ahead of the soft-max, which their way out of LDS then lies behind)
+      u32x4 ka[kQ * MB];
+      auto k_operand = [&](int n) { return (u32x4) * (const LdsU32x4*)(ks + 32 * (n % MB) * X::kKPitch + 32 * (n / MB)); };
 #pragma unroll
-      for (int mb = 0; mb < MB; ++mb) st[mb] = zero;
+      for (int n = 0; n < kAheadK; ++n) ka[n] = k_operand(n);
+      __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-      for (int s = 0; s < kQ; ++s)
+      for (int n = 0; n < kQ * MB; ++n) {
+        st[n % MB] = Mfma<S>::m32x32x16(ka[n], qreg[n / MB], n < MB ? zero : st[n % MB]);
+        if (n + kAheadK < kQ * MB) ka[n + kAheadK] = k_operand(n + kAheadK);
+      }
 #pragma unroll
-        for (int mb = 0; mb < MB; ++mb) {
-          const u32x4 a = *(const LdsU32x4*)(ks + 32 * mb * X::kKPitch + 32 * s);
-          st[mb] = Mfma<S>::m32x32x16(a, qreg[s], st[mb]);
-        }
+      for (int n = 0; n < kAhead; ++n) va[n] = v_operand(vs, n);
+      __builtin_amdgcn_sched_barrier(0);
     }
-    if (kb + kKeys - 1 > wave_first || kb + kKeys > end) {   // some pair of the step is masked
+    if (step >= mask_from) {   // some pair of the step is masked
 #pragma unroll
       for (int mb = 0; mb < MB; ++mb)
 #pragma unroll
@@ -354,19 +387,18 @@ void general_chunk_kernel(GeneralArgs p) {
           for (int e = 0; e < 4; ++e) v[e] = next[e];
       });
     } else {
-      u32x4 hi[2 * MB], lo[2 * MB];
-      // (the loop stands here and below: as a lambda it takes 9 registers more where LAZY is off)
-      if constexpr (!LAZY || !kFirst) {
+      f32x16 w[MB];
+      auto weigh = [&](int cc, float shift) __attribute__((always_inline)) {   // keys 16 cc .. + 15
 #pragma unroll
-        for (int cc = 0; cc < 2 * MB; ++cc)
+        for (int e = 8 * (cc & 1); e < 8 * (cc & 1) + 8; e += 2) {
+          w[cc >> 1][e] = fast_exp2(__builtin_fmaf(st[cc >> 1][e], p.c, shift));
+          w[cc >> 1][e + 1] = fast_exp2(__builtin_fmaf(st[cc >> 1][e + 1], p.c, shift));
+          psum += w[cc >> 1][e] + w[cc >> 1][e + 1];
+        }
+      };
+      if constexpr (LAZY && !kFirst) {
 #pragma unroll
-          for (int w = 0; w < 4; ++w) {
-            const int e = 8 * (cc & 1) + 2 * w;
-            uint32_t h, l;
-            psum += weigh_pair<S>(st[cc >> 1][e], st[cc >> 1][e + 1], p.c, neg_m, h, l);
-            hi[cc][w] = h;
-            lo[cc][w] = l;
-          }
+        for (int cc = 0; cc < 2 * MB; ++cc) weigh(cc, neg_m);
       }
       if constexpr (LAZY) {
         // (a row without a reference makes its sum infinite or NaN; a row moves by what its own two lanes saw)
@@ -388,29 +420,56 @@ void general_chunk_kernel(GeneralArgs p) {
           neg_m = (m_run == -INFINITY) ? 0.0f : kShift - m_run;
           psum = 0.0f;
 #pragma unroll
-          for (int cc = 0; cc < 2 * MB; ++cc)
-#pragma unroll
-            for (int w = 0; w < 4; ++w) {
-              const int e = 8 * (cc & 1) + 2 * w;
-              uint32_t h, l;
-              psum += weigh_pair<S>(st[cc >> 1][e], st[cc >> 1][e + 1], p.c, neg_m, h, l);
-              hi[cc][w] = h;
-              lo[cc][w] = l;
-            }
+          for (int cc = 0; cc < 2 * MB; ++cc) weigh(cc, neg_m);
         }
       }
+      u32x4 hi[2 * MB], lo[2 * MB];
+      auto split = [&](int cc) __attribute__((always_inline)) {
 #pragma unroll
-      for (int cc = 0; cc < 2 * MB; ++cc)
-#pragma unroll
-        for (int db = 0; db < NB; ++db) {
-          const uint32_t at = vs + 16 * cc * X::kVPitch + 64 * db;
-          const i16x4 a0 = __builtin_amdgcn_ds_read_tr16_b64_v4i16((LdsI16x4*)at);
-          const i16x4 a1 = __builtin_amdgcn_ds_read_tr16_b64_v4i16((LdsI16x4*)(at + 8 * X::kVPitch));
-          const u32x2 w0 = __builtin_bit_cast(u32x2, a0), w1 = __builtin_bit_cast(u32x2, a1);
-          const u32x4 a = {w0[0], w0[1], w1[0], w1[1]};
-          oacc[db] = Mfma<S>::m32x32x16(a, hi[cc], oacc[db]);
-          oacc[db] = Mfma<S>::m32x32x16(a, lo[cc], oacc[db]);
+        for (int x = 0; x < 4; ++x) {
+          const int e = 8 * (cc & 1) + 2 * x;
+          uint32_t h, l;
+          split_pair<S>(w[cc >> 1][e], w[cc >> 1][e + 1], h, l);
+          hi[cc][x] = h;
+          lo[cc][x] = l;
         }
+      };
+      auto product = [&](int n, const u32x4& weights) __attribute__((always_inline)) {
+        oacc[n % NB] = Mfma<S>::m32x32x16(va[n], weights, oacc[n % NB]);
+      };
+      auto more_operands = [&](int n) __attribute__((always_inline)) {
+        if (n + kAhead < 2 * MB * NB) va[n + kAhead] = v_operand(vs, n + kAhead);
+      };
+      if constexpr (NB <= kAhead) {
+        // sixteen keys at a time: their products run beside the splitting of the next ones' weights, and none waits for
+        // the one before it
+#pragma unroll
+        for (int cc = 0; cc < 2 * MB; ++cc) {
+          if constexpr (!LAZY) weigh(cc, neg_m);
+          split(cc);
+          __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+          for (int n = NB * cc; n < NB * cc + NB; ++n) product(n, hi[cc]);
+#pragma unroll
+          for (int n = NB * cc; n < NB * cc + NB; ++n) {
+            product(n, lo[cc]);
+            more_operands(n);
+          }
+          __builtin_amdgcn_sched_barrier(0);
+        }
+      } else {   // (wide heads have products enough: in that order 2 to 8 % slower)
+#pragma unroll
+        for (int cc = 0; cc < 2 * MB; ++cc) {
+          weigh(cc, neg_m);
+          split(cc);
+        }
+#pragma unroll
+        for (int n = 0; n < 2 * MB * NB; ++n) {
+          product(n, hi[n / NB]);
+          product(n, lo[n / NB]);
+          more_operands(n);
+        }
+      }
     }
     l_run += psum;
   };
