@@ -18,7 +18,7 @@
 // one burst and re-read the token rows from the caches in operand layout: raw sums of 2048 -> 5120, one
 // row 7.6 -> 6.2, 2048 -> 5120 with finished heads, 1 / 16 / 64 rows 9.4 / 9.9 / 17.0 -> 8.3 / 9.1 / 14.6;
 // 4096 -> 12288, 1 / 16 / 64 rows 24 / 29 / 62 -> 21 / 21 / 27; 8192 -> 10240, 1 / 16 / 64 rows 53 / 65 / 64 ->
-// 31 / 32 / 42 (raw, one row: 28.4 us, 5.9 TB/s).  What is left beside the stream is about 6 us a launch:
+// 31 / 32 / 42 (all before the workgroups walked K apart, below).  What is left beside the stream is about 6 us a launch:
 // start, first data, the sums, the store.
 #include "project_common.hpp"
 
@@ -89,7 +89,14 @@ __global__ __launch_bounds__(kStThreads, 2) void project_small_kernel(ProjectKer
   const int row8 = lane >> 3, piece = lane & 7;
   const uint32_t src = row8 * K * 2 + piece * 16, x_step = 8 * K * 2;
   u32x4 stg[kDepth][X::kPieces];
+  // Every workgroup starts its walk along K one chunk further than its neighbour: rows lie a power of two apart with
+  // the usual widths, and in step all of them would read the same few kilobytes of every row, that is, from a part of
+  // the memory channels (one token, 64 / 8 heads on 8192: 65.2 -> 57.7 us, 32 / 32 on 4096 35.2 -> 33.6; sixteenths of the
+  // row apart, or apart by XCD only, less: 61 to 64).
+  const uint32_t rot = blockIdx.x % n_chunks;
   auto load_chunk = [&](uint32_t chunk, u32x4 (&st)[X::kPieces]) {
+    chunk += rot;
+    chunk = chunk >= n_chunks ? chunk - n_chunks : chunk;
 #pragma unroll
     for (int i = 0; i < W8; ++i) st[i] = __builtin_amdgcn_raw_buffer_load_b128(w_rsrc[i], src, chunk * kLine, 2);   // 2: read once
 #pragma unroll
