@@ -30,7 +30,7 @@ fn main() {
         "api.hip", "attn_general.hip", "attn_general_chunk.hip", "attn_general_step.hip", "attn_general.hpp", "general_plan.hpp", "noalloc.hip", "decode.hip", "decode_balanced.hip", "prefill.hip", "kv_cache.hip",
         "project.hip", "project_mid.hip", "project_small.hip", "project_api.hip", "step.hip", "handles.hpp", "common.hpp",
         "kernels.hpp", "decode_common.hpp", "decode_plan.hpp", "decode_shares.hpp", "chunk_plan.hpp", "project_common.hpp",
-        "project_epilogue.hpp", "project_mid_tile.hpp", "Makefile",
+        "project_epilogue.hpp", "project_mid_tile.hpp", "project_plan.hpp", "Makefile",
     ] {
         println!("cargo:rerun-if-changed={}", csrc.join(f).display());
     }

@@ -36,6 +36,8 @@ struct ellm_matmul3 {
   int device;
   float* ws;
   uint32_t* counters;
+  float* part;         // inside ws, behind what the few-rows kernel takes; null: no room was taken for it
+  size_t part_floats;
   // destination with per-sequence capacities (ellm_matmul3_create_ragged); null / empty otherwise
   const size_t* seq_offsets;
   const uint32_t* seq_caps;

@@ -143,6 +143,9 @@ struct ProjectArgs {
   // workspace of the few-rows kernel (may be null: the tile kernel runs whatever the row count)
   float* ws;
   uint32_t* counters;
+  // room for the sums of tiles whose K is shared by several workgroups (null: none is)
+  float* part;
+  size_t part_floats;
   // raw_out: the few-rows kernel leaves the binary32 sums of every column in ws, laid out as
   // PendingRows describes (one part), and writes nothing else (requires project_raw_takes())
   uint32_t raw_out;
@@ -152,6 +155,8 @@ bool project_raw_takes(uint32_t rows, uint32_t heads, uint32_t K, bool has_works
 hipError_t launch_project(const ProjectArgs& a, hipStream_t stream);
 // Few-rows kernel: rows it handles at most, floats of partial sums and counters it needs.
 size_t project_workspace_floats(uint32_t heads);
+// Floats of a handle's `part`: calls of up to max_rows rows.
+size_t project_part_floats(uint32_t heads, uint32_t K, size_t max_rows);
 // The kernel a projection of this shape runs (heads = 128-wide output column groups).
 enum { kPathFewRows = 0, kPathTiles128 = 1, kPathTiles256x1 = 2, kPathTiles = 3 };
 int project_path(uint32_t rows, uint32_t heads, uint32_t K, bool has_workspace);

@@ -23,6 +23,7 @@
 // Calls with at most 64 rows go to the streaming kernel of project_small.hip, calls that would
 // leave these tiles fewer than the compute units to the 128-token tiles of project_mid.hip.
 #include "project_mid_tile.hpp"
+#include "project_plan.hpp"
 
 namespace ellm {
 using namespace proj;
@@ -134,13 +135,24 @@ hipError_t launch_project(const ProjectArgs& a, hipStream_t stream) {
   p.max_start = a.max_start;
   p.finalize0 = a.finalize0;
   p.eps = a.eps;
-  const int path = project_path(a.rows, a.heads0 + 2 * a.heads_kv, a.K, a.ws && a.counters);
+  p.k_split = 1;
+  p.part = nullptr;
+  const uint32_t heads = a.heads0 + 2 * a.heads_kv;
+  const int path = project_path(a.rows, heads, a.K, a.ws && a.counters);
   if (a.raw_out) {
     if (path != kPathFewRows || a.residual) return hipErrorInvalidValue;   // (project_raw_takes() said otherwise)
     return launch_project_small(p, a.ws, a.counters, g_n_cu, a.dtype, kModeRaw, stream);
   }
   if (path == kPathFewRows)
     return launch_project_small(p, a.ws, a.counters, g_n_cu, a.dtype, a.residual ? kModeAdd : kModeQkv, stream);
+  if (path == kPathTiles128 && a.part) {
+    const ProjectSplit split = project_split(a.rows, heads, a.K, g_n_cu, a.part_floats);
+    if (split.k_split > 1) {
+      p.k_split = split.k_split;
+      p.part = a.part;
+      return launch_project_mid(p, split.token_blocks, a.dtype, a.residual != nullptr, stream);
+    }
+  }
   if (path == kPathTiles128 || path == kPathTiles256x1)
     return launch_project_mid(p, path == kPathTiles128 ? 1 : 2, a.dtype, a.residual != nullptr, stream);
   // A last round of tiles that would leave half of the compute units without one, or three
@@ -184,5 +196,6 @@ hipError_t project_prepare() {
 }
 
 size_t project_workspace_floats(uint32_t heads) { return (size_t)heads * kHeadDim * kSmallRowsMax; }
+size_t project_part_floats(uint32_t heads, uint32_t K, size_t max_rows) { return project_split_room(heads, K, g_n_cu, max_rows); }
 
 }  // namespace ellm

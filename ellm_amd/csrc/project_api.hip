@@ -1,6 +1,7 @@
 // C ABI of the projections either side of attention (declared in
 // include/ellm_attn.h): validation and handles for ellm_matmul3_* and
-// ellm_matmul_add_*.  A handle owns the workspace of the few-rows kernel only.
+// ellm_matmul_add_*.  A handle owns the workspace of the few-rows kernel
+// and of calls whose K several workgroups share.
 #include <hip/hip_runtime.h>
 
 #include <cmath>
@@ -21,21 +22,27 @@ struct ellm_matmul_add {
   int device;
   float* ws;
   uint32_t* counters;
+  float* part;
+  size_t part_floats;
 };
 
 namespace {
 // Partial sums and arrival counters of the few-rows kernel; left null (the tile kernel then
-// runs every call) when they would take more than 64 MiB.
-int alloc_small_workspace(uint32_t heads, int* device, float** ws, uint32_t** counters) {
-  *ws = nullptr;
+// runs every call, K whole) when they would take more than 64 MiB.  Behind them, for handles that may run
+// more rows, room for the sums of tiles whose K is shared (project_plan.hpp).
+int alloc_small_workspace(uint32_t heads, size_t k, size_t max_rows, int* device, float** ws, uint32_t** counters, float** part,
+                          size_t* part_floats) {
+  *ws = *part = nullptr;
   *counters = nullptr;
+  *part_floats = 0;
   int n_cu = 0;
   if (int st = ellm::current_gfx950_device(device, &n_cu)) return st;
   const hipError_t prep = ellm::project_prepare();
   if (prep != hipSuccess) return ellm::set_error(ELLM_ERR_HIP, "projection kernels: %s", hipGetErrorString(prep));
   const size_t floats = ellm::project_workspace_floats(heads);
   if (floats * sizeof(float) > (size_t)64 << 20) return ELLM_OK;
-  hipError_t e = hipMalloc((void**)ws, floats * sizeof(float));
+  const size_t more = ellm::project_part_floats(heads, (uint32_t)k, max_rows);
+  hipError_t e = hipMalloc((void**)ws, (floats + more) * sizeof(float));
   if (e == hipSuccess) e = hipMalloc((void**)counters, heads * sizeof(uint32_t));
   if (e == hipSuccess) e = hipMemset(*counters, 0, heads * sizeof(uint32_t));
   if (e != hipSuccess) {
@@ -44,6 +51,10 @@ int alloc_small_workspace(uint32_t heads, int* device, float** ws, uint32_t** co
     *ws = nullptr;
     *counters = nullptr;
     return ellm::set_error(ELLM_ERR_HIP, "projection workspace: %s", hipGetErrorString(e));
+  }
+  if (more) {
+    *part = *ws + floats;
+    *part_floats = more;
   }
   return ELLM_OK;
 }
@@ -119,8 +130,8 @@ static int matmul3_create(const ellm_matmul3_desc* d, const ellm_kv_seq_table* t
     h->seq_caps = table->seq_capacity;
     h->caps_host.assign(table->seq_capacity_host, table->seq_capacity_host + d->batch_size);
   }
-  const int rc = alloc_small_workspace((uint32_t)(d->attention_head_num + 2 * d->kv_head_num), &h->device, &h->ws,
-                                       &h->counters);
+  const int rc = alloc_small_workspace((uint32_t)(d->attention_head_num + 2 * d->kv_head_num), d->hidden_size, rows, &h->device, &h->ws,
+                                       &h->counters, &h->part, &h->part_floats);
   if (rc != ELLM_OK) {
     delete h;
     return rc;
@@ -208,6 +219,8 @@ int ellm::matmul3_fill_args(const ellm_matmul3* h, size_t position_index, size_t
   a.dtype = d.dtype;
   a.ws = h->ws;
   a.counters = h->counters;
+  a.part = h->part;
+  a.part_floats = h->part_floats;
   *out = a;
   return ELLM_OK;
 }
@@ -266,7 +279,8 @@ int ellm_matmul_add_create(const ellm_matmul_add_desc* d, ellm_matmul_add** out_
   ellm_matmul_add* h = new (std::nothrow) ellm_matmul_add;
   if (!h) return ellm::set_error(ELLM_ERR_HIP, "out of host memory");
   h->d = *d;
-  const int rc = alloc_small_workspace((uint32_t)(d->n / 128), &h->device, &h->ws, &h->counters);
+  const int rc = alloc_small_workspace((uint32_t)(d->n / 128), d->k, d->max_position_interval * d->batch_size, &h->device, &h->ws,
+                                       &h->counters, &h->part, &h->part_floats);
   if (rc != ELLM_OK) {
     delete h;
     return rc;
@@ -318,6 +332,8 @@ int ellm_matmul_add_run(ellm_matmul_add* h, size_t position_index, size_t positi
   a.dtype = d.dtype;
   a.ws = h->ws;
   a.counters = h->counters;
+  a.part = h->part;
+  a.part_floats = h->part_floats;
   const hipError_t e = ellm::launch_project(a, (hipStream_t)stream);
   if (e != hipSuccess) return ellm::set_error(ELLM_ERR_HIP, "projection launch: %s", hipGetErrorString(e));
   return ELLM_OK;

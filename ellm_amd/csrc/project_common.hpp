@@ -31,6 +31,8 @@ struct ProjectKernelArgs {
   uint32_t tiles_m, tiles_n;
   uint32_t whole_tiles, tail_parts;   // project_kernel: tiles of 256 x 256; workgroups per tile of the rest
   uint32_t band_m;                    // project_mid_kernel: token tiles that take turns on one head
+  uint32_t k_split;                   // ... and workgroups that share a tile's K (one: 0 or 1)
+  float* part;                        // their sums, [k_split][rows][columns]
   uint32_t position_index, max_start;
   uint32_t finalize0;        // segment 0 rows are normalised and rotated
   float eps;
@@ -54,6 +56,7 @@ constexpr int kModeQkv = 0;  // heads normalised + rotated (or passed through), 
 constexpr int kModeAdd = 1;  // plain product plus a residual of the output's layout
 constexpr int kModeRaw = 2;  // the binary32 sums of every column to the workspace, [row][column]: a fused
                              // single-token step, whose attention kernel finishes the rows (few-rows kernel only)
+constexpr int kModePart = 3; // the binary32 sums of every column over a piece of K (project_mid_kernel)
 
 // Streaming kernel for a few rows (project_small.hip); from 65 rows on one 128-token tile per head
 // (project_mid.hip) runs.
@@ -66,7 +69,8 @@ hipError_t launch_project_small(const ProjectKernelArgs& p, float* ws, uint32_t*
 // Tile kernel with 128-token x one-head tiles (project_mid.hip), for row counts at which
 // the 256 x 256 tiles are fewer than the compute units.
 hipError_t mid_prepare();
-// token_blocks: 1 = 128-token tiles, 2 = 256-token tiles
+// token_blocks: 1 = 128-token tiles, 2 = 256-token tiles; with p.k_split > 1 every tile's K goes to that many workgroups,
+// which leave their sums in p.part for a second launch
 hipError_t launch_project_mid(ProjectKernelArgs p, uint32_t token_blocks, int dtype, bool add,
                               hipStream_t stream);
 

@@ -5,6 +5,10 @@
 // The same tile code (project_mid_tile.hpp) at 128 or 256 tokens x one head.  Tiles this small move up to twice
 // the LDS bytes per MFMA, and 128-bit LDS stores are slow (13 cycles an instruction against
 // 4.7 for a read), one more reason why operands go from memory straight into LDS.
+// Where even these tiles leave most units idle (79 rows of 4096 -> 2048: 16 of 256) several workgroups share a tile's K
+// and leave their sums for project_fold_kernel (project_plan.hpp: when, and both sides measured).  What bounds that form
+// is the second launch, 4 us, and the sums' way through the L2s; finishing a tile in the last workgroup to arrive would
+// read all of them through one unit at 60 to 100 GB/s, 5 to 8 us for eight pieces.
 #include "project_mid_tile.hpp"
 
 namespace ellm {
@@ -25,12 +29,71 @@ __global__ __launch_bounds__(64 * WAVES) void project_mid_kernel(ProjectKernelAr
   mid_tile<S, MODE, MB, WAVES, 1>(p, (first_m + in_band % here) * MidShape<MB, WAVES, 1>::kTokens, in_band / here, mid_smem);
 }
 
+// Sums of the pieces of K, in order, and what the tiles' epilogue does with a finished head: 16 lanes a (row, head),
+// eight columns each.
+template <typename S, int MODE>
+__global__ __launch_bounds__(256) void project_fold_kernel(ProjectKernelArgs p) {
+  using M = Mfma<S>;
+  const uint32_t heads = p.heads0 + 2 * p.heads_kv, n_cols = heads * kHeadDim;
+  const uint32_t item = blockIdx.x * 16 + threadIdx.x / 16, c8 = threadIdx.x % 16;
+  const uint32_t R = item / heads, head = item % heads, b = R % p.batch_pitch;
+  const bool live = R < p.rows && b < p.batch;
+  const size_t step = (size_t)p.rows * n_cols;
+  const float* from = p.part + (live ? (size_t)R * n_cols + head * kHeadDim + 8 * c8 : 0);
+  const bool rotated = MODE == kModeQkv && (head < p.heads0 ? p.finalize0 != 0 : head < p.heads0 + p.heads_kv);
+  const uint32_t hs = head < p.heads0 ? head : head < p.heads0 + p.heads_kv ? head - p.heads0 : head - p.heads0 - p.heads_kv;
+  const uint32_t pos = R / p.batch_pitch + (MODE == kModeQkv && live && p.positions ? min(p.positions[b], p.max_start) : p.position_index);
+  const uint32_t one_zero = M::pack2(1.0f, 0.0f);
+  u32x4 extra = {one_zero, one_zero, one_zero, one_zero};   // rotary row or residual
+  if (MODE == kModeAdd && live) extra = load16(p.residual + (size_t)R * p.ld0 + head * kHeadDim + 8 * c8);
+  if (MODE == kModeQkv && live && rotated) extra = load16(p.rope + (size_t)pos * p.rope_pos_stride + (size_t)hs * p.rope_head_stride + 8 * c8);
+  f32x4 lo = {0.0f, 0.0f, 0.0f, 0.0f}, hi = lo;
+  for (uint32_t s = 0; s < p.k_split; s += 4) {   // (four pieces' loads at once)
+    f32x4 a[4], c[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const float* at = from + min(s + i, p.k_split - 1) * step;
+      a[i] = *(const f32x4*)at;
+      c[i] = *(const f32x4*)(at + 4);
+    }
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+      if (s + i < p.k_split) {
+        lo += a[i];
+        hi += c[i];
+      }
+  }
+  float o[8] = {lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
+  u32x4 packed;
+  if constexpr (MODE == kModeAdd) {
+#pragma unroll
+    for (int e = 0; e < 4; ++e)
+      packed[e] = M::pack2(o[2 * e] + M::to_float((uint16_t)(extra[e] & 0xffffu)), o[2 * e + 1] + M::to_float((uint16_t)(extra[e] >> 16)));
+  } else {
+    float ss = squares8(o);
+#pragma unroll
+    for (int m = 1; m < 16; m <<= 1) ss += __shfl_xor(ss, m, 16);
+    if (rotated) {
+      packed = scale_rotate_pack8<S>(o, inverse_rms(ss, p.eps), extra);
+    } else {
+#pragma unroll
+      for (int e = 0; e < 4; ++e) packed[e] = M::pack2(o[2 * e], o[2 * e + 1]);
+    }
+  }
+  if (!live) return;
+  uint16_t* to = head < p.heads0 ? p.out0 + (size_t)R * p.ld0 + head * kHeadDim
+                                 : (head < p.heads0 + p.heads_kv ? p.k_out : p.v_out) + kv_row_offset(p, b, hs, pos);
+  store16(to + 8 * c8, packed);
+}
+
 template <int MB, int WAVES>
 hipError_t prepare_shape() {
   const void* kernels[] = {(const void*)project_mid_kernel<F16, kModeQkv, MB, WAVES>,
                            (const void*)project_mid_kernel<BF16, kModeQkv, MB, WAVES>,
                            (const void*)project_mid_kernel<F16, kModeAdd, MB, WAVES>,
-                           (const void*)project_mid_kernel<BF16, kModeAdd, MB, WAVES>};
+                           (const void*)project_mid_kernel<BF16, kModeAdd, MB, WAVES>,
+                           (const void*)project_mid_kernel<F16, kModePart, MB, WAVES>,
+                           (const void*)project_mid_kernel<BF16, kModePart, MB, WAVES>};
   for (const void* k : kernels) {
     const hipError_t e =
         hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, MidShape<MB, WAVES, 1>::kLdsBytes);
@@ -73,6 +136,17 @@ hipError_t launch_shape(ProjectKernelArgs p, int dtype, bool add, hipStream_t st
     hipLaunchKernelGGL(kernel, dim3(blocks), dim3(Shape::kThreads), Shape::kLdsBytes, stream, p);
     return hipGetLastError();
   };
+  if (p.k_split > 1) {
+    hipLaunchKernelGGL((dtype == 0 ? project_mid_kernel<F16, kModePart, MB, WAVES> : project_mid_kernel<BF16, kModePart, MB, WAVES>),
+                       dim3(blocks, p.k_split), dim3(Shape::kThreads), Shape::kLdsBytes, stream, p);
+    const hipError_t e = hipGetLastError();
+    if (e != hipSuccess) return e;
+    const dim3 grid((p.rows * p.tiles_n + 15) / 16);
+    auto fold = add ? (dtype == 0 ? project_fold_kernel<F16, kModeAdd> : project_fold_kernel<BF16, kModeAdd>)
+                    : (dtype == 0 ? project_fold_kernel<F16, kModeQkv> : project_fold_kernel<BF16, kModeQkv>);
+    hipLaunchKernelGGL(fold, grid, dim3(256), 0, stream, p);
+    return hipGetLastError();
+  }
   if (add)
     return dtype == 0 ? go(project_mid_kernel<F16, kModeAdd, MB, WAVES>) : go(project_mid_kernel<BF16, kModeAdd, MB, WAVES>);
   return dtype == 0 ? go(project_mid_kernel<F16, kModeQkv, MB, WAVES>) : go(project_mid_kernel<BF16, kModeQkv, MB, WAVES>);

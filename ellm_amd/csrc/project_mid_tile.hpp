@@ -61,7 +61,9 @@ __device__ __forceinline__ void mid_tile(const ProjectKernelArgs& p, uint32_t ro
   const int c16 = lane & 15, g = lane >> 4;
   const int wn = wave % HEADS, wm = wave / HEADS;
   const uint32_t K = p.K;
-  const uint32_t n_chunks = K / kMidKc;
+  // kModePart: piece blockIdx.y of K, as many chunks as the others or one more
+  const uint32_t all_chunks = K / kMidKc, first_chunk = MODE == kModePart ? blockIdx.y * all_chunks / p.k_split : 0u;
+  const uint32_t n_chunks = MODE == kModePart ? (blockIdx.y + 1) * all_chunks / p.k_split - first_chunk : all_chunks;
   const uint32_t rows_here = min(p.rows - row0, (uint32_t)Shape::kTokens);
   // (descriptors as four plain words: base, base >> 32, bytes, flags; they go into inline asm)
   auto make_rsrc = [](uint64_t base, uint32_t bytes) {
@@ -116,12 +118,12 @@ __device__ __forceinline__ void mid_tile(const ProjectKernelArgs& p, uint32_t ro
   uint32_t x_to = 0, w_to = 0, x_off = 0, w_off = 0;
   auto aim_x = [&](uint32_t chunk, uint32_t at) __attribute__((always_inline)) {   // what load_piece() takes, and where to
     x_to = st_wave + at;
-    x_off = chunk * (kMidKc * 2);
+    x_off = (first_chunk + chunk) * (kMidKc * 2);
     if (chunk >= n_chunks) x_rsrc[2] = 0;
   };
   auto aim_w = [&](uint32_t chunk, uint32_t at) __attribute__((always_inline)) {
     w_to = st_wave + at;
-    w_off = chunk * (kMidKc * 2);
+    w_off = (first_chunk + chunk) * (kMidKc * 2);
     if (chunk >= n_chunks) {
 #pragma unroll
       for (int h = 0; h < HEADS; ++h) w_rsrc[h][2] = 0;
@@ -181,7 +183,7 @@ __device__ __forceinline__ void mid_tile(const ProjectKernelArgs& p, uint32_t ro
   // (requested behind the first chunks where registers are left for it, used after the loop: destinations,
   // positions and the first rows of the rotary table or the residual)
   HeadRows<MB> head;
-  if constexpr (MB == 1) head = prepare_head<S, MODE, MB>(p, head0 + wn, row0 + 32 * MB * wm, lane);
+  if constexpr (MB == 1 && MODE != kModePart) head = prepare_head<S, MODE, MB>(p, head0 + wn, row0 + 32 * MB * wm, lane);
   if constexpr (kHalves)
     asm volatile("s_waitcnt vmcnt(12)" ::: "memory");
   else if constexpr (WAVES == 8)
@@ -276,9 +278,21 @@ __device__ __forceinline__ void mid_tile(const ProjectKernelArgs& p, uint32_t ro
     if (c + 1 < n_chunks) chunk_step(std::integral_constant<int, 1>{}, c + 1);
   }
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // the last (empty) requests still write LDS
+  if constexpr (MODE == kModePart) {   // a lane's four columns of its tokens, plain stores: the next launch reads them
+    const uint32_t n_cols = (p.heads0 + 2 * p.heads_kv) * kHeadDim;
+#pragma unroll
+    for (int t = 0; t < TB; ++t) {
+      const uint32_t row = row0 + 32 * MB * wm + 16 * t + c16;
+      if (row >= p.rows) continue;
+      float* to = p.part + ((size_t)blockIdx.y * p.rows + row) * n_cols + (head0 + wn) * kHeadDim + 4 * g;
+#pragma unroll
+      for (int nb = 0; nb < 8; ++nb) *(f32x4*)(to + 16 * nb) = acc[nb][t];
+    }
+    return;
+  }
   __syncthreads();
   if constexpr (MB != 1) head = prepare_head<S, MODE, MB>(p, head0 + wn, row0 + 32 * MB * wm, lane);
-  finish_head<S, MODE, MB>(p, acc, head, lds0 + wave * kEpWaveBytes, lane);
+  if constexpr (MODE != kModePart) finish_head<S, MODE, MB>(p, acc, head, lds0 + wave * kEpWaveBytes, lane);
 }
 
 }  // namespace proj

@@ -1,0 +1,73 @@
+// Projections of 65 to some hundred rows: whether, and into how many pieces, K is shared between workgroups
+// (host code, no device types: also compiled by the CPU tests).
+#pragma once
+
+#include <stddef.h>
+#include <stdint.h>
+
+namespace ellm {
+namespace proj {
+
+// Tiles of 128 token_blocks tokens x one head, k_split workgroups a tile (1: K stays whole).
+struct ProjectSplit {
+  uint32_t token_blocks, k_split;
+};
+
+inline size_t split_floats(const ProjectSplit& s, uint32_t rows, uint32_t heads) {
+  return s.k_split > 1 ? (size_t)s.k_split * rows * heads * 128 : 0;
+}
+
+// Estimated time (us, 256 units).  A chunk of 64 of K takes 0.5 us a workgroup of 128 tokens and 0.65 of 256 (weights
+// from memory); the operands of all tiles come out of the L2s at 14 TB/s and the weights from memory at 4.6; the second
+// launch and the partial sums, written and read, are 4 us and their bytes at 6 TB/s.
+inline double project_tiles_us(const ProjectSplit& s, uint32_t rows, uint32_t heads, uint32_t K) {
+  const double chunks = (K / 64 + s.k_split - 1) / s.k_split, tokens = 128.0 * s.token_blocks;
+  const double tiles = (rows + 128 * s.token_blocks - 1) / (128 * s.token_blocks) * (double)heads;
+  const double chain = chunks * (s.token_blocks == 1 ? 0.5 : 0.65);
+  if (s.k_split == 1) return 5.0 + chain;
+  const double operands = tiles * (tokens + 128) * K * 2 / 14e6, weights = (double)heads * 128 * K * 2 / 4.6e6;
+  const double walk = chain > operands ? chain : operands;
+  return 9.0 + (walk > weights ? walk : weights) + 2.0 * split_floats(s, rows, heads) * 4 / 6e6;
+}
+
+// Three to eight workgroups a tile, all of them at once, one per unit, pieces of at least four chunks, sums within
+// `room` floats; where that is estimated 5 % below one round of whole tiles.  Two a tile gained nothing that lasts
+// (2048 <- 4096, 700 rows 32.9 / 33.0).  Whole / shared, weights from memory, f16 (us; tokens a tile / pieces):
+//   2048 <- 4096   79 rows 32.4 / 14.6 (128 / 8)   128 37.2 / 16.0 (128 / 8)   234 35.2 / 18.6 (128 / 8)   400 30.0 / 22.6 (128 / 4)
+//                  700 32.9 / 28.1 (256 / 4)
+//   5120 <- 2048   79 21.0 / 15.5 (128 / 6)   128 23.4 / 17.8 (128 / 6)   400 stays whole: 20.3 / 26.2 and more
+//   4096 <- 4096   79 34.7 / 17.8 (128 / 8)   128 39.6 / 20.3   234 37.2 / 23.7 (128 / 4)   400 31.7 / 30.9 (256 / 3)
+//   10240 <- 8192  79 67.6 / 45.1 (128 / 3)   128 77.2 / 49.7   234 73.3 / 63.3 (256 / 3)
+//   8192 <- 8192   79 64.8 / 42.9 (128 / 4)   128 74.5 / 46.9   234 70.5 / 56.9 (256 / 4)
+inline ProjectSplit project_split(uint32_t rows, uint32_t heads, uint32_t K, uint32_t n_cu, size_t room) {
+  const ProjectSplit whole = {1, 1};
+  if (((size_t)rows + 127) / 128 * heads > n_cu) return whole;
+  ProjectSplit best = whole;
+  double best_us = 0.95 * project_tiles_us(whole, rows, heads, K);
+  for (uint32_t blocks = 1; blocks <= 2; ++blocks) {
+    const uint32_t tiles = (rows + 128 * blocks - 1) / (128 * blocks) * heads;
+    for (uint32_t n = 3; n <= 8 && n * tiles <= n_cu && 4 * n <= K / 64; ++n) {
+      const ProjectSplit s = {blocks, n};
+      if (split_floats(s, rows, heads) > room) break;
+      const double us = project_tiles_us(s, rows, heads, K);
+      if (us < best_us) {
+        best_us = us;
+        best = s;
+      }
+    }
+  }
+  return best;
+}
+
+// Room that the calls of up to max_rows rows of a matrix can use (at most 256 tokens x 128 columns a unit).
+inline size_t project_split_room(uint32_t heads, uint32_t K, uint32_t n_cu, size_t max_rows) {
+  size_t most = 0;
+  for (uint32_t rows = 65; rows <= max_rows && ((size_t)rows + 127) / 128 * heads <= n_cu; ++rows) {
+    const size_t f = split_floats(project_split(rows, heads, K, n_cu, (size_t)-1), rows, heads);
+    if (f > most) most = f;
+  }
+  return most;
+}
+
+}  // namespace proj
+}  // namespace ellm

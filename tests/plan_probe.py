@@ -15,7 +15,16 @@ SOURCE = r"""
 #include <cstdio>
 #include <cstdlib>
 #include "general_plan.hpp"
+#include "project_plan.hpp"
 using namespace ellm;
+static int project(char** v) {   // rows, heads, K, room (0: what a handle for that many rows takes)
+  uint32_t a[5];
+  for (int i = 1; i <= 4; ++i) a[i] = (uint32_t)strtoul(v[i + 1], nullptr, 10);
+  const size_t room = a[4] ? a[4] : proj::project_split_room(a[2], a[3], 256, a[1]);
+  const proj::ProjectSplit s = proj::project_split(a[1], a[2], a[3], 256, room);
+  printf("%u %u %zu %zu\n", s.token_blocks, s.k_split, proj::split_floats(s, a[1], a[2]), room);
+  return 0;
+}
 static int chunk(char** v) {   // batch capacity, batch, query heads, key-value heads, most positions a call, position_index, interval, bfloat16
   uint32_t a[9];
   for (int i = 1; i <= 8; ++i) a[i] = (uint32_t)strtoul(v[i + 1], nullptr, 10);
@@ -29,6 +38,7 @@ static int chunk(char** v) {   // batch capacity, batch, query heads, key-value 
 // position_index, interval, whole aligned pieces, and room for partial rows per query row (0: the workspace's)
 int main(int, char** v) {
   if (v[1][0] == 'c') return chunk(v);
+  if (v[1][0] == 'p') return project(v);
   uint32_t a[12];
   for (int i = 1; i <= 11; ++i) a[i] = (uint32_t)strtoul(v[i], nullptr, 10);
   const gen::GeneralWorkspace w = gen::general_workspace(a[7], a[3], a[5], a[6], a[1], 256);
@@ -70,6 +80,12 @@ def general_plan(head_size, element_bytes, batch_capacity, batch, q_heads, kv_he
     args = (head_size, element_bytes, batch_capacity, batch, q_heads, kv_heads, interval, position_index, interval, int(vec), room)
     out = subprocess.run([_program(), *map(str, args)], check=True, capture_output=True, text=True).stdout.split()
     return (("rows", "step", "chunk")[int(out[0])], *map(int, out[1:]))
+
+
+def project_split(rows, heads, k, room=0):
+    """Projection of 65 rows and more: (128-token blocks a tile, workgroups that share its K, their sums' floats, a handle's room)"""
+    out = subprocess.run([_program(), "p", *map(str, (rows, heads, k, room))], check=True, capture_output=True, text=True)
+    return tuple(map(int, out.stdout.split()))
 
 
 def _chunk(batch_capacity, batch, q_heads, kv_heads, position_index, interval, most=None, bf16=False):
