@@ -115,6 +115,10 @@ hipError_t launch_positions_advance(uint32_t* positions, uint32_t n, uint32_t by
 // p[i] = value for i < n: a kernel, not a memset node, so that it can be recorded into a graph.
 hipError_t launch_fill_u32(uint32_t* p, size_t n, uint32_t value, hipStream_t stream);
 
+// Merge launches of split chunk calls: lanes up to which several share a row's partials (more partials than a lane takes
+// at once); beyond, one lane takes them all.
+constexpr size_t kMergeLanes = (size_t)1 << 19;
+
 // Projection C = X . W^T on MFMA with the per-head epilogue (see project.hip).
 // Column segment 0 (heads0 heads, weights w0) goes row-major to out0 [rows][heads0 * 128],
 // optionally normalised + rotated (finalize0) and with `residual` added; segments 1 and 2

@@ -1336,7 +1336,7 @@ __global__ __launch_bounds__(WR* WK* kWave, 2) void short_prompt_kernel(PrefillK
 // its workgroup sees, as in the kernel above; a split whose keys are all masked for this row
 // left (max = -inf, sum = 0) and weighs nothing.  Split 0 always holds key 0, so the maximum
 // is finite.
-template <typename T, int G>
+template <typename T, int G, int TURN>
 __global__ __launch_bounds__(256) void prefill_merge_kernel(PrefillKernelArgs p, uint32_t batch) {
   const uint32_t quads = kHeadDim / 4;
   const size_t items = (size_t)p.interval * batch * p.n_q_heads * quads;
@@ -1355,26 +1355,10 @@ __global__ __launch_bounds__(256) void prefill_merge_kernel(PrefillKernelArgs p,
   const uint32_t all_tiles = (p.position_index + wg_last_tok) / kBK + 1;
   const uint32_t live = (all_tiles + p.split_tiles - 1) / p.split_tiles;
   const size_t row = ((size_t)tok * p.batch_pitch + seq) * p.n_q_heads + head;
-  const float* ml = p.part_ml + row * p.n_split * 2;
-  const float* po = p.part_o + row * p.n_split * kHeadDim + 4 * dq;
-  float m = -INFINITY;
-  for (uint32_t s = sub; s < live; s += G) m = fmaxf(m, ml[2 * s]);
-#pragma unroll
-  for (int x = 1; x < G; x <<= 1) m = fmaxf(m, __shfl_xor(m, x));
-  float l = 0.0f;
-  f32x4 o = {0.0f, 0.0f, 0.0f, 0.0f};
-  for (uint32_t s = sub; s < live; s += G) {
-    const float ms = ml[2 * s];
-    const float w = (ms == -INFINITY) ? 0.0f : fast_exp2(ms - m);
-    l += w * ml[2 * s + 1];
-    o += w * *(const f32x4*)(po + (size_t)s * kHeadDim);
-  }
-#pragma unroll
-  for (int x = 1; x < G; x <<= 1) {
-    l += __shfl_xor(l, x);
-#pragma unroll
-    for (int e = 0; e < 4; ++e) o[e] += __shfl_xor(o[e], x);
-  }
+  float l;
+  f32x4 o;
+  const float m = fold_splits<G, TURN>(p.part_ml + row * p.n_split * 2, p.part_o + row * p.n_split * kHeadDim + 4 * dq, kHeadDim,
+                                 sub, live, l, o);
   if (!valid || sub != 0) return;
   const float inv = 1.0f / l;
   u32x2 w;
@@ -1466,11 +1450,15 @@ hipError_t launch_chunk(const AttnArgs& a, hipStream_t stream) {
     hipLaunchKernelGGL(kernel, dim3((uint32_t)((items * lanes + 255) / 256)), dim3(256), 0, stream, p, a.batch);
     return hipGetLastError();
   };
-  // lanes per item: more when there are many splits to walk, as long as the grid stays small
-  constexpr size_t kLanesMax = (size_t)1 << 21;
-  if (p.n_split > 32 && items * 64 <= kLanesMax) return merge(prefill_merge_kernel<T, 64>, 64);
-  if (p.n_split > 8 && items * 8 <= kLanesMax) return merge(prefill_merge_kernel<T, 8>, 8);
-  return merge(prefill_merge_kernel<T, 1>, 1);
+  // Lanes a row's partials are shared by and partials a lane takes at once: eight lanes where there are more than eight
+  // and the grid stays small, 64 from 33 on; else one.  One partial a trip to memory / this (us, the call): 189 tokens on 4704,
+  // 32 / 4 heads, 10 pieces 37.8 / 30.7 (eight lanes there 36.0); 16 x 4 on 8000, 26 pieces 33.7 / 32.0; 34 x 5 on 28920, 13
+  // 127.8 / 123.5; 110 x 2 on 3656, 8 30.1 / 29.3 (eight at once 29.4); 24 x 24 on 8191, 3 114 / 113.
+  if (p.n_split > 8 && items * 8 <= kMergeLanes) {
+    if (p.n_split > 32) return merge(prefill_merge_kernel<T, 64, 4>, 64);
+    return p.n_split > 16 ? merge(prefill_merge_kernel<T, 8, 4>, 8) : merge(prefill_merge_kernel<T, 8, 2>, 8);
+  }
+  return p.n_split > 2 ? merge(prefill_merge_kernel<T, 1, 4>, 1) : merge(prefill_merge_kernel<T, 1, 2>, 1);
 }
 
 }  // namespace

@@ -138,6 +138,26 @@ def test_values_beyond_a_row_are_not_seen(dtype, hq, hkv, hs, p0, s):
     assert np.isposinf(got[-1]).all() and np.abs(lse[-1] - want_lse[-1]).max() <= 1e-4
 
 
+@pytest.mark.parametrize("dtype,hs", [(orc.F16, 64), (orc.BF16, 96), (orc.F16, 256)])
+@pytest.mark.parametrize("p0", [31, 32, 33, 63, 64, 95, 127])
+def test_one_value_beyond_a_row_at_the_edges_of_steps(dtype, hs, p0):
+    """The chunk kernel looks at values only from the first step on whose keys its first row must not see: one infinite
+    element, in either half of a register, in the value row right behind that row's position."""
+    s, hq, hkv = 40, 4, 1
+    q, k, v = (_rand(n, 71 + i, dtype) for i, n in enumerate(((s, 1, hq, hs), (1, hkv, p0 + s, hs), (1, hkv, p0 + s, hs))))
+    print("p0", p0, "head", hs, flush=True)
+    assert plan_probe.general_plan(hs, 2, 1, 1, hq, hkv, p0, s)[0] == "chunk"
+    want, want_lse = orc.attention(q, k, v, hs ** -0.5, dtype, position_index=p0)
+    for column in (0, hs - 1):
+        v2 = v.copy()
+        v2.view(np.uint16)[:, :, p0 + 1, column] = 0x7C00 if dtype == orc.F16 else 0x7F80
+        got, lse = _run(q, k, v2, hs ** -0.5, dtype, p0=p0)
+        _check("infinite_next_value", got[:1], lse[:1], want[:1], want_lse[:1], dtype, 1)
+        assert np.isposinf(got[1:, ..., column]).all()
+        keep = np.arange(hs) != column
+        _check("other_columns", got[1:][..., keep], lse[1:], want[1:][..., keep], want_lse[1:], dtype, 1)
+
+
 # (q heads, kv heads, head size, position_index, interval): chunk kernel with one, two and four key groups and with a
 # key split, step kernel with one and several splits, several tokens
 INFINITE = [(8, 8, 64, 20, 40), (8, 2, 64, 400, 40), (4, 4, 192, 300, 140), (8, 1, 96, 1500, 9), (4, 4, 80, 40, 1),
