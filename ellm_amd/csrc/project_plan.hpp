@@ -59,10 +59,13 @@ inline ProjectSplit project_split(uint32_t rows, uint32_t heads, uint32_t K, uin
   return best;
 }
 
-// Room that the calls of up to max_rows rows of a matrix can use (at most 256 tokens x 128 columns a unit).
+// Room that the calls of up to max_rows rows of a matrix can use (at most 256 tokens x 128 columns a unit): what the
+// plans at every 32nd row take.
 inline size_t project_split_room(uint32_t heads, uint32_t K, uint32_t n_cu, size_t max_rows) {
   size_t most = 0;
-  for (uint32_t rows = 65; rows <= max_rows && ((size_t)rows + 127) / 128 * heads <= n_cu; ++rows) {
+  for (uint32_t last = 96; last < max_rows + 32 && ((size_t)last + 127) / 128 * heads <= n_cu; last += 32) {
+    const uint32_t rows = last < max_rows ? last : (uint32_t)max_rows;
+    if (rows < 65) continue;
     const size_t f = split_floats(project_split(rows, heads, K, n_cu, (size_t)-1), rows, heads);
     if (f > most) most = f;
   }
