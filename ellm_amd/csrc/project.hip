@@ -138,6 +138,7 @@ hipError_t launch_project(const ProjectArgs& a, hipStream_t stream) {
   p.finalize0 = a.finalize0;
   p.eps = a.eps;
   p.k_split = 1;
+  p.half_heads = 0;
   p.part = nullptr;
   const uint32_t heads = a.heads0 + 2 * a.heads_kv;
   const int path = project_path(a.rows, heads, a.K, a.ws && a.counters);
@@ -151,6 +152,7 @@ hipError_t launch_project(const ProjectArgs& a, hipStream_t stream) {
     const ProjectSplit split = project_split(a.rows, heads, a.K, g_n_cu, a.part_floats);
     if (split.k_split > 1) {
       p.k_split = split.k_split;
+      p.half_heads = split.half_heads;
       p.part = a.part;
       return launch_project_mid(p, split.token_blocks, a.dtype, a.residual != nullptr, stream);
     }

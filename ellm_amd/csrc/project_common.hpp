@@ -32,6 +32,7 @@ struct ProjectKernelArgs {
   uint32_t whole_tiles, tail_parts;   // project_kernel: tiles of 256 x 256; workgroups per tile of the rest
   uint32_t band_m;                    // project_mid_kernel: token tiles that take turns on one head
   uint32_t k_split;                   // ... and workgroups that share a tile's K (one: 0 or 1)
+  uint32_t half_heads;                // ... 128-token tiles: eight waves of half a head each, not four of a head
   float* part;                        // their sums, [k_split][rows][columns]
   uint32_t position_index, max_start;
   uint32_t finalize0;        // segment 0 rows are normalised and rotated

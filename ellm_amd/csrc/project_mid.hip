@@ -15,7 +15,7 @@ namespace ellm {
 namespace proj {
 namespace {
 
-template <typename S, int MODE, int MB, int WAVES>
+template <typename S, int MODE, int MB, int WAVES, int CH = 1>
 __global__ __launch_bounds__(64 * WAVES) void project_mid_kernel(ProjectKernelArgs p) {
   extern __shared__ __attribute__((aligned(16))) uint8_t mid_smem[];
   // workgroup -> tile: ids that share id % 8 (one XCD, one L2) are made consecutive; a band of
@@ -26,7 +26,7 @@ __global__ __launch_bounds__(64 * WAVES) void project_mid_kernel(ProjectKernelAr
   const uint32_t per_band = p.band_m * p.tiles_n;
   const uint32_t first_m = pid / per_band * p.band_m, in_band = pid % per_band;
   const uint32_t here = min(p.tiles_m - first_m, p.band_m);
-  mid_tile<S, MODE, MB, WAVES, 1>(p, (first_m + in_band % here) * MidShape<MB, WAVES, 1>::kTokens, in_band / here, mid_smem);
+  mid_tile<S, MODE, MB, WAVES, 1, CH>(p, (first_m + in_band % here) * MidShape<MB, WAVES, 1, CH>::kTokens, in_band / here, mid_smem);
 }
 
 // Sums of the pieces of K, in order, and what the tiles' epilogue does with a finished head: 16 lanes a (row, head),
@@ -93,7 +93,9 @@ hipError_t prepare_shape() {
                            (const void*)project_mid_kernel<F16, kModeAdd, MB, WAVES>,
                            (const void*)project_mid_kernel<BF16, kModeAdd, MB, WAVES>,
                            (const void*)project_mid_kernel<F16, kModePart, MB, WAVES>,
-                           (const void*)project_mid_kernel<BF16, kModePart, MB, WAVES>};
+                           (const void*)project_mid_kernel<BF16, kModePart, MB, WAVES>,
+                           (const void*)project_mid_kernel<F16, kModePart, MB, 8, 8 / WAVES>,
+                           (const void*)project_mid_kernel<BF16, kModePart, MB, 8, 8 / WAVES>};
   for (const void* k : kernels) {
     const hipError_t e =
         hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, MidShape<MB, WAVES, 1>::kLdsBytes);
@@ -137,8 +139,18 @@ hipError_t launch_shape(ProjectKernelArgs p, int dtype, bool add, hipStream_t st
     return hipGetLastError();
   };
   if (p.k_split > 1) {
-    hipLaunchKernelGGL((dtype == 0 ? project_mid_kernel<F16, kModePart, MB, WAVES> : project_mid_kernel<BF16, kModePart, MB, WAVES>),
-                       dim3(blocks, p.k_split), dim3(Shape::kThreads), Shape::kLdsBytes, stream, p);
+    constexpr int kHalves = 8 / WAVES;   // (1: the same kernel)
+    using Halves = MidShape<MB, 8, 1, kHalves>;
+    static_assert(Halves::kTokens == Shape::kTokens && Halves::kRingBytes <= Shape::kLdsBytes, "the same tile");
+    auto pieces = [&](auto kernel, uint32_t threads) {
+      hipLaunchKernelGGL(kernel, dim3(blocks, p.k_split), dim3(threads), Shape::kLdsBytes, stream, p);
+    };
+    if (p.half_heads)
+      dtype == 0 ? pieces(project_mid_kernel<F16, kModePart, MB, 8, kHalves>, Halves::kThreads)
+                 : pieces(project_mid_kernel<BF16, kModePart, MB, 8, kHalves>, Halves::kThreads);
+    else
+      dtype == 0 ? pieces(project_mid_kernel<F16, kModePart, MB, WAVES>, Shape::kThreads)
+                 : pieces(project_mid_kernel<BF16, kModePart, MB, WAVES>, Shape::kThreads);
     const hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
     const dim3 grid((p.rows * p.tiles_n + 15) / 16);

@@ -2,7 +2,8 @@
 // project_kernel.  C^T = W . X^T on v_mfma_f32_16x16x32, a lane owns tokens; a wave owns one head (eight
 // blocks of 16 columns) x 32 MB tokens.  K runs in chunks of 64 (one 128-byte line of every operand row)
 // that go from memory straight into LDS, through two to four stages.
-// Every shape adds up K in the same order, so an output's bits do not depend on the shape that made it.
+// Every shape adds up K in the same order, so an output's bits do not depend on the shape that made it (pieces of K are
+// added to each other afterwards, in order: those bits depend on the plan, that is on the sizes, alone).
 //
 // What bounds it: on ordinary operands the board's power, and with it the time the matrix pipe idles.
 // A 256 x 256 x 64 loop on N(0,1) operands, probe kernels, TFLOP/s: 32x32x16 instructions 1494-1543 without
@@ -19,11 +20,12 @@ namespace proj {
 constexpr int kMidKc = 64;                        // K elements per chunk: one 128-byte line per row
 constexpr int kMidRowPitch = kMidKc * 2;          // unpadded; pieces permuted
 // Forms in use, all with 32 MB tokens a wave: 4 waves x (MB 1) x one head = 128 x 128; 8 x (MB 1) x one head =
-// 256 x 128; 8 x (MB 2) x two heads = 256 x 256.
-template <int MB, int WAVES, int HEADS>
+// 256 x 128; 8 x (MB 2) x two heads = 256 x 256.  CH 2: a wave owns half of a head's columns (kModePart, whose
+// epilogue needs no whole rows): 8 waves x (MB 1) x half a head = 128 x 128, two waves a SIMD.
+template <int MB, int WAVES, int HEADS, int CH = 1>
 struct MidShape {
   static constexpr int kThreads = 64 * WAVES;
-  static constexpr int kTokens = 32 * MB * WAVES / HEADS;
+  static constexpr int kTokens = 32 * MB * WAVES / (HEADS * CH);
   static constexpr int kStageBytes = (kTokens + HEADS * kHeadDim) * kMidRowPitch;  // X rows then W rows: 32, 48 or 64 KB
   // Small chunks: three or four stages, chunk c in stage c % kStages, chunk c + kStages - 1 requested early in
   // iteration c.  64 KB chunks (kHalves): five slots of half a chunk, weight rows of chunk c in slot 2 c % 5, token
@@ -44,22 +46,23 @@ struct MidShape {
   // loads a wave may still have outstanding where it waits for its pieces of the next chunk, and before the
   // loop for those of the first one (the literals of mid_tile's s_waitcnt)
   static constexpr int kMayBePending = kHalves ? kWLoads : (kStages - 2) * kLoads;
-  static_assert(kMayBePending == (kHalves ? 4 : (WAVES == 8 ? 6 : 16)), "s_waitcnt vmcnt literals in mid_tile");
-  static_assert((kXAhead - 1) * kXLoads + (kWAhead - 1) * kWLoads == (kHalves ? 12 : (WAVES == 8 ? 6 : 16)), "s_waitcnt vmcnt literals in mid_tile");
+  static_assert(kMayBePending == (kHalves ? 4 : CH == 2 ? 8 : (WAVES == 8 ? 6 : 16)), "s_waitcnt vmcnt literals in mid_tile");
+  static_assert((kXAhead - 1) * kXLoads + (kWAhead - 1) * kWLoads == (kHalves ? 12 : CH == 2 ? 8 : (WAVES == 8 ? 6 : 16)), "s_waitcnt vmcnt literals in mid_tile");
   static_assert(kLdsBytes <= 160 * 1024, "LDS of a compute unit");
 };
 
 // The tile of token rows row0.. x heads head0.., by a workgroup of WAVES waves.
-template <typename S, int MODE, int MB, int WAVES, int HEADS>
+template <typename S, int MODE, int MB, int WAVES, int HEADS, int CH = 1>
 __device__ __forceinline__ void mid_tile(const ProjectKernelArgs& p, uint32_t row0, uint32_t head0, uint8_t* mid_smem) {
   using M = Mfma<S>;
-  using Shape = MidShape<MB, WAVES, HEADS>;
+  using Shape = MidShape<MB, WAVES, HEADS, CH>;
+  static_assert(CH == 1 || (MODE == kModePart && HEADS == 1), "half heads");
   constexpr int kLoads = Shape::kLoads;
   constexpr bool kHalves = Shape::kHalves;
   constexpr int kXLoads = Shape::kXLoads, kHeadLoads = Shape::kWLoads / HEADS, TB = 2 * MB;
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int c16 = lane & 15, g = lane >> 4;
-  const int wn = wave % HEADS, wm = wave / HEADS;
+  const int wn = wave % HEADS, wm = wave / (HEADS * CH), half = CH == 2 ? wave % 2 : 0;
   const uint32_t K = p.K;
   // kModePart: piece blockIdx.y of K, as many chunks as the others or one more
   const uint32_t all_chunks = K / kMidKc, first_chunk = MODE == kModePart ? blockIdx.y * all_chunks / p.k_split : 0u;
@@ -141,9 +144,10 @@ __device__ __forceinline__ void mid_tile(const ProjectKernelArgs& p, uint32_t ro
   constexpr uint32_t kX0 = kHalves ? Shape::kSlotBytes : 0, kW0 = kHalves ? 0 : Shape::kTokens * kMidRowPitch;
   auto next_at = [](uint32_t at) { return at + kStep >= (uint32_t)Shape::kRingBytes ? at + kStep - Shape::kRingBytes : at + kStep; };
 
-  f32x4 acc[8][TB];  // [16 columns][16 tokens]
+  constexpr int kNb = 8 / CH, kOps = 2 * kNb;   // blocks of 16 columns; weight operands a chunk
+  f32x4 acc[kNb][TB];  // [16 columns][16 tokens]
 #pragma unroll
-  for (int nb = 0; nb < 8; ++nb)
+  for (int nb = 0; nb < kNb; ++nb)
 #pragma unroll
     for (int t = 0; t < TB; ++t) acc[nb][t] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
 
@@ -152,7 +156,7 @@ __device__ __forceinline__ void mid_tile(const ProjectKernelArgs& p, uint32_t ro
   // entered (opaque, so that every read is an immediate offset on top of it).
   const uint32_t swz = (c16 >> 1) & 7;
   const uint32_t x_row = lds0 + (wm * 32 * MB + c16) * kMidRowPitch;
-  const uint32_t w_row = lds0 + (wn * kHeadDim + c16) * kMidRowPitch;
+  const uint32_t w_row = lds0 + (wn * kHeadDim + half * 64 + c16) * kMidRowPitch;
   auto base = [&](uint32_t row, int st, uint32_t stage) __attribute__((always_inline)) {
     uint32_t at = row + ((4 * st + g) ^ swz) * 16 + stage;
     asm volatile("" : "+v"(at));
@@ -186,6 +190,8 @@ __device__ __forceinline__ void mid_tile(const ProjectKernelArgs& p, uint32_t ro
   if constexpr (MB == 1 && MODE != kModePart) head = prepare_head<S, MODE, MB>(p, head0 + wn, row0 + 32 * MB * wm, lane);
   if constexpr (kHalves)
     asm volatile("s_waitcnt vmcnt(12)" ::: "memory");
+  else if constexpr (CH == 2)
+    asm volatile("s_waitcnt vmcnt(8)" ::: "memory");
   else if constexpr (WAVES == 8)
     asm volatile("s_waitcnt vmcnt(6)" ::: "memory");
   else
@@ -198,9 +204,9 @@ __device__ __forceinline__ void mid_tile(const ProjectKernelArgs& p, uint32_t ro
   // it has returned, the wave waits for its own pieces of the next chunk and meets the others at the
   // iteration's one barrier, and the reads that would have touched the next stage in between are made up.
   // The barrier orders both hazards: the next chunk is complete, and the stage behind it is read.
-  constexpr int kRing = TB == 4 ? 6 : 8;
-  constexpr int kBarrier = TB == 4 ? 11 : 10;
-  static_assert(kBarrier > 15 - kRing && kBarrier < 15, "the barrier stands behind the last read of a stage");
+  constexpr int kRing = CH == 2 ? 4 : TB == 4 ? 6 : 8;
+  constexpr int kBarrier = CH == 2 ? 5 : TB == 4 ? 11 : 10;
+  static_assert(kBarrier > kOps - 1 - kRing && kBarrier < kOps - 1 && kRing <= kNb && (kHalves || kLoads <= kBarrier), "the barrier stands behind the last read of a stage");
   u32x4 xop[2][TB], wop[kRing];
 #pragma unroll
   for (int t = 0; t < TB; ++t) xop[0][t] = read_block(base(x_row, 0, kX0), t);
@@ -210,10 +216,10 @@ __device__ __forceinline__ void mid_tile(const ProjectKernelArgs& p, uint32_t ro
   uint32_t cur_x = kX0, cur_w = kW0;
   uint32_t prev = Shape::kRingBytes - kStep;   // stage of the chunk before (not kHalves)
   // (kRing may not divide 16: the ring index runs on over a period of chunks)
-  constexpr int kPeriod = 16 % kRing == 0 ? 1 : 3;
-  static_assert(16 * kPeriod % kRing == 0, "ring position at the start of a period");
+  constexpr int kPeriod = kOps % kRing == 0 ? 1 : 3;
+  static_assert(kOps * kPeriod % kRing == 0, "ring position at the start of a period");
   auto chunk_step = [&](auto phase_, uint32_t c) __attribute__((always_inline)) {
-    constexpr int at = 16 * decltype(phase_)::value;   // operands before this chunk in its period
+    constexpr int at = kOps * decltype(phase_)::value;   // operands before this chunk in its period
     const uint32_t nxt_x = next_at(cur_x), nxt_w = next_at(cur_w);
     if constexpr (kHalves) {
       aim_x(c + 2, cur_w);   // (slot 2 (c + 2) + 1 = 2 c modulo 5)
@@ -224,19 +230,21 @@ __device__ __forceinline__ void mid_tile(const ProjectKernelArgs& p, uint32_t ro
     }
     const uint32_t x1 = base(x_row, 1, cur_x), w1 = base(w_row, 1, cur_w), x0 = base(x_row, 0, nxt_x), w0 = base(w_row, 0, nxt_w);
     __builtin_amdgcn_sched_barrier(0);
-    static_for<16>([&](auto o_) {
+    static_for<kOps>([&](auto o_) {
       constexpr int o = decltype(o_)::value;
-      constexpr int st = o >> 3, nb = o & 7;
+      constexpr int st = o / kNb, nb = o % kNb;
 #pragma unroll
       for (int t = 0; t < TB; ++t) {
         const int tt = (nb & 1) ? TB - 1 - t : t;
         acc[nb][tt] = M::m16x16x32(wop[(at + o) % kRing], xop[st][tt], acc[nb][tt]);
       }
-      if constexpr (o + kRing < 16) wop[(at + o) % kRing] = o + kRing < 8 ? read_block(w_at, o + kRing) : read_block(w1, o + kRing - 8);
+      if constexpr (o + kRing < kOps) wop[(at + o) % kRing] = o + kRing < kNb ? read_block(w_at, o + kRing) : read_block(w1, o + kRing - kNb);
       if constexpr (o < TB) xop[1][o] = read_block(x1, o);
       if constexpr (o == kBarrier) {
         if constexpr (kHalves)
           asm volatile("s_waitcnt vmcnt(4) lgkmcnt(0)" ::: "memory");
+        else if constexpr (CH == 2)
+          asm volatile("s_waitcnt vmcnt(8) lgkmcnt(0)" ::: "memory");
         else if constexpr (WAVES == 8)
           asm volatile("s_waitcnt vmcnt(6) lgkmcnt(0)" ::: "memory");
         else
@@ -245,11 +253,11 @@ __device__ __forceinline__ void mid_tile(const ProjectKernelArgs& p, uint32_t ro
 #pragma unroll
         for (int t = 0; t < TB; ++t) xop[0][t] = read_block(x0, t);
 #pragma unroll
-        for (int k = 16; k <= o + kRing; ++k) wop[(at + k) % kRing] = read_block(w0, k - 16);
+        for (int k = kOps; k <= o + kRing; ++k) wop[(at + k) % kRing] = read_block(w0, k - kOps);
       }
-      if constexpr (o > kBarrier) wop[(at + o) % kRing] = read_block(w0, o + kRing - 16);
+      if constexpr (o > kBarrier) wop[(at + o) % kRing] = read_block(w0, o + kRing - kOps);
       if constexpr (kHalves) {
-        constexpr int kSlots = 15 - kBarrier, kEach = (kLoads + kSlots - 1) / kSlots;
+        constexpr int kSlots = kOps - 1 - kBarrier, kEach = (kLoads + kSlots - 1) / kSlots;
         if constexpr (o > kBarrier) {
 #pragma unroll
           for (int i = 0; i < kEach; ++i)
@@ -284,9 +292,9 @@ __device__ __forceinline__ void mid_tile(const ProjectKernelArgs& p, uint32_t ro
     for (int t = 0; t < TB; ++t) {
       const uint32_t row = row0 + 32 * MB * wm + 16 * t + c16;
       if (row >= p.rows) continue;
-      float* to = p.part + ((size_t)blockIdx.y * p.rows + row) * n_cols + (head0 + wn) * kHeadDim + 4 * g;
+      float* to = p.part + ((size_t)blockIdx.y * p.rows + row) * n_cols + (head0 + wn) * kHeadDim + 64 * half + 4 * g;
 #pragma unroll
-      for (int nb = 0; nb < 8; ++nb) *(f32x4*)(to + 16 * nb) = acc[nb][t];
+      for (int nb = 0; nb < kNb; ++nb) *(f32x4*)(to + 16 * nb) = acc[nb][t];
     }
     return;
   }

@@ -8,9 +8,11 @@
 namespace ellm {
 namespace proj {
 
-// Tiles of 128 token_blocks tokens x one head, k_split workgroups a tile (1: K stays whole).
+// Tiles of 128 token_blocks tokens x one head, k_split workgroups a tile (1: K stays whole), with 128 tokens of four waves
+// of a head each or eight of half a head.
 struct ProjectSplit {
   uint32_t token_blocks, k_split;
+  bool half_heads;
 };
 
 inline size_t split_floats(const ProjectSplit& s, uint32_t rows, uint32_t heads) {
@@ -32,23 +34,29 @@ inline double project_tiles_us(const ProjectSplit& s, uint32_t rows, uint32_t he
 
 // Three to eight workgroups a tile, all of them at once, one per unit, pieces of at least four chunks, sums within
 // `room` floats; where that is estimated 5 % below one round of whole tiles.  Two a tile gained nothing that lasts
-// (2048 <- 4096, 700 rows 32.9 / 33.0).  Whole / shared, weights from memory, f16 (us; tokens a tile / pieces):
+// (2048 <- 4096, 700 rows 32.9 / 33.0), nor did three of 256 tokens below 96 chunks (a layer of 800 rows, 2048 wide, 73.7 /
+// 75.0; 4096 <- 4096, 400 rows 31.7 / 30.9), nor any of 256 tokens on all units at once (those 800 rows, four, 73.1 / 78.0).  Whole / shared, weights from memory, f16 (us; tokens a tile / pieces):
 //   2048 <- 4096   79 rows 32.4 / 14.6 (128 / 8)   128 37.2 / 16.0 (128 / 8)   234 35.2 / 18.6 (128 / 8)   400 30.0 / 22.6 (128 / 4)
 //                  700 32.9 / 28.1 (256 / 4)
 //   5120 <- 2048   79 21.0 / 15.5 (128 / 6)   128 23.4 / 17.8 (128 / 6)   400 stays whole: 20.3 / 26.2 and more
-//   4096 <- 4096   79 34.7 / 17.8 (128 / 8)   128 39.6 / 20.3   234 37.2 / 23.7 (128 / 4)   400 31.7 / 30.9 (256 / 3)
+//   4096 <- 4096   79 34.7 / 17.8 (128 / 8)   128 39.6 / 20.3   234 37.2 / 23.7 (128 / 4)   400 stays whole
 //   10240 <- 8192  79 67.6 / 45.1 (128 / 3)   128 77.2 / 49.7   234 73.3 / 63.3 (256 / 3)
 //   8192 <- 8192   79 64.8 / 42.9 (128 / 4)   128 74.5 / 46.9   234 70.5 / 56.9 (256 / 4)
+// These with four waves a workgroup of 128 tokens.  One wave a SIMD waits for every operand; eight waves of half a head read
+// a fifth more from LDS, but take turns (layer of a chunk, four / eight waves: 2048 wide, 65 rows 32.5 / 28.1, 128 37.3 /
+// 33.0, 300 46.5 / 42.4; 4096 wide, 128 55.4 / 51.8; 8192 wide, 65 82.2 / 75.2, 128 93.7 / 90.7), except where all units are
+// at work: 500 rows 2048 wide, 256 workgroups, 52.5 / 55.5; 256 rows 4096 wide 62.7 / 64.2.
 inline ProjectSplit project_split(uint32_t rows, uint32_t heads, uint32_t K, uint32_t n_cu, size_t room) {
-  const ProjectSplit whole = {1, 1};
+  const ProjectSplit whole = {1, 1, false};
   if (((size_t)rows + 127) / 128 * heads > n_cu) return whole;
   ProjectSplit best = whole;
   double best_us = 0.95 * project_tiles_us(whole, rows, heads, K);
   for (uint32_t blocks = 1; blocks <= 2; ++blocks) {
     const uint32_t tiles = (rows + 128 * blocks - 1) / (128 * blocks) * heads;
-    for (uint32_t n = 3; n <= 8 && n * tiles <= n_cu && 4 * n <= K / 64; ++n) {
-      const ProjectSplit s = {blocks, n};
-      if (split_floats(s, rows, heads) > room) break;
+    for (uint32_t n = blocks == 2 && K / 64 < 96 ? 4 : 3; n <= 8 && n * tiles <= n_cu && 4 * n <= K / 64; ++n) {
+      const bool spare = 16 * n * tiles <= 15 * n_cu;
+      const ProjectSplit s = {blocks, n, blocks == 1 && spare};
+      if (split_floats(s, rows, heads) > room || (blocks == 2 && !spare)) break;
       const double us = project_tiles_us(s, rows, heads, K);
       if (us < best_us) {
         best_us = us;

@@ -22,7 +22,7 @@ static int project(char** v) {   // rows, heads, K, room (0: what a handle for t
   for (int i = 1; i <= 4; ++i) a[i] = (uint32_t)strtoul(v[i + 1], nullptr, 10);
   const size_t room = a[4] ? a[4] : proj::project_split_room(a[2], a[3], 256, a[1]);
   const proj::ProjectSplit s = proj::project_split(a[1], a[2], a[3], 256, room);
-  printf("%u %u %zu %zu\n", s.token_blocks, s.k_split, proj::split_floats(s, a[1], a[2]), room);
+  printf("%u %u %zu %zu %d\n", s.token_blocks, s.k_split, proj::split_floats(s, a[1], a[2]), room, (int)s.half_heads);
   return 0;
 }
 static int chunk(char** v) {   // batch capacity, batch, query heads, key-value heads, most positions a call, position_index, interval, bfloat16
@@ -83,7 +83,8 @@ def general_plan(head_size, element_bytes, batch_capacity, batch, q_heads, kv_he
 
 
 def project_split(rows, heads, k, room=0):
-    """Projection of 65 rows and more: (128-token blocks a tile, workgroups that share its K, their sums' floats, a handle's room)"""
+    """Projection of 65 rows and more: (128-token blocks a tile, workgroups that share its K, their sums' floats, a handle's room,
+    whether eight waves of half a head walk a tile)"""
     out = subprocess.run([_program(), "p", *map(str, (rows, heads, k, room))], check=True, capture_output=True, text=True)
     return tuple(map(int, out.stdout.split()))
 

@@ -12,20 +12,25 @@ from test_gpu_projection import TILES_128, _path, _rope_table, _run_matmul3, _we
 
 pytestmark = pytest.mark.gpu
 
-# interval, pitch, batch, K, q heads, kv heads, position_index, dtype, (128-token blocks a tile, pieces)
+# interval, pitch, batch, K, q heads, kv heads, position_index, dtype, (128-token blocks a tile, pieces, half heads)
 QKV = [
-    (65, 1, 1, 64 * 33, 1, 1, 3, orc.F16, (1, 7)),      # 33 chunks in seven pieces, one token tile a quarter empty and a row beyond half
-    (44, 3, 2, 64 * 40, 3, 1, 9, orc.BF16, (1, 8)),     # 131 rows: a second tile of three; a sequence beyond batch_size
-    (1, 100, 97, 2048, 32, 4, 40, orc.F16, (1, 4)),     # one token for a hundred sequences
-    (130, 1, 1, 8192, 52, 4, 0, orc.BF16, (2, 3)),      # 256-token tiles, half of them empty
+    (65, 1, 1, 64 * 33, 1, 1, 3, orc.F16, (1, 7, 1)),      # 33 chunks in seven pieces, one token tile a quarter empty and a row beyond half
+    (44, 3, 2, 64 * 40, 3, 1, 9, orc.BF16, (1, 8, 1)),     # 131 rows: a second tile of three; a sequence beyond batch_size
+    (1, 100, 97, 2048, 32, 4, 40, orc.F16, (1, 4, 1)),     # one token for a hundred sequences
+    (130, 1, 1, 8192, 52, 4, 0, orc.BF16, (2, 3, 0)),      # 256-token tiles, half of them empty
 ]
+
+
+def _plan(rows, heads, k):
+    plan = plan_probe.project_split(rows, heads, k)
+    return plan[0], plan[1], plan[4]
 
 
 @pytest.mark.parametrize("interval,pitch,batch,k,hq,hkv,p0,dtype,plan", QKV)
 def test_matmul3_pieces(interval, pitch, batch, k, hq, hkv, p0, dtype, plan):
     rows, heads, cap = (interval - 1) * pitch + batch, hq + 2 * hkv, p0 + interval + 5
     print("rows", rows, "heads", heads, "K", k, flush=True)
-    assert _path(rows, heads, k) == TILES_128 and plan_probe.project_split(rows, heads, k)[:2] == plan
+    assert _path(rows, heads, k) == TILES_128 and _plan(rows, heads, k) == plan
     hidden = rand_storage((interval, pitch, k), 11, dtype)
     w = _weights(k, hq, hkv, dtype, 20)
     positions = None if interval > 1 else (np.arange(pitch) % (cap - 1)).astype(np.uint32)
@@ -36,15 +41,15 @@ def test_matmul3_pieces(interval, pitch, batch, k, hq, hkv, p0, dtype, plan):
         assert r["ok"], (name, r)
 
 
-@pytest.mark.parametrize("rows,heads,k,dtype,plan", [(79, 16, 4096, orc.F16, (1, 8)), (385, 16, 64 * 63, orc.BF16, (2, 6)),
-                                                      (300, 12, 64 * 25, orc.F16, (1, 5))])
+@pytest.mark.parametrize("rows,heads,k,dtype,plan", [(79, 16, 4096, orc.F16, (1, 8, 1)), (480, 16, 64 * 61, orc.BF16, (1, 4, 0)), (385, 16, 64 * 63, orc.BF16, (2, 6, 0)),
+                                                      (300, 12, 64 * 25, orc.F16, (1, 5, 1))])
 def test_matmul_add_pieces(rows, heads, k, dtype, plan):
     import torch
 
     import ellm_amd
 
     print("rows", rows, "heads", heads, "K", k, flush=True)
-    assert _path(rows, heads, k) == TILES_128 and plan_probe.project_split(rows, heads, k)[:2] == plan
+    assert _path(rows, heads, k) == TILES_128 and _plan(rows, heads, k) == plan
     more = 128 * (256 // heads)       # whole tiles: a round of them
     assert _path(more, heads, k) == TILES_128 and plan_probe.project_split(more, heads, k)[1] == 1
     a = rand_storage((more, 1, k), 51, dtype)
