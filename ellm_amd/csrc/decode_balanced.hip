@@ -110,6 +110,11 @@ __global__ __launch_bounds__(kDecThreads, 2) void decode_balanced_kernel(DecodeK
     umin_all = uni(s_umin);
   }
 
+  // Units without keys in front of every plane's first (decode_shares.hpp).
+  const uint32_t charge = balanced_charge(umax_all, umin_all);
+  r_units += charge;
+  r_incl += charge * (t.lane + 1);
+  total_units += charge * B;
   // All of the index arithmetic is 32-bit (the launcher keeps calls with 2^31 units or more
   // away): a 64-bit division is a subroutine of a few hundred instructions, and a handful of
   // them per piece showed as 2 us on a 47 us launch.
@@ -128,7 +133,7 @@ __global__ __launch_bounds__(kDecThreads, 2) void decode_balanced_kernel(DecodeK
   // its own start-up that a second workgroup on the unit hides (400 planes of 100-4096 keys).
   // (decode_shares.hpp: balanced_workgroups, also walked by the CPU tests)
   const uint32_t planes_all = PL * B;
-  const uint32_t W = balanced_workgroups(gridDim.x, p.wgs_one, U, umax_all, umin_all, planes_all);
+  const uint32_t W = balanced_workgroups(gridDim.x, p.wgs_one, U, umax_all + charge, umin_all + charge, planes_all);
   // Workgroups are dealt to the eight XCDs by their id modulo 8.  Each XCD takes one contiguous
   // eighth of the shares, so that no two of them walk the same stretch of memory side by side
   // (with shares numbered like the workgroups and as many pieces per plane as XCDs, every XCD
@@ -161,30 +166,34 @@ __global__ __launch_bounds__(kDecThreads, 2) void decode_balanced_kernel(DecodeK
       uint32_t lo = 0, hi = B;
       while (hi - lo > 1) {
         const uint32_t mid = (lo + hi) >> 1;
-        if (PL * prefix[mid] <= x)
+        if (PL * (prefix[mid] + charge * mid) <= x)
           lo = mid;
         else
           hi = mid;
       }
       seq = uni(lo);
-      u_seq = uni(prefix[seq + 1] - prefix[seq]);
-      seq_start = uni(PL * prefix[seq]);
+      u_seq = uni(prefix[seq + 1] - prefix[seq] + charge);
+      seq_start = uni(PL * (prefix[seq] + charge * seq));
       pos = uni(s_pos[seq]);
     }
     const uint32_t r = x - seq_start;
     const uint32_t pl = r / u_seq, a = r - pl * u_seq;        // plane of the sequence, first unit in it
     const uint32_t S = seq_start + pl * u_seq, E = S + u_seq;
-    const uint32_t stop = min(x_end, E);
-    const uint32_t a_end = a + (stop - x);
+    const uint32_t stop = min(x_end, E), S_keys = S + charge;
+    if (stop <= S_keys) {   // (the share ends before the plane's first key)
+      x = uni(stop);
+      continue;
+    }
+    const uint32_t a_end = a + (stop - x) - charge;   // units of keys
     // the workgroups that hold the plane's first and last unit (this one, when the piece starts
     // or ends with the plane: no look-up then)
-    const uint32_t first_w = x == S ? w : holder(S);
+    const uint32_t first_w = x <= S_keys ? w : holder(S_keys);
     const uint32_t last_w = stop == E ? w : holder(E - 1);
     const uint32_t n_pieces = last_w - first_w + 1, piece = w - first_w;
     const uint32_t plane_id = seq * PL + pl;
     const uint32_t slot0 = balanced_slot0(first_w, plane_id);
 
-    const uint32_t k_begin = a * kUnitKeys;
+    const uint32_t k_begin = (max(a, charge) - charge) * kUnitKeys;
     const uint32_t k_end = min(pos + 1, a_end * kUnitKeys);
     const uint32_t kvh = pl / p.head_groups, hgrp = pl % p.head_groups;
     const uint32_t heads_here = min((uint32_t)kMaxHeadsPerGroup, p.group - hgrp * kMaxHeadsPerGroup);
@@ -260,7 +269,7 @@ bool decode_balanced_takes(const DecodeWorkspace& w, uint32_t batch, uint32_t n_
   const uint64_t head_groups = (group + kMaxHeadsPerGroup - 1) / kMaxHeadsPerGroup;
   const uint64_t planes = (uint64_t)batch * n_kv_heads * head_groups;
   const uint64_t units = planes * ((max_len + kUnitKeys - 1) / kUnitKeys);
-  if (units < 8ull * wgs || units + wgs >= (1ull << 31) || wgs >= (1u << 16)) return false;
+  if (units < 8ull * wgs || units + kBalancedCharge * planes + wgs >= (1ull << 31) || wgs >= (1u << 16)) return false;
   const uint64_t G = group < (uint32_t)kMaxHeadsPerGroup ? group : (uint32_t)kMaxHeadsPerGroup;
   const uint64_t slots = balanced_slots(wgs, (uint32_t)planes), cslots = balanced_cluster_slots(wgs, (uint32_t)planes);
   return slots * G <= w.rows && cslots * G <= w.rows2 && cslots + planes <= w.counters;

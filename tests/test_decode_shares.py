@@ -150,3 +150,38 @@ def test_a_walked_launch_numbers_its_pieces_without_collisions(tmp_path):
     launches, bad = (int(x) for x in subprocess.run([str(exe)], check=True, capture_output=True, text=True,
                                                     timeout=600).stdout.split())
     assert launches == 6000 and bad == 0
+
+
+# The same walk with what the start of a plane is charged: units without keys in front of its first.
+CHARGED = (
+    ("    const uint32_t U = PL * total, planes", """    const uint32_t charge = balanced_charge(umax, umin);
+    for (uint32_t b = 0; b < B; ++b) { units[b] += charge; prefix[b + 1] += charge * (b + 1); }
+    total += charge * B;
+    umax += charge;
+    umin += charge;
+    const uint32_t U = PL * total, planes"""),
+    ("        const uint32_t first_w = x == S ? w : shares.holder(S), last_w", """        if (stop <= S + charge) { covered += stop - x; x = stop; continue; }
+        const uint32_t first_w = x <= S + charge ? w : shares.holder(S + charge), last_w"""),
+    ("        pieces_of[plane_id] = n_pieces;", """        bad += ++seen[plane_id] > n_pieces || (pieces_of[plane_id] && pieces_of[plane_id] != n_pieces);
+        pieces_of[plane_id] = n_pieces;"""),
+    ("pieces_of(planes, 0), first_slot", "pieces_of(planes, 0), seen(planes, 0), first_slot"),
+    ("      if (n == 0) { ++bad; continue; }", "      if (n == 0 || seen[plane] != n) { ++bad; continue; }"),
+)
+
+
+def test_a_walked_launch_with_charged_starts(tmp_path):
+    """Shares that end inside a charge take no piece: every plane still has exactly the pieces its holders count."""
+    gxx = shutil.which("g++")
+    if not gxx:
+        pytest.skip("no g++")
+    text = WALK
+    for old, new in CHARGED:
+        assert text.count(old) == 1, old
+        text = text.replace(old, new)
+    src = tmp_path / "walk.cpp"
+    src.write_text(text)
+    exe = tmp_path / "walk"
+    subprocess.run([gxx, "-O2", "-std=c++17", "-Wall", "-I", CSRC, str(src), "-o", str(exe)], check=True, timeout=300)
+    launches, bad = (int(x) for x in subprocess.run([str(exe)], check=True, capture_output=True, text=True,
+                                                    timeout=600).stdout.split())
+    assert launches == 6000 and bad == 0
