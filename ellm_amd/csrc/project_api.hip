@@ -41,8 +41,13 @@ int alloc_small_workspace(uint32_t heads, size_t k, size_t max_rows, int* device
   if (prep != hipSuccess) return ellm::set_error(ELLM_ERR_HIP, "projection kernels: %s", hipGetErrorString(prep));
   const size_t floats = ellm::project_workspace_floats(heads);
   if (floats * sizeof(float) > (size_t)64 << 20) return ELLM_OK;
-  const size_t more = ellm::project_part_floats(heads, (uint32_t)k, max_rows);
+  size_t more = ellm::project_part_floats(heads, (uint32_t)k, max_rows);
   hipError_t e = hipMalloc((void**)ws, (floats + more) * sizeof(float));
+  if (e == hipErrorOutOfMemory && more) {   // K stays whole then
+    (void)hipGetLastError();
+    more = 0;
+    e = hipMalloc((void**)ws, floats * sizeof(float));
+  }
   if (e == hipSuccess) e = hipMalloc((void**)counters, heads * sizeof(uint32_t));
   if (e == hipSuccess) e = hipMemset(*counters, 0, heads * sizeof(uint32_t));
   if (e != hipSuccess) {
