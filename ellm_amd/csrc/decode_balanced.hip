@@ -111,7 +111,7 @@ __global__ __launch_bounds__(kDecThreads, 2) void decode_balanced_kernel(DecodeK
   }
 
   // Units without keys in front of every plane's first (decode_shares.hpp).
-  const uint32_t charge = balanced_charge(umax_all, umin_all);
+  const uint32_t charge = balanced_charge(umax_all, umin_all, total_units, B);
   r_units += charge;
   r_incl += charge * (t.lane + 1);
   total_units += charge * B;

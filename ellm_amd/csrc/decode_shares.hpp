@@ -56,9 +56,13 @@ ELLM_SHARES_FN uint32_t balanced_min_share(uint32_t longest_plane_units) {
 // on 4, f16, shares equal in keys / one / two / three units a start: 300 sequences of 64-2000 keys 110.1 / 103.7 / 104.6 /
 // 104.9 us, 200 of 1-600 38.2 / 31.7 / 31.2 / 31.4, 900 of 16-500 109.0 / 103.9 / 99.4 / 99.9, 28 of 115-3918 29.3 / 28.9 / 28.0 /
 // 28.5, 64 of 500-9000 101.0 / 99.9 / 98.7 / 98.9; 100 of 100-4096 71.8 / 71.1 / 71.6 / 71.8).  Planes of one length have as
-// many starts in every share, and their ends are to stay shares' ends: no charge.
+// many starts in every share, and their ends are to stay shares' ends: no charge.  Nor where planes have more than 512 units
+// on average: a start is below half a per cent of one, and the launch as often longer as shorter (32 of 1024-131072, two draws,
+// 662 / 657 and 488.5 / 491.7; below, 48 of 1000-30000 210.6 / 207.6, 10 of 1000-60000 184.2 / 183.0).
 constexpr uint32_t kBalancedCharge = 2;
-ELLM_SHARES_FN uint32_t balanced_charge(uint32_t umax, uint32_t umin) { return umax == umin ? 0 : kBalancedCharge; }
+ELLM_SHARES_FN uint32_t balanced_charge(uint32_t umax, uint32_t umin, uint32_t total, uint32_t sequences) {
+  return umax == umin || total > 512u * sequences ? 0 : kBalancedCharge;
+}
 // Workgroups that take part out of `limit`: at most one per unit of work and few enough for
 // balanced_min_share; with planes of equal length a whole number per plane (so that shares end
 // where planes end), else a multiple of eight (one contiguous eighth of the shares per XCD).

@@ -154,7 +154,7 @@ def test_a_walked_launch_numbers_its_pieces_without_collisions(tmp_path):
 
 # The same walk with what the start of a plane is charged: units without keys in front of its first.
 CHARGED = (
-    ("    const uint32_t U = PL * total, planes", """    const uint32_t charge = balanced_charge(umax, umin);
+    ("    const uint32_t U = PL * total, planes", """    const uint32_t charge = balanced_charge(umax, umin, total, B);
     for (uint32_t b = 0; b < B; ++b) { units[b] += charge; prefix[b + 1] += charge * (b + 1); }
     total += charge * B;
     umax += charge;
