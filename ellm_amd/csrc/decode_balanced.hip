@@ -6,7 +6,7 @@
 // sized for the longest sequence the call may hold; with lengths spread between 1k and 128k
 // (the single-token side of a mixed step) most workgroups then have a fraction of the longest
 // one's keys or none at all.  Here the unit of work is 64 keys of one plane; plane p has
-// u_p = ceil(length / 64) of them, all planes together U, and workgroup w of W takes units
+// u_p = ceil(length / 64) of them (and, for its start, up to two without keys: balanced_charge), all planes together U, and workgroup w of W takes units
 // [w U / W, (w + 1) U / W) of the concatenation: a stretch of one plane, or the end of one plane,
 // some whole planes and the start of another.  Each stretch (a "piece") runs the same stream, wave
 // merge and, where a plane has more than one piece, the same partial / arrival / fold steps as
