@@ -1452,8 +1452,8 @@ hipError_t launch_chunk(const AttnArgs& a, hipStream_t stream) {
   };
   // Lanes a row's partials are shared by and partials a lane takes at once: eight lanes where there are more than eight
   // and the grid stays small, 64 from 33 on; else one.  One partial a trip to memory / this (us, the call): 189 tokens on 4704,
-  // 32 / 4 heads, 10 pieces 37.8 / 30.7 (eight lanes there 36.0); 16 x 4 on 8000, 26 pieces 33.7 / 32.0; 34 x 5 on 28920, 13
-  // 127.8 / 123.5; 110 x 2 on 3656, 8 30.1 / 29.3 (eight at once 29.4); 24 x 24 on 8191, 3 114 / 113.
+  // 32 / 4 heads, 10 pieces 37.6 / 30.6 (eight lanes there 36.0); 16 x 4 on 8000, 26 pieces 33.7 / 31.8; 34 x 5 on 28920, 13
+  // 129.1 / 125.1; 110 x 2 on 3656, 8 29.5 / 28.6 (eight at once 28.7); 24 x 24 on 8191, 3 115.3 / 115.0.
   if (p.n_split > 8 && items * 8 <= kMergeLanes) {
     if (p.n_split > 32) return merge(prefill_merge_kernel<T, 64, 4>, 64);
     return p.n_split > 16 ? merge(prefill_merge_kernel<T, 8, 4>, 8) : merge(prefill_merge_kernel<T, 8, 2>, 8);

@@ -30,8 +30,8 @@ static int chunk(char** v) {   // batch capacity, batch, query heads, key-value 
   for (int i = 1; i <= 8; ++i) a[i] = (uint32_t)strtoul(v[i + 1], nullptr, 10);
   const ChunkCall c = {a[6], a[7], a[2], a[1], a[3], a[4], 256, prefill_workspace_rows(a[5], a[1], a[3], 256), a[8] != 0};
   const ChunkPlan p = plan_chunk(c);
-  printf("%d %u %u %u %d\n", (int)p.kernel, p.kernel == kChunkStream ? p.waves : p.kernel == kChunkShort ? p.row_blocks : 0, p.n_split, p.n_wg,
-         (int)p.form);
+  printf("%d %u %u %u %d %u\n", (int)p.kernel, p.kernel == kChunkStream ? p.waves : p.kernel == kChunkShort ? p.row_blocks : 0, p.n_split, p.n_wg,
+         (int)p.form, p.split_tiles * kChunkTile);
   return 0;
 }
 // head size, bytes an element, batch capacity, batch, query heads, key-value heads, most positions a call,
@@ -53,7 +53,7 @@ int main(int, char** v) {
   c.vec = a[10] != 0;
   c.room = a[11] ? a[11] : w.rows / (c.planes * c.rows());
   const gen::GeneralPlan p = gen::general_plan(c);
-  printf("%d %u %u %u %d %zu %d\n", (int)p.kernel, p.n_split, p.tile_rows, p.key_groups, p.nb, w.rows, (int)p.max_first);
+  printf("%d %u %u %u %d %zu %d %u\n", (int)p.kernel, p.n_split, p.tile_rows, p.key_groups, p.nb, w.rows, (int)p.max_first, p.split_len);
 }
 """
 
@@ -74,7 +74,7 @@ def _program():
 
 def general_plan(head_size, element_bytes, batch_capacity, batch, q_heads, kv_heads, position_index, interval, vec=None, room=0):
     """(kernel "rows" / "step" / "chunk", key splits, rows per workgroup, key groups, padded head blocks, the
-    workspace's partial rows, whether a chunk kernel looks for the row maximum every step)"""
+    workspace's partial rows, whether a chunk kernel looks for the row maximum every step, keys a split)"""
     if vec is None:
         vec = head_size * element_bytes % 16 == 0
     args = (head_size, element_bytes, batch_capacity, batch, q_heads, kv_heads, interval, position_index, interval, int(vec), room)
@@ -105,6 +105,11 @@ def chunk_form(*call, **more):
     """The form of the tile kernel that an unsplit call of it runs: "registers", "direct" or "wide"; for the last one
     the storage type counts (bf16=True)."""
     return ("registers", "direct", "wide")[int(_chunk(*call, **more)[4])]
+
+
+def chunk_piece_keys(*call, **more):
+    """Keys a piece of a split call."""
+    return int(_chunk(*call, **more)[5])
 
 
 def chunk_is_direct(*call, **more):
