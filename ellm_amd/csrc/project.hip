@@ -149,8 +149,8 @@ hipError_t launch_project(const ProjectArgs& a, hipStream_t stream) {
   if (path == kPathFewRows)
     return launch_project_small(p, a.ws, a.counters, g_n_cu, a.dtype, a.residual ? kModeAdd : kModeQkv, stream);
   if (path == kPathTiles128 && a.part) {
-    const ProjectSplit split = project_split(a.rows, heads, a.K, g_n_cu, a.part_floats);
-    if (split.k_split > 1) {
+    const ProjectSplit split = project_split(a.rows, heads, a.K, g_n_cu);
+    if (split.k_split > 1 && split_floats(split, a.rows, heads) <= a.part_floats) {
       p.k_split = split.k_split;
       p.half_heads = split.half_heads;
       p.part = a.part;

@@ -3,7 +3,8 @@
 // blocks of 16 columns) x 32 MB tokens.  K runs in chunks of 64 (one 128-byte line of every operand row)
 // that go from memory straight into LDS, through two to four stages.
 // Every shape adds up K in the same order, so an output's bits do not depend on the shape that made it (pieces of K are
-// added to each other afterwards, in order: those bits depend on the plan, that is on the sizes, alone).
+// added to each other afterwards, in order: those bits depend on the plan, that is on the sizes, and on whether the handle
+// has the room a plan's sums take: one made when memory was out has none and keeps K whole).
 //
 // What bounds it: on ordinary operands the board's power, and with it the time the matrix pipe idles.
 // A 256 x 256 x 64 loop on N(0,1) operands, probe kernels, TFLOP/s: 32x32x16 instructions 1494-1543 without

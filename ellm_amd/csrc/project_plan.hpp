@@ -32,8 +32,8 @@ inline double project_tiles_us(const ProjectSplit& s, uint32_t rows, uint32_t he
   return 9.0 + (walk > weights ? walk : weights) + 2.0 * split_floats(s, rows, heads) * 4 / 6e6;
 }
 
-// Three to eight workgroups a tile, all of them at once, one per unit, pieces of at least four chunks, sums within
-// `room` floats; where that is estimated 5 % below one round of whole tiles.  Two a tile gained nothing that lasts
+// Three to eight workgroups a tile, all of them at once, one per unit, pieces of at least four chunks; where that is
+// estimated 5 % below one round of whole tiles.  Follows from the sizes alone.  Two a tile gained nothing that lasts
 // (2048 <- 4096, 700 rows 32.9 / 33.0), nor did three of 256 tokens below 96 chunks (a layer of 800 rows, 2048 wide, 73.7 /
 // 75.0; 4096 <- 4096, 400 rows 31.7 / 30.9), nor any of 256 tokens on all units at once (those 800 rows, four, 73.1 / 78.0).  Whole / shared, weights from memory, f16 (us; tokens a tile / pieces):
 //   2048 <- 4096   79 rows 32.4 / 14.6 (128 / 8)   128 37.2 / 16.0 (128 / 8)   234 35.2 / 18.6 (128 / 8)   400 30.0 / 22.6 (128 / 4)
@@ -46,9 +46,9 @@ inline double project_tiles_us(const ProjectSplit& s, uint32_t rows, uint32_t he
 // a fifth more from LDS, but take turns (layer of a chunk, four / eight waves: 2048 wide, 65 rows 32.5 / 28.1, 128 37.3 /
 // 33.0, 300 46.5 / 42.4; 4096 wide, 128 55.4 / 51.8; 8192 wide, 65 82.2 / 75.2, 128 93.7 / 90.7), except where all units are
 // at work: 500 rows 2048 wide, 256 workgroups, 52.5 / 55.5; 256 rows 4096 wide 62.7 / 64.2.
-inline ProjectSplit project_split(uint32_t rows, uint32_t heads, uint32_t K, uint32_t n_cu, size_t room) {
+inline ProjectSplit project_split(uint32_t rows, uint32_t heads, uint32_t K, uint32_t n_cu) {
   const ProjectSplit whole = {1, 1, false};
-  if (((size_t)rows + 127) / 128 * heads > n_cu) return whole;
+  if (rows <= 64 || ((size_t)rows + 127) / 128 * heads > n_cu) return whole;
   ProjectSplit best = whole;
   double best_us = 0.95 * project_tiles_us(whole, rows, heads, K);
   for (uint32_t blocks = 1; blocks <= 2; ++blocks) {
@@ -56,7 +56,7 @@ inline ProjectSplit project_split(uint32_t rows, uint32_t heads, uint32_t K, uin
     for (uint32_t n = blocks == 2 && K / 64 < 96 ? 4 : 3; n <= 8 && n * tiles <= n_cu && 4 * n <= K / 64; ++n) {
       const bool spare = 16 * n * tiles <= 15 * n_cu;
       const ProjectSplit s = {blocks, n, blocks == 1 && spare};
-      if (split_floats(s, rows, heads) > room || (blocks == 2 && !spare)) break;
+      if (blocks == 2 && !spare) break;
       const double us = project_tiles_us(s, rows, heads, K);
       if (us < best_us) {
         best_us = us;
@@ -67,15 +67,26 @@ inline ProjectSplit project_split(uint32_t rows, uint32_t heads, uint32_t K, uin
   return best;
 }
 
-// Room that the calls of up to max_rows rows of a matrix can use (at most 256 tokens x 128 columns a unit): what the
-// plans at every 32nd row take.
+// Room for the sums of every call of up to max_rows rows of a matrix (at most 256 tokens x 128 columns a unit).  The
+// rows of a 128-token tile have the same tiles, and with them a plan's estimate is a straight line, the steeper the more
+// pieces: from row to row pieces only get fewer, and the rows that have as many end where a bisection finds it.
 inline size_t project_split_room(uint32_t heads, uint32_t K, uint32_t n_cu, size_t max_rows) {
   size_t most = 0;
-  for (uint32_t last = 96; last < max_rows + 32 && ((size_t)last + 127) / 128 * heads <= n_cu; last += 32) {
-    const uint32_t rows = last < max_rows ? last : (uint32_t)max_rows;
-    if (rows < 65) continue;
-    const size_t f = split_floats(project_split(rows, heads, K, n_cu, (size_t)-1), rows, heads);
+  for (size_t first = 65; first <= max_rows && (first + 127) / 128 * heads <= n_cu;) {
+    const size_t tile_end = (first + 127) / 128 * 128;
+    const uint32_t pieces = project_split((uint32_t)first, heads, K, n_cu).k_split;
+    size_t last = tile_end < max_rows ? tile_end : max_rows;
+    if (project_split((uint32_t)last, heads, K, n_cu).k_split != pieces) {
+      size_t same = first;   // and `last` has fewer
+      while (last - same > 1) {
+        const size_t mid = (same + last) / 2;
+        (project_split((uint32_t)mid, heads, K, n_cu).k_split == pieces ? same : last) = mid;
+      }
+      last = same;
+    }
+    const size_t f = split_floats({1, pieces, false}, (uint32_t)last, heads);
     if (f > most) most = f;
+    first = last + 1;
   }
   return most;
 }

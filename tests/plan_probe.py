@@ -17,12 +17,22 @@ SOURCE = r"""
 #include "general_plan.hpp"
 #include "project_plan.hpp"
 using namespace ellm;
-static int project(char** v) {   // rows, heads, K, room (0: what a handle for that many rows takes)
-  uint32_t a[5];
-  for (int i = 1; i <= 4; ++i) a[i] = (uint32_t)strtoul(v[i + 1], nullptr, 10);
-  const size_t room = a[4] ? a[4] : proj::project_split_room(a[2], a[3], 256, a[1]);
-  const proj::ProjectSplit s = proj::project_split(a[1], a[2], a[3], 256, room);
-  printf("%u %u %zu %zu %d\n", s.token_blocks, s.k_split, proj::split_floats(s, a[1], a[2]), room, (int)s.half_heads);
+static int project(char** v) {   // rows, heads, K
+  uint32_t a[4];
+  for (int i = 1; i <= 3; ++i) a[i] = (uint32_t)strtoul(v[i + 1], nullptr, 10);
+  const proj::ProjectSplit s = proj::project_split(a[1], a[2], a[3], 256);
+  printf("%u %u %zu %d\n", s.token_blocks, s.k_split, proj::split_floats(s, a[1], a[2]), (int)s.half_heads);
+  return 0;
+}
+static int project_room(char** v) {   // heads, K, units, least and most rows of a handle: each one's room and what its calls' sums take at most
+  uint32_t a[6];
+  for (int i = 1; i <= 5; ++i) a[i] = (uint32_t)strtoul(v[i + 1], nullptr, 10);
+  size_t need = 0;
+  for (uint32_t rows = 1; rows <= a[5]; ++rows) {
+    const size_t f = proj::split_floats(proj::project_split(rows, a[1], a[2], a[3]), rows, a[1]);
+    need = f > need ? f : need;
+    if (rows >= a[4]) printf("%zu %zu\n", proj::project_split_room(a[1], a[2], a[3], rows), need);
+  }
   return 0;
 }
 static int chunk(char** v) {   // batch capacity, batch, query heads, key-value heads, most positions a call, position_index, interval, bfloat16
@@ -39,6 +49,7 @@ static int chunk(char** v) {   // batch capacity, batch, query heads, key-value 
 int main(int, char** v) {
   if (v[1][0] == 'c') return chunk(v);
   if (v[1][0] == 'p') return project(v);
+  if (v[1][0] == 'r') return project_room(v);
   uint32_t a[12];
   for (int i = 1; i <= 11; ++i) a[i] = (uint32_t)strtoul(v[i], nullptr, 10);
   const gen::GeneralWorkspace w = gen::general_workspace(a[7], a[3], a[5], a[6], a[1], 256);
@@ -82,11 +93,17 @@ def general_plan(head_size, element_bytes, batch_capacity, batch, q_heads, kv_he
     return (("rows", "step", "chunk")[int(out[0])], *map(int, out[1:]))
 
 
-def project_split(rows, heads, k, room=0):
-    """Projection of 65 rows and more: (128-token blocks a tile, workgroups that share its K, their sums' floats, a handle's room,
+def project_split(rows, heads, k):
+    """Projection of 65 rows and more: (128-token blocks a tile, workgroups that share its K, their sums' floats,
     whether eight waves of half a head walk a tile)"""
-    out = subprocess.run([_program(), "p", *map(str, (rows, heads, k, room))], check=True, capture_output=True, text=True)
+    out = subprocess.run([_program(), "p", *map(str, (rows, heads, k))], check=True, capture_output=True, text=True)
     return tuple(map(int, out.stdout.split()))
+
+
+def project_room(heads, k, least, most, units=256):
+    """[(a handle's room, the most that the sums of any of its calls take)] for handles of `least` .. `most` rows"""
+    out = subprocess.run([_program(), "r", *map(str, (heads, k, units, least, most))], check=True, capture_output=True, text=True)
+    return [tuple(map(int, line.split())) for line in out.stdout.splitlines()]
 
 
 def _chunk(batch_capacity, batch, q_heads, kv_heads, position_index, interval, most=None, bf16=False):

@@ -23,7 +23,7 @@ QKV = [
 
 def _plan(rows, heads, k):
     plan = plan_probe.project_split(rows, heads, k)
-    return plan[0], plan[1], plan[4]
+    return plan[0], plan[1], plan[3]
 
 
 @pytest.mark.parametrize("interval,pitch,batch,k,hq,hkv,p0,dtype,plan", QKV)
