@@ -22,8 +22,6 @@
 // 59 | 53 -> 52 | 44.
 // Calls with at most 64 rows go to the streaming kernel of project_small.hip, calls that would
 // leave these tiles fewer than the compute units to the 128-token tiles of project_mid.hip.
-#include <atomic>
-
 #include "project_mid_tile.hpp"
 #include "project_plan.hpp"
 
@@ -184,27 +182,20 @@ hipError_t launch_project(const ProjectArgs& a, hipStream_t stream) {
 }
 
 // The kernels' LDS needs exceed the default limit; raised here, on the current device, when
-// a handle is created, not at launch (a launch may be recorded into a graph).  Once a device: creating a handle for few
-// rows takes 9 us instead of 11.
+// a handle is created, not at launch (a launch may be recorded into a graph).  With every handle (2 us): a mark that
+// it has been done once would outlive the device's reset.
 hipError_t project_prepare() {
-  static std::atomic<uint64_t> prepared{0};
-  int dev = 0, n_cu = 0;
-  hipError_t e = hipGetDevice(&dev);
-  if (e != hipSuccess) return e;
-  const uint64_t bit = dev >= 0 && dev < 64 ? (uint64_t)1 << dev : 0;
-  if (!(prepared.load(std::memory_order_acquire) & bit)) {
-    const void* kernels[] = {(const void*)project_kernel<F16, kModeQkv>, (const void*)project_kernel<BF16, kModeQkv>,
-                             (const void*)project_kernel<F16, kModeAdd>, (const void*)project_kernel<BF16, kModeAdd>};
-    for (const void* k : kernels) {
-      e = hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, kProjLdsBytes);
-      if (e != hipSuccess) return e;
-    }
-    e = mid_prepare();
+  const void* kernels[] = {(const void*)project_kernel<F16, kModeQkv>, (const void*)project_kernel<BF16, kModeQkv>,
+                           (const void*)project_kernel<F16, kModeAdd>, (const void*)project_kernel<BF16, kModeAdd>};
+  for (const void* k : kernels) {
+    const hipError_t e = hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, kProjLdsBytes);
     if (e != hipSuccess) return e;
-    prepared.fetch_or(bit, std::memory_order_release);
   }
-  if (hipDeviceGetAttribute(&n_cu, hipDeviceAttributeMultiprocessorCount, dev) == hipSuccess && n_cu > 0) g_n_cu = (uint32_t)n_cu;
-  return hipSuccess;
+  int dev = 0, n_cu = 0;
+  if (hipGetDevice(&dev) == hipSuccess &&
+      hipDeviceGetAttribute(&n_cu, hipDeviceAttributeMultiprocessorCount, dev) == hipSuccess && n_cu > 0)
+    g_n_cu = (uint32_t)n_cu;
+  return mid_prepare();
 }
 
 size_t project_workspace_floats(uint32_t heads) { return (size_t)heads * kHeadDim * kSmallRowsMax; }
