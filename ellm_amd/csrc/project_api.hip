@@ -11,6 +11,7 @@
 #include "../../include/ellm_attn.h"
 #include "handles.hpp"
 #include "kernels.hpp"
+#include "project_plan.hpp"
 
 namespace {
 bool aligned16(const void* p) { return ((uintptr_t)p & 15u) == 0; }
@@ -42,14 +43,17 @@ int alloc_small_workspace(uint32_t heads, size_t k, size_t max_rows, int* device
   const size_t floats = ellm::project_workspace_floats(heads);
   if (floats * sizeof(float) > (size_t)64 << 20) return ELLM_OK;
   size_t more = ellm::project_part_floats(heads, (uint32_t)k, max_rows);
-  hipError_t e = hipMalloc((void**)ws, (floats + more) * sizeof(float));
-  if (e == hipErrorOutOfMemory && more) {   // K stays whole then
-    (void)hipGetLastError();
-    more = 0;
-    e = hipMalloc((void**)ws, floats * sizeof(float));
-  }
-  if (e == hipSuccess) e = hipMalloc((void**)counters, heads * sizeof(uint32_t));
+  // (the counters first: the room is not to take the memory that a handle cannot do without)
+  hipError_t e = hipMalloc((void**)counters, heads * sizeof(uint32_t));
   if (e == hipSuccess) e = hipMemset(*counters, 0, heads * sizeof(uint32_t));
+  if (e == hipSuccess) e = (hipError_t)ellm::proj::project_block(floats, &more, [&](size_t bytes) {
+    const hipError_t got = hipMalloc((void**)ws, bytes);
+    if (got != hipSuccess) {
+      (void)hipGetLastError();
+      *ws = nullptr;
+    }
+    return (int)got;
+  });
   if (e != hipSuccess) {
     (void)hipFree(*ws);
     (void)hipFree(*counters);

@@ -91,5 +91,17 @@ inline size_t project_split_room(uint32_t heads, uint32_t K, uint32_t n_cu, size
   return most;
 }
 
+// A handle's one block of device memory: the few-rows kernel's workspace and, behind it, room for shared sums.
+// `alloc(bytes)` returns 0 and takes the block; where it does not, whatever the reason, the workspace alone is asked for, and K
+// stays whole: *part_floats becomes 0.  Returns alloc's last answer.
+template <typename Alloc>
+inline int project_block(size_t ws_floats, size_t* part_floats, Alloc alloc) {
+  if (*part_floats) {
+    if (alloc((ws_floats + *part_floats) * sizeof(float)) == 0) return 0;
+    *part_floats = 0;
+  }
+  return alloc(ws_floats * sizeof(float));
+}
+
 }  // namespace proj
 }  // namespace ellm

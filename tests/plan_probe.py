@@ -35,6 +35,16 @@ static int project_room(char** v) {   // heads, K, units, least and most rows of
   }
   return 0;
 }
+static int project_block(char** v) {   // the workspace's floats, the room's, bytes that an allocation may have, status of a larger one
+  const size_t most = strtoull(v[4], nullptr, 10);
+  size_t part = strtoull(v[3], nullptr, 10);
+  const int status = proj::project_block(strtoull(v[2], nullptr, 10), &part, [&](size_t bytes) {
+    printf("%zu ", bytes);
+    return bytes <= most ? 0 : atoi(v[5]);
+  });
+  printf("%zu %d\n", part, status);
+  return 0;
+}
 static int chunk(char** v) {   // batch capacity, batch, query heads, key-value heads, most positions a call, position_index, interval, bfloat16
   uint32_t a[9];
   for (int i = 1; i <= 8; ++i) a[i] = (uint32_t)strtoul(v[i + 1], nullptr, 10);
@@ -50,6 +60,7 @@ int main(int, char** v) {
   if (v[1][0] == 'c') return chunk(v);
   if (v[1][0] == 'p') return project(v);
   if (v[1][0] == 'r') return project_room(v);
+  if (v[1][0] == 'b') return project_block(v);
   uint32_t a[12];
   for (int i = 1; i <= 11; ++i) a[i] = (uint32_t)strtoul(v[i], nullptr, 10);
   const gen::GeneralWorkspace w = gen::general_workspace(a[7], a[3], a[5], a[6], a[1], 256);
@@ -104,6 +115,14 @@ def project_room(heads, k, least, most, units=256):
     """[(a handle's room, the most that the sums of any of its calls take)] for handles of `least` .. `most` rows"""
     out = subprocess.run([_program(), "r", *map(str, (heads, k, units, least, most))], check=True, capture_output=True, text=True)
     return [tuple(map(int, line.split())) for line in out.stdout.splitlines()]
+
+
+def project_block(ws, part, most, status):
+    """A handle's block where allocations beyond `most` bytes end with `status`: (bytes asked for in turn, the room it got
+    in floats, the last status)"""
+    out = subprocess.run([_program(), "b", *map(str, (ws, part, most, status))], check=True, capture_output=True, text=True)
+    *asked, room, last = map(int, out.stdout.split())
+    return asked, room, last
 
 
 def _chunk(batch_capacity, batch, q_heads, kv_heads, position_index, interval, most=None, bf16=False):

@@ -1,5 +1,5 @@
 """How projections share K between workgroups (ellm_amd/csrc/project_plan.hpp), on the CPU: every plan is one round of
-workgroups, its pieces hold at least four chunks, and a handle has room for the sums of every call it may run, whatever
+workgroups, its pieces hold at least four chunks, a handle without memory for shared sums is made without, and one with has room for the sums of every call it may run, whatever
 its most rows, and for no more."""
 import pytest
 
@@ -37,3 +37,11 @@ def test_few_rows_keep_k_whole():
     """Below 65 rows (hidden sizes the few-rows kernel does not take), whatever the handle's room."""
     for heads, k in ((1, 960), (16, 960), (40, 896)):
         assert all(plan_probe.project_split(rows, heads, k)[1] == 1 for rows in (1, 33, 64))
+
+
+@pytest.mark.parametrize("status", [2, 1, 999])   # out of memory, and any other reason
+def test_a_handle_without_memory_for_shared_sums(status):
+    assert plan_probe.project_block(1000, 5000, 24000, status) == ([24000], 5000, 0)
+    assert plan_probe.project_block(1000, 5000, 23999, status) == ([24000, 4000], 0, 0)      # K stays whole
+    assert plan_probe.project_block(1000, 5000, 3999, status) == ([24000, 4000], 0, status)  # no handle
+    assert plan_probe.project_block(1000, 0, 3999, status) == ([4000], 0, status)
