@@ -135,6 +135,58 @@ def test_cache_writes_land_on_the_same_rows(dtype):
 
 
 @pytest.mark.parametrize("dtype", [orc.F16, orc.BF16])
+@pytest.mark.parametrize("seqs", [4, 70])
+def test_shared_k_projection_writes_the_same_rows(dtype, seqs):
+    """The fused projection where several workgroups share K and a second launch finishes the rows: a chunk of 50 tokens for
+    four sequences, one token for seventy at positions of their own (up to their last row)."""
+    import torch
+
+    import ellm_amd
+    import plan_probe
+
+    hidden, caps = 2048, [CAPS[i % 4] + i for i in range(seqs)]
+    tokens = 50 if seqs == 4 else 1
+    assert plan_probe.project_split(tokens * seqs, HQ + 2 * HKV, hidden)[1] > 2
+    rope = to_dev(_rope_table(max(caps), dtype), dtype)
+    w = [to_dev(rand_storage((h * D, hidden), 20 + i, dtype, scale=hidden ** -0.5), dtype)
+         for i, h in enumerate((HQ, HKV, HKV))]
+    hid = to_dev(rand_storage((tokens, seqs, hidden), 30, dtype), dtype)
+    starts = np.array([c - 1 - i % 3 for i, c in enumerate(caps)], dtype=np.int32)
+    dstarts = torch.from_numpy(starts).cuda()
+    td, outs, planes = torch_dtype(dtype), [], []
+    for ragged in (False, True):
+        q = torch.zeros((tokens, seqs, HQ, D), dtype=td, device="cuda")
+        if ragged:
+            c = ellm_amd.KVCache.ragged(1, caps, HKV, _code(dtype))
+            view = c.layer_ragged(0)
+            kt, vt = c.layer_flat_tensors(0, td)
+            strides, cap, table = view.strides, 0, view
+        else:
+            c = ellm_amd.KVCache(1, seqs, HKV, max(caps), _code(dtype))
+            kt, vt = c.layer_tensors(0, td)
+            strides, cap, table = c.layer(0)[2], max(caps), None
+        kt.zero_()
+        vt.zero_()
+        op = ellm_amd.MatMul3(hid, w[0], q, w[1], kt, w[2], vt, rope, D, seqs, HQ, HKV, strides, cap, seq_table=table)
+        if tokens > 1:
+            op.run(10, tokens, seqs)
+        else:
+            op.run_ragged(dstarts, int(starts.max()), seqs)
+        torch.cuda.synchronize()
+        outs.append(_bits(q))
+        assert outs[-1].any(axis=-1).all()
+        at = np.cumsum([0] + caps)
+        planes.append([_bits(t[:, at[s]:at[s + 1]] if ragged else t[s, :, :caps[s]]) for s in range(seqs) for t in (kt, vt)])
+        op.close()
+        c.close()
+    assert np.array_equal(outs[0], outs[1])
+    assert all(np.array_equal(u, r) for u, r in zip(*planes))
+    for s in range(seqs):
+        rows = np.flatnonzero(planes[1][2 * s].any(axis=(0, 2)))
+        assert list(rows) == (list(range(10, 60)) if tokens > 1 else [starts[s]])
+
+
+@pytest.mark.parametrize("dtype", [orc.F16, orc.BF16])
 def test_attention_reads_the_same_rows(dtype):
     import torch
 
