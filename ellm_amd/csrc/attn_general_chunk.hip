@@ -22,7 +22,7 @@
 // Binary16 heads of 256 (one group: no registers for two): 1019 tokens, 32 / 4 heads 80 us.
 // Operands of both products read ahead of their use, values looked at for infinities only in the steps whose keys some
 // row must not see, a step's place worked out without vector compares; before -> with it: 2048 tokens, 32 / 8 heads of 64,
-// bf16 40.3 -> 36.5 us; 512 x 4 on 7680 220 -> 208; 2048, 32 / 32 heads of 96, f16 64.2 -> 55.7; 512 x 4 on 7680, 32 / 8
+// bf16 40.0 -> 37.0 us; 512 x 4 on 7680 220 -> 208; 2048, 32 / 32 heads of 96, f16 64.2 -> 55.7; 512 x 4 on 7680, 32 / 8
 // heads of 256, bf16 986 -> 895 (a step of 32 keys x 32 rows of 64: 126 vector instructions, 150 before).
 #include "attn_general.hpp"
 

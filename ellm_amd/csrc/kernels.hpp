@@ -115,8 +115,8 @@ hipError_t launch_positions_advance(uint32_t* positions, uint32_t n, uint32_t by
 // p[i] = value for i < n: a kernel, not a memset node, so that it can be recorded into a graph.
 hipError_t launch_fill_u32(uint32_t* p, size_t n, uint32_t value, hipStream_t stream);
 
-// Merge launches of split chunk calls: lanes up to which several share a row's partials (more partials than a lane takes
-// at once); beyond, one lane takes them all.
+// Merge launches of split chunk calls with more than eight partials a row: up to this many lanes eight share a row's four
+// columns (64 do from 33 partials on, in launches of up to eight times as many lanes); beyond, one lane takes them all.
 constexpr size_t kMergeLanes = (size_t)1 << 19;
 
 // Projection C = X . W^T on MFMA with the per-head epilogue (see project.hip).
