@@ -2,15 +2,23 @@
 launch.  Rows that end inside a token tile, pieces of unequal length, odd head counts, sequences beyond batch_size,
 per-sequence positions, a residual that is the output; then a call of fewer rows and one of whole tiles on the
 same handle.  Same oracle and bound as tests/test_gpu_projection.py."""
+import ctypes
+
 import numpy as np
 import pytest
 
 import oracle_lib as orc
 import plan_probe
+from ellm_amd import _lib
 from gpu_util import D, compare_ulps, rand_storage, to_dev, to_host
 from test_gpu_projection import TILES_128, _path, _rope_table, _run_matmul3, _weights
 
 pytestmark = pytest.mark.gpu
+
+
+class _MatMulAddHandle(ctypes.Structure):   # struct ellm_matmul_add of project_api.hip
+    _fields_ = [("d", _lib.MatMulAddDesc), ("device", ctypes.c_int), ("ws", ctypes.c_void_p), ("counters", ctypes.c_void_p),
+                ("part", ctypes.c_void_p), ("part_floats", ctypes.c_size_t)]
 
 # interval, pitch, batch, K, q heads, kv heads, position_index, dtype, (128-token blocks a tile, pieces, half heads)
 QKV = [
@@ -67,3 +75,38 @@ def test_matmul_add_pieces(rows, heads, k, dtype, plan):
         assert res["ok"], (n, res)
         assert np.array_equal(got[n:], orc.from_storage(r[n:], dtype))   # rows past the call are left alone
     op.close()
+
+
+def test_a_handle_without_room_keeps_k_whole():
+    """What a handle does that was made when memory was out: its room is taken away behind its back, then each call that
+    shared K runs with K whole and gives what the oracle gives.  That the room was there, and how much, first."""
+    import torch
+
+    import ellm_amd
+
+    heads, k, dtype = 16, 4096, orc.F16
+    rows = 300
+    a = rand_storage((rows, 1, k), 61, dtype)
+    w = rand_storage((heads * D, k), 62, dtype, scale=k ** -0.5)
+    r = rand_storage((rows, 1, heads * D), 63, dtype)
+    da, dw, dr = to_dev(a, dtype), to_dev(w, dtype), to_dev(r, dtype)
+    out = torch.empty_like(dr)
+    want = orc.from_storage(orc.matmul_add(a, w, r, dtype, batch_size=1), dtype)
+    op = ellm_amd.MatMulAdd(da, dw, dr, out)
+    handle = _MatMulAddHandle.from_address(op._handle.value)
+    room, = plan_probe.project_room(heads, k, rows, rows)
+    assert handle.part_floats == room[0] > 0 and handle.part == handle.ws + 4 * heads * D * 64
+    seen = []
+    for part, floats in ((handle.part, room[0]), (None, 0)):
+        handle.part, handle.part_floats = part, floats
+        for n in (rows, 79):
+            assert _plan(n, heads, k)[1] > 2
+            out.fill_(float("nan"))
+            op.run(0, n, 1)
+            torch.cuda.synchronize()
+            seen.append(to_host(out, dtype))
+            res = compare_ulps(seen[-1][:n], want[:n], dtype)
+            assert res["ok"], (n, part, res)
+    op.close()
+    # whole sums are those of a handle that could never share (no call of it is one round of that many workgroups): bits differ
+    assert not np.array_equal(seen[0], seen[2])
