@@ -33,7 +33,7 @@ __global__ __launch_bounds__(256) void general_merge_kernel(GeneralArgs p, uint3
   float l;
   f32x4 o;
   const float m = fold_splits<G, TURN>(p.part_ml + prow * p.n_split * 2, p.part_o + prow * p.n_split * pitch + 4 * dq, pitch, sub,
-                                 live, l, o);
+                                 live, p.n_split, l, o);
   if (!valid || sub != 0) return;
   const size_t row = query_row(p, seq, kvh, r);
   const float inv = 1.0f / l;

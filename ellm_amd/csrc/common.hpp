@@ -271,42 +271,44 @@ __device__ __forceinline__ u32x4 norm_rope_row16(u32x4 kraw, u32x4 rraw, float e
   return out;
 }
 
-// Folds `live` partial results of a row, (reference exponent, sum of weights) pairs at ml and four columns of weighted
-// sums at po, `pitch` floats apart: G lanes (sub: which of them) take them in turn, kTurn at a time, and combine through
-// lane exchanges.  All of a turn's loads are on their way before the first is used, and the references of the later turns
-// behind those of the first: what bounds a merge launch is its trips to memory.  The row's highest reference is known
-// before the first partial is added (added against the highest one so far and rescaled later, pieces with large sums
-// under low scores pass binary32's range before the piece that outweighs them is seen; up to eight pieces cost the same
-// either way, ten to 28 in one lane 0.3 to 0.7 us more: 100 tokens on 9000, 32 / 4 heads, 16 pieces 32.5 / 33.2).  A partial without keys left
-// (-inf, 0) and weighs nothing.  Returns the row's reference, every lane its sums.
+// Folds `live` partial results of a row (of at most `most`, the launch's own count), (reference exponent, sum of weights)
+// pairs at ml and four columns of weighted sums at po, `pitch` floats apart: G lanes (sub: which of them) take them in turn,
+// kTurn at a time, and combine through lane exchanges.  All of a turn's loads are on their way before the first is used:
+// what bounds a merge launch is its trips to memory.  The row's highest reference is known before the first partial is
+// added (added against the highest one so far and rescaled later, pieces with large sums under low scores pass binary32's
+// range before the piece that outweighs them is seen): the references behind the first turn are asked for ahead of it,
+// shared out over eight lanes, which have one row (pitch is a multiple of 32); each lane looking at all of them, two a load, 100
+// tokens on 9000, 32 / 4 heads, 16 pieces, took 33.3 us, this 33.0, as without looking.  A partial without keys left (-inf, 0) and weighs nothing.
+// Returns the row's reference, every lane its sums.
 template <int G, int kTurn>
 __device__ __forceinline__ float fold_splits(const float* ml, const float* po, uint32_t pitch, uint32_t sub, uint32_t live,
-                                             float& l_out, f32x4& o_out) {
-  typedef f32x4 Pairs __attribute__((aligned(8)));
-  constexpr int kLook = 8;   // loads of two pairs a trip, for the references behind the first turn
+                                             uint32_t most, float& l_out, f32x4& o_out) {
+  constexpr uint32_t kLook = 4;   // references a lane and trip
   f32x2 r[kTurn];
   f32x4 part[kTurn];
   auto fetch = [&](uint32_t s0) __attribute__((always_inline)) {
 #pragma unroll
-    for (int i = 0; i < kTurn; ++i) {
-      const uint32_t s = min(s0 + i * G, live - 1);
-      r[i] = *(const f32x2*)(ml + 2 * s);
-      part[i] = *(const f32x4*)(po + (size_t)s * pitch);
-    }
+    for (int i = 0; i < kTurn; ++i) r[i] = *(const f32x2*)(ml + 2 * min(s0 + i * G, live - 1));
+#pragma unroll
+    for (int i = 0; i < kTurn; ++i) part[i] = *(const f32x4*)(po + (size_t)min(s0 + i * G, live - 1) * pitch);
   };
-  fetch(sub);
   float m = -INFINITY;
-  for (uint32_t s0 = kTurn * G + 2 * sub; s0 < live; s0 += 2 * kLook * G) {
-    f32x4 x[kLook];
+  if (most > kTurn * G) {
+    for (uint32_t s0 = kTurn * G + threadIdx.x % 8; s0 < live; s0 += 8 * kLook) {
+      float x[kLook];
 #pragma unroll
-    for (int i = 0; i < kLook; ++i) x[i] = *(const Pairs*)(ml + 2 * min(s0 + 2 * i * G, live - 2));
+      for (uint32_t i = 0; i < kLook; ++i) x[i] = ml[2 * min(s0 + 8 * i, live - 1)];
 #pragma unroll
-    for (int i = 0; i < kLook; ++i) m = fmaxf(m, fmaxf(x[i][0], x[i][2]));
+      for (uint32_t i = 0; i < kLook; ++i) m = fmaxf(m, x[i]);
+    }
   }
+  fetch(sub);
 #pragma unroll
   for (int i = 0; i < kTurn; ++i) m = fmaxf(m, r[i][0]);
+  if (G > 1 || most > kTurn * G) {
 #pragma unroll
-  for (int x = 1; x < G; x <<= 1) m = fmaxf(m, __shfl_xor(m, x));
+    for (int x = 1; x < (G > 8 ? G : 8); x <<= 1) m = fmaxf(m, __shfl_xor(m, x));
+  }
   float l = 0.0f;
   f32x4 o = {0.0f, 0.0f, 0.0f, 0.0f};
   for (uint32_t s0 = sub; s0 < live;) {

@@ -1358,7 +1358,7 @@ __global__ __launch_bounds__(256) void prefill_merge_kernel(PrefillKernelArgs p,
   float l;
   f32x4 o;
   const float m = fold_splits<G, TURN>(p.part_ml + row * p.n_split * 2, p.part_o + row * p.n_split * kHeadDim + 4 * dq, kHeadDim,
-                                 sub, live, l, o);
+                                 sub, live, p.n_split, l, o);
   if (!valid || sub != 0) return;
   const float inv = 1.0f / l;
   u32x2 w;
