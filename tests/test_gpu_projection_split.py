@@ -108,5 +108,5 @@ def test_a_handle_without_room_keeps_k_whole():
             res = compare_ulps(seen[-1][:n], want[:n], dtype)
             assert res["ok"], (n, part, res)
     op.close()
-    # whole sums are those of a handle that could never share (no call of it is one round of that many workgroups): bits differ
+    # (another order of the sums: the second pass did not share K)
     assert not np.array_equal(seen[0], seen[2])
